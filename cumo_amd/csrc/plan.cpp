@@ -244,8 +244,8 @@ void plan_reduce(const cumo_na_reduction_arg_t* arg, const cumo_na_iarray_t* out
         for (; vec > 1; vec >>= 1) {
             // the input is only read: a 128-bit global load needs no more than the element's alignment
             const int align = in_elmsz >= 4 ? in_elmsz : vec * in_elmsz;
-            // (outputs along one dimension may end in part of a vector where the caller's kernel sees to it)
-            const bool whole = (plan->out_shape[L] % vec) == 0 || (allow_tail && no <= 2 && plan->out_shape[L] >= (uint64_t)vec * 16);
+            // (outputs along one dimension, 16 of them at least, may end in part of a vector where the caller's kernel sees to it)
+            const bool whole = (plan->out_shape[L] % vec) == 0 || (allow_tail && no <= 2);
             bool ok = plan->in_out_step[L] == in_elmsz && whole && ((uintptr_t)arg->in.ptr % align) == 0;
             for (int d = 0; d < L && ok; ++d) ok = (plan->in_out_step[d] % align) == 0;
             for (int d = 0; d < nr && ok; ++d) ok = (plan->in_red_step[d] % align) == 0;

@@ -260,6 +260,21 @@ struct MomentsImpl {
             acc[j].n = n_new;
         }
     }
+    // The same for two lanes' accumulators of VEC neighbouring outputs: one weight for all of them.
+    template <int VEC>
+    __device__ __forceinline__ void combine_columns(const Acc (&next)[VEC], Acc (&acc)[VEC]) const {
+        if (next[0].n == (T)0) return;
+        const T n = acc[0].n + next[0].n;
+        const T w = next[0].n / n;
+        const T nw = acc[0].n * w;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            const T delta = next[j].mean - acc[j].mean;
+            acc[j].mean = acc[j].mean + delta * w;
+            acc[j].m2 += next[j].m2 + delta * delta * nw;
+            acc[j].n = n;
+        }
+    }
     // U blocks of N at once: the same two passes over all U * N values, one merge (and one
     // division) for all of them.
     static constexpr bool GROUPED = true;

@@ -694,6 +694,58 @@ static void red_fold_partials(const ReducePlan& plan, const RedKParams& kp, type
     cumo_cuda_runtime_check_kernel_launch();
 }
 
+// How a column reduction of `groups` vectors of outputs over an axis of n positions is split (red_scol_kernel).
+struct ColumnSplit {
+    uint32_t width;       // groups side by side in a block
+    uint32_t slots;       // lanes of the block that share a group's rows (1: blocks of kRedBlock, a lane per group)
+    uint32_t col_blocks;  // blocks side by side
+    uint32_t n_split;     // parts the axis is cut into across blocks
+    uint64_t chunk;       // rows of a part
+};
+
+// The aim is one block of kRcBlock lanes on every compute unit and as few launches as that takes. whole_lines: every
+// row starts on a cache line. Times below: sum of 128 MiB (unless a size says otherwise) on fresh operands, both sides of each line.
+//  * from 65536 groups on a lane per group fills the device by itself ([100, 330000] SFloat 23.9 us; with two slots 25.8);
+//  * one launch, the width that gives every compute unit a block (whole cache lines of it), as long as the pieces of a row
+//    that a block reads stay wide: 16 groups where rows start on lines (2048 x 16384 22.0 us, in parts 25.3), 48 where they do
+//    not, since a piece then touches a line more at either end (1677 x 20001: 24 groups 27.9 us, in parts 24.6; DFloat
+//    1292 x 12985: 32 groups 25.9, in parts 24.4);
+//  * one launch for a short axis however narrow the pieces, as the second launch costs more than they do (500 x 500: 4.1 us,
+//    in parts 6.7): up to 1024 rows, and below 2048 while the array is small (2000 x 300: 5.9 us against 8.3;
+//    2000 x 2000: 10.8 against 9.3);
+//  * else equal shares of the row, at most 256 groups each, and as many parts as make 256 blocks at most (a few blocks
+//    more than compute units and some of them read twice as long: 5000 x 3300 DFloat in 259 blocks 30.2 us, in 256 24.9).
+static inline ColumnSplit red_split_columns(uint64_t groups, uint64_t n, bool whole_lines) {
+    constexpr uint64_t kWidest = 256;
+    ColumnSplit c;
+    c.n_split = 1;
+    c.chunk = n;
+    if (groups >= 65536 || n < 2 * kRcRows) {
+        c.width = kRedBlock;
+        c.slots = 1;
+        c.col_blocks = (uint32_t)((groups + kRedBlock - 1) / kRedBlock);
+        return c;
+    }
+    uint64_t w = ((groups + kNumCU - 1) / kNumCU + 7) & ~(uint64_t)7;
+    const bool one = w >= (whole_lines ? 16u : 48u) || n <= 1024 || (n < 2048 && groups * n <= ((uint64_t)1 << 18));
+    if (!one) {
+        const uint64_t cb = (groups + kWidest - 1) / kWidest;
+        w = (groups + cb - 1) / cb;
+        if (cb > 1) w = (w + 7) & ~(uint64_t)7;
+    }
+    c.width = (uint32_t)w;
+    c.col_blocks = (uint32_t)((groups + w - 1) / w);
+    c.slots = (uint32_t)(kRcBlock / w);
+    const uint64_t most = (n + kRcRows - 1) / kRcRows;
+    if (c.slots > most) c.slots = (uint32_t)most;
+    if (one) return c;
+    const uint64_t window = (uint64_t)c.slots * kRcRows;
+    const uint64_t parts = (uint64_t)kNumCU / c.col_blocks;
+    c.chunk = ((n + parts - 1) / parts + window - 1) / window * window;
+    c.n_split = (uint32_t)((n + c.chunk - 1) / c.chunk);
+    return c;
+}
+
 // The lean kernels of reduce_stream.h for the layouts they take. Returns 1 when the
 // reduction has been launched, 0 when the general kernels must take it, -1 when the
 // caller's fixed scratch is too small (nothing launched).
@@ -742,20 +794,17 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
 
     if (plan.kind == RED_COL) {
         if (plan.in_out_step[plan.out_ndim - 1] != (int64_t)sizeof(In)) return 0;
-        p.lsplit_bits = (uint32_t)plan.local_split_bits;
-        const uint64_t per_block = (uint64_t)kRedBlock >> p.lsplit_bits;
-        const uint64_t groups = (uint64_t)(p.n_out / p.out_inner) * (((uint64_t)p.out_inner + V - 1) / V);
-        uint64_t grid = (groups + per_block - 1) / per_block;
-        if (plan.n_split > 1) {
+        const uint64_t gpo = ((uint64_t)p.out_inner + V - 1) / V;
+        const bool whole_lines = (((uintptr_t)p.in | (uint64_t)p.red_step | (uint64_t)p.in_step[0]) & 127u) == 0;
+        const ColumnSplit cs = red_split_columns((p.n_out / p.out_inner) * gpo, plan.red_total, whole_lines);
+        p.width = cs.width;
+        p.slots = cs.slots;
+        if (cs.n_split > 1) {
             // The axis is cut across blocks as well: accumulators to scratch, a second launch folds them.
-            if (grid > 65535) return 0;
-            const uint64_t bchunk = (plan.red_total + (uint64_t)plan.n_split - 1) / (uint64_t)plan.n_split;
-            const uint64_t n_split = (plan.red_total + bchunk - 1) / bchunk;  // no part is empty
-            if (n_split < 2 || n_split > 65535) return 0;
-            p.n_split = (uint32_t)n_split;
-            p.chunk = bchunk;
+            p.n_split = cs.n_split;
+            p.chunk = cs.chunk;
             const size_t parts_row = rs_parts_row(p.n_out, p.out_inner, V);
-            const uint64_t scratch_bytes = sizeof(Acc) * parts_row * n_split;
+            const uint64_t scratch_bytes = sizeof(Acc) * parts_row * cs.n_split;
             if (fixed) {
                 if (scratch_bytes > fixed->bytes) return -1;
                 p.partial = fixed->ptr;
@@ -764,32 +813,29 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
                 p.partial = cumo_cuda_runtime_malloc(scratch_bytes);
                 if (!p.partial) return 1;  // the pool has reported it
             }
-            const dim3 g2((unsigned)grid, (unsigned)n_split);
-            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, true, 4, true>), g2, b, 0, stream, p, impl);
-            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, true, 4, true>), g2, b, 0, stream, p, impl);
+            const dim3 g2(cs.col_blocks * cs.n_split), b2(kRcBlock);
+            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, true, true>), g2, b2, 0, stream, p, impl);
+            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, true, true>), g2, b2, 0, stream, p, impl);
             cumo_cuda_runtime_check_kernel_launch();
-            // the fold: as many lanes to a group of outputs as give each at most eight parts (a group's 16 bytes of every
-            // part next to its neighbours': at least four groups side by side)
+            // the fold: as many lanes to an output as give each at most eight parts
             RedSParams pf = p;
-            pf.lsplit_bits = 0;
-            while (pf.lsplit_bits < 6 && (8ull << pf.lsplit_bits) < n_split) ++pf.lsplit_bits;
-            const uint64_t fold_groups = (uint64_t)kRedBlock >> pf.lsplit_bits;
-            const dim3 gf((unsigned)((parts_row / V + fold_groups - 1) / fold_groups));
-            hipLaunchKernelGGL((red_fold_parts_kernel<Impl, V>), gf, b, 0, stream, pf, impl);
+            pf.fold_bits = 0;
+            while (pf.fold_bits < 6 && (8ull << pf.fold_bits) < cs.n_split) ++pf.fold_bits;
+            const uint32_t fold_outputs = (uint32_t)kRedBlock >> pf.fold_bits;
+            const dim3 gf((p.n_out + fold_outputs - 1) / fold_outputs);
+            hipLaunchKernelGGL((red_fold_parts_kernel<Impl>), gf, b, 0, stream, pf, impl, parts_row);
             cumo_cuda_runtime_check_kernel_launch();
             if (!fixed) cumo_cuda_runtime_free(p.partial);
             return 1;
         }
-        if (grid > red_grid_cap()) grid = red_grid_cap();
-        const dim3 g((unsigned)grid);
-        // four positions of the axis in flight per lane: more of them (or narrower blocks) read
-        // more rows at a time and measured slower
-        if (p.lsplit_bits > 0) {
-            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, true, 4>), g, b, 0, stream, p, impl);
-            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, true, 4>), g, b, 0, stream, p, impl);
+        const dim3 g(cs.col_blocks < red_grid_cap() ? cs.col_blocks : red_grid_cap());
+        if (cs.slots > 1) {
+            const dim3 b2(kRcBlock);
+            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, true>), g, b2, 0, stream, p, impl);
+            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, true>), g, b2, 0, stream, p, impl);
         } else {
-            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, false, 4>), g, b, 0, stream, p, impl);
-            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, false, 4>), g, b, 0, stream, p, impl);
+            if (nt) hipLaunchKernelGGL((red_scol_kernel<Impl, V, true, false>), g, b, 0, stream, p, impl);
+            else hipLaunchKernelGGL((red_scol_kernel<Impl, V, false, false>), g, b, 0, stream, p, impl);
         }
         cumo_cuda_runtime_check_kernel_launch();
         return 1;

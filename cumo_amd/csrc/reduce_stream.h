@@ -11,8 +11,9 @@
 //                         of the fold does not depend on which block that is, so results
 //                         are the same bits on every run, as with a second launch.
 //  red_scol_kernel        the outputs run along memory; a lane owns VEC neighbouring
-//                         outputs and walks the axis; with LOCAL, 2^k lanes of a block
-//                         share the axis and combine through LDS in axis order.
+//                         outputs and walks the axis; with SHARE, lanes of a block share
+//                         the rows and combine through LDS; with PARTIAL, the axis is also
+//                         cut across blocks and red_fold_parts_kernel folds their parts.
 //
 // What makes them lean: a 136-byte argument block instead of 620 bytes; every load of
 // an unrolled step is unconditional (a position past the end is pulled back inside the
@@ -30,7 +31,8 @@ constexpr int kRsOneLevel = 128;        // up to this many blocks per output cou
 constexpr uint32_t kRsTicketWords = 16384;  // ticket words per stream slot
 
 // An Impl whose accumulate_columns<U, VEC>(x[U][VEC], acc[VEC]) folds U positions of VEC neighbouring outputs at once,
-// all of which have seen the same number of positions before
+// all of which have seen the same number of positions before, and whose combine_columns<VEC>(next, acc) folds two
+// lanes' accumulators of such outputs
 template <class I, class = void> struct folds_columns_together { static constexpr bool value = false; };
 template <class I> struct folds_columns_together<I, decltype((void)I::COLUMNS_TOGETHER)> { static constexpr bool value = I::COLUMNS_TOGETHER; };
 
@@ -56,7 +58,9 @@ struct RedSParams {
     uint32_t group;        // split form: blocks that count in on one first-level ticket
     uint32_t tstride;      // split form: words between two tickets (tickets in one cache line serialise in one memory channel)
     uint32_t tpr_bits;     // row form: 2^tpr_bits lanes share an output
-    uint32_t lsplit_bits;  // column form: 2^lsplit_bits lanes of a block share an output group
+    uint32_t width;        // column form: output groups side by side in a block
+    uint32_t slots;        // column form: lanes of a block that share an output group's part of the axis
+    uint32_t fold_bits;    // fold of the column form's parts: 2^fold_bits lanes share an output
     int32_t index_mode;    // what accumulate() gets as idx: 1 = position along the axis, 2 = element offset from `in`
     char* partial;         // split form: n_out * n_split accumulators
     uint32_t* tickets;     // split form: n_out + n_out * ceil(n_split / group) words, zero between launches
@@ -333,81 +337,71 @@ __global__ __launch_bounds__(kRedBlock) void red_srow_split_kernel(RedSParams p,
 }
 
 // Second launch of the column form cut across blocks: folds partial[part][output] (rows of rs_parts_row
-// accumulators) into the results. 2^p.lsplit_bits lanes share a group of VEC outputs, each with a run of its
-// parts in axis order, up to eight of them in flight, and combine pairwise through LDS, earlier parts on the left.
+// accumulators) into the results. A lane has one output and a run of its parts in axis order, up to eight in
+// flight; the 2^fold_bits lanes of an output combine pairwise through LDS, earlier parts on the left. What bounds
+// it is one chain of memory round trips (parts that another die wrote, the LDS rounds, the store), not bytes, so a
+// lane has at most eight parts however wide the accumulator is: with a group of four outputs per lane the
+// running moments of 512 parts of 257 columns took 12.4 us (four divisions in turn, eight times over), one
+// output per lane 5.0 us.
 __host__ __device__ __forceinline__ size_t rs_parts_row(uint32_t n_out, uint32_t out_inner, int vec) {
     const uint32_t gpo = (out_inner + vec - 1) / vec;
     return (size_t)gpo * vec * (n_out / out_inner);
 }
 
-template <class Impl, int VEC>
-__global__ __launch_bounds__(kRedBlock) void red_fold_parts_kernel(RedSParams p, Impl impl) {
-    typedef typename Impl::Acc Acc;
+// one output's parts through the fold of I; E(impl, part, k, acc) folds part k
+template <class I, class Part, class F>
+__device__ __forceinline__ typename I::Acc rs_fold_output(const I& impl, const Part* base, size_t row, uint32_t k0, uint32_t k1, unsigned pg, unsigned PG,
+                                                          unsigned OV, typename I::Acc* slots, F fold) {
     constexpr int B = 8;
-    __shared__ Acc slots[kRedBlock][VEC];
-    const unsigned pbits = p.lsplit_bits;
-    const unsigned PG = 1u << pbits, OV = (unsigned)kRedBlock >> pbits;
-    const unsigned ov = threadIdx.x & (OV - 1), pg = threadIdx.x >> (8u - pbits);
-    const size_t row = rs_parts_row(p.n_out, p.out_inner, VEC);
-    const uint32_t o = (blockIdx.x * OV + ov) * VEC;   // the group's first output (groups are whole here: 1-D outputs, or out_inner a multiple of VEC)
+    typename I::Acc total = impl.identity();
+    for (uint32_t k = k0; k < k1; k += B) {
+        Part v[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) v[b] = base[(size_t)(k + b < k1 ? k + b : k1 - 1) * row];
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            if (k + b < k1) fold(v[b], k + b, total);
+    }
+    for (unsigned d = 1; d < PG; d <<= 1) {
+        slots[threadIdx.x] = total;
+        __syncthreads();
+        if ((pg & (2 * d - 1)) == 0) impl.combine(slots[threadIdx.x + d * OV], total);
+        __syncthreads();
+    }
+    return total;
+}
+
+template <class Impl>
+__global__ __launch_bounds__(kRedBlock) void red_fold_parts_kernel(RedSParams p, Impl impl, size_t row) {
+    typedef typename Impl::Acc Acc;
+    __shared__ Acc slots[kRedBlock];
+    const unsigned PG = 1u << p.fold_bits, OV = (unsigned)kRedBlock >> p.fold_bits;
+    const unsigned ov = threadIdx.x & (OV - 1), pg = threadIdx.x / OV;
+    const uint32_t o = blockIdx.x * OV + ov;
     const bool ok = o < p.n_out;
     const uint32_t per = (p.n_split + PG - 1) / PG;
     const uint32_t k0 = pg * per < p.n_split ? pg * per : p.n_split;
     const uint32_t k1 = k0 + per < p.n_split ? k0 + per : p.n_split;
-    const Acc* base = reinterpret_cast<const Acc*>(p.partial) + (ok ? o : 0);
-    Acc total[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) total[j] = impl.identity();
-    for (uint32_t k = k0; k < k1; k += B) {
-        Acc v[B][VEC];
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            const uint32_t kk = k + b < k1 ? k + b : k1 - 1;
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) v[b][j] = base[(size_t)kk * row + j];
-        }
-#pragma unroll
-        for (int b = 0; b < B; ++b)
-            if (k + b < k1) {
-#pragma unroll
-                for (int j = 0; j < VEC; ++j) impl.combine(v[b][j], total[j]);
-            }
-    }
-    for (unsigned stride = 1; stride < PG; stride <<= 1) {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) slots[threadIdx.x][j] = total[j];
-        __syncthreads();
-        if ((pg & (2 * stride - 1)) == 0 && pg + stride < PG) {
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) impl.combine(slots[(pg + stride) * OV + ov][j], total[j]);
-        }
-        __syncthreads();
-    }
-    if (pg != 0 || !ok) return;
+    const Acc* base = reinterpret_cast<const Acc*>(p.partial) + (ok ? o : p.n_out - 1);
+    Acc total = rs_fold_output(impl, base, row, k0, k1, pg, PG, OV, slots, [&](const Acc& v, uint32_t, Acc& t) { impl.combine(v, t); });
     if constexpr (has_exact<Impl>::value) {
         // the parts are plain values in axis order: where the fast fold cannot tell which of two equal
-        // values came first, the exact rule over the same values
+        // values came first, the exact rule over the same values, by the same lanes
         typedef typename Impl::Exact Exact;
-        const Exact ex = impl.exact();
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-            if (impl.needs_exact(total[j])) {
-                typename Exact::Acc e = ex.identity();
-                for (uint32_t k = 0; k < p.n_split; ++k) ex.accumulate_acc(base[(size_t)k * row + j], (int64_t)k, e);
-                total[j] = impl.from_exact(e);
-            }
+        if (__syncthreads_or(ok && pg == 0 && impl.needs_exact(total))) {
+            __shared__ typename Exact::Acc exact_slots[kRedBlock];
+            const Exact ex = impl.exact();
+            const typename Exact::Acc e = rs_fold_output(ex, base, row, k0, k1, pg, PG, OV, exact_slots,
+                                                         [&](const Acc& v, uint32_t k, typename Exact::Acc& t) { ex.accumulate_acc(v, (int64_t)k, t); });
+            if (impl.needs_exact(total)) total = impl.from_exact(e);
         }
     }
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-        const uint32_t oj = o + j;
-        if (oj >= p.n_out) break;
-        const uint32_t q0 = p.out_inner == p.n_out ? 0u : oj / p.out_inner;
-        const uint32_t q1 = oj - q0 * p.out_inner;
-        const int64_t a = (int64_t)q0 * p.out_step[0] + (int64_t)q1 * p.out_step[1];
-        const int64_t b2 = (Impl::NOUT > 1) ? (int64_t)q0 * p.out2_step[0] + (int64_t)q1 * p.out2_step[1] : 0;
-        impl.store(total[j], p.out + a, (Impl::NOUT > 1) ? (p.out2 + b2) : nullptr);
-    }
+    if (pg != 0 || !ok) return;
+    const uint32_t q0 = p.out_inner == p.n_out ? 0u : o / p.out_inner;
+    const uint32_t q1 = o - q0 * p.out_inner;
+    const int64_t a = (int64_t)q0 * p.out_step[0] + (int64_t)q1 * p.out_step[1];
+    const int64_t b = (Impl::NOUT > 1) ? (int64_t)q0 * p.out2_step[0] + (int64_t)q1 * p.out2_step[1] : 0;
+    impl.store(total, p.out + a, (Impl::NOUT > 1) ? (p.out2 + b) : nullptr);
 }
 
 // The exact second fold by ONE wave over the tiles that a whole block (tpr_bits 8) folded: the
@@ -558,188 +552,193 @@ __global__ __launch_bounds__(kRedBlock) void red_srow_poll_kernel(RedSParams p, 
     }
 }
 
-// Column form. out_inner is a multiple of VEC, or the outputs span one dimension (n_out >= VEC).
-// U: positions of the axis a lane has in flight (more when the outputs alone give too few lanes
-// to keep the memory system busy: a block still reads 4 KiB runs of every row it touches).
-// PARTIAL: the axis is also cut across blocks, p.n_split ways (blockIdx.y says which part this
-// block has); a block leaves its accumulators in p.partial[part][output] and a second launch
-// (red_fold_parts_kernel) folds them. Blocks stay 128 or 256 vectors wide that way however few the outputs are.
-template <class Impl, int VEC, bool NT, bool LOCAL, int U, bool PARTIAL = false>
-__global__ __launch_bounds__(kRedBlock) void red_scol_kernel(RedSParams p, Impl impl) {
-    typedef typename Impl::In In;
+// Column form: a lane owns VEC neighbouring outputs (a group) and walks the reduce axis, four rows in flight.
+//
+// What bounds it is how memory sees the reads, so that is what the split is for. A block is `width` groups side by
+// side (as equal a share of the row as whole blocks give, 256 groups at most) times `slots` lanes that share the
+// rows: slot s takes four rows, then the four that come slots * 4 later, so the whole block moves down one window
+// of slots * 4 rows at a time. Neither number is a power of two: 65 groups of a 257-column row are one
+// block of 65 x 7 lanes (blocks of 64 groups left a second block beside the first with one lane of 64 at work), and
+// a slot that kept a stretch of the axis to itself opened one stream per slot (131072 x 64: 27.1 -> 22 us).
+// PARTIAL: the axis is also cut across blocks, p.n_split ways, so that 256 blocks run: one on each compute unit, half of
+// what fits, reads faster than a full device (131072 x 256, this launch alone: 20.7 us against 21.9 for 512 blocks and 22.3
+// for 1024). Neighbouring blocks are neighbouring parts of the same columns: with the columns going first, 4096 x 4095
+// DFloat took 28.5 us instead of 24.9 and 2048 x 16384 SFloat 32.9 instead of 25.4, since block numbers go round the eight dies
+// and each die then has the same columns of every row.
+// Column sums of 128 MiB of SFloat, fresh operands, the fold included, before and after: 131072 x 257 41.6 -> 25.2 us,
+// 8192 x 4096 26.5 -> 24.5, 8192 x 4095 27.9 -> 24.3, 2048 x 16384 30.4 -> 22.0, 65536 x 500 30.0 -> 24.2; stddev of
+// 131072 x 257 51.7 -> 28.4; 500 x 500 (one launch instead of two) 6.7 -> 4.1.
+constexpr int kRcBlock = 512;   // SHARE: lanes of a block (slots * width of them at work)
+constexpr int kRcRows = 4;      // rows a lane has in flight
+
+// the lane's rows [begin, end) in steps of `step`, kRcRows at a time, through the fold of I
+template <class I, int VEC, bool NT>
+__device__ __forceinline__ void rc_walk(const I& impl, const RedSParams& p, int64_t in_off, uint64_t begin, uint64_t end, uint64_t step,
+                                        typename I::Acc (&acc)[VEC]) {
+    typedef typename I::In In;
+    constexpr int U = kRcRows;
+    const char* base = p.in + in_off;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) acc[j] = impl.identity();
+    for (uint64_t i0 = begin; i0 < end; i0 += step) {
+        In x[U][VEC];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t i = i0 + u;
+            const uint64_t ic = i < end ? i : end - 1;
+            rs_load<In, VEC, NT>(base + (int64_t)ic * p.red_step, x[u]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all loads of the step issued before the first fold
+        if (i0 + U <= end && p.index_mode != 2) {
+            // a whole block of consecutive positions along the axis for each output
+            if constexpr (folds_columns_together<I>::value) {
+                // (the lane's outputs have had the same positions so far: what depends on the count alone is worked out once)
+                impl.template accumulate_columns<U, VEC>(x, acc);
+            } else if constexpr (folds_columns_by_position<I>::value) {
+                impl.template accumulate_columns_by_position<U, VEC>(x, (int64_t)i0, acc);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) {
+                    In t[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) t[u] = x[u][j];
+                    impl.template accumulate_n<U>(t, (int64_t)i0, acc[j]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint64_t i = i0 + u;
+                if (i < end) {
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) {
+                        int64_t idx = 0;
+                        if (I::USES_INDEX)
+                            idx = (p.index_mode == 2) ? ((in_off + (int64_t)i * p.red_step) / (int64_t)sizeof(In) + j) : (int64_t)i;
+                        impl.accumulate(x[u][j], idx, acc[j]);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The slots' accumulators of every group meet pairwise through LDS: log2(slots) rounds in which every left-hand
+// lane works. Slot 0 ends up with everything. (Slots hold interleaved rows: what depends on the order of the
+// axis rides in the accumulator as a position.)
+template <class I, int VEC>
+__device__ __forceinline__ void rc_meet(const I& impl, typename I::Acc (&acc)[VEC], unsigned s, unsigned slots, unsigned width, char* lds) {
+    typedef typename I::Acc Acc;
+    Acc(*part)[VEC] = reinterpret_cast<Acc(*)[VEC]>(lds);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = acc[j];
+    __syncthreads();
+    for (unsigned d = 1; d < slots; d <<= 1) {
+        if ((s & (2u * d - 1u)) == 0 && s + d < slots) {
+            Acc next[VEC];
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) next[j] = part[threadIdx.x + d * width][j];
+            if constexpr (folds_columns_together<I>::value) {
+                impl.template combine_columns<VEC>(next, acc);
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) impl.combine(next[j], acc[j]);
+            }
+            if (2u * d < slots) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = acc[j];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// LDS of a SHARE block: the wider of the accumulators that meet there
+template <class Impl, int VEC>
+constexpr size_t rc_lds_bytes() {
+    if constexpr (has_exact<Impl>::value) {
+        constexpr size_t a = sizeof(typename Impl::Acc), e = sizeof(typename Impl::Exact::Acc);
+        return (a > e ? a : e) * VEC * kRcBlock;
+    } else {
+        return sizeof(typename Impl::Acc) * VEC * kRcBlock;
+    }
+}
+
+template <class Impl, int VEC, bool NT, bool SHARE, bool PARTIAL = false>
+__global__ __launch_bounds__(SHARE ? kRcBlock : kRedBlock) void red_scol_kernel(RedSParams p, Impl impl) {
     typedef typename Impl::Acc Acc;
-    __shared__ Acc part[LOCAL ? kRedBlock : 1][VEC];
-    const unsigned lbits = LOCAL ? p.lsplit_bits : 0u;
-    const unsigned SB = 1u << lbits;
-    const unsigned cbits = 8u - lbits;
-    const unsigned CPB = 1u << cbits;
-    const unsigned c = threadIdx.x & (CPB - 1);
-    const unsigned s = threadIdx.x >> cbits;
+    static_assert(rc_lds_bytes<Impl, VEC>() <= 65536, "the accumulators of a block fit its share of LDS");
+    __shared__ __align__(16) char lds[SHARE ? rc_lds_bytes<Impl, VEC>() : 16];
+    const unsigned width = SHARE ? p.width : (unsigned)kRedBlock;
+    const unsigned slots = SHARE ? p.slots : 1u;
+    const unsigned s = SHARE ? threadIdx.x / width : 0u;
+    const unsigned c = threadIdx.x - s * width;
     // (the inner output dimension need not be a whole number of vectors: its last group is pulled
     // back to its last VEC outputs and stores only those the group before it does not)
     const uint32_t gpo = (p.out_inner + VEC - 1) / VEC;            // groups per position of the outer output dimension
     const uint32_t groups = (p.n_out / p.out_inner) * gpo;
-    const uint32_t n_cb = (groups + CPB - 1) / CPB;
-    // this block's stretch of the axis, then this lane's part of it
+    const uint32_t n_cb = (groups + width - 1) / width;
+    // this block's stretch of the axis
+    const uint32_t cb_first = PARTIAL ? blockIdx.x / p.n_split : blockIdx.x;
+    const uint32_t part_no = PARTIAL ? blockIdx.x - cb_first * p.n_split : 0u;
     uint64_t b0 = 0, b1 = p.n;
     if (PARTIAL) {
-        const uint64_t bchunk = p.chunk;
-        b0 = (uint64_t)blockIdx.y * bchunk;
+        b0 = (uint64_t)part_no * p.chunk;
         if (b0 > p.n) b0 = p.n;
-        b1 = b0 + bchunk;
+        b1 = b0 + p.chunk;
         if (b1 > p.n) b1 = p.n;
     }
-    const uint64_t lchunk = (b1 - b0 + SB - 1) / SB;
-    uint64_t begin = b0 + (uint64_t)s * lchunk;
-    if (begin > b1) begin = b1;
-    uint64_t end = begin + lchunk;
-    if (end > b1) end = b1;
-
-    for (uint32_t cb = blockIdx.x; cb < n_cb; cb += gridDim.x) {
-        const uint32_t g = cb * CPB + c;
-        const bool ok = g < groups;
-        const uint32_t gg = ok ? g : groups - 1;
+    for (uint32_t cb = cb_first; cb < n_cb; cb += gridDim.x) {
+        const uint32_t g = cb * width + c;
+        const bool ok = g < groups && s < slots;
+        const uint32_t gg = g < groups ? g : groups - 1;
         const uint32_t o0 = p.out_inner == p.n_out ? 0u : gg / gpo;
         const uint32_t own1 = (gg - o0 * gpo) * VEC;
         const uint32_t o1 = own1 + VEC <= p.out_inner ? own1 : p.out_inner - VEC;  // where the group's vector starts
         const uint32_t own0 = o0 * p.out_inner + own1;                // the group's first output
         const uint32_t i_out0 = o0 * p.out_inner + o1;
         const int64_t in_off = (int64_t)o0 * p.in_step[0] + (int64_t)o1 * p.in_step[1];
-        const char* base = p.in + in_off;
+        // (a lane without a group or a slot walks nothing)
+        const uint64_t begin = ok ? b0 + (uint64_t)s * kRcRows : b1;
+        const uint64_t step = (uint64_t)slots * kRcRows;
         Acc acc[VEC];
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) acc[j] = impl.identity();
-        for (uint64_t i0 = begin; i0 < end; i0 += U) {
-            In x[U][VEC];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint64_t i = i0 + u;
-                const uint64_t ic = i < end ? i : end - 1;
-                rs_load<In, VEC, NT>(base + (int64_t)ic * p.red_step, x[u]);
-            }
-            __builtin_amdgcn_sched_barrier(0);  // all loads of the step issued before the first fold
-            if (i0 + U <= end && p.index_mode != 2) {
-                // a whole block of consecutive positions along the axis for each output
-                if constexpr (folds_columns_together<Impl>::value) {
-                    // (the lane's outputs have had the same positions so far: what depends on the count alone is worked out once)
-                    impl.template accumulate_columns<U, VEC>(x, acc);
-                } else if constexpr (folds_columns_by_position<Impl>::value) {
-                    impl.template accumulate_columns_by_position<U, VEC>(x, (int64_t)i0, acc);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) {
-                        In t[U];
-#pragma unroll
-                        for (int u = 0; u < U; ++u) t[u] = x[u][j];
-                        impl.template accumulate_n<U>(t, (int64_t)i0, acc[j]);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint64_t i = i0 + u;
-                    if (i < end) {
-#pragma unroll
-                        for (int j = 0; j < VEC; ++j) {
-                            int64_t idx = 0;
-                            if (Impl::USES_INDEX)
-                                idx = (p.index_mode == 2) ? ((in_off + (int64_t)i * p.red_step) / (int64_t)sizeof(In) + j) : (int64_t)i;
-                            impl.accumulate(x[u][j], idx, acc[j]);
-                        }
-                    }
-                }
-            }
-        }
+        rc_walk<Impl, VEC, NT>(impl, p, in_off, begin, b1, step, acc);
+        if constexpr (SHARE) rc_meet<Impl, VEC>(impl, acc, s, slots, width, lds);
         if constexpr (has_exact<Impl>::value) {
-            // this lane walked its part of the axis in order, but its fast fold may have lost
-            // which of two equal elements came first: walk that output again, exactly
+            // folded by value; where an output may have lost which of two equal elements came first, its rows
+            // are walked again with the rule that carries the position (whole blocks together when lanes share rows)
+            bool again = false;
+            if (ok && s == 0) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                if (impl.needs_exact(acc[j])) {
-                    typedef typename Impl::Exact Exact;
-                    const Exact ex = impl.exact();
-                    typename Exact::Acc e = ex.identity();
-                    for (uint64_t i = begin; i < end; ++i)
-                        ex.accumulate(*reinterpret_cast<const In*>(base + (int64_t)i * p.red_step + (int64_t)j * (int64_t)sizeof(In)), (int64_t)i, e);
-                    acc[j] = impl.from_exact(e);
-                }
+                for (int j = 0; j < VEC; ++j) again = again || impl.needs_exact(acc[j]);
+            }
+            if (SHARE ? __syncthreads_or(again ? 1 : 0) != 0 : again) {
+                typedef typename Impl::Exact Exact;
+                const Exact ex = impl.exact();
+                typename Exact::Acc e[VEC];
+                rc_walk<Exact, VEC, false>(ex, p, in_off, begin, b1, step, e);
+                if constexpr (SHARE) rc_meet<Exact, VEC>(ex, e, s, slots, width, lds);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j)
+                    if (impl.needs_exact(acc[j])) acc[j] = impl.from_exact(e[j]);
             }
         }
-        if constexpr (LOCAL) {
-            // The SB parts of an output group meet pairwise through LDS, neighbours first and the earlier part
-            // on the left: log2 SB rounds in which every left-hand lane works, where one lane folding all the
-            // parts one after the other waited for SB reads of LDS in a row while the rest of the block idled
-            // (blocks start and end together here, so nothing else covers that time).
-            Acc own[has_exact<Impl>::value ? VEC : 1];
-            if constexpr (has_exact<Impl>::value) {
-#pragma unroll
-                for (int j = 0; j < VEC; ++j) own[j] = acc[j];
-            }
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = acc[j];
-            __syncthreads();
-            for (unsigned d = 1; d < SB; d <<= 1) {
-                if ((s & (2u * d - 1u)) == 0) {
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) impl.combine(part[(s + d) * CPB + c][j], acc[j]);
-                    if (2u * d < SB) {
-#pragma unroll
-                        for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = acc[j];
-                    }
-                }
-                __syncthreads();
-            }
-            if constexpr (has_exact<Impl>::value) {
-                // folded by value; an output that may have lost which of two equal parts came first is folded
-                // again from the lanes' own parts, plain values in axis order, with the exact rule
-                bool again = false;
-                if (s == 0) {
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) again = again || impl.needs_exact(acc[j]);
-                }
-                if (__syncthreads_or(again ? 1 : 0)) {
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = own[j];
-                    __syncthreads();
-                    if (s == 0) {
-#pragma unroll
-                        for (int j = 0; j < VEC; ++j) {
-                            if (!impl.needs_exact(acc[j])) continue;
-                            typedef typename Impl::Exact Exact;
-                            const Exact ex = impl.exact();
-                            typename Exact::Acc e = ex.identity();
-                            for (unsigned k = 0; k < SB; ++k) ex.accumulate_acc(part[k * CPB + c][j], (int64_t)k, e);
-                            acc[j] = impl.from_exact(e);
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
-        }
+        if (!ok || s != 0) continue;
         if (PARTIAL) {
             // partial[part][output], a part's outputs padded to whole groups: the lanes of a block write one run
-            if (ok && s == 0) {
-                Acc* mine = reinterpret_cast<Acc*>(p.partial) + (size_t)blockIdx.y * ((size_t)gpo * VEC * (p.n_out / p.out_inner)) + i_out0;
-                if (i_out0 == own0) {
+            Acc* mine = reinterpret_cast<Acc*>(p.partial) + (size_t)part_no * ((size_t)gpo * VEC * (p.n_out / p.out_inner)) + i_out0;
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) mine[j] = acc[j];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < VEC; ++j)
-                        if (i_out0 + j >= own0) mine[j] = acc[j];
-                }
-            }
+            for (int j = 0; j < VEC; ++j)
+                if (i_out0 + j >= own0) mine[j] = acc[j];
             continue;
         }
-        if (ok && s == 0) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                if (i_out0 + j < own0) continue;  // (the pulled-back last group: the group before it has these)
-                // the VEC outputs of a group are neighbours along the inner output dimension
-                const int64_t a = (int64_t)o0 * p.out_step[0] + (int64_t)(o1 + j) * p.out_step[1];
-                const int64_t b = (Impl::NOUT > 1) ? (int64_t)o0 * p.out2_step[0] + (int64_t)(o1 + j) * p.out2_step[1] : 0;
-                impl.store(acc[j], p.out + a, (Impl::NOUT > 1) ? (p.out2 + b) : nullptr);
-            }
+        for (int j = 0; j < VEC; ++j) {
+            if (i_out0 + j < own0) continue;  // (the pulled-back last group: the group before it has these)
+            // the VEC outputs of a group are neighbours along the inner output dimension
+            const int64_t a = (int64_t)o0 * p.out_step[0] + (int64_t)(o1 + j) * p.out_step[1];
+            const int64_t b = (Impl::NOUT > 1) ? (int64_t)o0 * p.out2_step[0] + (int64_t)(o1 + j) * p.out2_step[1] : 0;
+            impl.store(acc[j], p.out + a, (Impl::NOUT > 1) ? (p.out2 + b) : nullptr);
         }
     }
 }

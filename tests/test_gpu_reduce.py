@@ -506,3 +506,36 @@ def test_reductions_of_slices_that_start_off_a_16_byte_boundary(tname, dt):
     for axis in (0, 1, None):
         assert (di[:, 3:1027].sum(axis=axis).to_numpy() == oracle.reduce("sum", np.ascontiguousarray(i[:, 3:1027]), axis=axis)).all()
         assert (di[:, 3:1027].argmax(axis=axis).to_numpy() == oracle.reduce("argmax", np.ascontiguousarray(i[:, 3:1027]), axis=axis)).all()
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("shape,axis", [((7, 40), 0), ((8, 16), 0), ((9, 17), 0), ((1024, 18), 0), ((1025, 19), 0), ((2047, 516), 0), ((2048, 17), 0),
+                                        ((2049, 1029), 0), ((2051, 2050), 0), ((5, 1100, 23), 1), ((9, 262149), 0), ((12, 262140), 0), ((2050, 15392), 0),
+                                        ((2052, 12291), 0), ((300007, 16), 0), ((40003, 257), 0)])
+def test_column_reductions_at_the_edges_of_their_splits(tname, dt, shape, axis):
+    """Every way the column kernel splits its work (a lane per group, slots that share rows in one launch, parts folded by a
+    second launch), on either side of the lines between them: axes shorter than a step, last slots and last parts that are
+    nearly empty, a last group pulled back over its neighbour, pieces of rows that are no power of two. Values are multiples
+    of 1/4, so sums are exact in either type; the zeros of both signs are the ends of some columns."""
+    rng = np.random.default_rng(91)
+    h = (rng.integers(-8, 9, size=shape) / 4.0).astype(dt)
+    col = np.arange(shape[-1])
+    h[..., col % 5 == 1] = -np.abs(h[..., col % 5 == 1])     # columns that end on a zero, of either sign
+    h[..., col % 5 == 2] = np.abs(h[..., col % 5 == 2])
+    h[(h == 0) & (rng.random(shape) < 0.5)] = -0.0
+    d = cls_of(tname).cast(h)
+    n = shape[axis]
+
+    def first_of(i):
+        return np.take_along_axis(h, np.expand_dims(i, axis), axis).squeeze(axis)
+
+    assert_bits_equal(d.sum(axis=axis).to_numpy() + dt(0), h.sum(axis=axis, dtype=np.float64).astype(dt) + dt(0), "sum")
+    assert (d.argmax(axis=axis).to_numpy() == h.argmax(axis=axis)).all()
+    assert (d.argmin(axis=axis).to_numpy() == h.argmin(axis=axis)).all()
+    # of +0 and -0 the earlier one is the answer: the element at the first position of the extreme
+    assert_bits_equal(d.max(axis=axis).to_numpy(), first_of(h.argmax(axis=axis)), "max")
+    lo, hi = d.minmax(axis=axis)
+    assert_bits_equal(lo.to_numpy(), first_of(h.argmin(axis=axis)), "minmax lo")
+    assert_bits_equal(hi.to_numpy(), first_of(h.argmax(axis=axis)), "minmax hi")
+    want = h.var(axis=axis, ddof=1, dtype=np.float64)
+    assert_reduction_close(d.var(axis=axis).to_numpy(), want.astype(dt), n, np.abs(want) + 1e-30, "var")
