@@ -55,6 +55,11 @@ bool mixed_flat_binary(int op, int ta, const char* x, int tb, const char* y, cha
 // the same for a contiguous Int32 run and one DFloat number (on the left when scalar_is_left), into a DFloat run
 bool mixed_flat_binary_s(int op, const char* x, double sv, bool scalar_is_left, char* z, uint64_t n);
 
+// mulsum.hip: the product sum of one run, and of many rows (see cumo_hip_mulsum_rows_t), from zero: what p3 / d->out
+// hold is not read. mulsum_rows is false when the layout is not one it takes; with fresh false it adds onto the result.
+void mulsum_run_fresh(int type, bool nan, char* p1, char* p2, char* p3, ssize_t s1, ssize_t s2, uint64_t n);
+bool mulsum_rows(int type, bool nan, const cumo_hip_mulsum_rows_t* d, bool fresh);
+
 // x cmp y (cmp: 0 == 1 != 2 > 3 >= 4 < 5 <=) for two such runs into the bits of z from its first word on
 bool mixed_flat_compare(int cmp, int ta, const char* x, int tb, const char* y, CUMO_BIT_DIGIT* z, uint64_t n);
 

@@ -1360,24 +1360,32 @@ int cumo_hip_na_mulsum(const cumo_hip_narray_t* x, const cumo_hip_narray_t* y, u
             total *= lp.n[d];
             if (d < lp.ndim - 1) launches *= lp.n[d];
         }
-        // many short contiguous runs: every row in one launch
+        // many short contiguous runs: every row in one launch (each with a result of its own: rows that add onto
+        // one element, the whole of a view that is not one run, are walked one after the other below)
+        const bool skip_nan = nan != 0 && is_float(up);
         bool rows_done = false;
-        if (!rc && total_of(z) != 0 && total != 0 && lp.ndim == 2 && lp.args[2].step[1] == 0 && launches >= 2 &&
+        if (!rc && total_of(z) != 0 && total != 0 && lp.ndim == 2 && lp.args[2].step[1] == 0 && launches >= 2 && lp.args[2].step[0] != 0 &&
             (launches > 1024 || lp.n[1] * (size_t)kElmsz[up] <= (1u << 20)) && lp.args[0].step[1] == (ssize_t)kElmsz[up] &&
             lp.args[1].step[1] == (ssize_t)kElmsz[up]) {
-            rc = cumo_hip_na_fill(z, 0.0);
+            // (a result given by the caller may be one of the operands: it is zeroed first, as it always was)
+            if (!fresh) rc = cumo_hip_na_fill(z, 0.0);
             if (!rc) {
                 cumo_hip_mulsum_rows_t g = {lp.n[0], lp.n[1], lp.args[0].step[0], lp.args[1].step[0], lp.args[2].step[0],
                                             lp.args[0].ptr, lp.args[1].ptr, lp.args[2].ptr};
-                const int t = up == CUMO_HIP_SFLOAT ? 0 : (up == CUMO_HIP_DFLOAT ? 1 : 2);
-                rows_done = cumo_hip_mulsum_rows_kernel_launch(t, nan != 0 && is_float(up), &g) == 1;
+                rows_done = cumo_hip::mulsum_rows(up, skip_nan, &g, fresh);
             }
+        } else if (!rc && fresh && total != 0 && lp.ndim >= 1 && launches == 1 && lp.args[2].step[lp.ndim - 1] == 0) {
+            // one run into one new element
+            char* p[3];
+            for (int a = 0; a < 3; ++a) p[a] = lp.args[a].ptr;
+            cumo_hip::mulsum_run_fresh(up, skip_nan, p[0], p[1], p[2], lp.args[0].step[lp.ndim - 1], lp.args[1].step[lp.ndim - 1], lp.n[lp.ndim - 1]);
+            rows_done = true;
         }
         if (!rc && total_of(z) != 0 && !rows_done) {
             if (launches <= 1024 || total == 0) {
                 rc = cumo_hip_na_fill(z, 0.0);
                 if (!rc && total != 0) {
-                    MulsumOpt opt = {up, nan != 0 && is_float(up)};
+                    MulsumOpt opt = {up, skip_nan};
                     mulsum_walk(&lp, 0, lp.args[0].ptr, lp.args[1].ptr, lp.args[2].ptr, &opt);
                 }
             } else {

@@ -501,3 +501,23 @@ def test_cum_and_mulsum_launchers_called_directly():
     _lib.call(g, px, py, pacc, 4, 0, 0)                       # an empty run adds nothing
     assert float(fetch(pacc, (1,), np.float32)[0]) == 100.0 + 2.0 * float(h[3:3 + 2 * n:2].astype(np.float64).sum())
     free(px, py, pz, pacc)
+
+
+@pytest.mark.parametrize("tname,dt", ALL)
+def test_mulsum_starts_from_zero_whatever_its_result_memory_held(tname, dt):
+    """The sum goes straight into a fresh element (or one per row) of pool memory that was in use before; rows of a
+    view that is not one run all add onto one element."""
+    cls = cls_of(tname)
+    rng = np.random.default_rng(54)
+    dirt = 77 if dt == np.int32 else float("nan")
+    for shape, axis in (((1,), None), ((1000,), None), ((100003,), None), ((300, 64), 1), ((700, 513), 1), ((40, 100), 0)):
+        hx, hy = (rng.integers(-8, 8, size=shape).astype(dt) for _ in range(2))
+        x, y = cls.cast(hx), cls.cast(hy)
+        want = (hx.astype(np.int64) * hy.astype(np.int64)).sum(axis=axis)
+        for _ in range(3):
+            cls(*np.shape(want)).fill(dirt)   # released again at once: the next result of this size is this memory
+            assert (x.mulsum(y, axis=axis).to_numpy() == want).all(), (shape, axis)
+    hx, hy = (rng.integers(-8, 8, size=(200, 301)).astype(dt) for _ in range(2))
+    x, y = cls.cast(hx), cls.cast(hy)
+    want = (hx[:, 1:].astype(np.int64) * hy[:, :-1].astype(np.int64)).sum()
+    assert (x[:, 1:].mulsum(y[:, :-1]).to_numpy() == want).all()
