@@ -852,3 +852,25 @@ def test_float_classification(tname, dt):
     x = np.array([1.0, 1.0 + 1e-7, 1.001, 0.0], dtype=dt)
     y = np.array([1.0, 1.0, 1.0, 0.0], dtype=dt)
     assert (cls.cast(x).nearly_eq(cls.cast(y)).to_numpy() == oracle.compare("nearly_eq", x, y)).all()
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS + [("int32", np.int32)])
+@pytest.mark.parametrize("shape", [(2, 5), (1000, 5), (4096, 7), (3001, 33), (2049, 257), (1023, 1023), (1500, 1027), (3, 700, 259), (8193, 513)])
+def test_matrix_with_one_row_repeated(tname, dt, shape):
+    """Rows that are no whole number of vectors against one row that repeats: where two rounds of whole rows
+    make the run each lane reads the row once for two vectors, elsewhere once a vector; either side, a strided
+    row, a zero divisor."""
+    cls = cls_of(tname)
+    rng = np.random.default_rng(12)
+    hx = rng.integers(-50, 50, size=shape).astype(dt)
+    hr = rng.integers(1, 50, size=(1, 2 * shape[-1])).astype(dt)
+    x, r = cls.cast(hx), cls.cast(hr)
+    for dr, h in ((r[:, :shape[-1]], hr[:, :shape[-1]]), (r[:, ::2], hr[:, ::2]), (r[:, ::-1][:, :shape[-1]], hr[:, ::-1][:, :shape[-1]])):
+        for op in ("add", "sub", "div"):
+            for want, got in ((oracle.binary(op, hx, h), getattr(x, PYOP[op])(dr)),
+                              (oracle.binary(op, h, np.where(hx == 0, 1, hx).astype(dt)), getattr(dr, PYOP[op])(cls.cast(np.where(hx == 0, 1, hx).astype(dt))))):
+                assert_bits_equal(got.to_numpy(), want, (op, shape))
+    if dt == np.int32:
+        hr[0, shape[-1] - 1] = 0
+        with pytest.raises(ZeroDivisionError):
+            (x / cls.cast(hr)[:, :shape[-1]]).to_numpy()
