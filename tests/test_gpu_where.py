@@ -232,3 +232,22 @@ def test_where_beyond_two_to_the_32_elements_answers_int64():
     assert int(tail.count_false()) == 72 - 3
     del b, tail, got
     cumo_amd.MemoryPool.free_all_blocks()
+
+
+@pytest.mark.parametrize("tname,dt", [("SFloat", np.float32), ("DFloat", np.float64), ("Int32", np.int32)])
+def test_mask_around_whole_vectors_chunks_and_tiles(tname, dt):
+    """A contiguous run is read in vectors (4 or 2 elements), chunks (32), a wave's 1024 and a block's 4096
+    elements, over 1024 blocks' stretches at most; masks and runs that start off their boundaries."""
+    import cumo_amd
+    cls = getattr(cumo_amd, tname)
+    rng = np.random.default_rng(94)
+    for n in (1, 2, 3, 5, 31, 33, 1023, 1025, 4095, 4097, 8191, 8193, (1 << 23) + 4099):
+        hx = rng.integers(-1000, 1000, size=n + 7).astype(dt)
+        x = cls.cast(hx)
+        for density in (0.0, 0.003, 0.4, 1.0):
+            hm = rng.random(n + 7) < density
+            m = cumo_amd.Bit.cast(hm.astype(np.uint8))
+            for a, b in ((0, 0), (3, 1), (1, 5)) if n < 100000 else ((0, 0), (3, 1)):
+                got = m[a:a + n].mask(x[b:b + n]).to_numpy()
+                want = hx[b:b + n][hm[a:a + n]]
+                assert got.shape == want.shape and (got == want).all(), (n, density, a, b)
