@@ -115,6 +115,8 @@ if not os.path.exists(LIB_PATH):
 
 lib = C.CDLL(LIB_PATH, mode=C.RTLD_GLOBAL)
 
+from . import _native  # noqa: E402  (built beside the library and linked against it)
+
 P = C.POINTER
 _sig = {
     "cumo_cuda_runtime_malloc": (C.c_void_p, [C.c_size_t]),
@@ -229,9 +231,12 @@ def check():
     """Raises what the Ruby extension would have raised for a latched error."""
     msg = C.c_char_p()
     kind = lib.cumo_hip_last_error(C.byref(msg))
-    if kind == 0:
-        return
-    text = msg.value.decode("utf-8", "replace") if msg.value else ""
+    if kind:
+        raise_latched(kind, msg.value or b"")
+
+
+def raise_latched(kind, message):
+    text = message.decode("utf-8", "replace")
     if kind == 2:
         raise OutOfMemoryError(text)
     if kind in (3, 7):
@@ -281,12 +286,14 @@ class record:
         global _recording
         self._prev = _recording
         _recording = _Calls()
+        _native.set_recording(_recording)
         self.calls = _recording
         return self.calls
 
     def __exit__(self, *exc):
         global _recording
         _recording = self._prev
+        _native.set_recording(_recording)
         return False
 
 

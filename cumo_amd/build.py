@@ -1,4 +1,5 @@
-"""Builds cumo_amd/libcumo_hip.so (gfx950) from cumo_amd/csrc with hipcc.
+"""Builds cumo_amd/libcumo_hip.so (gfx950) from cumo_amd/csrc with hipcc, and
+cumo_amd/_native.so (the object layer of the Python classes) from cumo_amd/native.
 
 One hipcc invocation per translation unit, run in parallel, then one link. The
 library is kept in-tree next to this file; nothing is installed.
@@ -12,12 +13,14 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libcumo_hip.so")
+NATIVE = os.path.join(HERE, "_native.so")
 HOST_COST_TOOL = os.path.join(HERE, "bench_host_cost")
 
 ARCH = "gfx950"
@@ -111,8 +114,20 @@ def build(jobs=None, force=False, verbose=True):
     if p.returncode:
         print(p.stdout)
         raise RuntimeError("link failed")
+    build_native()
     build_host_cost_tool()
     return LIB
+
+
+def build_native():
+    """native/arrays.cpp -> cumo_amd/_native.so, a CPython module linked against the library (host code only)."""
+    src = os.path.join(HERE, "native", "arrays.cpp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-I" + os.path.join(ROOT, "include"),
+           "-I" + sysconfig.get_paths()["include"], src, "-o", NATIVE, "-L" + HERE, "-lcumo_hip", "-Wl,-rpath,$ORIGIN"]
+    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if p.returncode:
+        print(p.stdout)
+        raise RuntimeError("_native: g++ failed")
 
 
 def build_host_cost_tool():

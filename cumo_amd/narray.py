@@ -22,39 +22,14 @@ import numbers
 import numpy as np
 
 from . import _lib
+from . import _native
 from ._lib import MAX_DIM, DimensionError, NArrayDesc, ShapeError, call
 
 _L = _lib.lib
 
 
-class _Buffer:
-    """One pool allocation; returned to the pool when the last view dies
-    (reference: gen/tmpl/alloc_func.c:33-56)."""
-
-    __slots__ = ("ptr", "nbytes")
-
-    def __init__(self, nbytes, ptr=None):
-        self.nbytes = int(nbytes)
-        if ptr is not None:
-            self.ptr = ptr or None  # adopted from the library
-            return
-        self.ptr = call(_L.cumo_cuda_runtime_malloc, self.nbytes) if nbytes else None
-        if nbytes and not self.ptr:
-            raise _lib.OutOfMemoryError("allocation of %d bytes failed" % nbytes)
-
-    def __del__(self):
-        try:
-            rec = _lib._recording
-            if self.ptr and rec is not None:
-                # released inside a recording: the recorded calls still name this memory
-                rec.keep.append(_Buffer(self.nbytes, ptr=self.ptr))
-                self.ptr = None
-                return
-            if self.ptr:
-                _L.cumo_cuda_runtime_free_no_raise(self.ptr)
-                self.ptr = None
-        except Exception:
-            pass
+# One pool allocation; returned to the pool when the last view dies (reference: gen/tmpl/alloc_func.c:33-56)
+_Buffer = _native.Buffer
 
 
 def _prod(shape):
@@ -86,7 +61,8 @@ def _wrap(desc):
 
 def _run(f, *args, results=()):
     """Calls one host-layer function; `results` are the descriptors it may have
-    allocated, released again if the call fails."""
+    allocated, released again if the call fails. The calls that nearly every program is made of go through
+    _native, which does the same without ctypes, and come here for the forms it leaves (and to be recorded)."""
     try:
         call(f, *args)
     except BaseException:
@@ -179,7 +155,7 @@ def _index_launchers():
 _IX = _index_launchers()
 
 
-class NArray:
+class NArray(_native.View):
     """Base of the typed arrays. shape/strides/offset describe a view into a
     pool buffer; strides and offset are bytes (bits for Bit)."""
 
@@ -254,11 +230,11 @@ class NArray:
 
     contiguous_p = is_contiguous
 
-    def _ptr(self):
-        return (self._buf.ptr or 0) + self._offset
-
     def _view(self, shape, strides, offset):
         return type(self)(*shape, _buffer=self._buf, _offset=offset, _strides=strides)
+
+    def __copy__(self):
+        return self._view(self.shape, self._strides, self._offset)
 
     def _desc(self):
         """This view as the library's cumo_hip_narray_t."""
@@ -697,16 +673,16 @@ class _Numeric(NArray):
         d, z = self._desc(), NArrayDesc()
         return _run(_L.cumo_hip_na_poly, C.byref(d), len(descs), ptrs, C.byref(z), results=(z,))
 
-    def __add__(self, o): return self._binary(o, "add")
-    def __radd__(self, o): return self._binary(o, "add", True)
-    def __sub__(self, o): return self._binary(o, "sub")
-    def __rsub__(self, o): return self._binary(o, "sub", True)
-    def __mul__(self, o): return self._binary(o, "mul")
-    def __rmul__(self, o): return self._binary(o, "mul", True)
-    def __truediv__(self, o): return self._binary(o, "div")
-    def __rtruediv__(self, o): return self._binary(o, "div", True)
-    def __mod__(self, o): return self._binary(o, "mod")
-    def __rmod__(self, o): return self._binary(o, "mod", True)
+    def __add__(self, o): return _native.binary(self, o, "add", False)
+    def __radd__(self, o): return _native.binary(self, o, "add", True)
+    def __sub__(self, o): return _native.binary(self, o, "sub", False)
+    def __rsub__(self, o): return _native.binary(self, o, "sub", True)
+    def __mul__(self, o): return _native.binary(self, o, "mul", False)
+    def __rmul__(self, o): return _native.binary(self, o, "mul", True)
+    def __truediv__(self, o): return _native.binary(self, o, "div", False)
+    def __rtruediv__(self, o): return _native.binary(self, o, "div", True)
+    def __mod__(self, o): return _native.binary(self, o, "mod", False)
+    def __rmod__(self, o): return _native.binary(self, o, "mod", True)
 
     # -- pow, clip, maximum / minimum -------------------------------------------
     def __pow__(self, other):
@@ -770,6 +746,9 @@ class _Numeric(NArray):
     # -- mulsum, cumsum / cumprod ---------------------------------------------------
     def mulsum(self, other, axis=None, keepdims=False, nan=False):
         """reference: gen/tmpl/accum_binary.c:62-110"""
+        return _native.mulsum(self, other, axis, keepdims, nan)
+
+    def _mulsum(self, other, axis, keepdims, nan):
         if not isinstance(other, _Numeric):
             other = type(self).cast(other)
         nd = max(self.ndim, other.ndim)
@@ -786,21 +765,21 @@ class _Numeric(NArray):
 
     def cumsum(self, axis=None, nan=False):
         """reference: gen/tmpl/cum.c:48-80"""
-        return self._cum("cumsum", axis, nan)
+        return _native.cum(self, "cumsum", axis, nan)
 
-    def cumprod(self, axis=None, nan=False): return self._cum("cumprod", axis, nan)
+    def cumprod(self, axis=None, nan=False): return _native.cum(self, "cumprod", axis, nan)
 
     # -- unary ----------------------------------------------------------------
     def _unary(self, op):
         x, z = self._desc(), NArrayDesc()
         return _run(_L.cumo_hip_na_unary, op.encode(), C.byref(x), C.byref(z), results=(z,))
 
-    def __neg__(self): return self._unary("minus")
-    def minus(self): return self._unary("minus")
-    def square(self): return self._unary("square")
-    def sign(self): return self._unary("sign")
-    def reciprocal(self): return self._unary("reciprocal")
-    def abs(self): return self._unary("abs")
+    def __neg__(self): return _native.unary(self, "minus")
+    def minus(self): return _native.unary(self, "minus")
+    def square(self): return _native.unary(self, "square")
+    def sign(self): return _native.unary(self, "sign")
+    def reciprocal(self): return _native.unary(self, "reciprocal")
+    def abs(self): return _native.unary(self, "abs")
 
     __abs__ = abs
 
@@ -816,19 +795,19 @@ class _Numeric(NArray):
         x, y = self._desc(), other._desc()
         return _run(_L.cumo_hip_na_compare, op.encode(), C.byref(x), C.byref(y), C.byref(z), results=(z,))
 
-    def eq(self, o): return self._compare(o, "eq")
-    def ne(self, o): return self._compare(o, "ne")
-    def gt(self, o): return self._compare(o, "gt")
-    def ge(self, o): return self._compare(o, "ge")
-    def lt(self, o): return self._compare(o, "lt")
-    def le(self, o): return self._compare(o, "le")
+    def eq(self, o): return _native.compare(self, o, "eq")
+    def ne(self, o): return _native.compare(self, o, "ne")
+    def gt(self, o): return _native.compare(self, o, "gt")
+    def ge(self, o): return _native.compare(self, o, "ge")
+    def lt(self, o): return _native.compare(self, o, "lt")
+    def le(self, o): return _native.compare(self, o, "le")
     __gt__ = gt
     __ge__ = ge
     __lt__ = lt
     __le__ = le
 
     def nearly_eq(self, o):
-        return self._compare(o, "nearly_eq" if self.is_float else "eq")
+        return _native.compare(self, o, "nearly_eq" if self.is_float else "eq")
 
     # -- reductions ------------------------------------------------------------
     def _reduce(self, name, axis=None, keepdims=False, nan=False):
@@ -841,37 +820,37 @@ class _Numeric(NArray):
         return _run(_L.cumo_hip_na_reduce, name.encode(), C.byref(x), mask, int(bool(keepdims)), int(bool(nan)),
                     C.byref(z), None, results=(z,))
 
-    def sum(self, axis=None, keepdims=False, nan=False): return self._reduce("sum", axis, keepdims, nan)
-    def prod(self, axis=None, keepdims=False, nan=False): return self._reduce("prod", axis, keepdims, nan)
-    def min(self, axis=None, keepdims=False, nan=False): return self._reduce("min", axis, keepdims, nan)
-    def max(self, axis=None, keepdims=False, nan=False): return self._reduce("max", axis, keepdims, nan)
-    def ptp(self, axis=None, keepdims=False, nan=False): return self._reduce("ptp", axis, keepdims, nan)
-    def minmax(self, axis=None, keepdims=False, nan=False): return self._reduce("minmax", axis, keepdims, nan)
-    def argmin(self, axis=None, keepdims=False, nan=False): return self._reduce("argmin", axis, keepdims, nan)
-    def argmax(self, axis=None, keepdims=False, nan=False): return self._reduce("argmax", axis, keepdims, nan)
-    def min_index(self, axis=None, keepdims=False, nan=False): return self._reduce("min_index", axis, keepdims, nan)
-    def max_index(self, axis=None, keepdims=False, nan=False): return self._reduce("max_index", axis, keepdims, nan)
+    def sum(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "sum", axis, keepdims, nan)
+    def prod(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "prod", axis, keepdims, nan)
+    def min(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "min", axis, keepdims, nan)
+    def max(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "max", axis, keepdims, nan)
+    def ptp(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "ptp", axis, keepdims, nan)
+    def minmax(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "minmax", axis, keepdims, nan)
+    def argmin(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "argmin", axis, keepdims, nan)
+    def argmax(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "argmax", axis, keepdims, nan)
+    def min_index(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "min_index", axis, keepdims, nan)
+    def max_index(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "max_index", axis, keepdims, nan)
 
 
 class _Float(_Numeric):
     is_float = True
 
-    def mean(self, axis=None, keepdims=False, nan=False): return self._reduce("mean", axis, keepdims, nan)
-    def var(self, axis=None, keepdims=False, nan=False): return self._reduce("var", axis, keepdims, nan)
-    def stddev(self, axis=None, keepdims=False, nan=False): return self._reduce("stddev", axis, keepdims, nan)
-    def rms(self, axis=None, keepdims=False, nan=False): return self._reduce("rms", axis, keepdims, nan)
+    def mean(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "mean", axis, keepdims, nan)
+    def var(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "var", axis, keepdims, nan)
+    def stddev(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "stddev", axis, keepdims, nan)
+    def rms(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "rms", axis, keepdims, nan)
 
     def modf(self):
         """[fraction, integral part], each with the sign of the element (reference: gen/tmpl/unary_ret2.c)."""
         d, f, w = self._desc(), NArrayDesc(), NArrayDesc()
         return _run(_L.cumo_hip_na_modf, C.byref(d), C.byref(f), C.byref(w), results=(f, w))
 
-    def floor(self): return self._unary("floor")
-    def round(self): return self._unary("round")
-    def ceil(self): return self._unary("ceil")
-    def trunc(self): return self._unary("trunc")
-    def rint(self): return self._unary("rint")
-    def copysign(self, o): return self._binary(o, "copysign")
+    def floor(self): return _native.unary(self, "floor")
+    def round(self): return _native.unary(self, "round")
+    def ceil(self): return _native.unary(self, "ceil")
+    def trunc(self): return _native.unary(self, "trunc")
+    def rint(self): return _native.unary(self, "rint")
+    def copysign(self, o): return _native.binary(self, o, "copysign", False)
 
     def _cond_unary(self, op):
         x, z = self._desc(), NArrayDesc()
@@ -892,7 +871,7 @@ class SFloat(_Float):
 class DFloat(_Float):
     type_name, type_code, np_dtype, elmsz = "dfloat", 1, np.float64, 8
 
-    def kahan_sum(self, axis=None, keepdims=False, nan=False): return self._reduce("kahan_sum", axis, keepdims, nan)
+    def kahan_sum(self, axis=None, keepdims=False, nan=False): return _native.reduce(self, "kahan_sum", axis, keepdims, nan)
 
 
 class Int64(NArray):
@@ -908,13 +887,13 @@ class UInt64(NArray):
 class Int32(_Numeric):
     type_name, type_code, np_dtype, elmsz = "int32", 2, np.int32, 4
 
-    def __and__(self, o): return self._binary(o, "bit_and")
-    def __or__(self, o): return self._binary(o, "bit_or")
-    def __xor__(self, o): return self._binary(o, "bit_xor")
-    def __lshift__(self, o): return self._binary(o, "left_shift")
-    def __rshift__(self, o): return self._binary(o, "right_shift")
-    def __invert__(self): return self._unary("bit_not")
-    def __floordiv__(self, o): return self._binary(o, "div")
+    def __and__(self, o): return _native.binary(self, o, "bit_and", False)
+    def __or__(self, o): return _native.binary(self, o, "bit_or", False)
+    def __xor__(self, o): return _native.binary(self, o, "bit_xor", False)
+    def __lshift__(self, o): return _native.binary(self, o, "left_shift", False)
+    def __rshift__(self, o): return _native.binary(self, o, "right_shift", False)
+    def __invert__(self): return _native.unary(self, "bit_not")
+    def __floordiv__(self, o): return _native.binary(self, o, "div", False)
 
 
 # ---------------------------------------------------------------------------
@@ -996,10 +975,10 @@ class Bit(NArray):
         x, y, z = self._desc(), other._desc(), NArrayDesc()
         return _run(_L.cumo_hip_na_bit_binary, op.encode(), C.byref(x), C.byref(y), C.byref(z), results=(z,))
 
-    def __and__(self, o): return self._bit_op2(o, "and")
-    def __or__(self, o): return self._bit_op2(o, "or")
-    def __xor__(self, o): return self._bit_op2(o, "xor")
-    def eq(self, o): return self._bit_op2(o, "eq")
+    def __and__(self, o): return _native.bit_binary(self, o, "and")
+    def __or__(self, o): return _native.bit_binary(self, o, "or")
+    def __xor__(self, o): return _native.bit_binary(self, o, "xor")
+    def eq(self, o): return _native.bit_binary(self, o, "eq")
 
     def __invert__(self):
         x, z = self._desc(), NArrayDesc()
@@ -1031,8 +1010,8 @@ class Bit(NArray):
         m, x, z = self._desc(), array._desc(), NArrayDesc()
         return _run(_L.cumo_hip_na_mask, C.byref(m), C.byref(x), C.byref(z), results=(z,))
 
-    def count_true(self, axis=None, keepdims=False): return self._count(False, axis, keepdims)
-    def count_false(self, axis=None, keepdims=False): return self._count(True, axis, keepdims)
+    def count_true(self, axis=None, keepdims=False): return _native.bit_count(self, False, axis, keepdims)
+    def count_false(self, axis=None, keepdims=False): return _native.bit_count(self, True, axis, keepdims)
 
     count = count_true
     count_1 = count_true
@@ -1084,12 +1063,17 @@ class _NMath:
             "asinh acosh atanh sinc erf erfc log1p expm1").split()
     _TWO = ("atan2", "hypot", "ldexp")
 
-    def __getattr__(self, name):
-        if name in self._ONE:
-            return lambda x: self._call1(name, x)
-        if name in self._TWO:
-            return lambda x, y: self._call2(name, x, y)
-        raise AttributeError(name)
+    def __init__(self):
+        for name in self._ONE:
+            setattr(self, name, self._one(name))
+        for name in self._TWO:
+            setattr(self, name, self._two(name))
+
+    def _one(self, name):
+        return lambda x: _native.math(name, x)
+
+    def _two(self, name):
+        return lambda x, y: self._call2(name, x, y)
 
     @staticmethod
     def _check(x):
@@ -1121,6 +1105,8 @@ class _NMath:
 
 
 NMath = _NMath()
+
+_native.setup(_CLASS_BY_CODE, _lib.raise_latched, NMath)
 
 
 class _Fused:
