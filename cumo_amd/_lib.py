@@ -142,6 +142,7 @@ _sig = {
     "cumo_hip_memset": (None, [C.c_void_p, C.c_int, C.c_size_t]),
     "cumo_hip_copy_to_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t]),
     "cumo_hip_copy_from_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t]),
+    "cumo_hip_index_from_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_ssize_t, C.c_int, C.c_size_t]),
     "cumo_hip_pool_malloc": (C.c_int, [C.c_size_t, C.c_void_p, P(C.c_void_p)]),
     "cumo_hip_pool_free": (C.c_int, [C.c_void_p]),
     "cumo_hip_pool_free_all_blocks": (None, []),

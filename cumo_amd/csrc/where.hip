@@ -21,6 +21,7 @@
 
 #include <type_traits>
 
+#include <chrono>
 #include <cstring>
 
 namespace cumo_hip {
@@ -126,9 +127,8 @@ __global__ __launch_bounds__(kWhBlock) void where_count_kernel(const CUMO_BIT_DI
     wh_block_exscan(cnt, &total);
     if (threadIdx.x == 0) {
         block_sums[blockIdx.x] = total;
-        // a copy straight into the caller's pinned host memory: the host then only has to wait for
-        // the stream, not for a copy queued behind the kernel
-        if (host_sums) host_sums[blockIdx.x] = total;
+        // a copy straight into the caller's pinned host memory, one up so that no count is the 0 the host looks for
+        if (host_sums) __hip_atomic_store(host_sums + blockIdx.x, total + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -429,25 +429,53 @@ void cumo_hip_bit_where_count_kernel_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t
     cumo_cuda_runtime_check_kernel_launch();
 }
 
-// The same, and the counts on the host when the call returns (it waits for the stream): the kernel
-// writes them into pinned host memory of the calling thread as well, so no copy is queued behind
-// it. host_counts: cumo_hip_bit_where_blocks(n) words of ordinary host memory.
+// The same, and the counts on the host when the call returns: the kernel writes them into pinned host memory of the
+// calling thread as well, and the host looks at that memory until every block's count is there. They are the last thing
+// the stream has been given, so nothing earlier is still running then. A stream that has not come this far within
+// kWhLookNs is waited for instead, which also reports what may have gone wrong on it. Looking costs the caller's core
+// what the runtime's own wait costs it, and saves the wait's way through a signal: SFloat 104 x 96 x[mask]
+// 20.9 -> 15.8 us, mask.where() 20.0 -> 15.2 us.
+// host_counts: cumo_hip_bit_where_blocks(n) words of ordinary host memory.
+constexpr int64_t kWhLookNs = 2000000;
 int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts) {
     if (n == 0) return CUMO_HIP_OK;
     const WhGeometry g = wh_geometry(n);
     static thread_local uint64_t* pinned = nullptr;   // kWhMaxBlocks words, kept for the thread's lifetime
     if (pinned == nullptr) {
         void* m = nullptr;
-        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable), "hipHostMalloc")) return CUMO_HIP_ERROR_RUNTIME;
+        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc"))
+            return CUMO_HIP_ERROR_RUNTIME;
         pinned = static_cast<uint64_t*>(m);
     }
+    std::memset(pinned, 0, g.nblocks * sizeof(uint64_t));
     hipStream_t st = current_stream();
     hipLaunchKernelGGL(where_count_kernel, dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s, (const size_t*)nullptr, n,
                        s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, counts, pinned);
-    cumo_cuda_runtime_check_kernel_launch();
-    if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+    const hipError_t launched = hipGetLastError();
+    if (launched != hipSuccess) {
+        report_hip_error(launched, "kernel launch");
+        return CUMO_HIP_ERROR_RUNTIME;
+    }
+    const auto begin = std::chrono::steady_clock::now();
+    uint64_t b = 0;
+    for (unsigned looks = 0; b < g.nblocks; ++looks) {
+        while (b < g.nblocks && __atomic_load_n(pinned + b, __ATOMIC_ACQUIRE) != 0) ++b;
+        if (b == g.nblocks) break;
+        __builtin_ia32_pause();
+        if ((looks & 63u) == 63u && (std::chrono::steady_clock::now() - begin) > std::chrono::nanoseconds(kWhLookNs)) {
+            if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+            break;
+        }
+    }
     if (!wait_trouble_check()) return CUMO_HIP_ERROR_RUNTIME;
-    std::memcpy(host_counts, pinned, g.nblocks * sizeof(uint64_t));
+    for (b = 0; b < g.nblocks; ++b) {
+        const uint64_t word = __atomic_load_n(pinned + b, __ATOMIC_RELAXED);
+        if (word == 0) {
+            report_error(CUMO_HIP_ERROR_RUNTIME, 0, "where: a block left no count");
+            return CUMO_HIP_ERROR_RUNTIME;
+        }
+        host_counts[b] = word - 1;
+    }
     return CUMO_HIP_OK;
 }
 

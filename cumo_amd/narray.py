@@ -136,12 +136,21 @@ def _upload_index(pos):
     return buf
 
 
+def _upload_offsets(pos, st, n):
+    """The byte offsets of positions in a dimension of n elements and stride st; a reversed dimension counts from its
+    far end (narray/index.c:580-590)."""
+    buf = _Buffer(8 * max(len(pos), 1))
+    if len(pos):
+        pos = np.ascontiguousarray(pos, dtype=np.uint64)
+        call(_L.cumo_hip_index_from_host, buf.ptr, pos.ctypes.data, len(pos), abs(st), 1 if st < 0 else 0, n - 1)
+    return buf
+
+
 def _index_launchers():
     v, sz, ss, u64 = C.c_void_p, C.c_size_t, C.c_ssize_t, C.c_uint64
     P = C.POINTER
     return {
         "aref_nadata_index_stride": _lib.fn("cumo_na_index_aref_nadata_index_stride_kernel_launch", None, [v, ss, u64]),
-        "aref_naview_index_stride": _lib.fn("cumo_na_index_aref_naview_index_stride_kernel_launch", None, [v, ss, u64]),
         "aref_naview_index_stride_last": _lib.fn("cumo_na_index_aref_naview_index_stride_last_kernel_launch", None, [v, ss, sz, u64]),
         "at_nadata_index_stride_add": _lib.fn("cumo_na_index_at_nadata_index_stride_add_kernel_launch", None, [v, v, ss, u64]),
         "at_nadata_index_beg_step_stride": _lib.fn("cumo_na_index_at_nadata_index_beg_step_stride_kernel_launch", None, [v, sz, ss, ss, u64]),
@@ -326,15 +335,10 @@ class NArray(_native.View):
                 a.stridx[d] = ((st * step) << 1) | 1
             else:
                 pos = _index_positions(k, n)
-                buf = _upload_index(pos)
+                buf = _upload_offsets(pos, st, n)
                 keep.append(buf)
-                if len(pos):
-                    if st < 0:
-                        # a reversed dimension counts from its far end (index.c:580-590)
-                        offset += st * (n - 1)
-                        call(_IX["aref_naview_index_stride_last"], buf.ptr, -st, n - 1, len(pos))
-                    else:
-                        call(_IX["aref_naview_index_stride"], buf.ptr, st, len(pos))
+                if len(pos) and st < 0:
+                    offset += st * (n - 1)
                 shape.append(len(pos))
                 a.stridx[d] = buf.ptr or 0
             d += 1

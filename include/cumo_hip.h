@@ -517,6 +517,11 @@ void cumo_na_index_aref_nadata_index_stride_kernel_launch(size_t *idx, ssize_t s
 void cumo_na_index_aref_naview_index_index_kernel_launch(size_t *idx, size_t *idx1, uint64_t n);
 void cumo_na_index_aref_naview_index_stride_last_kernel_launch(size_t *idx, ssize_t s1, size_t last, uint64_t n);
 void cumo_na_index_aref_naview_index_stride_kernel_launch(size_t *idx, ssize_t s1, uint64_t n);
+/* idx[i] = pos[i] * s1, or (last - pos[i]) * s1 with from_last: the two kernels above on n positions in ordinary
+ * host memory, which may change as soon as the call returns (not a reference symbol: there the index array is
+ * written through managed memory, narray/index.c:201-233). Few positions go without a wait; many, or those of a
+ * stream that has sixteen such calls ahead, are copied first. Returns CUMO_HIP_OK or an error kind. */
+int cumo_hip_index_from_host(size_t *idx, const size_t *pos, size_t n, ssize_t s1, int from_last, size_t last);
 void cumo_na_index_aref_naview_index_index_beg_step_kernel_launch(size_t *idx, size_t *idx1, size_t beg, ssize_t step, uint64_t n);
 void cumo_na_index_at_nadata_index_stride_add_kernel_launch(size_t *idx, size_t *idx1, ssize_t s1, uint64_t n);
 void cumo_na_index_at_nadata_index_beg_step_stride_kernel_launch(size_t *idx, size_t beg, ssize_t step, ssize_t s1, uint64_t n);
@@ -655,9 +660,10 @@ int cumo_hip_mulsum_rows_kernel_launch(int type, int nan, const cumo_hip_mulsum_
 size_t cumo_hip_bit_where_blocks(uint64_t n);
 void cumo_hip_bit_where_count_kernel_launch(CUMO_BIT_DIGIT *a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t *counts);
 /* count, and the counts in host_counts[0 .. blocks - 1] when the call returns: the kernel also writes
- * them to pinned host memory of the calling thread, and the call waits for the stream (the one
- * synchronisation that sizing the result costs, tmpl_bit/where.c:13-28) instead of queueing a copy
- * behind the kernel. Returns CUMO_HIP_OK or an error kind. */
+ * them to pinned host memory of the calling thread, and the call waits until they are there, that is
+ * for everything the stream was given before (the one synchronisation that sizing the result costs,
+ * tmpl_bit/where.c:13-28), instead of queueing a copy behind the kernel. Returns CUMO_HIP_OK or an
+ * error kind. */
 int  cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT *a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t *counts, uint64_t *host_counts);
 void cumo_hip_bit_where_place_kernel_launch(CUMO_BIT_DIGIT *a, size_t p, ssize_t s, uint64_t n, int invert, const uint64_t *counts,
                                             const char *x, ssize_t sx, size_t elmsz, char *out);

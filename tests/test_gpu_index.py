@@ -9,6 +9,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import cumo_amd
+
 import kat_adjacent as K
 from helpers import assert_bits_equal
 from test_gpu_raw_abi import dev, fetch, free, indexer
@@ -403,3 +405,37 @@ def test_a_bit_array_as_the_index_of_one_dimension(tname, dt):
     v[v.eq(7)] = cls.cast(np.arange(int((wantv == 7).sum()), dtype=dt))
     wantv[wantv == 7] = np.arange(int((wantv == 7).sum()), dtype=dt)
     assert_bits_equal(v.to_numpy(), wantv)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 1023, 1024, 1025, 8191, 8192, 8193, 20000])
+def test_index_arrays_of_every_size_reach_the_device(n):
+    # (8192 positions is where the slots of pinned memory end)
+    rng = np.random.default_rng(n)
+    a = rng.integers(0, 1 << 30, size=(n + 5, 3), dtype=np.int32)
+    x = cumo_amd.Int32.cast(a)
+    pos = rng.integers(-(n + 5), n + 5, size=n)
+    assert (x[pos].to_numpy() == a[pos]).all()
+    assert (x.reverse(0)[pos].to_numpy() == a[::-1][pos]).all()
+    assert (x[pos, [2, 0]].to_numpy() == a[pos][:, [2, 0]]).all()
+
+
+def test_many_index_arrays_in_a_row_and_from_two_threads():
+    # more of them in flight than there are slots, each with positions of its own in host memory that is then overwritten
+    import threading
+    a = np.arange(4000, dtype=np.float64)
+    bad = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        x = cumo_amd.DFloat.cast(a)
+        pos = np.empty(1000, dtype=np.int64)
+        got = []
+        for _ in range(60):
+            pos[:] = rng.integers(0, 4000, size=1000)
+            got.append((pos.copy(), x[pos]))
+        bad.extend(1 for p, g in got if not (g.to_numpy() == a[p]).all())
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
