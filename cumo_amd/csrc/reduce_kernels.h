@@ -526,7 +526,8 @@ struct CombineImpl {
 // Device memory a caller lends for the partial results of a split reduction.
 struct RedScratch {
     char* ptr;
-    size_t bytes;
+    size_t bytes;          // partial results of a planned split that are still taken
+    size_t column_bytes;   // what ptr holds: red_split_columns cuts an axis into more parts than the planner's count that `bytes` bounds
     mutable size_t used;   // set by the launch: bytes of ptr that its kernels write and read (0: none)
 };
 
@@ -795,6 +796,12 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
     if (plan.kind == RED_COL) {
         if (plan.in_out_step[plan.out_ndim - 1] != (int64_t)sizeof(In)) return 0;
         const uint64_t gpo = ((uint64_t)p.out_inner + V - 1) / V;
+        // A caller's array takes the calls that the planner's own count of parts fits, however many parts the axis is cut into
+        // below: 65536 groups over all parts at most, which column_bytes holds.
+        if (fixed && plan.n_split > 1) {
+            const uint64_t part = (plan.red_total + (uint64_t)plan.n_split - 1) / (uint64_t)plan.n_split;
+            if (sizeof(Acc) * rs_parts_row(p.n_out, p.out_inner, V) * ((plan.red_total + part - 1) / part) > fixed->bytes) return -1;
+        }
         const bool whole_lines = (((uintptr_t)p.in | (uint64_t)p.red_step | (uint64_t)p.in_step[0]) & 127u) == 0;
         const ColumnSplit cs = red_split_columns((p.n_out / p.out_inner) * gpo, plan.red_total, whole_lines);
         p.width = cs.width;
@@ -806,7 +813,7 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
             const size_t parts_row = rs_parts_row(p.n_out, p.out_inner, V);
             const uint64_t scratch_bytes = sizeof(Acc) * parts_row * cs.n_split;
             if (fixed) {
-                if (scratch_bytes > fixed->bytes) return -1;
+                if (scratch_bytes > fixed->column_bytes) return -1;
                 p.partial = fixed->ptr;
                 fixed->used = scratch_bytes;
             } else {

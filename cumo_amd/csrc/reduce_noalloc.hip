@@ -13,7 +13,7 @@ using namespace cumo_hip;
 
 namespace {
 
-constexpr size_t kScratchBytes = CUMO_HIP_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kScratchBytes = 4 * CUMO_HIP_NOALLOC_SCRATCH_BYTES;  // a column split of 65536 groups of four sums, the most there are
 constexpr int kMaxDevices = 64;
 
 // One copy per GPU the library runs on, held until the process ends. Host code never
@@ -66,7 +66,7 @@ extern "C" int cumo_hip_sfloat_sum_noalloc_kernel_launch(cumo_na_reduction_arg_t
     int kind = CUMO_HIP_OK;
     char* p = scratch_of_current_device(&kind);
     if (p == nullptr) return kind;
-    const RedScratch fixed = {p, kScratchBytes, 0};
+    const RedScratch fixed = {p, CUMO_HIP_NOALLOC_SCRATCH_BYTES, kScratchBytes, 0};
     if (!reduce_launch(arg, nullptr, SumImpl<float, float, false, false>{0.0f}, 0, &fixed)) {
         report_error(CUMO_HIP_ERROR_ARGUMENT, 0,
                      "cumo_hip_sfloat_sum_noalloc_kernel_launch: the partial sums of this reduction do not fit the fixed "

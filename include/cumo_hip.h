@@ -414,13 +414,14 @@ CUMO_HIP_DECL_REDUCE_PAIR(dfloat, minmax_nan)
  * reference, whose split reductions always take their scratch from the memory pool
  * (include/cumo/reduce_kernel.h:493-496). Same descriptors, planner, kernels and
  * result bits as cumo_sfloat_sum_kernel_launch, but the partial sums of a split
- * reduction go to a fixed array of CUMO_HIP_NOALLOC_SCRATCH_BYTES that lives in the
+ * reduction go to a fixed array of four times CUMO_HIP_NOALLOC_SCRATCH_BYTES that lives in the
  * library's device image (each GPU the library runs on holds its own copy until the
  * process ends); the call makes no hipMalloc / hipFree and does not touch the pool.
  * Returns CUMO_HIP_OK, or CUMO_HIP_ERROR_ARGUMENT (also latched / handed to the error
  * handler) without launching anything when the partial sums would not fit: a split
  * reduction with more than CUMO_HIP_NOALLOC_SCRATCH_BYTES / 4 partial sums, i.e.
- * outputs x chunks of the reduce axis. Every call on a GPU shares that GPU's array:
+ * outputs x chunks of the reduce axis as planned (column sums are cut into more chunks
+ * than that, which the array holds). Every call on a GPU shares that GPU's array:
  * calls that can overlap on one GPU (different streams or threads) race and must be
  * serialised by the caller. Nothing in the array has to start at zero; it keeps the
  * last call's partial sums. */

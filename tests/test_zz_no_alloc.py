@@ -115,6 +115,17 @@ def test_two_calls_in_a_row_second_one_smaller():
     assert (want == got).all()
 
 
+@pytest.mark.parametrize("rows,cols", [(5498, 1020), (4138, 1876), (1040, 1300), (14161, 584)])
+def test_column_sums_whose_planned_split_fits_are_taken(rows, cols):
+    # the axis is cut into more parts than the planner's count, which is what the limit is stated in
+    plan = _plan(_arg(0x1000, 0x2000, (cols,), (rows,), (4, 4 * cols), (4,)))
+    assert plan.n_split > 1 and 4 * cols * plan.n_split <= SCRATCH_BYTES
+    h = np.random.default_rng(rows).standard_normal((rows, cols)).astype(np.float32)
+    want, got, status, d_mallocs, d_used, plan = _both(h, (cols,), (rows,), (4, 4 * cols), (4,))
+    assert status == 0 and d_mallocs == 0 and d_used == 0
+    assert (want == got).all()
+
+
 def test_partial_sums_beyond_the_fixed_array_are_refused():
     from cumo_amd import _lib
     rng = np.random.default_rng(12)
