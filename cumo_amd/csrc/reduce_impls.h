@@ -235,6 +235,8 @@ struct MomentsImpl {
     // U positions of VEC neighbouring outputs at once (the column form: a lane's outputs have all seen the same
     // number of positions): each output's own two passes over its U values, and one merge each with the ONE weight
     // U / (n + U) that the count gives all of them (one division a step instead of one an output).
+    // The first step merges into an accumulator of no elements: nw is 0, and delta, the step's own mean, may have a square
+    // past the type's range (1e20 in SFloat), so it meets nw before it meets itself.
     static constexpr bool COLUMNS_TOGETHER = !SKIP_NAN;
     template <int U, int VEC>
     __device__ __forceinline__ void accumulate_columns(const T (&x)[U][VEC], Acc (&acc)[VEC]) const {
@@ -256,11 +258,11 @@ struct MomentsImpl {
             }
             const T delta = mb - acc[j].mean;
             acc[j].mean = acc[j].mean + delta * w;
-            acc[j].m2 += m2 + delta * delta * nw;
+            acc[j].m2 += m2 + delta * (delta * nw);
             acc[j].n = n_new;
         }
     }
-    // The same for two lanes' accumulators of VEC neighbouring outputs: one weight for all of them.
+    // The same for two lanes' accumulators of VEC neighbouring outputs: one weight for all of them (either may be empty).
     template <int VEC>
     __device__ __forceinline__ void combine_columns(const Acc (&next)[VEC], Acc (&acc)[VEC]) const {
         if (next[0].n == (T)0) return;
@@ -271,7 +273,7 @@ struct MomentsImpl {
         for (int j = 0; j < VEC; ++j) {
             const T delta = next[j].mean - acc[j].mean;
             acc[j].mean = acc[j].mean + delta * w;
-            acc[j].m2 += next[j].m2 + delta * delta * nw;
+            acc[j].m2 += next[j].m2 + delta * (delta * nw);
             acc[j].n = n;
         }
     }

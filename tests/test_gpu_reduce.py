@@ -539,3 +539,26 @@ def test_column_reductions_at_the_edges_of_their_splits(tname, dt, shape, axis):
     assert_bits_equal(hi.to_numpy(), first_of(h.argmax(axis=axis)), "minmax hi")
     want = h.var(axis=axis, ddof=1, dtype=np.float64)
     assert_reduction_close(d.var(axis=axis).to_numpy(), want.astype(dt), n, np.abs(want) + 1e-30, "var")
+
+
+@pytest.mark.parametrize("tname,dt,base,grain", [("sfloat", np.float32, 2.0 ** 65, 2.0 ** -12), ("dfloat", np.float64, 2.0 ** 520, 2.0 ** -20)])
+@pytest.mark.parametrize("shape", [(3, 24), (1024, 18), (1025, 64), (9, 262149), (2049, 1029), (40003, 257)])
+def test_column_moments_of_values_whose_squares_leave_the_range(tname, dt, base, grain, shape):
+    """var / stddev down columns of finite values with a mean whose square is infinite: a lane's first step merges into an
+    accumulator of no elements, whose weight is 0. Shapes of each split (a lane per group, one launch, parts), rows that are
+    whole vectors and rows that are not. Even columns are constant (a power of two: every mean is exact, the variance 0)."""
+    rng = np.random.default_rng(92)
+    k = rng.integers(-8, 9, size=shape)
+    k[:, ::2] = 0
+    h = (base * (1.0 + k * grain)).astype(dt)
+    d = cls_of(tname).cast(h)
+    want = (k * grain).var(axis=0, ddof=1) * base * base
+    # a merge sees two means, each off by a few units in the last place of the mean: relative to a deviation delta that is
+    # u * mean / delta, and m2 takes delta squared. 16 units for the whole chain.
+    u = np.finfo(dt).eps / 2
+    for got, ref in ((d.var(axis=0), want), (d.stddev(axis=0), np.sqrt(want)), (d.var(axis=0, nan=True), want)):
+        g = got.to_numpy().astype(np.float64)
+        assert np.isfinite(g).all()
+        assert (g[::2] == 0).all()
+        dev = np.sqrt(want[1::2])
+        assert (np.abs(g[1::2] - ref[1::2]) <= 16 * u * base / dev * ref[1::2]).all()
