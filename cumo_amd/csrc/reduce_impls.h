@@ -109,6 +109,8 @@ struct SumImpl {
     typedef TA Acc;
     static constexpr bool USES_INDEX = false;
     static constexpr int NOUT = 1;
+    // a sum in floating point loses a rounding per row of a column (see rc_walk); a product's roundings are relative, whatever their order
+    static constexpr int ROUNDS_EVERY = is_float_t<TA>::value && !PROD ? 1 : 0;
     TA divisor;
     // results have the input's type: a reduction may go through results of its own (rows first, then the rows' results),
     // the division only at the end
@@ -133,6 +135,7 @@ template <class T>
 struct MeanNanImpl {
     typedef T In;
     struct Acc { T sum; int64_t n; };
+    static constexpr int ROUNDS_EVERY = 1;
     static constexpr bool USES_INDEX = false;
     static constexpr int NOUT = 1;
     __device__ __forceinline__ Acc identity() const { return Acc{(T)0, 0}; }
@@ -157,6 +160,7 @@ struct RmsImpl {
     struct Counted { T sum; int64_t n; };
     struct Plain { T sum; };
     typedef typename std::conditional<SKIP_NAN, Counted, Plain>::type Acc;
+    static constexpr int ROUNDS_EVERY = 1;
     static constexpr bool USES_INDEX = false;
     static constexpr int NOUT = 1;
     T count;
@@ -187,6 +191,7 @@ template <class T, bool SKIP_NAN>
 struct MomentsImpl {
     typedef T In;
     struct Acc { T n; T mean; T m2; };
+    static constexpr int ROUNDS_EVERY = 4;   // (accumulate_n / accumulate_columns: four rows to a merge)
     static constexpr bool USES_INDEX = false;
     static constexpr int NOUT = 1;
     int take_sqrt;

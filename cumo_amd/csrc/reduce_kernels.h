@@ -45,6 +45,7 @@
 #include "plan.h"
 #include "wait_ctl.h"
 
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 
@@ -716,6 +717,7 @@ struct ColumnSplit {
 //    2000 x 2000: 10.8 against 9.3);
 //  * else equal shares of the row, at most 256 groups each, and as many parts as make 256 blocks at most (a few blocks
 //    more than compute units and some of them read twice as long: 5000 x 3300 DFloat in 259 blocks 30.2 us, in 256 24.9).
+// How many lanes share an axis is thereby a matter of time alone: what long walks would cost in rounding, rc_walk's runs give back.
 static inline ColumnSplit red_split_columns(uint64_t groups, uint64_t n, bool whole_lines) {
     constexpr uint64_t kWidest = 256;
     ColumnSplit c;
@@ -806,6 +808,7 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
         const ColumnSplit cs = red_split_columns((p.n_out / p.out_inner) * gpo, plan.red_total, whole_lines);
         p.width = cs.width;
         p.slots = cs.slots;
+        if constexpr (rounds_every<Impl>::value != 0) p.run = rc_run_steps((cs.chunk + cs.slots - 1) / cs.slots, rounds_every<Impl>::value);
         if (cs.n_split > 1) {
             // The axis is cut across blocks as well: accumulators to scratch, a second launch folds them.
             p.n_split = cs.n_split;

@@ -41,6 +41,10 @@ template <class I> struct folds_columns_together<I, decltype((void)I::COLUMNS_TO
 template <class I, class = void> struct folds_columns_by_position { static constexpr bool value = false; };
 template <class I> struct folds_columns_by_position<I, decltype((void)I::COLUMNS_BY_POSITION)> { static constexpr bool value = I::COLUMNS_BY_POSITION; };
 
+// An Impl whose accumulator is rounded by every ROUNDS_EVERY rows of a column (0, or none given: not at all, or it does not matter)
+template <class I, class = void> struct rounds_every { static constexpr int value = 0; };
+template <class I> struct rounds_every<I, decltype((void)I::ROUNDS_EVERY)> { static constexpr int value = I::ROUNDS_EVERY; };
+
 struct RedSParams {
     const char* in;
     char* out;
@@ -60,6 +64,7 @@ struct RedSParams {
     uint32_t tpr_bits;     // row form: 2^tpr_bits lanes share an output
     uint32_t width;        // column form: output groups side by side in a block
     uint32_t slots;        // column form: lanes of a block that share an output group's part of the axis
+    uint32_t run;          // column form: steps of kRcRows rows that a lane folds by themselves (where the Impl rounds)
     uint32_t fold_bits;    // fold of the column form's parts: 2^fold_bits lanes share an output
     int32_t index_mode;    // what accumulate() gets as idx: 1 = position along the axis, 2 = element offset from `in`
     char* partial;         // split form: n_out * n_split accumulators
@@ -358,9 +363,23 @@ __device__ __forceinline__ typename I::Acc rs_fold_output(const I& impl, const P
         Part v[B];
 #pragma unroll
         for (int b = 0; b < B; ++b) v[b] = base[(size_t)(k + b < k1 ? k + b : k1 - 1) * row];
+        if constexpr (rounds_every<I>::value != 0) {
+            // neighbours first: one behind the other, a lane's eight lose as much as all before them have (error of the column
+            // sums of 1677 x 20001, 12 parts, in norm: 4.2e-8 that way, 3.9e-8 this way)
 #pragma unroll
-        for (int b = 0; b < B; ++b)
-            if (k + b < k1) fold(v[b], k + b, total);
+            for (int b = 0; b < B; ++b)
+                if (k + b >= k1) v[b] = impl.identity();
+#pragma unroll
+            for (int d = 1; d < B; d <<= 1) {
+#pragma unroll
+                for (int b = 0; b < B; b += 2 * d) impl.combine(v[b + d], v[b]);
+            }
+            impl.combine(v[0], total);
+        } else {
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+                if (k + b < k1) fold(v[b], k + b, total);
+        }
     }
     for (unsigned d = 1; d < PG; d <<= 1) {
         slots[threadIdx.x] = total;
@@ -571,15 +590,46 @@ __global__ __launch_bounds__(kRedBlock) void red_srow_poll_kernel(RedSParams p, 
 constexpr int kRcBlock = 512;   // SHARE: lanes of a block (slots * width of them at work)
 constexpr int kRcRows = 4;      // rows a lane has in flight
 
-// the lane's rows [begin, end) in steps of `step`, kRcRows at a time, through the fold of I
+// two accumulators of VEC outputs each, `next` of later rows
+template <class I, int VEC>
+__device__ __forceinline__ void rc_combine(const I& impl, const typename I::Acc (&next)[VEC], typename I::Acc (&acc)[VEC]) {
+    if constexpr (folds_columns_together<I>::value) {
+        impl.template combine_columns<VEC>(next, acc);
+    } else {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) impl.combine(next[j], acc[j]);
+    }
+}
+
+// Steps of a run of a lane that walks `rows` rows (see rc_walk) and rounds every `every` of them. m roundings in runs of L leave
+// an error that goes with the root of L^2 / 3m inside the runs and of m / 3L between them: least at L^3 = m^2 / 2. Few rows stay one
+// run (var of 500 x 500, eight rows a lane, costs 0.4 of its 6.6 us more in runs).
+static inline uint32_t rc_run_steps(uint64_t rows, int every) {
+    if (rows <= 32) return 0xffffffffu;
+    const double m = (double)rows / every;
+    const uint64_t steps = ((uint64_t)std::ceil(std::cbrt(m * m / 2)) * every + kRcRows - 1) / kRcRows;
+    return steps < 1 ? 1u : (steps > 0xffffffffull ? 0xffffffffu : (uint32_t)steps);
+}
+
+// The lane's rows [begin, end) in steps of `step`, kRcRows at a time, through the fold of I.
+// Where that rounds, it goes in runs of p.run steps, each folded by itself and then into what the lane has: all rows in one chain
+// would lose the more the fewer lanes share them. Error of the sum of uniform SFloat columns, in norm, one chain / runs:
+// 128 x 262144 1.6e-7 / 5.4e-8, 4096 x 262144 8.4e-7 / 8.2e-8 (a lane per group); 4096 x 65536 1.1e-7 / 4.5e-8 (eight slots).
+// The times stay what they are: it is memory that a lane waits for.
 template <class I, int VEC, bool NT>
 __device__ __forceinline__ void rc_walk(const I& impl, const RedSParams& p, int64_t in_off, uint64_t begin, uint64_t end, uint64_t step,
                                         typename I::Acc (&acc)[VEC]) {
     typedef typename I::In In;
+    typedef typename I::Acc Acc;
     constexpr int U = kRcRows;
+    constexpr bool RUNS = rounds_every<I>::value != 0;
     const char* base = p.in + in_off;
+    Acc own[VEC];
+    Acc(&to)[VEC] = RUNS ? own : acc;
+    uint32_t left = p.run;
+    bool several = false;
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) acc[j] = impl.identity();
+    for (int j = 0; j < VEC; ++j) acc[j] = own[j] = impl.identity();
     for (uint64_t i0 = begin; i0 < end; i0 += step) {
         In x[U][VEC];
 #pragma unroll
@@ -593,16 +643,16 @@ __device__ __forceinline__ void rc_walk(const I& impl, const RedSParams& p, int6
             // a whole block of consecutive positions along the axis for each output
             if constexpr (folds_columns_together<I>::value) {
                 // (the lane's outputs have had the same positions so far: what depends on the count alone is worked out once)
-                impl.template accumulate_columns<U, VEC>(x, acc);
+                impl.template accumulate_columns<U, VEC>(x, to);
             } else if constexpr (folds_columns_by_position<I>::value) {
-                impl.template accumulate_columns_by_position<U, VEC>(x, (int64_t)i0, acc);
+                impl.template accumulate_columns_by_position<U, VEC>(x, (int64_t)i0, to);
             } else {
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) {
                     In t[U];
 #pragma unroll
                     for (int u = 0; u < U; ++u) t[u] = x[u][j];
-                    impl.template accumulate_n<U>(t, (int64_t)i0, acc[j]);
+                    impl.template accumulate_n<U>(t, (int64_t)i0, to[j]);
                 }
             }
         } else {
@@ -615,10 +665,27 @@ __device__ __forceinline__ void rc_walk(const I& impl, const RedSParams& p, int6
                         int64_t idx = 0;
                         if (I::USES_INDEX)
                             idx = (p.index_mode == 2) ? ((in_off + (int64_t)i * p.red_step) / (int64_t)sizeof(In) + j) : (int64_t)i;
-                        impl.accumulate(x[u][j], idx, acc[j]);
+                        impl.accumulate(x[u][j], idx, to[j]);
                     }
                 }
             }
+        }
+        if constexpr (RUNS) {
+            if (--left == 0) {
+                left = p.run;
+                several = true;
+                rc_combine<I, VEC>(impl, own, acc);
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) own[j] = impl.identity();
+            }
+        }
+    }
+    if constexpr (RUNS) {
+        if (several) {
+            rc_combine<I, VEC>(impl, own, acc);
+        } else {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) acc[j] = own[j];
         }
     }
 }
@@ -638,12 +705,7 @@ __device__ __forceinline__ void rc_meet(const I& impl, typename I::Acc (&acc)[VE
             Acc next[VEC];
 #pragma unroll
             for (int j = 0; j < VEC; ++j) next[j] = part[threadIdx.x + d * width][j];
-            if constexpr (folds_columns_together<I>::value) {
-                impl.template combine_columns<VEC>(next, acc);
-            } else {
-#pragma unroll
-                for (int j = 0; j < VEC; ++j) impl.combine(next[j], acc[j]);
-            }
+            rc_combine<I, VEC>(impl, next, acc);
             if (2u * d < slots) {
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) part[threadIdx.x][j] = acc[j];

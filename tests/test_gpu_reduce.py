@@ -562,3 +562,32 @@ def test_column_moments_of_values_whose_squares_leave_the_range(tname, dt, base,
         assert (g[::2] == 0).all()
         dev = np.sqrt(want[1::2])
         assert (np.abs(g[1::2] - ref[1::2]) <= 16 * u * base / dev * ref[1::2]).all()
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("shape,lanes", [((128, 262144), 1), ((512, 262148), 1), ((1024, 131072), 4)])
+def test_column_sums_lose_no_more_than_short_chains_do(tname, dt, shape, lanes):
+    """The rounding error of sums and moments down columns where few lanes (or one) share an axis. `lanes` is how many do for
+    rows of vectors of four; DFloat has half the columns, so as many vectors. Values with all bits set at random."""
+    rng = np.random.default_rng(93)
+    n, cols = shape[0], shape[1] // (2 if tname == "dfloat" else 1)
+    bits = 24 if tname == "sfloat" else 53
+    k = rng.integers(0, 1 << bits, size=(n, cols), dtype=np.int64)
+    h = np.ldexp(k.astype(dt), -bits)
+    d = cls_of(tname).cast(h)
+    # Rounding errors are uniform, so a sum of size S_i has one of u / sqrt(3) * S_i at most in root mean square, each on its own;
+    # relative to the result, m roundings in runs of L = cbrt(m^2 / 2) add up to the root of L^2 / 3m + m / 3L = 0.63 cbrt(m), and
+    # the lanes' parts meeting pairwise to less than 2.
+    u = np.finfo(dt).eps / 2
+
+    def off(got, want):
+        got = got.to_numpy().astype(np.longdouble)
+        return float(np.sqrt(((got - want) ** 2).sum() / (want * want).sum()))
+
+    exact = np.ldexp(k.sum(axis=0).astype(np.longdouble), -bits)   # (below 2^63: whole numbers)
+    assert off(d.sum(axis=0), exact) <= u / 3 ** 0.5 * (0.63 * (n / lanes) ** (1 / 3) / lanes + 2) ** 0.5
+    assert off(d.mean(axis=0), exact / n) <= u / 3 ** 0.5 * (0.63 * (n / lanes) ** (1 / 3) / lanes + 3) ** 0.5
+    if tname == "sfloat":
+        # (four rows to a merge; 6 for the rounding of the squares, of a merge's products and of the division)
+        m = n / lanes / 4
+        assert off(d.var(axis=0), h.astype(np.float64).var(axis=0, ddof=1)) <= u / 3 ** 0.5 * (0.63 * m ** (1 / 3) / lanes + 6) ** 0.5
