@@ -109,16 +109,19 @@ std::mutex g_ix_lock;
 IxSlot* g_ix_slots = nullptr;
 int g_ix_next = 0;
 
-// true when the upload has been launched; false when it has to go the general way
-bool index_upload(size_t* idx, const size_t* pos, size_t n, ssize_t s1, int from_last, size_t last) {
+// true when the upload has been launched, or has failed to be (*failed); false when it has to go the general way. Reports nothing
+// itself: the error handler need not return, and the lock is held here.
+bool index_upload(size_t* idx, const size_t* pos, size_t n, ssize_t s1, int from_last, size_t last, hipError_t* failed) {
+    *failed = hipSuccess;
     if (n > kIxUpMost) return false;
     hipStream_t st = current_stream();
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     // (a replay would read what the slot holds by then)
-    if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
+    if (capturing != hipStreamCaptureStatusNone) return false;
     std::lock_guard<std::mutex> hold(g_ix_lock);
     if (g_ix_slots == nullptr) {
         void* m = nullptr;
@@ -132,11 +135,18 @@ bool index_upload(size_t* idx, const size_t* pos, size_t n, ssize_t s1, int from
     IxSlot& slot = g_ix_slots[g_ix_next];
     if (__atomic_load_n(&slot.done, __ATOMIC_ACQUIRE) != slot.number) return false;   // still to be read: a queue this deep can wait for a copy
     std::memcpy(slot.pos, pos, n * sizeof(uint64_t));
-    hipLaunchKernelGGL(index_upload_kernel, dim3(1), dim3(kIxUpBlock), 0, st, idx, (const uint64_t*)slot.pos, (uint32_t)n, (uint64_t)last, from_last,
-                       (int64_t)s1, &slot.done, slot.number + 1);
-    if (hipGetLastError() != hipSuccess) return false;
+    // The slot belongs to this launch from here on, whatever the runtime says of it: were it given out again, positions that a
+    // queued kernel has yet to read could be overwritten. What decides whether there is one is the launch's own
+    // status: hipGetLastError would answer for an earlier call of the thread as well.
     slot.number += 1;
     g_ix_next = (g_ix_next + 1) % kIxSlots;
+    const uint64_t* from = slot.pos;
+    uint32_t count = (uint32_t)n;
+    uint64_t end = last;
+    int64_t step = s1;
+    uint32_t* done = &slot.done;
+    void* args[] = {&idx, &from, &count, &end, &from_last, &step, &done, &slot.number};
+    *failed = hipLaunchKernel(reinterpret_cast<const void*>(index_upload_kernel), dim3(1), dim3(kIxUpBlock), args, 0, st);
     return true;
 }
 
@@ -403,7 +413,16 @@ int cumo_hip_index_from_host(size_t* idx, const size_t* pos, size_t n, ssize_t s
         report_error(CUMO_HIP_ERROR_ARGUMENT, 0, "index_from_host: null pointer");
         return CUMO_HIP_ERROR_ARGUMENT;
     }
-    if (index_upload(idx, pos, n, s1, from_last, last)) return CUMO_HIP_OK;
+    hipError_t failed;
+    if (index_upload(idx, pos, n, s1, from_last, last, &failed)) {
+        if (failed != hipSuccess) {
+            (void)hipGetLastError();
+            report_hip_error(failed, "kernel launch");
+            return CUMO_HIP_ERROR_RUNTIME;
+        }
+        cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
+        return CUMO_HIP_OK;
+    }
     const int rc = cumo_hip_copy_from_host(idx, pos, n * sizeof(size_t));
     if (rc) return rc;
     if (from_last) index_arith<IX_LAST_MUL_STRIDE>(idx, nullptr, nullptr, last, 0, s1, 0, n);

@@ -439,3 +439,44 @@ def test_many_index_arrays_in_a_row_and_from_two_threads():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+def hip_runtime():
+    """The HIP runtime the library is linked against, as this process has loaded it."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    return C.CDLL(path)
+
+
+def queue_work(x, launches=200):
+    """Some 15 ms of work on the calling thread's stream."""
+    for _ in range(launches):
+        cumo_amd.NMath.erfc(x)
+
+
+def busy(hip, stream=None):
+    hip.hipStreamQuery.argtypes = [C.c_void_p]
+    left = hip.hipStreamQuery(stream)
+    hip.hipGetLastError()
+    assert left in (0, 600)      # hipSuccess, hipErrorNotReady
+    return left == 600
+
+
+def test_an_error_left_by_an_earlier_call_is_reported_and_costs_no_slot():
+    hip = hip_runtime()
+    a = np.arange(3000, dtype=np.float64)
+    x = cumo_amd.DFloat.cast(a)
+    long = cumo_amd.DFloat.cast(np.linspace(0.1, 2, 1 << 24))
+    pos = [np.random.default_rng(k).integers(0, 3000, size=100) for k in range(40)]
+    for p in pos:
+        assert (x[p].to_numpy() == a[p]).all()
+    for _ in range(3):
+        hip.hipSetDevice(1 << 20)          # no such device: refused by the runtime, which keeps the error for the thread
+        with pytest.raises(RuntimeError):
+            x[pos[0]]
+    cumo_amd.synchronize()
+    # every slot is still given out: as many uploads as there are go behind queued work without waiting for it
+    queue_work(long)
+    got = [x[p] for p in pos[:16]]
+    assert busy(hip)
+    assert all((g.to_numpy() == a[p]).all() for g, p in zip(got, pos))
