@@ -97,7 +97,7 @@ __global__ __launch_bounds__(kIxUpBlock) void index_upload_kernel(size_t* idx, c
 }
 
 // The slots that index arrays travel through: pinned memory for kIxSlots of them, allocated at first use, kept. A slot
-// is free again when the kernel that read it has said so; the next one to use it looks for that.
+// is free again when the kernel that read it has said so; whoever needs one looks for that.
 constexpr int kIxSlots = 16;
 struct IxSlot {
     uint32_t done;      // written by the kernel
@@ -132,14 +132,20 @@ bool index_upload(size_t* idx, const size_t* pos, size_t n, ssize_t s1, int from
         std::memset(m, 0, kIxSlots * sizeof(IxSlot));
         g_ix_slots = static_cast<IxSlot*>(m);
     }
-    IxSlot& slot = g_ix_slots[g_ix_next];
-    if (__atomic_load_n(&slot.done, __ATOMIC_ACQUIRE) != slot.number) return false;   // still to be read: a queue this deep can wait for a copy
+    // the next slot whose last kernel has read it: those that wait behind long work on some stream are passed over
+    int at = g_ix_next, left = kIxSlots;
+    while (left > 0 && __atomic_load_n(&g_ix_slots[at].done, __ATOMIC_ACQUIRE) != g_ix_slots[at].number) {
+        at = (at + 1) % kIxSlots;
+        --left;
+    }
+    if (left == 0) return false;   // all of them have yet to be read: a queue this deep can wait for a copy
+    IxSlot& slot = g_ix_slots[at];
     std::memcpy(slot.pos, pos, n * sizeof(uint64_t));
     // The slot belongs to this launch from here on, whatever the runtime says of it: were it given out again, positions that a
     // queued kernel has yet to read could be overwritten. What decides whether there is one is the launch's own
     // status: hipGetLastError would answer for an earlier call of the thread as well.
     slot.number += 1;
-    g_ix_next = (g_ix_next + 1) % kIxSlots;
+    g_ix_next = (at + 1) % kIxSlots;
     const uint64_t* from = slot.pos;
     uint32_t count = (uint32_t)n;
     uint64_t end = last;
@@ -404,8 +410,8 @@ void cumo_na_index_at_naview_index_index_beg_step_add_kernel_launch(size_t* idx,
 void cumo_na_index_at_naview_index_stride_last_add_kernel_launch(size_t* idx, ssize_t s1, size_t last, uint64_t n) { index_arith<IX_ADD_LAST_MUL_STRIDE>(idx, nullptr, nullptr, last, 0, s1, 0, n); }
 
 // Up to kIxUpMost positions go through a slot of pinned memory that a kernel reads: nothing is waited for. More of them
-// are copied and multiplied, as do those of a stream that is being captured (where the copy is refused) or that has all slots
-// ahead of it. SFloat x[26 rows of 96] 33.0 -> 19.5 us, x[2048 rows of 4096] 36.6 -> 22.6 us: the copy
+// are copied and multiplied, as are those of a stream that is being captured (where the copy is refused) and those that find every
+// slot of the process still to be read. SFloat x[26 rows of 96] 33.0 -> 19.5 us, x[2048 rows of 4096] 36.6 -> 22.6 us: the copy
 // waited for the stream, moved 16 KB by a kernel of its own and had the multiplication behind it.
 int cumo_hip_index_from_host(size_t* idx, const size_t* pos, size_t n, ssize_t s1, int from_last, size_t last) {
     if (n == 0) return CUMO_HIP_OK;

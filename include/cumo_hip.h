@@ -520,8 +520,8 @@ void cumo_na_index_aref_naview_index_stride_last_kernel_launch(size_t *idx, ssiz
 void cumo_na_index_aref_naview_index_stride_kernel_launch(size_t *idx, ssize_t s1, uint64_t n);
 /* idx[i] = pos[i] * s1, or (last - pos[i]) * s1 with from_last: the two kernels above on n positions in ordinary
  * host memory, which may change as soon as the call returns (not a reference symbol: there the index array is
- * written through managed memory, narray/index.c:201-233). Few positions go without a wait; many, or those of a
- * stream that has sixteen such calls ahead, are copied first. Returns CUMO_HIP_OK or an error kind. */
+ * written through managed memory, narray/index.c:201-233). Few positions go without a wait; many, or any while
+ * sixteen such calls of the process are still to run, are copied first. Returns CUMO_HIP_OK or an error kind. */
 int cumo_hip_index_from_host(size_t *idx, const size_t *pos, size_t n, ssize_t s1, int from_last, size_t last);
 void cumo_na_index_aref_naview_index_index_beg_step_kernel_launch(size_t *idx, size_t *idx1, size_t beg, ssize_t step, uint64_t n);
 void cumo_na_index_at_nadata_index_stride_add_kernel_launch(size_t *idx, size_t *idx1, ssize_t s1, uint64_t n);

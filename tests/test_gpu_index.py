@@ -448,18 +448,22 @@ def hip_runtime():
     return C.CDLL(path)
 
 
-def queue_work(x, launches=200):
-    """Some 15 ms of work on the calling thread's stream."""
+def queue_work(hip, x, launches=200):
+    """Some 15 ms of work on the calling thread's stream; the event behind it."""
+    from cumo_amd import _lib
     for _ in range(launches):
         cumo_amd.NMath.erfc(x)
+    event = C.c_void_p()
+    assert hip.hipEventCreate(C.byref(event)) == 0
+    assert hip.hipEventRecord(event, C.c_void_p(_lib.lib.cumo_hip_get_stream())) == 0
+    return event
 
 
-def busy(hip, stream=None):
-    hip.hipStreamQuery.argtypes = [C.c_void_p]
-    left = hip.hipStreamQuery(stream)
+def running(hip, event):
+    state = hip.hipEventQuery(event)
     hip.hipGetLastError()
-    assert left in (0, 600)      # hipSuccess, hipErrorNotReady
-    return left == 600
+    assert state in (0, 600)      # hipSuccess, hipErrorNotReady
+    return state == 600
 
 
 def test_an_error_left_by_an_earlier_call_is_reported_and_costs_no_slot():
@@ -476,7 +480,57 @@ def test_an_error_left_by_an_earlier_call_is_reported_and_costs_no_slot():
             x[pos[0]]
     cumo_amd.synchronize()
     # every slot is still given out: as many uploads as there are go behind queued work without waiting for it
-    queue_work(long)
+    work = queue_work(hip, long)
     got = [x[p] for p in pos[:16]]
-    assert busy(hip)
+    assert running(hip, work)
     assert all((g.to_numpy() == a[p]).all() for g, p in zip(got, pos))
+
+
+@pytest.fixture
+def side_stream():
+    """A stream of its own for the calling thread; the thread is back on the default one afterwards."""
+    from cumo_amd import _lib
+    st = _lib.lib.cumo_hip_stream_create()
+    yield st
+    _lib.lib.cumo_hip_set_stream(None)
+    cumo_amd.synchronize()
+    _lib.lib.cumo_hip_stream_destroy(st)
+
+
+def test_more_index_arrays_behind_long_work_than_there_are_slots():
+    a = np.arange(3000, dtype=np.float64)
+    x = cumo_amd.DFloat.cast(a)
+    long = cumo_amd.DFloat.cast(np.linspace(0.1, 2, 1 << 24))
+    pos = [np.random.default_rng(k).integers(0, 3000, size=100) for k in range(40)]
+    queue_work(hip_runtime(), long)
+    got = [x[p] for p in pos]          # (from the seventeenth on by a copy that waits)
+    assert all((g.to_numpy() == a[p]).all() for g, p in zip(got, pos))
+
+
+def test_a_stream_behind_long_work_leaves_the_other_slots_to_the_others(side_stream):
+    from cumo_amd import _lib
+    hip = hip_runtime()
+    a = np.arange(3000, dtype=np.float64)
+    x = cumo_amd.DFloat.cast(a)
+    long = cumo_amd.DFloat.cast(np.linspace(0.1, 2, 1 << 24))
+    pos = [np.random.default_rng(k).integers(0, 3000, size=100) for k in range(40)]
+
+    def on_side(pos, launches):
+        _lib.lib.cumo_hip_set_stream(side_stream)
+        work = queue_work(hip, long, launches)
+        got = [x[p] for p in pos]
+        ahead = running(hip, work)
+        ok = all((g.to_numpy() == a[p]).all() for g, p in zip(got, pos))
+        cumo_amd.synchronize()
+        _lib.lib.cumo_hip_set_stream(None)
+        return ok, ahead
+
+    cumo_amd.synchronize()
+    assert on_side(pos, 4)[0]          # (the side stream's memory is there from here on)
+    theirs = queue_work(hip, long, 900)
+    mine = x[pos[0]]
+    assert on_side(pos[:8], 0)[0]
+    # the ring has come round to the slot that the default stream has yet to read: these neither take it nor wait for their stream
+    assert on_side(pos[:12], 200) == (True, True)
+    assert running(hip, theirs)
+    assert (mine.to_numpy() == a[pos[0]]).all()
