@@ -449,10 +449,17 @@ int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uin
     }
     std::memset(pinned, 0, g.nblocks * sizeof(uint64_t));
     hipStream_t st = current_stream();
-    hipLaunchKernelGGL(where_count_kernel, dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s, (const size_t*)nullptr, n,
-                       s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, counts, pinned);
-    const hipError_t launched = hipGetLastError();
+    // The launch's own status: hipGetLastError would answer for an earlier call of the thread as well, and a kernel that has been
+    // queued must be waited for, or its counts could be taken for the next call's.
+    uint64_t first = p, words = n, *host = pinned;
+    int64_t step = s;
+    const size_t* idx = nullptr;
+    int contiguous = s == 1 ? 1 : 0;
+    WhGeometry kg = g;
+    void* args[] = {&a, &first, &step, &idx, &words, &contiguous, &invert, &kg.nchunks, &kg.cpb, &counts, &host};
+    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(where_count_kernel), dim3((unsigned)g.nblocks), dim3(kWhBlock), args, 0, st);
     if (launched != hipSuccess) {
+        (void)hipGetLastError();
         report_hip_error(launched, "kernel launch");
         return CUMO_HIP_ERROR_RUNTIME;
     }
@@ -476,6 +483,7 @@ int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uin
         }
         host_counts[b] = word - 1;
     }
+    cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
     return CUMO_HIP_OK;
 }
 

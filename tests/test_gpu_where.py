@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import kat_adjacent as K
+from test_gpu_index import hip_runtime, queue_work, side_stream  # noqa: F401  (a fixture among them)
 
 oracle = K.OracleEngine().o
 
@@ -251,3 +252,26 @@ def test_mask_around_whole_vectors_chunks_and_tiles(tname, dt):
                 got = m[a:a + n].mask(x[b:b + n]).to_numpy()
                 want = hx[b:b + n][hm[a:a + n]]
                 assert got.shape == want.shape and (got == want).all(), (n, density, a, b)
+
+
+def masks(k):
+    import cumo_amd
+    rng = np.random.default_rng(700 + k)
+    h = (rng.random(100000) < rng.random()).astype(np.uint8)
+    return h, cumo_amd.Bit.cast(h)
+
+
+def test_an_error_left_by_an_earlier_call_is_reported_and_leaves_no_kernel_behind():
+    import cumo_amd
+    hip = hip_runtime()
+    long = cumo_amd.DFloat.cast(np.linspace(0.1, 2, 1 << 24))
+    many = [masks(k) for k in range(12)]
+    many[0][1].where()
+    cumo_amd.synchronize()
+    queue_work(hip, long)
+    hip.hipSetDevice(1 << 20)          # no such device: refused by the runtime, which keeps the error for the thread
+    with pytest.raises(RuntimeError):
+        many[0][1].where()
+    # (a count still to come from the refused call's kernel would be taken for one of these)
+    for h, b in many[1:]:
+        assert (b.where().to_numpy() == oracle.where(h)).all()
