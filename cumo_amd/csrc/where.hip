@@ -463,6 +463,13 @@ int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uin
         report_hip_error(launched, "kernel launch");
         return CUMO_HIP_ERROR_RUNTIME;
     }
+    // (under capture nothing has been queued that could leave a count: the runtime's wait refuses at once, as it always has)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;
+    }
+    if (capturing != hipStreamCaptureStatusNone && !hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
     const auto begin = std::chrono::steady_clock::now();
     uint64_t b = 0;
     for (unsigned looks = 0; b < g.nblocks; ++looks) {

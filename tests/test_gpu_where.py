@@ -4,6 +4,7 @@ arrays, views that start inside a word, strided and reversed views, and through
 the reference's launcher symbols with a device index array and a cursor carried
 across calls (narray/gen/tmpl_bit/where_kernel.cu:91-107, mask_kernel.cu:36-54)."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -275,3 +276,49 @@ def test_an_error_left_by_an_earlier_call_is_reported_and_leaves_no_kernel_behin
     # (a count still to come from the refused call's kernel would be taken for one of these)
     for h, b in many[1:]:
         assert (b.where().to_numpy() == oracle.where(h)).all()
+
+
+def test_a_stream_under_capture_is_refused_at_once():
+    from cumo_amd import _lib
+    hip = hip_runtime()
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    h, b = masks(0)
+    took = []
+    for _ in range(3):
+        # (left alone afterwards: the runtime goes on to take a stream whose capture has failed for one under capture)
+        stream = _lib.lib.cumo_hip_stream_create()
+        _lib.lib.cumo_hip_set_stream(stream)
+        assert (b.where().to_numpy() == oracle.where(h)).all()
+        assert hip.hipStreamBeginCapture(stream, 2) == 0           # (relaxed: only the wait is refused)
+        begin = time.perf_counter()
+        with pytest.raises(RuntimeError):
+            b.where()
+        took.append(time.perf_counter() - begin)
+        graph = C.c_void_p()
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) != 0 and not graph.value
+        hip.hipGetLastError()
+        _lib.lib.cumo_hip_set_stream(None)
+    assert min(took) < 1.5e-3          # without the 2 ms that a running stream is looked at
+    assert (b.where().to_numpy() == oracle.where(h)).all()
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_masks_behind_more_work_than_the_host_looks_for(side, side_stream):
+    import cumo_amd
+    from cumo_amd import _lib
+    hip = hip_runtime()
+    if side:
+        _lib.lib.cumo_hip_set_stream(side_stream)
+    long = cumo_amd.DFloat.cast(np.linspace(0.1, 2, 1 << 24))
+    x = np.arange(100000, dtype=np.float32)
+    dx = cumo_amd.SFloat.cast(x)
+    for k in range(3):
+        h, b = masks(k)
+        begin = time.perf_counter()
+        queue_work(hip, long)
+        got = dx[b]
+        assert time.perf_counter() - begin > 2e-3                  # (it was the runtime's wait that ended)
+        queue_work(hip, long)
+        at = b.where()
+        assert (got.to_numpy() == x[h != 0]).all() and (at.to_numpy() == oracle.where(h)).all()
