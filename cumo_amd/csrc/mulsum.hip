@@ -391,8 +391,8 @@ CUMO_DEF_MULSUM(int32, int32_t, mulsum, false)
 
 // type: 0 SFloat, 1 DFloat, 2 Int32. out[r] += sum over the row of p1 * p2, for every
 // row in one launch. Returns 1 when launched, 0 when the layout is outside what the
-// kernel takes (rows not a whole number of 128-bit vectors, or not 16-byte aligned):
-// the caller then launches the rows one by one.
+// kernel takes (rows shorter than sixteen 128-bit vectors, anything not aligned to its
+// element): the caller then launches the rows one by one.
 int cumo_hip_mulsum_rows_kernel_launch(int type, int nan, const cumo_hip_mulsum_rows_t* d) {
     return mulsum_rows(type, nan != 0, d, false) ? 1 : 0;
 }

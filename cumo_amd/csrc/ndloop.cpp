@@ -1360,20 +1360,40 @@ int cumo_hip_na_mulsum(const cumo_hip_narray_t* x, const cumo_hip_narray_t* y, u
             total *= lp.n[d];
             if (d < lp.ndim - 1) launches *= lp.n[d];
         }
-        // many short contiguous runs: every row in one launch (each with a result of its own: rows that add onto
-        // one element, the whole of a view that is not one run, are walked one after the other below)
+        // many short contiguous runs: every row in one launch. Rows that all add onto one element (the whole of a view that is not one
+        // run) leave their sums in an array of their own, which is then added up: SFloat [8192,4095] of [8192,4096] 82 -> 44 us,
+        // [1000,1000] of [1000,1001] 3902 -> 8.5 (one launch per row, or from 1025 rows on an array of all the products).
         const bool skip_nan = nan != 0 && is_float(up);
         bool rows_done = false;
-        if (!rc && total_of(z) != 0 && total != 0 && lp.ndim == 2 && lp.args[2].step[1] == 0 && launches >= 2 && lp.args[2].step[0] != 0 &&
+        if (!rc && total_of(z) != 0 && total != 0 && lp.ndim == 2 && lp.args[2].step[1] == 0 && launches >= 2 &&
             (launches > 1024 || lp.n[1] * (size_t)kElmsz[up] <= (1u << 20)) && lp.args[0].step[1] == (ssize_t)kElmsz[up] &&
             lp.args[1].step[1] == (ssize_t)kElmsz[up]) {
+            const bool one = lp.args[2].step[0] == 0;
             // (a result given by the caller may be one of the operands: it is zeroed first, as it always was)
             if (!fresh) rc = cumo_hip_na_fill(z, 0.0);
+            NA sums;
+            sums.ptr = NULL;
+            const size_t rows = lp.n[0];
+            if (!rc && one) rc = cumo_hip_na_alloc(&sums, up, 1, &rows);
             if (!rc) {
-                cumo_hip_mulsum_rows_t g = {lp.n[0], lp.n[1], lp.args[0].step[0], lp.args[1].step[0], lp.args[2].step[0],
-                                            lp.args[0].ptr, lp.args[1].ptr, lp.args[2].ptr};
-                rows_done = cumo_hip::mulsum_rows(up, skip_nan, &g, fresh);
+                cumo_hip_mulsum_rows_t g = {lp.n[0], lp.n[1], lp.args[0].step[0], lp.args[1].step[0], one ? (ssize_t)kElmsz[up] : lp.args[2].step[0],
+                                            lp.args[0].ptr, lp.args[1].ptr, one ? sums.ptr + sums.offset : lp.args[2].ptr};
+                rows_done = cumo_hip::mulsum_rows(up, skip_nan, &g, fresh || one);
             }
+            if (!rc && one && rows_done) {
+                NA zs = *z;   // (one element, whatever its dimensions)
+                zs.ndim = 0;
+                if (up == CUMO_HIP_INT32) {
+                    NA sum64;   // (as below)
+                    sum64.ptr = NULL;
+                    rc = cumo_hip_na_reduce("sum", &sums, 0, 0, 0, &sum64, NULL);
+                    if (!rc) rc = cumo_hip_na_store(&zs, &sum64);
+                    free_tmp(&sum64);
+                } else {
+                    rc = cumo_hip_na_reduce("sum", &sums, 0, 0, 0, &zs, NULL);
+                }
+            }
+            free_tmp(&sums);
         } else if (!rc && fresh && total != 0 && lp.ndim >= 1 && launches == 1 && lp.args[2].step[lp.ndim - 1] == 0) {
             // one run into one new element
             char* p[3];

@@ -637,9 +637,10 @@ int cumo_hip_fused_rows_kernel_launch(int type, int mode, const cumo_hip_fused_r
  * cumo_<type>_mulsum_reduce_kernel_launch once per row from a host loop,
  * gen/tmpl/accum_binary.c:20-45): out[r] += sum_i p1[r][i] * p2[r][i] for rows of n
  * contiguous elements, row r of an operand at p + r * row_step (0 repeats the row).
- * type 0 SFloat, 1 DFloat, 2 Int32; nan skips NaN factors. Returns 1 when launched,
- * 0 when the layout is outside what the kernel takes (n not a whole number of
- * 128-bit vectors, operands or row steps not 16-byte aligned). */
+ * type 0 SFloat, 1 DFloat, 2 Int32; nan skips NaN factors. Rows add onto their elements
+ * side by side, so an out_step of 0 is not for this. Returns 1 when launched, 0 when the
+ * layout is outside what the kernel takes (rows shorter than sixteen 128-bit vectors,
+ * anything not aligned to its element). */
 typedef struct {
     uint64_t rows, n;
     ssize_t  row_step1, row_step2, out_step;

@@ -521,3 +521,36 @@ def test_mulsum_starts_from_zero_whatever_its_result_memory_held(tname, dt):
     x, y = cls.cast(hx), cls.cast(hy)
     want = (hx[:, 1:].astype(np.int64) * hy[:, :-1].astype(np.int64)).sum()
     assert (x[:, 1:].mulsum(y[:, :-1]).to_numpy() == want).all()
+
+
+@pytest.mark.parametrize("tname,dt", ALL)
+@pytest.mark.parametrize("shape", [(2, 64), (2, 63), (3, 1001), (1023, 65), (1024, 200), (1025, 200), (5000, 77), (1030, 15), (2, 300001)])
+def test_mulsum_of_all_of_a_view_whose_rows_do_not_follow_one_another(tname, dt, shape):
+    """All rows add onto one element: through their own sums where the rows' kernel takes them, whatever their number, one after
+    the other where it does not (rows shorter than sixteen vectors, rows of more than 1 MiB)."""
+    import ctypes as C
+    from cumo_amd import _lib
+    cls = cls_of(tname)
+    rng = np.random.default_rng(55)
+    rows, n = shape
+    hx, hy = (rng.integers(-8, 8, size=(rows, n + 1)).astype(dt) for _ in range(2))
+    x, y = cls.cast(hx)[:, 1:], cls.cast(hy)[:, :-1]
+    px, py = hx[:, 1:].astype(np.int64), hy[:, :-1].astype(np.int64)
+    want = (px * py).sum()
+    for _ in range(2):
+        assert x.mulsum(y).to_numpy() == want
+        got = x.mulsum(y, keepdims=True)
+        assert got.shape == (1, 1) and (got.to_numpy() == want).all()
+    # (one operand repeats its row)
+    assert x.mulsum(y[:1]).to_numpy() == (px * py[:1]).sum()
+    if dt != np.int32:
+        hx[rows - 1, n] = np.nan
+        x = cls.cast(hx)[:, 1:]
+        assert np.isnan(x.mulsum(y).to_numpy())
+        assert x.mulsum(y, nan=True).to_numpy() == want - px[-1, -1] * py[-1, -1]
+    # into a result that the caller gives
+    z = cls().fill(55)
+    x = cls.cast(np.where(np.isnan(hx), 0, hx).astype(dt))[:, 1:]
+    d, e, o = x._desc(), y._desc(), z._desc()
+    _lib.call(_lib.lib.cumo_hip_na_mulsum, C.byref(d), C.byref(e), 0, 0, 0, C.byref(o))
+    assert z.to_numpy() == want - (px[-1, -1] * py[-1, -1] if dt != np.int32 else 0)
