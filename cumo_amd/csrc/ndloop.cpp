@@ -1699,8 +1699,7 @@ int where_single_run(const LP& lp, int invert, int rtype, const char* x, ssize_t
     bool allocated = false;
     if (!rc) rc = result_1d(z, rtype, (size_t)n_hit, &allocated);
     if (!rc && n_hit != 0)
-        cumo_hip_bit_where_place_kernel_launch((CUMO_BIT_DIGIT*)in.ptr, in.bitpos, in.step[0], n, invert, counts, x, sx, (size_t)kElmsz[rtype],
-                                               z->ptr + z->offset);
+        cumo_hip::where_place((CUMO_BIT_DIGIT*)in.ptr, in.bitpos, in.step[0], n, invert, counts, n_hit, x, sx, (size_t)kElmsz[rtype], z->ptr + z->offset);
     cumo_cuda_runtime_free(reinterpret_cast<char*>(counts));
     return rc;
 }

@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kWhBlock) void where_scatter_kernel(const CUMO_BIT_
 // LDS-only barrier, so the next tile's vectors stay in flight while this one's hits are written.
 // Bound by memory: where_scatter_kernel asks for one element per hit and lane, which is a third of the cache lines' worth
 // of bytes at a hit in three: 2^25 SFloat at 33 % hits, fresh operands, 45.5 -> 35.8 us. Of sparse masks both read the lines
-// that hold a hit.
+// that hold a hit, and what a wave does for every 1024 elements here costs more than its few hits do there: where_place.
 template <int ES, bool NT>
 __global__ __launch_bounds__(kWhBlock) void mask_pack_kernel(const CUMO_BIT_DIGIT* a, uint64_t p, uint64_t n, int invert, uint64_t nchunks, uint64_t cpb,
                                                              char* out, const char* x, const uint64_t* block_sums) {
@@ -386,6 +386,38 @@ __global__ __launch_bounds__(256) void gather_flat_kernel(GatherParams g) {
 }
 
 }  // namespace
+// What cumo_hip_bit_where_place_kernel_launch does, for a mask that is known to have `hits` of them.
+// Elements of a contiguous run are packed as vectors from one hit in 40 on: 2^25 SFloat, fresh operands, at 3 % hits 37.4 us one by one,
+// 36.4 packed; at 2 % 33.7 and 35.0, at 0.1 % 25.2 and 30.7 (DFloat 2^24: 30.2 / 30.5, 26.8 / 29.6, 23.0 / 25.3).
+void where_place(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, const uint64_t* counts, uint64_t hits, const char* x, ssize_t sx,
+                 size_t elmsz, char* out) {
+    if (n == 0) return;
+    const WhGeometry g = wh_geometry(n);
+    const int contiguous = s == 1 ? 1 : 0;
+    hipStream_t st = current_stream();
+#define WH_PLACE(MODE, ES, P2, S2)                                                                                                     \
+    hipLaunchKernelGGL((where_scatter_kernel<MODE, ES, true>), dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s, \
+                       (const size_t*)nullptr, n, contiguous, invert, g.nchunks, g.cpb, out, (uint64_t)0, (size_t)(P2), (int64_t)(S2),      \
+                       (const size_t*)nullptr, counts)
+    if (x && contiguous && sx == (ssize_t)elmsz && ((uintptr_t)x & (elmsz - 1)) == 0 && hits >= n / 40) {
+        const bool nt = stream_past_caches(n * elmsz);
+#define WH_PACK(ES, NT)                                                                                                                 \
+    hipLaunchKernelGGL((mask_pack_kernel<ES, NT>), dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, n, invert, g.nchunks, g.cpb, \
+                       out, x, counts)
+        if (elmsz == 4) { if (nt) WH_PACK(4, true); else WH_PACK(4, false); }
+        else { if (nt) WH_PACK(8, true); else WH_PACK(8, false); }
+#undef WH_PACK
+    } else if (x) {
+        if (elmsz == 4) WH_PLACE(2, 4, (uintptr_t)x, sx);
+        else WH_PLACE(2, 8, (uintptr_t)x, sx);
+    } else {
+        if (elmsz == 4) WH_PLACE(0, 4, 0, 0);
+        else WH_PLACE(0, 8, 0, 0);
+    }
+#undef WH_PLACE
+    cumo_cuda_runtime_check_kernel_launch();
+}
+
 }  // namespace cumo_hip
 
 using namespace cumo_hip;
@@ -498,31 +530,7 @@ int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uin
 // otherwise out[o] = the element (elmsz 4 or 8 bytes) at x + j*sx of the o-th hit j.
 void cumo_hip_bit_where_place_kernel_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, const uint64_t* counts, const char* x,
                                             ssize_t sx, size_t elmsz, char* out) {
-    if (n == 0) return;
-    const WhGeometry g = wh_geometry(n);
-    const int contiguous = s == 1 ? 1 : 0;
-    hipStream_t st = current_stream();
-#define WH_PLACE(MODE, ES, P2, S2)                                                                                                     \
-    hipLaunchKernelGGL((where_scatter_kernel<MODE, ES, true>), dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s, \
-                       (const size_t*)nullptr, n, contiguous, invert, g.nchunks, g.cpb, out, (uint64_t)0, (size_t)(P2), (int64_t)(S2),      \
-                       (const size_t*)nullptr, counts)
-    if (x && contiguous && sx == (ssize_t)elmsz && ((uintptr_t)x & (elmsz - 1)) == 0) {
-        const bool nt = stream_past_caches(n * elmsz);
-#define WH_PACK(ES, NT)                                                                                                                 \
-    hipLaunchKernelGGL((mask_pack_kernel<ES, NT>), dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, n, invert, g.nchunks, g.cpb, \
-                       out, x, counts)
-        if (elmsz == 4) { if (nt) WH_PACK(4, true); else WH_PACK(4, false); }
-        else { if (nt) WH_PACK(8, true); else WH_PACK(8, false); }
-#undef WH_PACK
-    } else if (x) {
-        if (elmsz == 4) WH_PLACE(2, 4, (uintptr_t)x, sx);
-        else WH_PLACE(2, 8, (uintptr_t)x, sx);
-    } else {
-        if (elmsz == 4) WH_PLACE(0, 4, 0, 0);
-        else WH_PLACE(0, 8, 0, 0);
-    }
-#undef WH_PLACE
-    cumo_cuda_runtime_check_kernel_launch();
+    where_place(a, p, s, n, invert, counts, n, x, sx, elmsz, out);   // (as of a mask with many hits)
 }
 
 void cumo_hip_gather_flat_kernel_launch(const cumo_hip_gather_flat_t* d) {

@@ -255,6 +255,21 @@ def test_mask_around_whole_vectors_chunks_and_tiles(tname, dt):
                 assert got.shape == want.shape and (got == want).all(), (n, density, a, b)
 
 
+@pytest.mark.parametrize("tname,dt", [("SFloat", np.float32), ("DFloat", np.float64)])
+def test_masks_on_either_side_of_one_hit_in_forty(tname, dt):
+    """Where elements are placed one by one and where they are packed as vectors; hits spread out and all at one end."""
+    import cumo_amd
+    rng = np.random.default_rng(95)
+    for n in (39, 40, 80, 4000, 400040):
+        x = rng.integers(-1000, 1000, size=n).astype(dt)
+        dx = getattr(cumo_amd, tname).cast(x)
+        for hits in (max(n // 40 - 1, 0), n // 40, n // 40 + 1):
+            for spread in (True, False):
+                h = np.zeros(n, np.uint8)
+                h[rng.permutation(n)[:hits] if spread else np.arange(n - hits, n)] = 1
+                assert (dx[cumo_amd.Bit.cast(h)].to_numpy() == x[h != 0]).all(), (n, hits, spread)
+
+
 def masks(k):
     import cumo_amd
     rng = np.random.default_rng(700 + k)
