@@ -115,7 +115,12 @@ if not os.path.exists(LIB_PATH):
 
 lib = C.CDLL(LIB_PATH, mode=C.RTLD_GLOBAL)
 
-from . import _native  # noqa: E402  (built beside the library and linked against it)
+try:
+    from . import _native  # built beside the library and linked against it
+except ImportError as e:
+    raise ImportError(
+        "cumo_amd: the native module of the array classes (cumo_amd/_native*.so, for this interpreter) is missing or does not load: %s. "
+        "Build it with `python cumo_amd/build.py` and the interpreter that imports it." % e) from e
 
 P = C.POINTER
 _sig = {

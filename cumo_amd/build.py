@@ -1,5 +1,6 @@
 """Builds cumo_amd/libcumo_hip.so (gfx950) from cumo_amd/csrc with hipcc, and
-cumo_amd/_native.so (the object layer of the Python classes) from cumo_amd/native.
+cumo_amd/_native.<interpreter>.so (the object layer of the Python classes) from
+cumo_amd/native.
 
 One hipcc invocation per translation unit, run in parallel, then one link. The
 library is kept in-tree next to this file; nothing is installed.
@@ -20,7 +21,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libcumo_hip.so")
-NATIVE = os.path.join(HERE, "_native.so")
+# (the suffix says which interpreter it is for: one of another version does not pick it up)
+NATIVE = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 HOST_COST_TOOL = os.path.join(HERE, "bench_host_cost")
 
 ARCH = "gfx950"
@@ -120,14 +122,16 @@ def build(jobs=None, force=False, verbose=True):
 
 
 def build_native():
-    """native/arrays.cpp -> cumo_amd/_native.so, a CPython module linked against the library (host code only)."""
+    """native/arrays.cpp -> NATIVE, a CPython module linked against the library (host code only). Put in place whole: a process that
+    has the last one loaded keeps it."""
     src = os.path.join(HERE, "native", "arrays.cpp")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-I" + os.path.join(ROOT, "include"),
-           "-I" + sysconfig.get_paths()["include"], src, "-o", NATIVE, "-L" + HERE, "-lcumo_hip", "-Wl,-rpath,$ORIGIN"]
+           "-I" + sysconfig.get_paths()["include"], src, "-o", NATIVE + ".new", "-L" + HERE, "-lcumo_hip", "-Wl,-rpath,$ORIGIN"]
     p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if p.returncode:
         print(p.stdout)
         raise RuntimeError("_native: g++ failed")
+    os.replace(NATIVE + ".new", NATIVE)
 
 
 def build_host_cost_tool():

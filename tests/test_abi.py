@@ -108,3 +108,15 @@ def test_missing_library_fails_loudly(tmp_path):
     p.write_text(src)
     r = subprocess.run(["python", "-c", code % str(p)], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0 and "IMPORTERROR" in r.stdout
+
+
+def test_missing_native_module_fails_loudly(tmp_path):
+    # the library is there, the module of the array classes is not (or is another interpreter's)
+    pkg = tmp_path / "pkg"
+    pkg.mkdir()
+    (pkg / "__init__.py").write_text("")
+    (pkg / "_lib.py").write_text(open(os.path.join(ROOT, "cumo_amd", "_lib.py")).read())
+    os.symlink(os.path.join(ROOT, "cumo_amd", "libcumo_hip.so"), str(pkg / "libcumo_hip.so"))
+    (pkg / "_native.cpython-20-x86_64-linux-gnu.so").write_bytes(b"")
+    r = subprocess.run(["python", "-c", "import pkg._lib"], cwd=str(tmp_path), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode != 0 and "ImportError" in r.stdout and "cumo_amd/build.py" in r.stdout.splitlines()[-1]

@@ -1,4 +1,4 @@
-"""The native object layer (cumo_amd/_native.so): the same arrays, bit for bit, as the general Python methods give, for every
+"""The native object layer (cumo_amd/native/arrays.cpp): the same arrays, bit for bit, as the general Python methods give, for every
 form it takes, and what it leaves to them."""
 import copy
 import gc
