@@ -591,3 +591,88 @@ def test_column_sums_lose_no_more_than_short_chains_do(tname, dt, shape, lanes):
         # (four rows to a merge; 6 for the rounding of the squares, of a merge's products and of the division)
         m = n / lanes / 4
         assert off(d.var(axis=0), h.astype(np.float64).var(axis=0, ddof=1)) <= u / 3 ** 0.5 * (0.63 * m ** (1 / 3) / lanes + 6) ** 0.5
+
+
+COLUMN_SPLITS = [(7, 40), (9, 17), (1024, 18), (1025, 19), (2047, 516), (2049, 1029), (5000, 64), (40003, 257), (9, 262149)]
+ROW_VIEWS = [lambda a: a, lambda a: a[1::2], lambda a: a[::-1], lambda a: a[:, 1:]]
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("shape", COLUMN_SPLITS)
+def test_special_values_down_columns_over_every_split(tname, dt, shape):
+    """NaN, infinities and columns of nothing but NaN through each way the column kernel splits its work, whole arrays and views whose
+    rows are every other one, run backwards or start off a vector. Finite values are multiples of 1/4: sums are exact."""
+    rng = np.random.default_rng(94)
+    full = (rng.integers(-8, 9, size=shape) / 4.0).astype(dt)
+    col = np.arange(shape[1])
+    row = rng.integers(0, shape[0], size=shape[1])
+    for k, v in ((0, np.nan), (2, np.inf), (3, -np.inf)):
+        full[row[col % 7 == k], col[col % 7 == k]] = v
+    full[:, col % 7 == 1] = np.nan
+    both = col[col % 7 == 4]                       # an infinity of either sign
+    full[row[both], both] = np.inf
+    full[(row[both] + 3) % shape[0], both] = -np.inf
+    dfull = cls_of(tname).cast(full)
+    for view in ROW_VIEWS:
+        h, d = view(full), view(dfull)
+        n = h.shape[0]
+        f64 = h.astype(np.float64)
+        some = ~np.isnan(h).all(axis=0)
+        with np.errstate(all="ignore"):
+            want = f64.sum(axis=0).astype(dt)
+            assert_bits_equal(d.sum(axis=0).to_numpy() + dt(0), want + dt(0), "sum")
+            assert_bits_equal(d.mean(axis=0).to_numpy() + dt(0), want / dt(n) + dt(0), "mean")
+            want = np.nansum(f64, axis=0).astype(dt)
+            left = (~np.isnan(h)).sum(axis=0)
+            assert_bits_equal(d.sum(axis=0, nan=True).to_numpy() + dt(0), want + dt(0), "sum nan")
+            assert_bits_equal(d.mean(axis=0, nan=True).to_numpy() + dt(0), want / left.astype(dt) + dt(0), "mean nan")
+            assert_reduction_close(d.rms(axis=0).to_numpy(), np.sqrt((f64 * f64).mean(axis=0)).astype(dt), n, None, "rms")
+            assert_reduction_close(d.rms(axis=0, nan=True).to_numpy(), np.sqrt(np.nansum(f64 * f64, axis=0) / left).astype(dt), n, None, "rms nan")
+            # (an infinity leaves no deviation; a column of nothing but NaN answers 0 where NaN is skipped, as Numo does)
+            want = f64.var(axis=0, ddof=1)
+            assert_reduction_close(d.var(axis=0).to_numpy(), want.astype(dt), n, np.abs(want) + 1e-30, "var")
+            kept = np.where(np.isnan(f64), 0, f64 - np.nansum(f64, axis=0) / left)
+            want = np.where(some, (kept * kept).sum(axis=0) / (left - 1), 0)
+            assert_reduction_close(d.var(axis=0, nan=True).to_numpy(), want.astype(dt), n, np.abs(want) + 1e-30, "var nan")
+        # NaN loses to everything, a column of nothing else answers its first; with nan: the first NaN wins
+        filled_lo, filled_hi = np.where(np.isnan(h), -np.inf, h), np.where(np.isnan(h), np.inf, h)
+        nan_free_max = np.where(some, filled_lo.max(axis=0), np.nan).astype(dt)
+        nan_free_min = np.where(some, filled_hi.min(axis=0), np.nan).astype(dt)
+        assert_bits_equal(d.max(axis=0).to_numpy() + dt(0), nan_free_max + dt(0), "max")
+        lo, hi = d.minmax(axis=0)
+        assert_bits_equal(lo.to_numpy() + dt(0), nan_free_min + dt(0), "minmax lo")
+        assert_bits_equal(hi.to_numpy() + dt(0), nan_free_max + dt(0), "minmax hi")
+        assert_bits_equal(d.max(axis=0, nan=True).to_numpy() + dt(0), h.max(axis=0) + dt(0), "max nan")
+        lo, hi = d.minmax(axis=0, nan=True)
+        assert_bits_equal(lo.to_numpy() + dt(0), h.min(axis=0) + dt(0), "minmax nan lo")
+        assert_bits_equal(hi.to_numpy() + dt(0), h.max(axis=0) + dt(0), "minmax nan hi")
+        first = np.where(some, (h == nan_free_max).argmax(axis=0), 0)
+        assert (d.argmax(axis=0).to_numpy() == first).all()
+        assert (d.argmax(axis=0, nan=True).to_numpy() == h.argmax(axis=0)).all()
+        first = np.where(some, (h == nan_free_min).argmax(axis=0), 0)
+        assert (d.argmin(axis=0).to_numpy() == first).all()
+        assert (d.argmin(axis=0, nan=True).to_numpy() == h.argmin(axis=0)).all()
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("shape", COLUMN_SPLITS)
+def test_products_and_compensated_sums_down_columns_over_every_split(tname, dt, shape):
+    rng = np.random.default_rng(95)
+    # powers of two whose partial products stay in the range: exact whatever the order
+    h = (rng.integers(0, 2, size=shape) * 2 - 1).astype(dt)
+    for _ in range(20):
+        h[rng.integers(0, shape[0], size=shape[1]), np.arange(shape[1])] *= dt(2)
+    h[0, ::5] = np.nan
+    d = cls_of(tname).cast(h)
+    assert_bits_equal(d.prod(axis=0).to_numpy(), h.prod(axis=0), "prod")
+    assert_bits_equal(d.prod(axis=0, nan=True).to_numpy(), np.nanprod(h, axis=0).astype(dt), "prod nan")
+    if dt == np.float64:
+        # whole numbers and large ones that cancel: the sum is the whole numbers' own, which a plain sum loses
+        small = rng.integers(-8, 9, size=shape).astype(np.float64)
+        big = np.ldexp(1.0, rng.integers(60, 70, size=shape[1]))
+        h = small.copy()
+        cols = np.arange(shape[1])
+        r = rng.permuted(np.tile(np.arange(min(shape[0], 64)), (shape[1], 1)), axis=1)[:, :2]
+        h[r[:, 0], cols], h[r[:, 1], cols] = big, -big
+        small[r[:, 0], cols] = small[r[:, 1], cols] = 0
+        assert_bits_equal(cls_of(tname).cast(h).kahan_sum(axis=0).to_numpy() + 0.0, small.sum(axis=0) + 0.0, "kahan_sum")
