@@ -245,6 +245,9 @@ class NArray(_native.View):
     def __copy__(self):
         return self._view(self.shape, self._strides, self._offset)
 
+    def __deepcopy__(self, memo):
+        return self.copy()
+
     def _desc(self):
         """This view as the library's cumo_hip_narray_t."""
         d = NArrayDesc()

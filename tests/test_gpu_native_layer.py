@@ -118,3 +118,17 @@ def test_threads_call_and_release_at_once():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+@pytest.mark.parametrize("cls", [SFloat, DFloat, Int32, cumo_amd.Int64, cumo_amd.UInt64, Bit])
+def test_a_deep_copy_has_memory_of_its_own(cls):
+    h = (np.arange(60).reshape(5, 12) % 2).astype(cls.np_dtype or np.uint8)
+    x = cls.cast(h)
+    for v, want in ((x, h), (x.transpose(), h.T), (x[1:, 3:9], h[1:, 3:9])):
+        y = copy.deepcopy({"a": [v, v]})["a"]
+        assert y[0] is y[1] and type(y[0]) is cls and y[0]._ptr() != v._ptr()
+        assert (y[0].to_numpy() == want).all()
+        _lib.call(_lib.lib.cumo_hip_memset, y[0]._buf.ptr, 0xff, y[0]._buf.nbytes)
+        assert (v.to_numpy() == want).all()
+        del y
+    assert (x.to_numpy() == h).all()
