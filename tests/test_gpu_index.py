@@ -420,7 +420,8 @@ def test_index_arrays_of_every_size_reach_the_device(n):
 
 
 def test_many_index_arrays_in_a_row_and_from_two_threads():
-    # more of them in flight than there are slots, each with positions of its own in host memory that is then overwritten
+    # more of them in a row than there are slots, each with positions of its own in host memory that is then overwritten (slots still to
+    # be read: the tests with queued work below)
     import threading
     a = np.arange(4000, dtype=np.float64)
     bad = []
