@@ -17,6 +17,9 @@ void report_error(int kind, int hip_status, const char* message);
 void report_hip_error(hipError_t status, const char* what);
 
 hipStream_t current_stream();
+// whether the current stream is being captured (taken for so when the runtime cannot say): a replay would use memory that has gone back
+// to the pool by then
+bool stream_under_capture();
 
 // A number in [0, kStreamSlots) that belongs to this stream until it is destroyed
 // through cumo_hip_stream_destroy, or -1 when every number is taken. Kernels that

@@ -1362,13 +1362,14 @@ int cumo_hip_na_mulsum(const cumo_hip_narray_t* x, const cumo_hip_narray_t* y, u
         }
         // many short contiguous runs: every row in one launch. Rows that all add onto one element (the whole of a view that is not one
         // run) leave their sums in an array of their own, which is then added up: SFloat [8192,4095] of [8192,4096] 82 -> 44 us,
-        // [1000,1000] of [1000,1001] 3902 -> 8.5 (one launch per row, or from 1025 rows on an array of all the products).
+        // [1000,1000] of [1000,1001] 3902 -> 8.5 (one launch per row, or from 1025 rows on an array of all the products). Under capture, where a
+        // replay must not depend on an array that has been given back, up to 1024 rows are launched one by one all the same.
         const bool skip_nan = nan != 0 && is_float(up);
         bool rows_done = false;
+        const bool one = lp.ndim == 2 && lp.args[2].step[0] == 0;
         if (!rc && total_of(z) != 0 && total != 0 && lp.ndim == 2 && lp.args[2].step[1] == 0 && launches >= 2 &&
             (launches > 1024 || lp.n[1] * (size_t)kElmsz[up] <= (1u << 20)) && lp.args[0].step[1] == (ssize_t)kElmsz[up] &&
-            lp.args[1].step[1] == (ssize_t)kElmsz[up]) {
-            const bool one = lp.args[2].step[0] == 0;
+            lp.args[1].step[1] == (ssize_t)kElmsz[up] && !(one && launches <= 1024 && cumo_hip::stream_under_capture())) {
             // (a result given by the caller may be one of the operands: it is zeroed first, as it always was)
             if (!fresh) rc = cumo_hip_na_fill(z, 0.0);
             NA sums;

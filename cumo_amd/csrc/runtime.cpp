@@ -47,6 +47,15 @@ void report_hip_error(hipError_t status, const char* what) {
 
 hipStream_t current_stream() { return t_stream; }
 
+bool stream_under_capture() {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(t_stream, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return capturing != hipStreamCaptureStatusNone;
+}
+
 bool force_wide_indices() {
     static const bool on = [] {
         const char* e = std::getenv("CUMO_HIP_FORCE_WIDE");

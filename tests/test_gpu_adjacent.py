@@ -554,3 +554,35 @@ def test_mulsum_of_all_of_a_view_whose_rows_do_not_follow_one_another(tname, dt,
     d, e, o = x._desc(), y._desc(), z._desc()
     _lib.call(_lib.lib.cumo_hip_na_mulsum, C.byref(d), C.byref(e), 0, 0, 0, C.byref(o))
     assert z.to_numpy() == want - (px[-1, -1] * py[-1, -1] if dt != np.int32 else 0)
+
+
+def test_mulsum_of_such_a_view_can_be_replayed():
+    """Captured into a given result and replayed, with the pool's memory in use in between: nothing of it is part of the graph."""
+    import ctypes as C
+    import cumo_amd
+    from cumo_amd import _lib
+    from test_gpu_index import hip_runtime
+    hip = hip_runtime()
+    rng = np.random.default_rng(56)
+    hx, hy = (rng.integers(-8, 8, size=(50, 201)).astype(np.float32) for _ in range(2))
+    x, y, z = cumo_amd.SFloat.cast(hx), cumo_amd.SFloat.cast(hy), cumo_amd.SFloat().fill(55)
+    stream = C.c_void_p(_lib.lib.cumo_hip_stream_create())
+    graph, ready = C.c_void_p(), C.c_void_p()
+    d, e, o = x[:, 1:]._desc(), y[:, :-1]._desc(), z._desc()
+    cumo_amd.synchronize()
+    _lib.lib.cumo_hip_set_stream(stream)
+    try:
+        assert hip.hipStreamBeginCapture(stream, 2) == 0
+        _lib.call(_lib.lib.cumo_hip_na_mulsum, C.byref(d), C.byref(e), 0, 0, 0, C.byref(o))
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(ready), graph, None, None, C.c_size_t(0)) == 0
+        for k in range(4):
+            x.fill(float(k))
+            dirt = [cumo_amd.SFloat(n).fill(float("nan")) for n in (1, 50, 201, 10000)]
+            assert hip.hipGraphLaunch(ready, stream) == 0
+            [a.fill(1e30) for a in dirt]
+            cumo_amd.synchronize()
+            assert z.to_numpy() == k * hy[:, :-1].astype(np.int64).sum()
+            del dirt
+    finally:
+        _lib.lib.cumo_hip_set_stream(None)
