@@ -130,27 +130,9 @@ __device__ __forceinline__ void raw_load(const char* p, T (&out)[VEC]) {
     for (int j = 0; j < VEC; ++j) out[j] = u.t[j];
 }
 
-// A 128-bit store for tiles that are written once, far apart from one another, by an operation
-// too large for the caches: non-temporal AND written through at device scope (`nt sc1`), so the
-// second-level cache does not collect the partly written lines of many rows before it lets them
-// go. Measured on the transposed 8192 x 4096 SFloat copy, every launch on fresh operands: 47.2 us
-// with `nt` alone, 46.3 us with `nt sc1` (plain stores: 50.9 us); a contiguous stream gains
-// nothing from it (43.5 us either way for 128 MiB -> 128 MiB). No builtin spells the pair.
-template <class T, int VEC>
-__device__ __forceinline__ void raw_store_scattered_stream(char* p, const T (&in)[VEC]) {
-    static_assert(sizeof(T) * VEC == 16, "one 128-bit store");
-    union U {
-        T t[VEC];
-        u32x4 q;
-        __device__ U() {}
-    } u;
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) u.t[j] = in[j];
-    asm volatile("global_store_dwordx4 %0, %1, off nt sc1" ::"v"(p), "v"(u.q) : "memory");
-}
-
+// `pieces`: the lanes' vectors together are whole 64-byte pieces (see store_vector)
 template <class T, int VEC, bool NT>
-__device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC]) {
+__device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC], bool pieces = false) {
     constexpr int BYTES = (int)sizeof(T) * VEC;
     union U {
         T t[VEC];
@@ -164,9 +146,8 @@ __device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC]) {
     if constexpr (BYTES % 16 == 0) {
 #pragma unroll
         for (int k = 0; k < BYTES / 16; ++k) {
-            u32x4* dst = reinterpret_cast<u32x4*>(p) + k;
-            if (NT) __builtin_nontemporal_store(u.q[k], dst);
-            else *dst = u.q[k];
+            // (a lane that stores several vectors leaves gaps between them)
+            store_vector<NT>(reinterpret_cast<u32x4*>(p) + k, u.q[k], pieces && BYTES == 16);
         }
     } else if constexpr (BYTES == 8) {
         u32x2* dst = reinterpret_cast<u32x2*>(p);
@@ -549,7 +530,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_flat_period_kernel(const char* __
         ok = ok && okj;
     }
     if (cnt == VEC && (!Op::CHECKED || ok)) {
-        raw_store<R, VEC, NT>(pz + (uint64_t)i * sizeof(R), zv);
+        raw_store<R, VEC, NT>(pz + (uint64_t)i * sizeof(R), zv, store_pieces(pz));
         return;
     }
     // the run's last, ragged vector, or a vector with a rejected element: one by one
@@ -617,7 +598,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_flat_row_kernel(const char* __res
             }
         }
         if (ok) {
-            raw_store<R, VEC, NT>(pz + (uint64_t)i * sizeof(R), zv);
+            raw_store<R, VEC, NT>(pz + (uint64_t)i * sizeof(R), zv, store_pieces(pz));
             continue;
         }
         // the run's last, ragged vector, or a vector with a rejected element: one by one
@@ -711,7 +692,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_flat_addressed_kernel(EwAddressed
         ok = ok && (okv[j] || (uint32_t)j >= cnt);
     }
     if (cnt == VEC && (!Op::CHECKED || ok)) {
-        raw_store<R, VEC, NT>(p.out + (uint64_t)i * sizeof(R), zv);
+        raw_store<R, VEC, NT>(p.out + (uint64_t)i * sizeof(R), zv, store_pieces(p.out));
         return;
     }
     // the run's last, ragged vector, or a vector with a rejected element: one by one
@@ -847,7 +828,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_flat_kernel(const char* __restric
     for (int u = 0; u < UNR; ++u) {
         const uint64_t i = i0 + (uint64_t)u * (kEwBlock * VEC);
         if (whole[u] && (!Op::CHECKED || ok[u])) {
-            raw_store<R, VEC, NT>(pz + i * sizeof(R), zv[u]);
+            raw_store<R, VEC, NT>(pz + i * sizeof(R), zv[u], store_pieces(pz));
             continue;
         }
         if (i >= n) continue;
@@ -1222,7 +1203,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_rows2_kernel(EwR2Params p, Op op,
         char* o = p.ptr[2] + roff[2] + (uint64_t)cv * (VEC * sizeof(R));
         constexpr uint32_t full = (1u << VEC) - 1u;
         if (!Op::CHECKED || okmask == full) {
-            raw_store<R, VEC, (NTM & 4) != 0>(o, zv);
+            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, store_pieces(p.ptr[2], p.rstep[2], p.ostep[2]));
         } else {
             if (p.flag) *p.flag = 1;
 #pragma unroll
@@ -1309,7 +1290,7 @@ __device__ __forceinline__ void ew_rows2_lean_body(const EwR2LeanParams& p, Op o
         char* o = p.ptr[2] + (int64_t)row[u] * p.rstep[2] + (uint64_t)cv * (VEC * sizeof(R));
         constexpr uint32_t full = (1u << VEC) - 1u;
         if (!Op::CHECKED || okmask == full) {
-            raw_store<R, VEC, (NTM & 4) != 0>(o, zv);
+            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, store_pieces(p.ptr[2], p.rstep[2]));
         } else {
             if (p.flag) *p.flag = 1;
 #pragma unroll
@@ -1631,8 +1612,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
 #pragma unroll
                     for (int q = 0; q < V; ++q) zr[q] = tile_r[lg][fv * V + q];
                     char* dstr = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
-                    if constexpr (NT && sizeof(R) * V == 16) raw_store_scattered_stream<R, V>(dstr, zr);
-                    else raw_store<R, V, NT>(dstr, zr);
+                    raw_store<R, V, NT>(dstr, zr, store_pieces(p.ptr[2] + off[2], p.gstep[2]));
                     continue;
                 }
                 A x[V];
@@ -1669,8 +1649,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
                 }
                 char* dst = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
                 if (!Op::CHECKED || ok) {
-                    if constexpr (NT && sizeof(R) * V == 16) raw_store_scattered_stream<R, V>(dst, z);
-                    else raw_store<R, V, NT>(dst, z);
+                    raw_store<R, V, NT>(dst, z, store_pieces(p.ptr[2] + off[2], p.gstep[2]));
                 } else {
                     // some element was rejected: store the others one by one
                     if (p.flag) *p.flag = 1;

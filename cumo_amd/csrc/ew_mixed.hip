@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kMxBlock) void ew_mixed_flat_kernel(const char* __r
             TR zv[kMxVec];
 #pragma unroll
             for (int j = 0; j < kMxVec; ++j) zv[j] = mixed_apply<OP, TR>((TR)xv[u][j], (TR)yv[u][j]);
-            raw_store<TR, kMxVec, NT>(pz + i * sizeof(TR), zv);
+            raw_store<TR, kMxVec, NT>(pz + i * sizeof(TR), zv, store_pieces(pz));
         } else if (i < n) {
             // the run's last elements, fewer than a vector
             for (uint64_t k = i; k < n; ++k)
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kMxBlock) void ew_mixed_scalar_kernel(const char* _
 #pragma unroll
             for (int j = 0; j < kMxVec; ++j)
                 zv[j] = LEFT ? mixed_apply<OP, double>(sv, (double)xv[u][j]) : mixed_apply<OP, double>((double)xv[u][j], sv);
-            raw_store<double, kMxVec, NT>(pz + i * sizeof(double), zv);
+            raw_store<double, kMxVec, NT>(pz + i * sizeof(double), zv, store_pieces(pz));
         } else if (i < n) {
             for (uint64_t k = i; k < n; ++k) {
                 const double x = (double)reinterpret_cast<const int32_t*>(px)[k];

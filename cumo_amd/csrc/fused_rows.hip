@@ -153,9 +153,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
         auto put = [&](int k) {
             const uint64_t col = ((uint64_t)k * TPR + lane_r) * V;
             if (cnt[k] == V) {
-                u4* st = reinterpret_cast<u4*>(dst + col * sizeof(T));
-                if (NT) __builtin_nontemporal_store(x[k].q, st);
-                else *st = x[k].q;
+                store_vector<NT>(reinterpret_cast<u4*>(dst + col * sizeof(T)), x[k].q, store_pieces(p.out, p.out_row_step));
             } else {
 #pragma unroll
                 for (int j = 0; j < V; ++j)

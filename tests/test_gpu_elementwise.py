@@ -874,3 +874,29 @@ def test_matrix_with_one_row_repeated(tname, dt, shape):
         hr[0, shape[-1] - 1] = 0
         with pytest.raises(ZeroDivisionError):
             (x / cls.cast(hr)[:, :shape[-1]]).to_numpy()
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("rows,step,first,width", [
+    (37, 64, 0, 64), (37, 64, 16, 32), (37, 64, 4, 36), (37, 68, 16, 36), (37, 65, 1, 60), (300, 1040, 16, 1024), (300, 1040, 8, 1000),
+    (3300, 4160, 16, 4128), (3300, 4160, 4, 4128),
+])
+def test_results_on_and_off_whole_pieces_of_memory(tname, dt, rows, step, first, width):
+    # windows whose rows start on 64-byte pieces of memory and beside them, below and above the size from which
+    # loads are non-temporal; through the flat, row and transposed kernels; what lies around the window stays as it was
+    rng = np.random.default_rng(rows + step + first)
+    cls = cls_of(tname)
+    h = rng.standard_normal((rows, width)).astype(dt)
+    x = cls.cast(h)
+    for source, want in ((x, h), (cls.cast(np.ascontiguousarray(h.T)).transpose(), h)):
+        z = cls(rows, step).fill(5)
+        z[:, first:first + width].store(source)
+        whole = np.full((rows, step), 5, dtype=dt)
+        whole[:, first:first + width] = want
+        assert_bits_equal(z.to_numpy(), whole)
+    flat = cls(rows * step).fill(5)
+    flat[first:first + rows * width // 2].store(x.reshape(rows * width)[:rows * width // 2])
+    whole = np.full(rows * step, 5, dtype=dt)
+    whole[first:first + rows * width // 2] = h.reshape(-1)[:rows * width // 2]
+    assert_bits_equal(flat.to_numpy(), whole)
+    assert_bits_equal((x.transpose() * 3.0).to_numpy(), oracle.binary("mul", h.T, dt(3.0)))
