@@ -355,22 +355,6 @@ __device__ __forceinline__ bool chain_peek(const uint64_t* slot, T& value, uint3
     return all;
 }
 
-// (x, has) of the 64 lanes folded in a fixed shape; every lane ends with the result
-template <class T, class Op>
-__device__ __forceinline__ void chain_wave_fold(T& x, bool& has) {
-    const unsigned lane = threadIdx.x & 63u;
-#pragma unroll
-    for (unsigned m = 1; m < 64; m <<= 1) {
-        const T o = scan_shfl_xor(x, m);
-        const bool oh = __shfl_xor((int)has, (int)m) != 0;
-        if (oh) {
-            if (!has) x = o;
-            else x = (lane & m) ? Op::apply(o, x) : Op::apply(x, o);
-            has = true;
-        }
-    }
-}
-
 template <class T, class Op>
 __device__ __forceinline__ void chain_join(T& a, bool& a_has, T b, bool b_has) {  // a = a (+) b, a the earlier
     if (b_has) {
@@ -379,20 +363,55 @@ __device__ __forceinline__ void chain_join(T& a, bool& a_has, T b, bool b_has) {
     }
 }
 
+// v of another lane by data-parallel primitive (no trip through the LDS unit that shuffles take); lanes without a source keep their own
+template <int CTRL, class T>
+__device__ __forceinline__ T scan_dpp(T v) {
+    constexpr int W = (int)(sizeof(T) / 4);
+    union { T t; int w[W]; } a, b;
+    a.t = v;
+#pragma unroll
+    for (int i = 0; i < W; ++i) b.w[i] = __builtin_amdgcn_update_dpp(a.w[i], a.w[i], CTRL, 0xf, 0xf, false);
+    return b.t;
+}
+
+// v of one lane, the same lane for the whole wave
 template <class T>
-__device__ __forceinline__ T scan_shfl_idx(T v, int src) {
-    if constexpr (sizeof(T) == 8) {
-        union { T t; uint32_t w[2]; } a, b;
-        a.t = v;
-        b.w[0] = __shfl(a.w[0], src);
-        b.w[1] = __shfl(a.w[1], src);
-        return b.t;
-    } else {
-        union { T t; uint32_t w; } a, b;
-        a.t = v;
-        b.w = __shfl(a.w, src);
-        return b.t;
+__device__ __forceinline__ T scan_read_lane(T v, uint32_t lane) {
+    constexpr int W = (int)(sizeof(T) / 4);
+    union { T t; int w[W]; } a;
+    a.t = v;
+#pragma unroll
+    for (int i = 0; i < W; ++i) a.w[i] = __builtin_amdgcn_readlane(a.w[i], (int)lane);
+    return a.t;
+}
+
+// Inclusive scan of K values of every lane across the wave, side by side: inside quarters of 16 lanes, then the
+// quarters' totals from lane 15 of the first and third, then the half's from lane 31.
+template <class T, class Op, int K>
+__device__ __forceinline__ void scan_across_wave(T (&x)[K]) {
+    const unsigned lane = threadIdx.x & 63u;
+#define CUMO_SCAN_STEP(CTRL, COND)                        \
+    _Pragma("unroll") for (int k = 0; k < K; ++k) {       \
+        const T o = scan_dpp<CTRL>(x[k]);                 \
+        x[k] = (COND) ? Op::apply(o, x[k]) : x[k];        \
     }
+    CUMO_SCAN_STEP(0x111, (lane & 15u) >= 1)   // row_shr:1
+    CUMO_SCAN_STEP(0x112, (lane & 15u) >= 2)   // row_shr:2
+    CUMO_SCAN_STEP(0x114, (lane & 15u) >= 4)   // row_shr:4
+    CUMO_SCAN_STEP(0x118, (lane & 15u) >= 8)   // row_shr:8
+    CUMO_SCAN_STEP(0x142, (lane & 16u) != 0)   // row_bcast:15
+    CUMO_SCAN_STEP(0x143, lane >= 32)          // row_bcast:31
+#undef CUMO_SCAN_STEP
+}
+
+// x of the first `count` lanes folded in a fixed shape, the same for the whole wave; has: whether there is one
+template <class T, class Op>
+__device__ __forceinline__ void chain_fold_lanes(T& x, bool& has, uint32_t count) {
+    has = count > 0;
+    if (!has) return;
+    T k[1] = {x};
+    scan_across_wave<T, Op, 1>(k);
+    x = scan_read_lane(k[0], count - 1);
 }
 
 // What a tile needs from the tiles before it, through the published totals (wave 0 of the
@@ -405,6 +424,7 @@ template <class T, class Op>
 __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t t, T total, bool total_has, T& prefix, bool& prefix_has) {
     constexpr int W = ScanChain<T>::W;
     const unsigned lane = threadIdx.x & 63u;
+    t = (uint32_t)__builtin_amdgcn_readfirstlane(t);
     const uint32_t pos = t & 63u, g = t >> 6, gpos = g & 63u, sg = g >> 6;
     if (lane == 0) chain_publish<T>(c.tile + (size_t)t * W, total, c.flag);
     T x = T(), y = T(), z = T();
@@ -432,7 +452,7 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
     // otherwise every group would wait for the group before it, one memory round trip each.
     const bool closes_group = pos == 63u, closes_super = closes_group && gpos == 63u;
     bool group_out = !closes_group, super_out = !closes_super;
-    bool xh = has_x, yh = has_y, zh = has_z;
+    bool xh = false, yh = false, zh = false;
     bool x_folded = false, y_folded = false;
     T gt = T();
     bool gt_has = false;
@@ -441,7 +461,7 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
         if (need_y) need_y = !chain_peek<T>(py, y, c.flag);
         if (need_z) need_z = !chain_peek<T>(pz, z, c.flag);
         if (!x_folded && __ballot(need_x) == 0) {
-            chain_wave_fold<T, Op>(x, xh);
+            chain_fold_lanes<T, Op>(x, xh, pos);
             x_folded = true;
             if (!group_out) {
                 gt = x;
@@ -452,7 +472,7 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
             }
         }
         if (!y_folded && x_folded && __ballot(need_y) == 0) {
-            chain_wave_fold<T, Op>(y, yh);
+            chain_fold_lanes<T, Op>(y, yh, gpos);
             y_folded = true;
             if (!super_out) {
                 T st = y;
@@ -469,9 +489,9 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
         }
         __builtin_amdgcn_s_sleep(16);
     }
-    if (!x_folded) chain_wave_fold<T, Op>(x, xh);  // (only after giving up)
-    if (!y_folded) chain_wave_fold<T, Op>(y, yh);
-    chain_wave_fold<T, Op>(z, zh);
+    if (!x_folded) chain_fold_lanes<T, Op>(x, xh, pos);  // (only after giving up)
+    if (!y_folded) chain_fold_lanes<T, Op>(y, yh, gpos);
+    chain_fold_lanes<T, Op>(z, zh, sg);
     chain_join<T, Op>(z, zh, y, yh);
     chain_join<T, Op>(z, zh, x, xh);
     prefix = z;
@@ -484,11 +504,13 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
 // four waves meet once, in LDS, and what is left to add after the look-back is one value per
 // wave, so only the tile's elements stay in registers while the block waits. The ragged last
 // tile of a run goes sub-tile by sub-tile through the block-wide scan, reading its input twice.
-// Measured on 2^26 SFloat (fresh operands): 116 us with 64 KiB tiles, against 139 us with
-// 32 KiB tiles (twice the tickets and look-backs, each a trip through memory with nothing else
-// for the block to do), 155 us for the three launches, and 92 us for the same kernel with
-// neither ticket nor look-back. Blocks that keep a second tile's loads in flight while they
-// wait were slower still (170 us): the registers that takes cost more blocks than it wins.
+// Bound by what a block waits for with nothing in flight: its ticket and the look-back. The
+// steps across a wave go by data-parallel primitives: shuffles put 16 rows times six steps through
+// the LDS unit (2^24 DFloat 75 -> 63 us, 2^22 24.1 -> 20.4, 2^26 SFloat 111 -> 109; with 128 KiB
+// tiles 57.8, 16.4, 102). The three launches take 155 us for 2^26 SFloat. Slower, measured: 32 KiB
+// tiles; persistent blocks that stage the next tile into LDS with a wave of their own for tickets
+// and look-backs (2^24 DFloat 67 us with 64 KiB tiles, 89 with 32, 141 with 16: the tickets; with
+// tiles dealt out by block index, which could wait for a block that is not running, 63 with 32).
 template <class T>
 struct ChainVec {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
@@ -534,43 +556,46 @@ __device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first
 // The tile in v (already loaded) scanned by itself: afterwards every element holds the running
 // value from the start of its wave's quarter, `total` is the tile's total and `wave_pre` the
 // total of the waves before this one (for wave 0: nothing). One barrier, met by every thread.
-template <class T, class Op, int R, int NW = kScanBlock / 64>
-__device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
+// The rows of one wave in v (already loaded) scanned by themselves; returns their total. Eight rows at a time: with the
+// lane totals of sixteen rows of doubles beside the tile 128 registers do not hold it.
+template <class T, class Op, int R>
+__device__ __forceinline__ T chain_scan_wave(ChainVec<T> (&v)[R]) {
     constexpr int V = ChainVec<T>::V;
+    constexpr int K = R < 8 ? R : 8;
+    static_assert(R % K == 0, "rows in whole groups");
     const unsigned lane = threadIdx.x & 63u;
-    const int w = threadIdx.x >> 6;
-    T inc[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-#pragma unroll
-        for (int e = 1; e < V; ++e) v[r].e[e] = Op::apply(v[r].e[e - 1], v[r].e[e]);
-        inc[r] = v[r].e[V - 1];
-    }
-    // the lane totals of each row, scanned across the wave (the rows are independent)
-#pragma unroll
-    for (unsigned d = 1; d < 64; d <<= 1) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const T o = scan_shfl_up(inc[r], d);
-            if (lane >= d) inc[r] = Op::apply(o, inc[r]);
-        }
-    }
-    // every element takes on what precedes its vector inside the wave's quarter
     T run = T();  // the rows so far
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const T ex = scan_shfl_up(inc[r], 1);       // the lanes before, in this row
-        const T row = scan_shfl_idx(inc[r], 63);    // the whole row
-        T before = ex;
-        if (r > 0) before = lane > 0 ? Op::apply(run, ex) : run;
-        if (r > 0 || lane > 0) {
+    for (int r0 = 0; r0 < R; r0 += K) {
+        T inc[K];
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[r].e[e] = Op::apply(before, v[r].e[e]);
+        for (int k = 0; k < K; ++k) {
+#pragma unroll
+            for (int e = 1; e < V; ++e) v[r0 + k].e[e] = Op::apply(v[r0 + k].e[e - 1], v[r0 + k].e[e]);
+            inc[k] = v[r0 + k].e[V - 1];
         }
-        run = r == 0 ? row : Op::apply(run, row);
+        scan_across_wave<T, Op, K>(inc);   // the lane totals of each row (the rows are independent)
+        // every element takes on what precedes its vector inside the wave's part
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const T ex = scan_dpp<0x138>(inc[k]);        // the lanes before, in this row (wave_shr:1)
+            const T row = scan_read_lane(inc[k], 63);    // the whole row
+            T before = ex;
+            if (r0 + k > 0) before = lane > 0 ? Op::apply(run, ex) : run;
+            if (r0 + k > 0 || lane > 0) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[r0 + k].e[e] = Op::apply(before, v[r0 + k].e[e]);
+            }
+            run = r0 + k == 0 ? row : Op::apply(run, row);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
-    if (lane == 0) s_wave_tot[w] = run;
-    __syncthreads();
+    return run;
+}
+
+// the total of a tile from its waves' totals, and what precedes wave w in it (for wave 0: nothing)
+template <class T, class Op, int NW>
+__device__ __forceinline__ void chain_fold_waves(const T* s_wave_tot, int w, T& total, T& wave_pre) {
     total = s_wave_tot[0];
     wave_pre = T();
 #pragma unroll
@@ -578,6 +603,15 @@ __device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_t
         if (j == w) wave_pre = total;
         total = Op::apply(total, s_wave_tot[j]);
     }
+}
+
+template <class T, class Op, int R, int NW = kScanBlock / 64>
+__device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
+    const int w = threadIdx.x >> 6;
+    const T run = chain_scan_wave<T, Op, R>(v);
+    if ((threadIdx.x & 63u) == 0) s_wave_tot[w] = run;
+    __syncthreads();
+    chain_fold_waves<T, Op, NW>(s_wave_tot, w, total, wave_pre);
 }
 
 // adds what precedes the tile (if anything) and the earlier waves' total, and stores
@@ -609,8 +643,7 @@ __device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, Chai
                 continue;
             }
         }
-        if (NT) __builtin_nontemporal_store(v[r].q, dst + r * 64);
-        else dst[r * 64] = v[r].q;
+        store_vector<NT>(dst + r * 64, v[r].q, store_pieces(out));
     }
 }
 
@@ -849,17 +882,19 @@ static void chain_words_release(const ChainWords& w) {
 template <class T, class Op>
 int scan_chain_launch(const char* p1, char* p2, ssize_t s1, ssize_t s2, uint64_t n, hipStream_t stream) {
     constexpr int W = ScanChain<T>::W;
-    // Blocks of eight waves and 128 KiB tiles for four-byte elements wherever that leaves 64 tiles (half the
-    // tickets and look-backs per byte: 2^26 SFloat 115 -> 111 us, 2^24 39 -> 33 us), else blocks of four waves
-    // and 64 KiB tiles; eight-byte elements always those (their kernel needs 168 registers, and one block of
-    // eight waves would have a compute unit to itself: 2^26 DFloat 224 us against 260 us).
+    // Blocks of eight waves and 128 KiB tiles wherever that leaves 64 tiles of four-byte elements or 128 to 3072 of eight-byte
+    // ones (half the tickets, which one word hands out at about 10 ns each, and half the look-backs per byte), else blocks of
+    // four waves and 64 KiB tiles. Wide / narrow, us on fresh operands: SFloat 2^20 8.8 / 6.5, 2^22 11.2 / 11.4, 2^24 29.1 /
+    // 35.3, 2^26 102 / 109; DFloat 2^20 9.0 / 8.5, 2^21 11.7 / 12.1, 2^22 16.4 / 20.3, 2^24 57.8 / 63.4, 2^25 107.5 / 110, 2^26
+    // 212 / 203 (one wide block of doubles has a compute unit to itself, three narrow ones share it).
     // CUMO_HIP_SCAN_CHAIN_WAVES=4 or 8, read once, fixes the choice.
     static const int forced_waves = [] {
         const char* e = std::getenv("CUMO_HIP_SCAN_CHAIN_WAVES");
         return e ? std::atoi(e) : 0;
     }();
     const uint64_t wide_tile = 2ull * ScanChain<T>::TILE;
-    const bool wide = forced_waves == 8 || (forced_waves != 4 && sizeof(T) == 4 && (n + wide_tile - 1) / wide_tile >= 64);
+    const uint64_t wide_tiles = (n + wide_tile - 1) / wide_tile;
+    const bool wide = forced_waves == 8 || (forced_waves != 4 && (sizeof(T) == 4 ? wide_tiles >= 64 : wide_tiles >= 128 && wide_tiles <= 3072));
     const uint64_t tile = wide ? wide_tile : (uint64_t)ScanChain<T>::TILE;
     const uint64_t n_tiles = (n + tile - 1) / tile;
     if (n_tiles < 64 || n_tiles > kChainMaxTiles) return -1;

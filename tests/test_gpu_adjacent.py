@@ -301,6 +301,11 @@ def test_one_long_run_in_one_pass(tname, dt):
             h[::3] = 0   # keeps the running float sums far below 2^24
         d = cls.cast(h)
         assert_bits_equal(d.cumsum().to_numpy(), oracle.cum("cumsum", h), (n, "cumsum"))
+    if dt == np.float64:
+        # eight-byte elements: blocks of eight waves from 128 to 3072 of their tiles
+        for n in (254 * tile, 254 * tile + 1, 257 * tile - 1, 6144 * tile, 6144 * tile + 1):
+            h = rng.integers(-3, 4, size=n).astype(dt)
+            assert_bits_equal(cls.cast(h).cumsum().to_numpy(), oracle.cum("cumsum", h), (n, "cumsum"))
     n = 64 * tile * 3 + 17
     f = rng.choice(np.array([1, -1], dtype=dt), size=n)
     f[rng.integers(0, n, 25)] = 2
