@@ -275,6 +275,10 @@ class NArray(_native.View):
     def __getitem__(self, key):
         if isinstance(key, NArray) and type(key).__name__ == "Bit":
             return key.mask(self)  # a[mask]: the elements where the mask is set
+        if type(key) is np.ndarray:
+            taken = _native.take(self, key)  # one array of 64-bit positions; None: the general way
+            if taken is not None:
+                return taken
         key = self._expand_key(key)
         if any(_is_index_array(k) for k in key):
             return self._gather(key)

@@ -13,7 +13,10 @@
 #include <Python.h>
 #include <structmember.h>
 
+#include <cstdint>
 #include <cstring>
+#include <memory>
+#include <new>
 
 #include "cumo_hip.h"
 #include "cumo_hip_ndloop.h"
@@ -525,6 +528,71 @@ PyObject* na_bit_count(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return run(&z, 1, [&] { cumo_hip_na_bit_count(&dx, mask, keep, count_false, &z); });
 }
 
+// (self, positions): self[positions] for a one-dimensional array of 64-bit positions in the first dimension; None where the general
+// form answers (other kinds of positions, positions out of range, empty results). x[2048 rows] 27.4 -> 8.5 us of the caller's time.
+PyObject* na_take(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (!arity(n, 2)) return nullptr;
+    const View* x = as_view(a[0]);
+    if (!x || x->code < 0 || x->code > 4 || g_recording || ndim_of(x) < 1) Py_RETURN_NONE;
+    static const size_t element[5] = {4, 8, 4, 8, 8};
+    const size_t elmsz = element[x->code];
+    Desc dx, z;
+    if (describe(x, &dx) < 0) return nullptr;
+    size_t row = elmsz, bytes;
+    for (int k = 1; k < dx.ndim; k++) row *= dx.shape[k];
+    Py_buffer b;
+    if (PyObject_GetBuffer(a[1], &b, PyBUF_FORMAT | PyBUF_ND) < 0) {
+        PyErr_Clear();   // (not contiguous, say)
+        Py_RETURN_NONE;
+    }
+    const size_t count = static_cast<size_t>(b.len) / sizeof(int64_t);
+    bool taken = b.ndim == 1 && b.itemsize == sizeof(int64_t) && b.format && (!std::strcmp(b.format, "l") || !std::strcmp(b.format, "q")) &&
+                 reinterpret_cast<uintptr_t>(b.buf) % alignof(int64_t) == 0 && count > 0 && row > 0 && dx.shape[0] > 0 &&
+                 !__builtin_mul_overflow(row, count, &bytes);
+    std::unique_ptr<size_t[]> pos(taken ? new (std::nothrow) size_t[count] : nullptr);
+    taken = taken && pos;
+    if (taken) {
+        // a negative position counts from the end
+        const int64_t* from = static_cast<const int64_t*>(b.buf);
+        const int64_t len = static_cast<int64_t>(dx.shape[0]);
+        for (size_t i = 0; i < count; i++) {
+            const int64_t k = from[i] < 0 ? from[i] + len : from[i];
+            taken = taken && k >= 0 && k < len;
+            pos[i] = static_cast<size_t>(k);
+        }
+    }
+    PyBuffer_Release(&b);
+    if (!taken) Py_RETURN_NONE;
+    return run(&z, 1, [&] {
+        const ssize_t st = dx.stride[0];
+        const size_t last = dx.shape[0] - 1;
+        size_t* off = reinterpret_cast<size_t*>(cumo_cuda_runtime_malloc(count * sizeof(size_t)));
+        char* out = off ? reinterpret_cast<char*>(cumo_cuda_runtime_malloc(bytes)) : nullptr;
+        if (out) {
+            z.type = dx.type;
+            z.ndim = dx.ndim;
+            z.ptr = out;
+            cumo_na_iarray_stridx_t view;
+            cumo_na_indexer_t ix;
+            std::memset(&view, 0, sizeof(view));
+            std::memset(&ix, 0, sizeof(ix));
+            ix.ndim = dx.ndim;
+            ix.total_size = bytes / elmsz;
+            for (int k = 0; k < dx.ndim; k++) {
+                z.shape[k] = ix.shape[k] = k == 0 ? count : dx.shape[k];
+                CUMO_SDX_SET_STRIDE(view.stridx[k], dx.stride[k]);
+            }
+            // (a reversed dimension counts from its far end)
+            CUMO_SDX_SET_INDEX(view.stridx[0], off);
+            view.ptr = static_cast<char*>(dx.ptr) + dx.offset + (st < 0 ? st * static_cast<ssize_t>(last) : 0);
+            if (cumo_hip_index_from_host(off, pos.get(), count, st < 0 ? -st : st, st < 0 ? 1 : 0, last) == CUMO_HIP_OK)
+                cumo_ndloop_copy_to_buffer_kernel_launch(&view, &ix, out, elmsz);
+        }
+        // (stream-ordered: whoever gets it next can only touch it from later work)
+        if (off) cumo_cuda_runtime_free_no_raise(reinterpret_cast<char*>(off));
+    });
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // set-up
 // ---------------------------------------------------------------------------------------------------------------
@@ -565,7 +633,7 @@ PyObject* set_recording(PyObject*, PyObject* rec) {
 
 #define CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(na_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {CALL(binary), CALL(compare), CALL(unary), CALL(math), CALL(reduce), CALL(mulsum), CALL(cum), CALL(bit_binary),
-                         CALL(bit_count), {"setup", setup, METH_VARARGS, nullptr}, {"set_recording", set_recording, METH_O, nullptr}, {}};
+                         CALL(bit_count), CALL(take), {"setup", setup, METH_VARARGS, nullptr}, {"set_recording", set_recording, METH_O, nullptr}, {}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "cumo_amd._native", "Buffers, views and calls of the array classes.", -1, methods};
 

@@ -65,6 +65,34 @@ def test_native_calls_answer_like_the_general_methods(tname, shape):
     assert empty.count_true() == 0 and empty.count_true(axis=0) == 0
 
 
+@pytest.mark.parametrize("tname", sorted(TYPES) + ["int64"])
+def test_rows_by_position_answer_like_the_general_form(tname):
+    rng = np.random.default_rng(5)
+    x = TYPES[tname].cast(rng.integers(-99, 99, size=(7, 6, 5)).astype(TYPES[tname].np_dtype)) if tname in TYPES else \
+        DFloat.cast(rng.standard_normal((7, 6, 5))).argmax(axis=2)
+    for v in (x, x.transpose(), x.reverse(0), x.reverse(1), x[::2], x[1], x[:, 1:4], x[3:4], x.reshape(x.size), x.reverse(0)[1::3]):
+        n = v.shape[0]
+        for k in (np.arange(n), np.array([0]), np.array([-1, 0, n - 1, -n, 0]), rng.integers(-n, n, 300), rng.integers(0, n, 9000)):
+            got, want = _native.take(v, k), v._gather(v._expand_key(k))
+            assert same(got, want) and same(v[k], want)
+        one = np.zeros(4, np.int64)
+        # what it leaves to the general form, and what that refuses
+        for k in (one.astype(np.int32), one.astype(np.uint64), one.astype(float), one[::2], one[:0], one.reshape(2, 2), one.astype(">i8"),
+                  np.array(0), np.array([0, n]), np.array([-n - 1])):
+            assert _native.take(v, k) is None
+        for k in (np.array([0, n]), np.array([-n - 1]), one.reshape(2, 2), np.array([0.5])):
+            with pytest.raises(IndexError):
+                v[k]
+        assert same(v[one.astype(np.int32)], v._gather(v._expand_key(one)))
+        assert v[one[:0]].size == 0
+    with pytest.raises(TypeError):
+        Bit(8)[np.array([0])]
+    assert _native.take(SFloat(0, 3), np.array([0])) is None and _native.take(SFloat(3, 0), np.array([0])) is None
+    with _lib.record() as calls:
+        x[np.array([1, 0])]
+    assert len(calls) > 0
+
+
 def test_what_is_refused_stays_refused_and_leaks_nothing():
     x = SFloat.cast(np.ones((4, 5), np.float32))
     i = Int32.cast(np.zeros(6, np.int32))
