@@ -269,7 +269,7 @@ struct StridxRows {
     uint64_t row_bytes;
 };
 
-typedef store_u4 ix_u4;
+typedef uint32_t ix_u4 __attribute__((ext_vector_type(4)));
 
 template <bool TO_BUFFER, int LPR, bool NT>
 __global__ __launch_bounds__(kIxBlock) void stridx_rows_kernel(StridxView v, StridxRows g, char* buf) {
@@ -291,9 +291,6 @@ __global__ __launch_bounds__(kIxBlock) void stridx_rows_kernel(StridxView v, Str
         char* in_buf = buf + (uint64_t)row * g.row_bytes + (uint64_t)first * 16;
         const char* src = TO_BUFFER ? in_view : in_buf;
         char* dst = TO_BUFFER ? in_buf : in_view;
-        // rows of the buffer that start on whole pieces are written through the second-level cache (see store_vector;
-        // 2048 rows of 4096 SFloat 15.0 -> 13.4 us)
-        const bool pieces = TO_BUFFER && store_pieces(buf, g.row_bytes);
         // (a 128-bit access works on any 4-byte boundary)
         if (((uintptr_t)in_view & 3) == 0) {
             if (seg + 1 == g.segs_per_row && lane < g.tail_words) {
@@ -313,7 +310,8 @@ __global__ __launch_bounds__(kIxBlock) void stridx_rows_kernel(StridxView v, Str
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     if (b + k * LPR + lane < nv) {
-                        store_vector<NT>(d4 + (b + k * LPR + lane), x[k], pieces);
+                        if (NT) __builtin_nontemporal_store(x[k], d4 + (b + k * LPR + lane));
+                        else d4[b + k * LPR + lane] = x[k];
                     }
                 }
             }
