@@ -115,22 +115,59 @@ __device__ __forceinline__ uint32_t wh_block_exscan32(uint32_t v, uint32_t* tota
     return before + inc - v;
 }
 
-__global__ __launch_bounds__(kWhBlock) void where_count_kernel(const CUMO_BIT_DIGIT* a, uint64_t p, int64_t s, const size_t* idx, uint64_t n,
-                                                               int contiguous, int invert, uint64_t nchunks, uint64_t cpb, uint64_t* block_sums,
-                                                               uint64_t* host_sums) {
-    uint64_t start = (uint64_t)blockIdx.x * cpb;
+// The hits of every placing block's share of the chunks: a block counts for kWhGroups of them, 256 lanes each. host_words: pinned
+// host memory that the caller looks at, for each share's count (host_each) or for the block's total, one up so that no count is
+// the 0 the host looks for. Every word is a write across the link and every line of them a miss of the caller's, one behind
+// the other: a pass over 8192 x 4096 SFloat that reads back two masks' counts takes 164 us by 1024 words each, 158 by 256 totals.
+constexpr int kWhGroups = 4;
+__global__ __launch_bounds__(kWhBlock * kWhGroups) void where_count_kernel(const CUMO_BIT_DIGIT* a, uint64_t p, int64_t s, const size_t* idx, uint64_t n,
+                                                                           int contiguous, int invert, uint64_t nchunks, uint64_t cpb, uint64_t nshares,
+                                                                           uint64_t* sums, uint64_t* host_words, int host_each) {
+    __shared__ uint64_t wave_sum[kWhBlock * kWhGroups / 64];
+    const unsigned t = threadIdx.x % kWhBlock;
+    const uint64_t share = (uint64_t)blockIdx.x * kWhGroups + threadIdx.x / kWhBlock;
+    uint64_t start = share * cpb;
     if (start > nchunks) start = nchunks;
     const uint64_t end = (nchunks - start < cpb) ? nchunks : start + cpb;
     uint64_t cnt = 0;
-    for (uint64_t c = start + threadIdx.x; c < end; c += kWhBlock) cnt += (uint64_t)__popc(wh_chunk(a, p, s, idx, n, c, contiguous, invert));
-    uint64_t total;
-    wh_block_exscan(cnt, &total);
-    if (threadIdx.x == 0) {
-        block_sums[blockIdx.x] = total;
-        // a copy straight into the caller's pinned host memory, one up so that no count is the 0 the host looks for
-        if (host_sums) __hip_atomic_store(host_sums + blockIdx.x, total + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    uint64_t c = start + t;
+    if (contiguous && (p & 31) == 0) {
+        // whole words, four in flight a lane; a run's last chunk, partly there, comes below
+        const uint64_t whole = (end == nchunks && (n & 31) != 0) ? end - 1 : end;
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(a) + (p >> 5);
+        const uint32_t flip = invert ? 0xffffffffu : 0u;
+        for (; c + 3 * kWhBlock < whole; c += 4 * kWhBlock) {
+            uint32_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = w[c + k * kWhBlock];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cnt += (uint64_t)__popc(v[k] ^ flip);
+        }
+    }
+    for (; c < end; c += kWhBlock) cnt += (uint64_t)__popc(wh_chunk(a, p, s, idx, n, c, contiguous, invert));
+    for (int m = 32; m > 0; m >>= 1) {
+        const uint32_t lo = __shfl_xor((uint32_t)cnt, m), hi = __shfl_xor((uint32_t)(cnt >> 32), m);
+        cnt += ((uint64_t)hi << 32) | lo;
+    }
+    if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    constexpr unsigned WPS = kWhBlock / 64;   // waves of a share
+    if (threadIdx.x < kWhGroups) {
+        uint64_t mine = 0;
+        for (unsigned k = 0; k < WPS; ++k) mine += wave_sum[threadIdx.x * WPS + k];
+        const uint64_t at = (uint64_t)blockIdx.x * kWhGroups + threadIdx.x;
+        if (at < nshares) {
+            sums[at] = mine;
+            if (host_words && host_each) __hip_atomic_store(host_words + at, mine + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    if (threadIdx.x == 0 && host_words && !host_each) {
+        uint64_t all = 0;
+        for (unsigned k = 0; k < WPS * kWhGroups; ++k) all += wave_sum[k];
+        __hip_atomic_store(host_words + blockIdx.x, all + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
+inline unsigned wh_count_grid(uint64_t nblocks) { return (unsigned)((nblocks + kWhGroups - 1) / kWhGroups); }
 
 // block_sums[b] becomes the output position of block b's first hit; *running moves on
 __global__ __launch_bounds__(kWhBlock) void where_scan_kernel(uint64_t* block_sums, uint64_t nblocks, uint64_t* running) {
@@ -324,8 +361,8 @@ void where_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, size_t* idx, uint64_t 
     const uint64_t nchunks = g.nchunks, nblocks = g.nblocks, cpb = g.cpb;
     const int contiguous = (idx == nullptr && s == 1) ? 1 : 0;
     hipStream_t st = current_stream();
-    hipLaunchKernelGGL(where_count_kernel, dim3((unsigned)nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s, (const size_t*)idx, n, contiguous,
-                       invert, nchunks, cpb, block_sums, (uint64_t*)nullptr);
+    hipLaunchKernelGGL(where_count_kernel, dim3(wh_count_grid(nblocks)), dim3(kWhBlock * kWhGroups), 0, st, a, (uint64_t)p, (int64_t)s, (const size_t*)idx, n,
+                       contiguous, invert, nchunks, cpb, nblocks, block_sums, (uint64_t*)nullptr, 0);
     hipLaunchKernelGGL(where_scan_kernel, dim3(1), dim3(kWhBlock), 0, st, block_sums, nblocks, running);
 #define WH_SCATTER(ES)                                                                                                                      \
     hipLaunchKernelGGL((where_scatter_kernel<MODE, ES, false>), dim3((unsigned)nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s,     \
@@ -420,6 +457,74 @@ void where_place(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert,
     cumo_cuda_runtime_check_kernel_launch();
 }
 
+// The counts in device memory, and on the host when the call returns each of them (host_counts) or their sum (*total): the
+// kernel writes into pinned host memory of the calling thread as well, and the host looks at that memory until every word is there. They are the last thing
+// the stream has been given, so nothing earlier is still running then. A stream that has not come this far within
+// kWhLookNs is waited for instead, which also reports what may have gone wrong on it. Looking costs the caller's core
+// what the runtime's own wait costs it, and saves the wait's way through a signal: SFloat 104 x 96 x[mask]
+// 20.9 -> 15.8 us, mask.where() 20.0 -> 15.2 us.
+constexpr int64_t kWhLookNs = 2000000;
+int where_count_wait(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts, uint64_t* total) {
+    if (total) *total = 0;
+    if (n == 0) return CUMO_HIP_OK;
+    const WhGeometry g = wh_geometry(n);
+    static thread_local uint64_t* pinned = nullptr;   // kWhMaxBlocks words, kept for the thread's lifetime
+    if (pinned == nullptr) {
+        void* m = nullptr;
+        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc"))
+            return CUMO_HIP_ERROR_RUNTIME;
+        pinned = static_cast<uint64_t*>(m);
+    }
+    int each = host_counts != nullptr ? 1 : 0;
+    const uint64_t nwords = each ? g.nblocks : wh_count_grid(g.nblocks);
+    std::memset(pinned, 0, nwords * sizeof(uint64_t));
+    hipStream_t st = current_stream();
+    // The launch's own status: hipGetLastError would answer for an earlier call of the thread as well, and a kernel that has been
+    // queued must be waited for, or its counts could be taken for the next call's.
+    uint64_t first = p, words = n, *host = pinned;
+    int64_t step = s;
+    const size_t* idx = nullptr;
+    int contiguous = s == 1 ? 1 : 0;
+    WhGeometry kg = g;
+    void* args[] = {&a, &first, &step, &idx, &words, &contiguous, &invert, &kg.nchunks, &kg.cpb, &kg.nblocks, &counts, &host, &each};
+    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(where_count_kernel), dim3(wh_count_grid(g.nblocks)), dim3(kWhBlock * kWhGroups), args, 0, st);
+    if (launched != hipSuccess) {
+        (void)hipGetLastError();
+        report_hip_error(launched, "kernel launch");
+        return CUMO_HIP_ERROR_RUNTIME;
+    }
+    // (under capture nothing has been queued that could leave a count: the runtime's wait refuses at once, as it always has)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;
+    }
+    if (capturing != hipStreamCaptureStatusNone && !hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+    const auto begin = std::chrono::steady_clock::now();
+    uint64_t b = 0;
+    for (unsigned looks = 0; b < nwords; ++looks) {
+        while (b < nwords && __atomic_load_n(pinned + b, __ATOMIC_ACQUIRE) != 0) ++b;
+        if (b == nwords) break;
+        __builtin_ia32_pause();
+        if ((looks & 63u) == 63u && (std::chrono::steady_clock::now() - begin) > std::chrono::nanoseconds(kWhLookNs)) {
+            if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+            break;
+        }
+    }
+    if (!wait_trouble_check()) return CUMO_HIP_ERROR_RUNTIME;
+    for (b = 0; b < nwords; ++b) {
+        const uint64_t word = __atomic_load_n(pinned + b, __ATOMIC_RELAXED);
+        if (word == 0) {
+            report_error(CUMO_HIP_ERROR_RUNTIME, 0, "where: a block left no count");
+            return CUMO_HIP_ERROR_RUNTIME;
+        }
+        if (host_counts) host_counts[b] = word - 1;
+        if (total) *total += word - 1;
+    }
+    cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
+    return CUMO_HIP_OK;
+}
+
 }  // namespace cumo_hip
 
 using namespace cumo_hip;
@@ -458,74 +563,14 @@ size_t cumo_hip_bit_where_blocks(uint64_t n) { return (size_t)wh_geometry(n).nbl
 void cumo_hip_bit_where_count_kernel_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts) {
     if (n == 0) return;
     const WhGeometry g = wh_geometry(n);
-    hipLaunchKernelGGL(where_count_kernel, dim3((unsigned)g.nblocks), dim3(kWhBlock), 0, current_stream(), a, (uint64_t)p, (int64_t)s,
-                       (const size_t*)nullptr, n, s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, counts, (uint64_t*)nullptr);
+    hipLaunchKernelGGL(where_count_kernel, dim3(wh_count_grid(g.nblocks)), dim3(kWhBlock * kWhGroups), 0, current_stream(), a, (uint64_t)p, (int64_t)s,
+                       (const size_t*)nullptr, n, s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, g.nblocks, counts, (uint64_t*)nullptr, 0);
     cumo_cuda_runtime_check_kernel_launch();
 }
 
-// The same, and the counts on the host when the call returns: the kernel writes them into pinned host memory of the
-// calling thread as well, and the host looks at that memory until every block's count is there. They are the last thing
-// the stream has been given, so nothing earlier is still running then. A stream that has not come this far within
-// kWhLookNs is waited for instead, which also reports what may have gone wrong on it. Looking costs the caller's core
-// what the runtime's own wait costs it, and saves the wait's way through a signal: SFloat 104 x 96 x[mask]
-// 20.9 -> 15.8 us, mask.where() 20.0 -> 15.2 us.
 // host_counts: cumo_hip_bit_where_blocks(n) words of ordinary host memory.
-constexpr int64_t kWhLookNs = 2000000;
 int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts) {
-    if (n == 0) return CUMO_HIP_OK;
-    const WhGeometry g = wh_geometry(n);
-    static thread_local uint64_t* pinned = nullptr;   // kWhMaxBlocks words, kept for the thread's lifetime
-    if (pinned == nullptr) {
-        void* m = nullptr;
-        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc"))
-            return CUMO_HIP_ERROR_RUNTIME;
-        pinned = static_cast<uint64_t*>(m);
-    }
-    std::memset(pinned, 0, g.nblocks * sizeof(uint64_t));
-    hipStream_t st = current_stream();
-    // The launch's own status: hipGetLastError would answer for an earlier call of the thread as well, and a kernel that has been
-    // queued must be waited for, or its counts could be taken for the next call's.
-    uint64_t first = p, words = n, *host = pinned;
-    int64_t step = s;
-    const size_t* idx = nullptr;
-    int contiguous = s == 1 ? 1 : 0;
-    WhGeometry kg = g;
-    void* args[] = {&a, &first, &step, &idx, &words, &contiguous, &invert, &kg.nchunks, &kg.cpb, &counts, &host};
-    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(where_count_kernel), dim3((unsigned)g.nblocks), dim3(kWhBlock), args, 0, st);
-    if (launched != hipSuccess) {
-        (void)hipGetLastError();
-        report_hip_error(launched, "kernel launch");
-        return CUMO_HIP_ERROR_RUNTIME;
-    }
-    // (under capture nothing has been queued that could leave a count: the runtime's wait refuses at once, as it always has)
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        capturing = hipStreamCaptureStatusActive;
-    }
-    if (capturing != hipStreamCaptureStatusNone && !hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
-    const auto begin = std::chrono::steady_clock::now();
-    uint64_t b = 0;
-    for (unsigned looks = 0; b < g.nblocks; ++looks) {
-        while (b < g.nblocks && __atomic_load_n(pinned + b, __ATOMIC_ACQUIRE) != 0) ++b;
-        if (b == g.nblocks) break;
-        __builtin_ia32_pause();
-        if ((looks & 63u) == 63u && (std::chrono::steady_clock::now() - begin) > std::chrono::nanoseconds(kWhLookNs)) {
-            if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
-            break;
-        }
-    }
-    if (!wait_trouble_check()) return CUMO_HIP_ERROR_RUNTIME;
-    for (b = 0; b < g.nblocks; ++b) {
-        const uint64_t word = __atomic_load_n(pinned + b, __ATOMIC_RELAXED);
-        if (word == 0) {
-            report_error(CUMO_HIP_ERROR_RUNTIME, 0, "where: a block left no count");
-            return CUMO_HIP_ERROR_RUNTIME;
-        }
-        host_counts[b] = word - 1;
-    }
-    cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
-    return CUMO_HIP_OK;
+    return where_count_wait(a, p, s, n, invert, counts, host_counts, nullptr);
 }
 
 // x == NULL: out[o] = the position in the run of the o-th hit, as an elmsz-byte integer (4 or 8);

@@ -163,6 +163,34 @@ def test_count_then_place_launchers(nbits):
     free(pw, px, pxd)
 
 
+@pytest.mark.parametrize("lead", [64, 37])   # a run that starts on a word, and inside one
+@pytest.mark.parametrize("nbits", [1, 33, 8192, 8193, 1 << 15, (1 << 15) + 1, (1 << 20) - 5, (1 << 25) + 32 * 1024 + 77])
+def test_counts_of_shares_on_device_and_host(nbits, lead):
+    """The blocks of the count take four placing blocks' shares each: every share's count, on the device and on
+    the host, at sizes that end inside a share, a block and a word; and the positions that the total sizes."""
+    from cumo_amd import Bit, _lib
+    from test_gpu_raw_abi import dev, fetch, free
+    rng = np.random.default_rng(nbits)
+    h = (rng.random(lead + nbits) < 0.4).astype(np.uint8)
+    words = np.frombuffer(np.packbits(np.concatenate([h, np.ones((-h.size) % 32, np.uint8)]), bitorder="little").tobytes(), dtype=np.uint32)
+    pw = dev(words)
+    nb = _lib.fn("cumo_hip_bit_where_blocks", C.c_size_t, [C.c_uint64])(nbits)
+    to_host = _lib.fn("cumo_hip_bit_where_count_to_host", C.c_int, [C.c_void_p, C.c_size_t, C.c_ssize_t, C.c_uint64, C.c_int, C.c_void_p, C.c_void_p])
+    chunks = -(-nbits // 32)
+    share = -(-chunks // nb) * 32
+    for invert in (0, 1):
+        run = h[lead:] ^ invert
+        want = np.array([run[k * share:(k + 1) * share].sum(dtype=np.uint64) for k in range(nb)], dtype=np.uint64)
+        pc, on_host = dev(np.full(nb + 1, 12345, dtype=np.uint64)), np.full(nb + 1, 777, dtype=np.uint64)
+        _lib.call(to_host, pw, lead, 1, nbits, invert, pc, on_host.ctypes.data)
+        counts = fetch(pc, (nb + 1,), np.uint64)
+        assert (counts[:nb] == want).all() and counts[nb] == 12345 and (on_host[:nb] == want).all() and on_host[nb] == 777
+        free(pc)
+    free(pw)
+    b = Bit.cast(h)[lead:]
+    assert (b.where().to_numpy() == np.flatnonzero(h[lead:])).all()
+
+
 def test_where_and_mask_into_a_given_result():
     """A result array of exactly the count's length is written in place; any other length is a shape error."""
     import ctypes as C
