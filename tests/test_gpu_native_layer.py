@@ -93,6 +93,20 @@ def test_rows_by_position_answer_like_the_general_form(tname):
     assert len(calls) > 0
 
 
+@pytest.mark.parametrize("tname", sorted(TYPES))
+def test_selections_of_a_derived_class_are_of_that_class(tname):
+    class Derived(TYPES[tname]):
+        pass
+    h = np.arange(24).reshape(4, 6).astype(TYPES[tname].np_dtype)
+    w = Derived.cast(h)
+    for key in (slice(1, 3), [0, 2], np.array([0, 2]), np.array([0, 2], dtype=np.int32), np.array([-1, 0, 3]), (np.array([1]), slice(None))):
+        got = w[key]
+        assert type(got) is Derived
+        assert (got.to_numpy() == h[key]).all()
+    assert type(w.reshape(24)[np.array([5])]) is Derived
+    assert type(TYPES[tname].cast(h)[np.array([0, 2])]) is TYPES[tname]
+
+
 def test_what_is_refused_stays_refused_and_leaks_nothing():
     x = SFloat.cast(np.ones((4, 5), np.float32))
     i = Int32.cast(np.zeros(6, np.int32))
