@@ -283,15 +283,15 @@ def test_cum_along_contiguous_runs_of_whole_chunks(tname, dt):
 
 @pytest.mark.parametrize("tname,dt", ALL)
 def test_one_long_run_in_one_pass(tname, dt):
-    """Runs from 64 tiles of 64 KiB on are scanned in one pass (four-byte elements: by blocks of
-    eight waves with tiles of 128 KiB once there are 64 of those), tiles handing their totals on
-    through groups of 64 and supergroups of 64 groups: sizes that end exactly on a group, one
-    element past it, the same for the larger tiles, and 4096 small (2048 large) tiles with
-    a ragged tail; small integers (float sums
+    """Runs from 64 tiles of 64 KiB on are scanned in one pass (by blocks of eight waves with
+    tiles of 128 KiB once there are 64 of those, of eight-byte elements from 128 to 3072), tiles
+    handing their totals on through groups of 64 and supergroups of 64 groups: sizes that end
+    exactly on a group, one element past it, the same for the larger tiles, and 4096 small
+    (2048 large) tiles with a ragged tail; small integers (float sums
     exact in any order), so every result is compared bit for bit with the sequential scan.
-    Then what only the order-free comparison can hold: products of +-1 and 2, NaN skipped
-    (the run starts with a tile of nothing but NaN) and carried, a strided view on each side,
-    and the same call twice giving the same bits on random floats."""
+    Then, by small and by large tiles, what only the order-free comparison can hold: products
+    of +-1 and 2, NaN skipped (the run starts with a tile of nothing but NaN) and carried, a
+    strided view on each side, and the same call twice giving the same bits on random floats."""
     cls = cls_of(tname)
     rng = np.random.default_rng(57)
     tile = 65536 // np.dtype(dt).itemsize
@@ -306,27 +306,28 @@ def test_one_long_run_in_one_pass(tname, dt):
         for n in (254 * tile, 254 * tile + 1, 257 * tile - 1, 6144 * tile, 6144 * tile + 1):
             h = rng.integers(-3, 4, size=n).astype(dt)
             assert_bits_equal(cls.cast(h).cumsum().to_numpy(), oracle.cum("cumsum", h), (n, "cumsum"))
-    n = 64 * tile * 3 + 17
-    f = rng.choice(np.array([1, -1], dtype=dt), size=n)
-    f[rng.integers(0, n, 25)] = 2
-    assert_bits_equal(cls.cast(f).cumprod().to_numpy(), oracle.cum("cumprod", f), "cumprod")
-    h = rng.integers(-3, 4, size=2 * n).astype(dt)
-    hv = np.ascontiguousarray(h[::2])
-    assert_bits_equal(cls.cast(h)[::2].cumsum().to_numpy(), oracle.cum("cumsum", hv), "strided input")
-    if dt != np.int32:
-        g = rng.integers(-3, 4, size=n).astype(dt)
-        g[rng.integers(0, n, 3000)] = np.nan
-        g[:5000] = np.nan
-        d = cls.cast(g)
-        assert_bits_equal(d.cumsum(nan=True).to_numpy(), oracle.cum("cumsum", g, nan=True), "nan: true")
-        assert_bits_equal(d.cumsum().to_numpy(), oracle.cum("cumsum", g), "NaN carried")
-        r = rng.standard_normal(n).astype(dt)
-        d = cls.cast(r)
-        first = d.cumsum().to_numpy()
-        for _ in range(3):
-            assert_bits_equal(d.cumsum().to_numpy(), first, "same bits from launch to launch")
-        exact = np.cumsum(r.astype(np.float64)) if dt == np.float32 else np.asarray(np.cumsum(r.astype(np.longdouble))).astype(np.float64)
-        _cum_close(first, exact, np.cumsum(np.abs(r).astype(np.float64)), n, dt, "random floats")
+    # 192 small tiles (96 large ones: eight-byte elements take the small), and 150 large ones of either size
+    for n in (192 * tile + 17, 300 * tile + 17):
+        f = rng.choice(np.array([1, -1], dtype=dt), size=n)
+        f[rng.integers(0, n, 25)] = 2
+        assert_bits_equal(cls.cast(f).cumprod().to_numpy(), oracle.cum("cumprod", f), (n, "cumprod"))
+        h = rng.integers(-3, 4, size=2 * n).astype(dt)
+        hv = np.ascontiguousarray(h[::2])
+        assert_bits_equal(cls.cast(h)[::2].cumsum().to_numpy(), oracle.cum("cumsum", hv), (n, "strided input"))
+        if dt != np.int32:
+            g = rng.integers(-3, 4, size=n).astype(dt)
+            g[rng.integers(0, n, 3000)] = np.nan
+            g[:2 * tile] = np.nan
+            d = cls.cast(g)
+            assert_bits_equal(d.cumsum(nan=True).to_numpy(), oracle.cum("cumsum", g, nan=True), (n, "nan: true"))
+            assert_bits_equal(d.cumsum().to_numpy(), oracle.cum("cumsum", g), (n, "NaN carried"))
+            r = rng.standard_normal(n).astype(dt)
+            d = cls.cast(r)
+            first = d.cumsum().to_numpy()
+            for _ in range(3):
+                assert_bits_equal(d.cumsum().to_numpy(), first, (n, "same bits from launch to launch"))
+            exact = np.cumsum(r.astype(np.float64)) if dt == np.float32 else np.asarray(np.cumsum(r.astype(np.longdouble))).astype(np.float64)
+            _cum_close(first, exact, np.cumsum(np.abs(r).astype(np.float64)), n, dt, (n, "random floats"))
 
 
 @pytest.mark.parametrize("tname,dt", ALL)

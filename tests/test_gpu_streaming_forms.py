@@ -80,6 +80,11 @@ def test_one_long_run_by_blocks_of_four_waves():
     run_child({"CUMO_HIP_SCAN_CHAIN_WAVES": "4"}, ["tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass"])
 
 
+def test_one_long_run_by_blocks_of_eight_waves():
+    """Also the sizes of eight-byte elements that take blocks of four: 64 to 127 large tiles, and more than 3072."""
+    run_child({"CUMO_HIP_SCAN_CHAIN_WAVES": "8"}, ["tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass"])
+
+
 def test_bit_vector_kernels_with_lanes_that_loop():
     run_child({"CUMO_HIP_BIT_VEC_GRID": "1", "CUMO_HIP_NT": "1"},
               ["tests/test_gpu_bit.py::test_rows_of_bits_in_views_word_by_word", "tests/test_gpu_bit.py::test_long_runs_of_bits_by_whole_vectors",
