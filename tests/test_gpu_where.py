@@ -167,7 +167,8 @@ def test_count_then_place_launchers(nbits):
 @pytest.mark.parametrize("nbits", [1, 33, 8192, 8193, 1 << 15, (1 << 15) + 1, (1 << 20) - 5, (1 << 25) + 32 * 1024 + 77])
 def test_counts_of_shares_on_device_and_host(nbits, lead):
     """The blocks of the count take four placing blocks' shares each: every share's count, on the device and on
-    the host, at sizes that end inside a share, a block and a word; and the positions that the total sizes."""
+    the host, at sizes that end inside a share, a block and a word; and the total of the blocks, which sizes the
+    positions, of the set and of the clear bits, of the run and of every third bit of it."""
     from cumo_amd import Bit, _lib
     from test_gpu_raw_abi import dev, fetch, free
     rng = np.random.default_rng(nbits)
@@ -187,8 +188,9 @@ def test_counts_of_shares_on_device_and_host(nbits, lead):
         assert (counts[:nb] == want).all() and counts[nb] == 12345 and (on_host[:nb] == want).all() and on_host[nb] == 777
         free(pc)
     free(pw)
-    b = Bit.cast(h)[lead:]
-    assert (b.where().to_numpy() == np.flatnonzero(h[lead:])).all()
+    for b, run in ((Bit.cast(h)[lead:], h[lead:]), (Bit.cast(h)[lead::3], h[lead::3])):
+        for got, want in zip(b.where2(), (np.flatnonzero(run), np.flatnonzero(run == 0))):
+            assert got.shape == want.shape and (got.to_numpy() == want).all()
 
 
 def test_where_and_mask_into_a_given_result():
