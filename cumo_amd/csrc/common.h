@@ -63,8 +63,7 @@ bool mixed_flat_binary_s(int op, const char* x, double sv, bool scalar_is_left, 
 void mulsum_run_fresh(int type, bool nan, char* p1, char* p2, char* p3, ssize_t s1, ssize_t s2, uint64_t n);
 bool mulsum_rows(int type, bool nan, const cumo_hip_mulsum_rows_t* d, bool fresh);
 
-// where.hip: the hits of a mask counted, and waited for; their positions or elements placed, their number being known
-int where_count_wait(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts, uint64_t* total);
+// where.hip: places the positions or elements of a mask's hits, whose number the caller knows
 void where_place(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, const uint64_t* counts, uint64_t hits, const char* x, ssize_t sx,
                  size_t elmsz, char* out);
 

@@ -1682,17 +1682,21 @@ int result_1d(NA* z, int type, size_t n, bool* allocated) {
         return fail(CUMO_HIP_ERROR_SHAPE, "the given result must be a contiguous 1-D array of the result's type and exact length");
     return 0;
 }
-// A mask that walks as one run: its hits are counted block by block, their total read back
-// (the one stream synchronisation) to size the result, and the same counts then place the hits: positions (x == NULL, as itype) or the elements of the run
+// A mask that walks as one run: its hits are counted block by block, the counts read back
+// (the one stream synchronisation) and added up here to size the result, and the same
+// counts then place the hits: positions (x == NULL, as itype) or the elements of the run
 // (x, sx) of xtype.
 int where_single_run(const LP& lp, int invert, int rtype, const char* x, ssize_t sx, NA* z) {
     const cumo_hip_loop_args_t& in = lp.args[0];
     const uint64_t n = lp.n[0];
     const size_t nb = cumo_hip_bit_where_blocks(n);
+    uint64_t host_counts[1024];
+    if (nb > sizeof(host_counts) / sizeof(host_counts[0])) return fail(CUMO_HIP_ERROR_ARGUMENT, "where: more block counts than expected");
     uint64_t* counts = reinterpret_cast<uint64_t*>(cumo_cuda_runtime_malloc(nb * sizeof(uint64_t)));
     if (!counts) return CUMO_HIP_ERROR_OUT_OF_MEMORY;
+    int rc = cumo_hip_bit_where_count_to_host((CUMO_BIT_DIGIT*)in.ptr, in.bitpos, in.step[0], n, invert, counts, host_counts);
     uint64_t n_hit = 0;
-    int rc = cumo_hip::where_count_wait((CUMO_BIT_DIGIT*)in.ptr, in.bitpos, in.step[0], n, invert, counts, nullptr, &n_hit);
+    for (size_t b = 0; !rc && b < nb; ++b) n_hit += host_counts[b];
     bool allocated = false;
     if (!rc) rc = result_1d(z, rtype, (size_t)n_hit, &allocated);
     if (!rc && n_hit != 0)

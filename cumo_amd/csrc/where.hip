@@ -115,14 +115,15 @@ __device__ __forceinline__ uint32_t wh_block_exscan32(uint32_t v, uint32_t* tota
     return before + inc - v;
 }
 
-// The hits of every placing block's share of the chunks: a block counts for kWhGroups of them, 256 lanes each. host_words: pinned
-// host memory that the caller looks at, for each share's count (host_each) or for the block's total, one up so that no count is
-// the 0 the host looks for. Every word is a write across the link and every line of them a miss of the caller's, one behind
-// the other: a pass over 8192 x 4096 SFloat that reads back two masks' counts takes 164 us by 1024 words each, 158 by 256 totals.
+// The hits of every placing block's share of the chunks: a block counts for kWhGroups of them, 256 lanes each, four words in
+// flight a lane. host_sums: pinned host memory that the caller looks at, which gets a copy of each count, one up so that no count
+// is the 0 the host looks for. Measured with x.where and x[mask] of 2^25 SFloat, the host's time, us a call: blocks of one share
+// and one word in flight a lane 27.3 and (a hit in a thousand) 22.8, this 23.7 and 18.9; the total of a block's four counts to
+// the host in their place, a quarter of the words, 24.5 and 19.7.
 constexpr int kWhGroups = 4;
 __global__ __launch_bounds__(kWhBlock * kWhGroups) void where_count_kernel(const CUMO_BIT_DIGIT* a, uint64_t p, int64_t s, const size_t* idx, uint64_t n,
                                                                            int contiguous, int invert, uint64_t nchunks, uint64_t cpb, uint64_t nshares,
-                                                                           uint64_t* sums, uint64_t* host_words, int host_each) {
+                                                                           uint64_t* sums, uint64_t* host_sums) {
     __shared__ uint64_t wave_sum[kWhBlock * kWhGroups / 64];
     const unsigned t = threadIdx.x % kWhBlock;
     const uint64_t share = (uint64_t)blockIdx.x * kWhGroups + threadIdx.x / kWhBlock;
@@ -158,13 +159,8 @@ __global__ __launch_bounds__(kWhBlock * kWhGroups) void where_count_kernel(const
         const uint64_t at = (uint64_t)blockIdx.x * kWhGroups + threadIdx.x;
         if (at < nshares) {
             sums[at] = mine;
-            if (host_words && host_each) __hip_atomic_store(host_words + at, mine + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (host_sums) __hip_atomic_store(host_sums + at, mine + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
-    }
-    if (threadIdx.x == 0 && host_words && !host_each) {
-        uint64_t all = 0;
-        for (unsigned k = 0; k < WPS * kWhGroups; ++k) all += wave_sum[k];
-        __hip_atomic_store(host_words + blockIdx.x, all + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 inline unsigned wh_count_grid(uint64_t nblocks) { return (unsigned)((nblocks + kWhGroups - 1) / kWhGroups); }
@@ -362,7 +358,7 @@ void where_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, size_t* idx, uint64_t 
     const int contiguous = (idx == nullptr && s == 1) ? 1 : 0;
     hipStream_t st = current_stream();
     hipLaunchKernelGGL(where_count_kernel, dim3(wh_count_grid(nblocks)), dim3(kWhBlock * kWhGroups), 0, st, a, (uint64_t)p, (int64_t)s, (const size_t*)idx, n,
-                       contiguous, invert, nchunks, cpb, nblocks, block_sums, (uint64_t*)nullptr, 0);
+                       contiguous, invert, nchunks, cpb, nblocks, block_sums, (uint64_t*)nullptr);
     hipLaunchKernelGGL(where_scan_kernel, dim3(1), dim3(kWhBlock), 0, st, block_sums, nblocks, running);
 #define WH_SCATTER(ES)                                                                                                                      \
     hipLaunchKernelGGL((where_scatter_kernel<MODE, ES, false>), dim3((unsigned)nblocks), dim3(kWhBlock), 0, st, a, (uint64_t)p, (int64_t)s,     \
@@ -457,74 +453,6 @@ void where_place(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert,
     cumo_cuda_runtime_check_kernel_launch();
 }
 
-// The counts in device memory, and on the host when the call returns each of them (host_counts) or their sum (*total): the
-// kernel writes into pinned host memory of the calling thread as well, and the host looks at that memory until every word is there. They are the last thing
-// the stream has been given, so nothing earlier is still running then. A stream that has not come this far within
-// kWhLookNs is waited for instead, which also reports what may have gone wrong on it. Looking costs the caller's core
-// what the runtime's own wait costs it, and saves the wait's way through a signal: SFloat 104 x 96 x[mask]
-// 20.9 -> 15.8 us, mask.where() 20.0 -> 15.2 us.
-constexpr int64_t kWhLookNs = 2000000;
-int where_count_wait(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts, uint64_t* total) {
-    if (total) *total = 0;
-    if (n == 0) return CUMO_HIP_OK;
-    const WhGeometry g = wh_geometry(n);
-    static thread_local uint64_t* pinned = nullptr;   // kWhMaxBlocks words, kept for the thread's lifetime
-    if (pinned == nullptr) {
-        void* m = nullptr;
-        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc"))
-            return CUMO_HIP_ERROR_RUNTIME;
-        pinned = static_cast<uint64_t*>(m);
-    }
-    int each = host_counts != nullptr ? 1 : 0;
-    const uint64_t nwords = each ? g.nblocks : wh_count_grid(g.nblocks);
-    std::memset(pinned, 0, nwords * sizeof(uint64_t));
-    hipStream_t st = current_stream();
-    // The launch's own status: hipGetLastError would answer for an earlier call of the thread as well, and a kernel that has been
-    // queued must be waited for, or its counts could be taken for the next call's.
-    uint64_t first = p, words = n, *host = pinned;
-    int64_t step = s;
-    const size_t* idx = nullptr;
-    int contiguous = s == 1 ? 1 : 0;
-    WhGeometry kg = g;
-    void* args[] = {&a, &first, &step, &idx, &words, &contiguous, &invert, &kg.nchunks, &kg.cpb, &kg.nblocks, &counts, &host, &each};
-    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(where_count_kernel), dim3(wh_count_grid(g.nblocks)), dim3(kWhBlock * kWhGroups), args, 0, st);
-    if (launched != hipSuccess) {
-        (void)hipGetLastError();
-        report_hip_error(launched, "kernel launch");
-        return CUMO_HIP_ERROR_RUNTIME;
-    }
-    // (under capture nothing has been queued that could leave a count: the runtime's wait refuses at once, as it always has)
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        capturing = hipStreamCaptureStatusActive;
-    }
-    if (capturing != hipStreamCaptureStatusNone && !hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
-    const auto begin = std::chrono::steady_clock::now();
-    uint64_t b = 0;
-    for (unsigned looks = 0; b < nwords; ++looks) {
-        while (b < nwords && __atomic_load_n(pinned + b, __ATOMIC_ACQUIRE) != 0) ++b;
-        if (b == nwords) break;
-        __builtin_ia32_pause();
-        if ((looks & 63u) == 63u && (std::chrono::steady_clock::now() - begin) > std::chrono::nanoseconds(kWhLookNs)) {
-            if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
-            break;
-        }
-    }
-    if (!wait_trouble_check()) return CUMO_HIP_ERROR_RUNTIME;
-    for (b = 0; b < nwords; ++b) {
-        const uint64_t word = __atomic_load_n(pinned + b, __ATOMIC_RELAXED);
-        if (word == 0) {
-            report_error(CUMO_HIP_ERROR_RUNTIME, 0, "where: a block left no count");
-            return CUMO_HIP_ERROR_RUNTIME;
-        }
-        if (host_counts) host_counts[b] = word - 1;
-        if (total) *total += word - 1;
-    }
-    cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
-    return CUMO_HIP_OK;
-}
-
 }  // namespace cumo_hip
 
 using namespace cumo_hip;
@@ -564,13 +492,73 @@ void cumo_hip_bit_where_count_kernel_launch(CUMO_BIT_DIGIT* a, size_t p, ssize_t
     if (n == 0) return;
     const WhGeometry g = wh_geometry(n);
     hipLaunchKernelGGL(where_count_kernel, dim3(wh_count_grid(g.nblocks)), dim3(kWhBlock * kWhGroups), 0, current_stream(), a, (uint64_t)p, (int64_t)s,
-                       (const size_t*)nullptr, n, s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, g.nblocks, counts, (uint64_t*)nullptr, 0);
+                       (const size_t*)nullptr, n, s == 1 ? 1 : 0, invert, g.nchunks, g.cpb, g.nblocks, counts, (uint64_t*)nullptr);
     cumo_cuda_runtime_check_kernel_launch();
 }
 
+// The same, and the counts on the host when the call returns: the kernel writes them into pinned host memory of the
+// calling thread as well, and the host looks at that memory until every share's count is there. They are the last thing
+// the stream has been given, so nothing earlier is still running then. A stream that has not come this far within
+// kWhLookNs is waited for instead, which also reports what may have gone wrong on it. Looking costs the caller's core
+// what the runtime's own wait costs it, and saves the wait's way through a signal: SFloat 104 x 96 x[mask]
+// 20.9 -> 15.8 us, mask.where() 20.0 -> 15.2 us.
 // host_counts: cumo_hip_bit_where_blocks(n) words of ordinary host memory.
+constexpr int64_t kWhLookNs = 2000000;
 int cumo_hip_bit_where_count_to_host(CUMO_BIT_DIGIT* a, size_t p, ssize_t s, uint64_t n, int invert, uint64_t* counts, uint64_t* host_counts) {
-    return where_count_wait(a, p, s, n, invert, counts, host_counts, nullptr);
+    if (n == 0) return CUMO_HIP_OK;
+    const WhGeometry g = wh_geometry(n);
+    static thread_local uint64_t* pinned = nullptr;   // kWhMaxBlocks words, kept for the thread's lifetime
+    if (pinned == nullptr) {
+        void* m = nullptr;
+        if (!hip_ok(hipHostMalloc(&m, kWhMaxBlocks * sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent), "hipHostMalloc"))
+            return CUMO_HIP_ERROR_RUNTIME;
+        pinned = static_cast<uint64_t*>(m);
+    }
+    std::memset(pinned, 0, g.nblocks * sizeof(uint64_t));
+    hipStream_t st = current_stream();
+    // The launch's own status: hipGetLastError would answer for an earlier call of the thread as well, and a kernel that has been
+    // queued must be waited for, or its counts could be taken for the next call's.
+    uint64_t first = p, words = n, *host = pinned;
+    int64_t step = s;
+    const size_t* idx = nullptr;
+    int contiguous = s == 1 ? 1 : 0;
+    WhGeometry kg = g;
+    void* args[] = {&a, &first, &step, &idx, &words, &contiguous, &invert, &kg.nchunks, &kg.cpb, &kg.nblocks, &counts, &host};
+    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(where_count_kernel), dim3(wh_count_grid(g.nblocks)), dim3(kWhBlock * kWhGroups), args, 0, st);
+    if (launched != hipSuccess) {
+        (void)hipGetLastError();
+        report_hip_error(launched, "kernel launch");
+        return CUMO_HIP_ERROR_RUNTIME;
+    }
+    // (under capture nothing has been queued that could leave a count: the runtime's wait refuses at once, as it always has)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;
+    }
+    if (capturing != hipStreamCaptureStatusNone && !hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+    const auto begin = std::chrono::steady_clock::now();
+    uint64_t b = 0;
+    for (unsigned looks = 0; b < g.nblocks; ++looks) {
+        while (b < g.nblocks && __atomic_load_n(pinned + b, __ATOMIC_ACQUIRE) != 0) ++b;
+        if (b == g.nblocks) break;
+        __builtin_ia32_pause();
+        if ((looks & 63u) == 63u && (std::chrono::steady_clock::now() - begin) > std::chrono::nanoseconds(kWhLookNs)) {
+            if (!hip_ok(hipStreamSynchronize(st), "hipStreamSynchronize")) return CUMO_HIP_ERROR_RUNTIME;
+            break;
+        }
+    }
+    if (!wait_trouble_check()) return CUMO_HIP_ERROR_RUNTIME;
+    for (b = 0; b < g.nblocks; ++b) {
+        const uint64_t word = __atomic_load_n(pinned + b, __ATOMIC_RELAXED);
+        if (word == 0) {
+            report_error(CUMO_HIP_ERROR_RUNTIME, 0, "where: a block left no count");
+            return CUMO_HIP_ERROR_RUNTIME;
+        }
+        host_counts[b] = word - 1;
+    }
+    cumo_cuda_runtime_check_kernel_launch();   // (what an earlier call left on the thread, as behind every other launch)
+    return CUMO_HIP_OK;
 }
 
 // x == NULL: out[o] = the position in the run of the o-th hit, as an elmsz-byte integer (4 or 8);

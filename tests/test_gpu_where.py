@@ -167,7 +167,7 @@ def test_count_then_place_launchers(nbits):
 @pytest.mark.parametrize("nbits", [1, 33, 8192, 8193, 1 << 15, (1 << 15) + 1, (1 << 20) - 5, (1 << 25) + 32 * 1024 + 77])
 def test_counts_of_shares_on_device_and_host(nbits, lead):
     """The blocks of the count take four placing blocks' shares each: every share's count, on the device and on
-    the host, at sizes that end inside a share, a block and a word; and the total of the blocks, which sizes the
+    the host, at sizes that end inside a share, a block and a word; and their sum, which sizes the
     positions, of the set and of the clear bits, of the run and of every third bit of it."""
     from cumo_amd import Bit, _lib
     from test_gpu_raw_abi import dev, fetch, free
