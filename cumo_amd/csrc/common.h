@@ -7,6 +7,7 @@
 #include <stdint.h>
 #include <stddef.h>
 #include "cumo_hip.h"
+#include "store_form.h"
 
 namespace cumo_hip {
 
@@ -102,35 +103,6 @@ WaitCtl* wait_ctl();
 bool wait_trouble_check();
 // Compute units of the current device (queried once).
 int device_compute_units();
-
-// Vector stores of results, 128 bits a lane. Where the lanes of a wave fill whole 64-byte pieces of memory
-// (`pieces`: the result, and each of its rows, starts on one) they are written through the second-level cache at
-// device scope (`sc1`): the last-level cache has the line as it is written, so the operation that reads the result
-// next finds up to about 200 MB of it there, and the second-level cache keeps nothing dirty that it would write back
-// later, in an order of its own, beside what the next operation reads. Measured with a 1R+1W kernel (four vectors in
-// flight a lane, operands loaded non-temporally, every launch on fresh operands), us a launch on the MI355X:
-//   array      copy, plain / nt / sc1    a copy and a copy of its result    a copy and a sum of its result
-//   1 MiB      2.8 / 2.9 / 2.4           5.1 / 5.4 / 4.7                    4.7 / 5.0 / 4.4
-//   16 MiB     7.4 / 6.6 / 7.0           14.1 / 13.3 / 12.9                 10.8 / 10.5 / 10.5
-//   128 MiB    46.8 / 44.2 / 43.4        85.8 / 88.3 / 82.0                 59.6 / 64.4 / 58.0
-//   512 MiB    185 / 175.5 / 175.8       371 / 349 / 351                    248 / 253 / 236
-// From other boundaries every wave would leave part of a piece at each end (128 MiB, 32 bytes off: 47.6 / 45.5 /
-// 49.9), so those results go as they did: non-temporally where NT, from stream_past_caches, says so, else plainly.
-typedef uint32_t store_u4 __attribute__((ext_vector_type(4)));
-constexpr uintptr_t kStorePiece = 64;
-
-// whether every one of these (an address, byte steps) is a whole number of pieces
-template <class... S>
-__device__ __forceinline__ bool store_pieces(const void* p, S... steps) {
-    return (((uintptr_t)p | ... | (uintptr_t)steps) & (kStorePiece - 1)) == 0;
-}
-
-template <bool NT>
-__device__ __forceinline__ void store_vector(store_u4* p, store_u4 v, bool pieces) {
-    if (pieces) __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) store_u4*)p, v, "agent");
-    else if (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
 
 static inline bool hip_ok(hipError_t status, const char* what) {
     if (status == hipSuccess) return true;

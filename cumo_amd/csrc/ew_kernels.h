@@ -130,7 +130,7 @@ __device__ __forceinline__ void raw_load(const char* p, T (&out)[VEC]) {
     for (int j = 0; j < VEC; ++j) out[j] = u.t[j];
 }
 
-// `pieces`: the lanes' vectors together are whole 64-byte pieces (see store_vector)
+// `pieces`: the lanes' vectors together are whole 64-byte pieces (see store_form.h)
 template <class T, int VEC, bool NT>
 __device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC], bool pieces = false) {
     constexpr int BYTES = (int)sizeof(T) * VEC;
@@ -1115,6 +1115,7 @@ struct EwR2Params {
     uint32_t n_tiles;
     int tx_bits;
     int use_scalar;
+    bool through;        // see StoreRows
     int* flag;
 };
 
@@ -1203,7 +1204,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_rows2_kernel(EwR2Params p, Op op,
         char* o = p.ptr[2] + roff[2] + (uint64_t)cv * (VEC * sizeof(R));
         constexpr uint32_t full = (1u << VEC) - 1u;
         if (!Op::CHECKED || okmask == full) {
-            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, store_pieces(p.ptr[2], p.rstep[2], p.ostep[2]));
+            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, p.through && store_pieces(p.ptr[2], p.rstep[2], p.ostep[2]));
         } else {
             if (p.flag) *p.flag = 1;
 #pragma unroll
@@ -1229,6 +1230,7 @@ struct EwR2LeanParams {
     uint32_t col_tiles;
     int tx_bits;
     int mode;            // see ew_rows2_lean_body
+    bool through;        // see StoreRows
     int* flag;
 };
 
@@ -1290,7 +1292,7 @@ __device__ __forceinline__ void ew_rows2_lean_body(const EwR2LeanParams& p, Op o
         char* o = p.ptr[2] + (int64_t)row[u] * p.rstep[2] + (uint64_t)cv * (VEC * sizeof(R));
         constexpr uint32_t full = (1u << VEC) - 1u;
         if (!Op::CHECKED || okmask == full) {
-            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, store_pieces(p.ptr[2], p.rstep[2]));
+            raw_store<R, VEC, (NTM & 4) != 0>(o, zv, p.through && store_pieces(p.ptr[2], p.rstep[2]));
         } else {
             if (p.flag) *p.flag = 1;
 #pragma unroll
@@ -1339,6 +1341,7 @@ struct EwTParams {
     int use_scalar;
     int tr[2];                // input k goes through LDS
     int order;                // how block index maps to tiles: 0 F fastest, 1 G fastest, 2 8x8 super-tiles, 3 F fastest along diagonals
+    bool through;             // see StoreRows
     int* flag;
     uint64_t oshape[kMaxDim - 2];
     int64_t ostep[3][kMaxDim - 2];
@@ -1612,7 +1615,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
 #pragma unroll
                     for (int q = 0; q < V; ++q) zr[q] = tile_r[lg][fv * V + q];
                     char* dstr = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
-                    raw_store<R, V, NT>(dstr, zr, store_pieces(p.ptr[2] + off[2], p.gstep[2]));
+                    raw_store<R, V, NT>(dstr, zr, p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2]));
                     continue;
                 }
                 A x[V];
@@ -1649,7 +1652,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
                 }
                 char* dst = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
                 if (!Op::CHECKED || ok) {
-                    raw_store<R, V, NT>(dst, z, store_pieces(p.ptr[2] + off[2], p.gstep[2]));
+                    raw_store<R, V, NT>(dst, z, p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2]));
                 } else {
                     // some element was rejected: store the others one by one
                     if (p.flag) *p.flag = 1;
@@ -1934,6 +1937,9 @@ static void ew_launch(Op op, const cumo_na_iarray_t* in1, const cumo_na_iarray_t
                 tp.tr[s] = (gs != 0 && fs != 0 && gs < fs) ? 1 : 0;
             }
         }
+        StoreRows out_rows(tp.ptr[2], tp.nf * sizeof(R));
+        for (int d = 0; d < n - 1; ++d) out_rows.dimension(plan.shape[d], d < n - 2 ? tp.ostep[2][d] : tp.gstep[2]);
+        tp.through = out_rows.through(tr_nt);
         uint64_t grid = tp.n_tiles;
         if (grid > 0x7fffffffull) grid = 0x7fffffffull;
         // 128-bit form: same element size everywhere, whole vectors in both tile
@@ -2364,6 +2370,10 @@ static void ew_launch(Op op, const cumo_na_iarray_t* in1, const cumo_na_iarray_t
                 rp.tx_bits = txb;
                 rp.use_scalar = use_scalar;
                 rp.flag = flag;
+                StoreRows out_rows(rp.ptr[2], kp.inner * sizeof(R));
+                out_rows.dimension(plan.shape[n - 2], rp.rstep[2]);
+                if (n == 3) out_rows.dimension(plan.shape[0], rp.ostep[2]);
+                rp.through = out_rows.through(nt);
                 // non-temporal for what streams past once; an operand that repeats along the rows stays cached
                 int ntm = 0;
                 if (nt) {
@@ -2396,6 +2406,7 @@ static void ew_launch(Op op, const cumo_na_iarray_t* in1, const cumo_na_iarray_t
                     lp.col_div = div31_make(rp.col_tiles);
                     lp.tx_bits = txb;
                     lp.mode = use_scalar == 1 ? 3 : (use_scalar == 2 ? 4 : (!rp.walk[1] ? 2 : (rp.rstep[1] == 0 ? 1 : 0)));
+                    lp.through = rp.through;
                     lp.flag = flag;
                     const dim3 g((unsigned)lean_tiles);
 #define CUMO_R2_LAUNCH(V, M) hipLaunchKernelGGL((ew_rows2_lean_kernel<Op, V, M>), g, b, 0, stream, lp, op, sv)

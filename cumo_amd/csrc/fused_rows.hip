@@ -109,6 +109,7 @@ struct FusedRowsParams {
     const char* in;
     char* out;
     double eps;
+    bool through;  // see StoreRows
 };
 
 // MODE 0 softmax, 1 layernorm. TPR lanes share a row, each holding NV vectors of V
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
         auto put = [&](int k) {
             const uint64_t col = ((uint64_t)k * TPR + lane_r) * V;
             if (cnt[k] == V) {
-                store_vector<NT>(reinterpret_cast<u4*>(dst + col * sizeof(T)), x[k].q, store_pieces(p.out, p.out_row_step));
+                store_vector<NT>(reinterpret_cast<u4*>(dst + col * sizeof(T)), x[k].q, p.through && store_pieces(p.out, p.out_row_step));
             } else {
 #pragma unroll
                 for (int j = 0; j < V; ++j)
@@ -235,12 +236,15 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
 }
 
 template <class T, int MODE, int TPR, int NV>
-void fr_launch_one(const FusedRowsParams& p, hipStream_t stream) {
+void fr_launch_one(FusedRowsParams p, hipStream_t stream) {
     constexpr int RPB = kFrBlock / TPR;
     uint64_t grid = (p.rows + RPB - 1) / RPB;
     if (grid > 256u * 64u) grid = 256u * 64u;
     // one read and one write of the array: beyond the 256 MB last-level cache, stream past it
     const bool nt = stream_past_caches(2 * p.rows * p.n * sizeof(T));
+    StoreRows out_rows(p.out, p.n * sizeof(T));
+    out_rows.dimension(p.rows, p.out_row_step);
+    p.through = out_rows.through(nt);
     if (nt) hipLaunchKernelGGL((fused_rows_kernel<T, MODE, TPR, NV, true>), dim3((unsigned)grid), dim3(kFrBlock), 0, stream, p);
     else hipLaunchKernelGGL((fused_rows_kernel<T, MODE, TPR, NV, false>), dim3((unsigned)grid), dim3(kFrBlock), 0, stream, p);
 }
@@ -292,6 +296,7 @@ extern "C" int cumo_hip_fused_rows_kernel_launch(int type, int mode, const cumo_
     p.in = d->in;
     p.out = d->out;
     p.eps = d->eps;
+    p.through = false;  // (fr_launch_one says)
     hipStream_t stream = current_stream();
     bool ok;
     if (type == 0) ok = mode == 0 ? fr_launch<float, 0>(p, stream) : fr_launch<float, 1>(p, stream);

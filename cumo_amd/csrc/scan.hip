@@ -196,6 +196,7 @@ struct ScanRowsParams {
     int64_t s_in, s_out;
     const char* in;
     char* out;
+    bool through;   // see StoreRows (scan_rows_whole_kernel)
 };
 
 template <class T, class Op>
@@ -614,9 +615,10 @@ __device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_t
     chain_fold_waves<T, Op, NW>(s_wave_tot, w, total, wave_pre);
 }
 
-// adds what precedes the tile (if anything) and the earlier waves' total, and stores
+// adds what precedes the tile (if anything) and the earlier waves' total, and stores (pieces: see store_form.h)
 template <class T, class Op, bool NT, int R, bool RAGGED = false>
-__device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, ChainVec<T> (&v)[R], T head, bool head_has, T wave_pre, uint32_t nelem = 0) {
+__device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, ChainVec<T> (&v)[R], T head, bool head_has, T wave_pre, bool pieces,
+                                                 uint32_t nelem = 0) {
     typedef typename ChainVec<T>::u4 u4;
     constexpr int V = ChainVec<T>::V;
     const unsigned lane = threadIdx.x & 63u;
@@ -643,7 +645,7 @@ __device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, Chai
                 continue;
             }
         }
-        store_vector<NT>(dst + r * 64, v[r].q, store_pieces(out));
+        store_vector<NT>(dst + r * 64, v[r].q, pieces);
     }
 }
 
@@ -663,7 +665,7 @@ __device__ __forceinline__ void chain_finish_tile(char* out, uint64_t first, uin
         }
     }
     __syncthreads();
-    chain_store_tile<T, Op, NT, R>(out, first, v, *s_prefix, sh->prefix_has != 0, wave_pre);
+    chain_store_tile<T, Op, NT, R>(out, first, v, *s_prefix, sh->prefix_has != 0, wave_pre, store_pieces(out));
 }
 
 // Many runs, each contiguous on both sides (64 vectors at least, aligned as their elements are):
@@ -687,19 +689,20 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
         }
         T carry = T();
         bool has_carry = false;
+        const bool pieces = p.through && store_pieces(p.out + oo);
         for (uint64_t first = 0; first < p.n; first += CHUNK) {
             ChainVec<T> v[R];
             T total, wave_pre;
             if (p.n - first >= CHUNK) {
                 chain_issue_loads<T, NT, R>(p.in + oi, first, v);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R>(p.out + oo, first, v, carry, has_carry, wave_pre);
+                chain_store_tile<T, Op, NT, R>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces);
             } else {
                 // the run's last chunk, partly there
                 const uint32_t nelem = (uint32_t)(p.n - first);
                 chain_issue_loads<T, NT, R, true>(p.in + oi, first, v, nelem);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R, true>(p.out + oo, first, v, carry, has_carry, wave_pre, nelem);
+                chain_store_tile<T, Op, NT, R, true>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces, nelem);
             }
             carry = has_carry ? Op::apply(carry, total) : total;
             has_carry = true;
@@ -1460,7 +1463,7 @@ void scan_cols_dispatch(int prod, int nan, ScanColsParams& p, hipStream_t stream
 }
 
 template <class T, class Op>
-void scan_rows_launch(const ScanRowsParams& p, hipStream_t stream) {
+void scan_rows_launch(ScanRowsParams& p, hipStream_t stream) {
     if (p.rows == 0 || p.n == 0) return;
     uint64_t grid = p.rows;
     if (grid > 65536) grid = 65536;
@@ -1472,6 +1475,9 @@ void scan_rows_launch(const ScanRowsParams& p, hipStream_t stream) {
     if (whole) {
         const uint64_t vec_rows = (p.n + kScanBlock * V - 1) / (kScanBlock * V);  // rows of 256 vectors in a run, the last one maybe partly there
         const bool nt = stream_past_caches(2 * p.rows * p.n * sizeof(T));
+        StoreRows out_rows(p.out, p.n * sizeof(T));
+        for (int d = 0; d < p.nouter; ++d) out_rows.dimension(p.oshape[d], p.ostep_out[d]);
+        p.through = out_rows.through(nt);
         const dim3 g((unsigned)grid), b(kScanBlock);
 #define CUMO_SCAN_WHOLE(R_) do { if (nt) hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, true, R_>), g, b, 0, stream, p); \
                                  else hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, false, R_>), g, b, 0, stream, p); } while (0)
@@ -1542,7 +1548,7 @@ int scan_run_launch(const char* p1, char* p2, ssize_t s1, ssize_t s2, uint64_t n
 }
 
 template <class T>
-void scan_rows_dispatch(int prod, int nan, const ScanRowsParams& p, hipStream_t stream) {
+void scan_rows_dispatch(int prod, int nan, ScanRowsParams& p, hipStream_t stream) {
     if (prod) {
         if (nan) scan_rows_launch<T, ScanOp<T, 1, true> >(p, stream);
         else scan_rows_launch<T, ScanOp<T, 1, false> >(p, stream);
