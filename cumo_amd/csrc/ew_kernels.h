@@ -130,8 +130,8 @@ __device__ __forceinline__ void raw_load(const char* p, T (&out)[VEC]) {
     for (int j = 0; j < VEC; ++j) out[j] = u.t[j];
 }
 
-// `pieces`: the lanes' vectors together are whole 64-byte pieces (see store_form.h)
-template <class T, int VEC, bool NT>
+// `pieces`: the lanes' vectors together are whole 64-byte pieces; TILE: a tile of many rows at a time (see store_form.h)
+template <class T, int VEC, bool NT, bool TILE = false>
 __device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC], bool pieces = false) {
     constexpr int BYTES = (int)sizeof(T) * VEC;
     union U {
@@ -147,7 +147,8 @@ __device__ __forceinline__ void raw_store(char* p, const T (&in)[VEC], bool piec
 #pragma unroll
         for (int k = 0; k < BYTES / 16; ++k) {
             // (a lane that stores several vectors leaves gaps between them)
-            store_vector<NT>(reinterpret_cast<u32x4*>(p) + k, u.q[k], pieces && BYTES == 16);
+            if constexpr (TILE && BYTES == 16) store_tile_vector<NT>(reinterpret_cast<u32x4*>(p) + k, u.q[k], pieces);
+            else store_vector<NT>(reinterpret_cast<u32x4*>(p) + k, u.q[k], pieces && BYTES == 16);
         }
     } else if constexpr (BYTES == 8) {
         u32x2* dst = reinterpret_cast<u32x2*>(p);
@@ -1611,24 +1612,34 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
                     else if (p.flag) *p.flag = 1;
                 }
             }
+        } else if (EARLY && f < p.nf) {
+            // (the form of the stores picked once a tile: windows of transposed SFloat, whose stores are `nt sc1`, 1 % faster than
+            // with the choice at each)
+            R(*tile_r)[TF + 1] = reinterpret_cast<R(*)[TF + 1]>(ew_transpose_lds);
+            char* const dst0 = p.ptr[2] + off[2] + (int64_t)f * (int64_t)sizeof(R);
+            auto put = [&](auto pieces) {
+#pragma unroll
+                for (unsigned k = 0; k < NQ; ++k) {
+                    const unsigned lg = lg0 + k * GP;
+                    const uint64_t g = g0 + lg;
+                    if (g >= p.ng) continue;
+                    R zr[V];
+#pragma unroll
+                    for (int q = 0; q < V; ++q) zr[q] = tile_r[lg][fv * V + q];
+                    raw_store<R, V, NT, true>(dst0 + (int64_t)g * p.gstep[2], zr, decltype(pieces)::value);
+                }
+            };
+            if (p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2])) put(std::true_type());
+            else put(std::false_type());
         } else if (f < p.nf) {
             // an op with many instructions per element is not unrolled over the rows:
             // its V elements side by side already fill the registers eight waves can have
-            constexpr int UNROLL_ROWS = (op_is_heavy<Op>::value && !EARLY) ? 1 : (int)NQ;
+            constexpr int UNROLL_ROWS = op_is_heavy<Op>::value ? 1 : (int)NQ;
 #pragma unroll UNROLL_ROWS
             for (unsigned k = 0; k < NQ; ++k) {
                 const unsigned lg = lg0 + k * GP;
                 const uint64_t g = g0 + lg;
                 if (g >= p.ng) continue;
-                if constexpr (EARLY) {
-                    R(*tile_r)[TF + 1] = reinterpret_cast<R(*)[TF + 1]>(ew_transpose_lds);
-                    R zr[V];
-#pragma unroll
-                    for (int q = 0; q < V; ++q) zr[q] = tile_r[lg][fv * V + q];
-                    char* dstr = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
-                    raw_store<R, V, NT>(dstr, zr, p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2]));
-                    continue;
-                }
                 A x[V];
                 B y[V];
                 if (NIN >= 1) {
@@ -1663,7 +1674,7 @@ __global__ __launch_bounds__(kEwBlock) void ew_transpose_vec_kernel(EwTParams p,
                 }
                 char* dst = p.ptr[2] + off[2] + (int64_t)g * p.gstep[2] + (int64_t)f * (int64_t)sizeof(R);
                 if (!Op::CHECKED || ok) {
-                    raw_store<R, V, NT>(dst, z, p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2]));
+                    raw_store<R, V, NT, true>(dst, z, p.through && store_pieces(p.ptr[2] + off[2], p.gstep[2]));
                 } else {
                     // some element was rejected: store the others one by one
                     if (p.flag) *p.flag = 1;

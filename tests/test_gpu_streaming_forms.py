@@ -5,8 +5,8 @@ run on the ordinary suites' small inputs in child processes:
                            non-temporal gather / scatter, mulsum, scans and fused rows;
   CUMO_HIP_RED_POLL=0      split reductions with tickets instead of the hand-over words;
   CUMO_HIP_SCAN_CHAIN=0    long runs scanned by the three launches instead of the one pass;
-  CUMO_HIP_SCAN_CHAIN_WAVES=4 the one pass over one long run by blocks of four waves at every size (4097 tiles: the
-                           second supergroup);
+  CUMO_HIP_SCAN_CHAIN_WAVES=4, 8 the one pass over one long run by blocks of four waves, of eight waves, at every size
+                           (4097 tiles of four: the second supergroup);
   CUMO_HIP_SCAN_COLS_CHAIN=0  long runs across memory scanned in two passes over segments;
   CUMO_HIP_SCAN_KEEP_WORDS=0  the one-pass scans with their words from the pool, cleared by a kernel
                            before each launch (what a stream under capture gets);
@@ -32,7 +32,8 @@ ELEMENTWISE = ["tests/test_gpu_elementwise.py::test_float_binary_over_views", "t
                "tests/test_gpu_elementwise.py::test_many_dims_and_permuted_views", "tests/test_gpu_elementwise.py::test_sizes_and_tails",
                "tests/test_gpu_elementwise.py::test_unary_and_rounding", "tests/test_gpu_elementwise.py::test_int32_arithmetic",
                "tests/test_gpu_elementwise.py::test_int32_error_flags", "tests/test_gpu_elementwise.py::test_casts_and_copies",
-               "tests/test_gpu_elementwise.py::test_compare_into_bit", "tests/test_gpu_elementwise.py::test_nmath"]
+               "tests/test_gpu_elementwise.py::test_compare_into_bit", "tests/test_gpu_elementwise.py::test_nmath",
+               "tests/test_gpu_elementwise.py::test_results_on_and_off_whole_pieces_of_memory"]
 REDUCE = ["tests/test_gpu_reduce.py::test_float_reductions_every_axis", "tests/test_gpu_reduce.py::test_random_float_sums",
           "tests/test_gpu_reduce.py::test_nan_rules", "tests/test_gpu_reduce.py::test_int32_reductions",
           "tests/test_gpu_reduce.py::test_min_max_keep_the_zero_that_came_first"]
