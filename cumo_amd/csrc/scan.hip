@@ -297,7 +297,7 @@ __global__ __launch_bounds__(kScanBlock) void scan_apply_kernel(const char* in, 
 // needs the total of everything before it. That comes in a fixed shape, so that results
 // do not change from launch to launch: tiles form groups of 64 and groups form supergroups
 // of 64; the last tile of a group also publishes the group's total and the last tile of a
-// supergroup the supergroup's. A tile folds, each with one wave-wide butterfly, the totals
+// supergroup the supergroup's. A tile folds, each with one scan across a wave, the totals
 // of the earlier tiles of its group, of the earlier groups of its supergroup and of the
 // earlier supergroups. Reads the input once and writes the output once.
 // A published value travels as 64-bit words {the launch's number, 32 bits of the value},
@@ -499,16 +499,16 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
     prefix_has = zh;
 }
 
-// Both sides are contiguous and 16-byte aligned. A whole tile goes wave by wave: a wave owns a
-// quarter of the tile as R rows of 64 vectors, lane l holding vector l of every row (each load
-// and store covers 1 KiB without gaps); the rows are scanned side by side with shuffles, the
-// four waves meet once, in LDS, and what is left to add after the look-back is one value per
+// Both sides are contiguous and 16-byte aligned. A whole tile goes wave by wave: each of the block's
+// four or eight waves owns a part of the tile as R rows of 64 vectors, lane l holding vector l of every
+// row (each load and store covers 1 KiB without gaps); the rows are scanned side by side, the
+// waves meet once, in LDS, and what is left to add after the look-back is one value per
 // wave, so only the tile's elements stay in registers while the block waits. The ragged last
 // tile of a run goes sub-tile by sub-tile through the block-wide scan, reading its input twice.
 // Bound by what a block waits for with nothing in flight: its ticket and the look-back. The
 // steps across a wave go by data-parallel primitives: shuffles put 16 rows times six steps through
-// the LDS unit (2^24 DFloat 75 -> 63 us, 2^22 24.1 -> 20.4, 2^26 SFloat 111 -> 109; with 128 KiB
-// tiles 57.8, 16.4, 102). The three launches take 155 us for 2^26 SFloat. Slower, measured: 32 KiB
+// the LDS unit (64 KiB tiles: 2^24 DFloat 75 -> 63 us, 2^22 24.1 -> 20.2, 2^26 SFloat 114 -> 109; 128 KiB
+// tiles: 72 -> 57, 20.5 -> 16.4, 111 -> 103). The three launches take 155 us for 2^26 SFloat. Slower, measured: 32 KiB
 // tiles; persistent blocks that stage the next tile into LDS with a wave of their own for tickets
 // and look-backs (2^24 DFloat 67 us with 64 KiB tiles, 89 with 32, 141 with 16: the tickets; with
 // tiles dealt out by block index, which could wait for a block that is not running, 63 with 32).
@@ -554,11 +554,8 @@ __device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first
     }
 }
 
-// The tile in v (already loaded) scanned by itself: afterwards every element holds the running
-// value from the start of its wave's quarter, `total` is the tile's total and `wave_pre` the
-// total of the waves before this one (for wave 0: nothing). One barrier, met by every thread.
-// The rows of one wave in v (already loaded) scanned by themselves; returns their total. Eight rows at a time: with the
-// lane totals of sixteen rows of doubles beside the tile 128 registers do not hold it.
+// The rows of one wave in v (already loaded) scanned by themselves; returns their total. Eight rows at a time, so that what
+// is in flight beside the tile stays in registers (a lane of doubles has 168 of them; none is spilled).
 template <class T, class Op, int R>
 __device__ __forceinline__ T chain_scan_wave(ChainVec<T> (&v)[R]) {
     constexpr int V = ChainVec<T>::V;
@@ -606,6 +603,9 @@ __device__ __forceinline__ void chain_fold_waves(const T* s_wave_tot, int w, T& 
     }
 }
 
+// The tile in v (already loaded) scanned by itself: afterwards every element holds the running
+// value from the start of its wave's part, `total` is the tile's total and `wave_pre` the
+// total of the waves before this one (for wave 0: nothing). One barrier, met by every thread.
 template <class T, class Op, int R, int NW = kScanBlock / 64>
 __device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
     const int w = threadIdx.x >> 6;
@@ -887,9 +887,9 @@ int scan_chain_launch(const char* p1, char* p2, ssize_t s1, ssize_t s2, uint64_t
     constexpr int W = ScanChain<T>::W;
     // Blocks of eight waves and 128 KiB tiles wherever that leaves 64 tiles of four-byte elements or 128 to 3072 of eight-byte
     // ones (half the tickets, which one word hands out at about 10 ns each, and half the look-backs per byte), else blocks of
-    // four waves and 64 KiB tiles. Wide / narrow, us on fresh operands: SFloat 2^20 8.8 / 6.5, 2^22 11.2 / 11.4, 2^24 29.1 /
-    // 35.3, 2^26 102 / 109; DFloat 2^20 9.0 / 8.5, 2^21 11.7 / 12.1, 2^22 16.4 / 20.3, 2^24 57.8 / 63.4, 2^25 107.5 / 110, 2^26
-    // 212 / 203 (one wide block of doubles has a compute unit to itself, three narrow ones share it).
+    // four waves and 64 KiB tiles. Wide / narrow, us on fresh operands: SFloat 2^22 11.2 / 11.6, 2^24 29.1 /
+    // 35.2, 2^26 103 / 109; DFloat 2^20 9.0 / 8.6, 2^21 11.8 / 12.2, 2^22 16.4 / 20.2, 2^24 56.5 / 63.2, 2^25 106 / 110, 2^26
+    // 207 / 202 (one wide block of doubles has a compute unit to itself, three narrow ones share it).
     // CUMO_HIP_SCAN_CHAIN_WAVES=4 or 8, read once, fixes the choice.
     static const int forced_waves = [] {
         const char* e = std::getenv("CUMO_HIP_SCAN_CHAIN_WAVES");

@@ -119,7 +119,8 @@ __device__ __forceinline__ uint32_t wh_block_exscan32(uint32_t v, uint32_t* tota
 // flight a lane. host_sums: pinned host memory that the caller looks at, which gets a copy of each count, one up so that no count
 // is the 0 the host looks for. Measured with x.where and x[mask] of 2^25 SFloat, the host's time, us a call: blocks of one share
 // and one word in flight a lane 27.3 and (a hit in a thousand) 22.8, this 23.7 and 18.9; the total of a block's four counts to
-// the host in their place, a quarter of the words, 24.5 and 19.7.
+// the host in their place, a quarter of the words, 24.5 and 19.7. (Masks of a few thousand bits: 14.5 against 14.3; blocks of no
+// more waves than there are shares changed nothing there.)
 constexpr int kWhGroups = 4;
 __global__ __launch_bounds__(kWhBlock * kWhGroups) void where_count_kernel(const CUMO_BIT_DIGIT* a, uint64_t p, int64_t s, const size_t* idx, uint64_t n,
                                                                            int contiguous, int invert, uint64_t nchunks, uint64_t cpb, uint64_t nshares,
