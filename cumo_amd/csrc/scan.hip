@@ -12,11 +12,11 @@
 //                           carried along: many runs (an axis of a matrix), or short ones;
 //   scan_rows_whole_kernel  the same for contiguous runs of whole 256-vector chunks, held
 //                           in registers wave by wave;
-//   scan_chain_kernel       one long contiguous run in one pass: tiles hand their totals on
-//                           through words in memory (read once, written once);
-//   three launches          one long run that is strided or unaligned: per-tile totals, a
-//                           scan of the totals, then every tile scans itself from its
-//                           offset (reads the input twice);
+//   scan_chain_kernel       one contiguous run, or a few long ones, in one pass: tiles hand their
+//                           totals on through words in memory (read once, written once);
+//   three launches          one long run that is strided: per-tile totals, a scan of the
+//                           totals, then every tile scans itself from its offset (reads the
+//                           input twice);
 //   scan_cols_chain_kernel  long runs that lie across memory (down the rows of a matrix) in
 //                           one pass, tiles of 256 rows handing on their column totals;
 //   scan_cols_kernel        other runs across memory, in segments and two passes.
@@ -199,28 +199,37 @@ struct ScanRowsParams {
     bool through;   // see StoreRows (scan_rows_whole_kernel)
 };
 
+// where run `row` starts on either side
+__device__ __forceinline__ void scan_run_start(const ScanRowsParams& p, uint64_t row, const char*& in, char*& out) {
+    int64_t oi = 0, oo = 0;
+#pragma unroll 1
+    for (int d = p.nouter - 1; d >= 0; --d) {
+        const uint64_t m = p.oshape[d];
+        const uint64_t q = row / m;
+        const int64_t k = (int64_t)(row - q * m);
+        row = q;
+        oi += k * p.ostep_in[d];
+        oo += k * p.ostep_out[d];
+    }
+    in = p.in + oi;
+    out = p.out + oo;
+}
+
 template <class T, class Op>
 __global__ __launch_bounds__(kScanBlock) void scan_rows_kernel(ScanRowsParams p) {
     for (uint64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
-        int64_t oi = 0, oo = 0;
-        uint64_t r = row;
-        for (int d = p.nouter - 1; d >= 0; --d) {
-            const uint64_t m = p.oshape[d];
-            const uint64_t q = r / m;
-            const int64_t k = (int64_t)(r - q * m);
-            r = q;
-            oi += k * p.ostep_in[d];
-            oo += k * p.ostep_out[d];
-        }
+        const char* in;
+        char* out;
+        scan_run_start(p, row, in, out);
         T carry = T();
         bool has_carry = false;
         for (uint64_t first = 0; first < p.n; first += kScanTile) {
             const uint64_t left = p.n - first;
             const int cnt = left < (uint64_t)kScanTile ? (int)left : kScanTile;
             T v[kScanPer];
-            scan_load<T>(p.in + oi, p.s_in, first, cnt, v);
+            scan_load<T>(in, p.s_in, first, cnt, v);
             scan_tile<T, Op>(v, cnt, carry, has_carry);
-            scan_store<T>(p.out + oo, p.s_out, first, cnt, v);
+            scan_store<T>(out, p.s_out, first, cnt, v);
         }
     }
 }
@@ -313,17 +322,17 @@ __global__ __launch_bounds__(kScanBlock) void scan_apply_kernel(const char* in, 
 // a tile publishes travels whole in its tagged words.
 constexpr uint32_t kChainSpinLimit = 1u << 22;
 constexpr uint64_t kChainMaxTiles = 64ull * 64ull * 64ull;
+constexpr uint64_t kChainSmallBytes = 16 << 10;
 
 template <class T>
 struct ScanChain {
     static constexpr int W = (int)(sizeof(T) / 4);
-    static constexpr int SUB = 64 / (int)sizeof(T) / 2;        // sub-tiles of the block-wide scan per tile: 64 KiB of elements
-    static constexpr int TILE = kScanTile * SUB;
     WaitCtl* wait;     // where a look-back that gives up reports it
     uint32_t* ticket;
-    uint64_t* tile;    // [n_tiles * W]
-    uint64_t* group;   // [n_groups * W]
-    uint64_t* super;   // [n_supers * W]
+    uint64_t* tile;    // [run][n_tiles][W]
+    uint64_t* group;   // [run][n_groups][W]
+    uint64_t* super;   // [run][n_supers][W]
+    uint32_t n_tiles, n_groups, n_supers;  // of one run
     uint32_t flag;         // the upper half of a word of this launch
     uint32_t ticket_base;  // what the ticket word held before this launch
 };
@@ -499,13 +508,17 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
     prefix_has = zh;
 }
 
-// Both sides are contiguous and 16-byte aligned. A whole tile goes wave by wave: each of the block's
+// Both sides are contiguous and aligned as their elements are. A tile goes wave by wave: each of the block's
 // four or eight waves owns a part of the tile as R rows of 64 vectors, lane l holding vector l of every
 // row (each load and store covers 1 KiB without gaps); the rows are scanned side by side, the
 // waves meet once, in LDS, and what is left to add after the look-back is one value per
 // wave, so only the tile's elements stay in registers while the block waits. The ragged last
-// tile of a run goes sub-tile by sub-tile through the block-wide scan, reading its input twice.
-// Bound by what a block waits for with nothing in flight: its ticket and the look-back. The
+// tile of a run goes the same way with what it lacks read as zeros (sub-tile by sub-tile through the block-wide
+// scan, its input read twice, it took as long as everything before it: SFloat 1975200 19.1 -> 8.9 us, 7489984 28.8 -> 14.0; and
+// without that code a block of doubles needs 110 registers a lane instead of 165, so two wide ones share a compute unit: DFloat 2^24
+// 58.3 -> 54.6, 7489984 29.8 -> 25.7).
+// Several runs (MANY) go level by level: the first tile of every run, then the second of every run, so that a tile waits only for
+// tiles whose blocks are running, as with one run. Bound by what a block waits for with nothing in flight: its ticket and the look-back. The
 // steps across a wave go by data-parallel primitives: shuffles put 16 rows times six steps through
 // the LDS unit (64 KiB tiles: 2^24 DFloat 75 -> 63 us, 2^22 24.1 -> 20.2, 2^26 SFloat 114 -> 109; 128 KiB
 // tiles: 72 -> 57, 20.5 -> 16.4, 111 -> 103). The three launches take 155 us for 2^26 SFloat. Slower, measured: 32 KiB
@@ -649,25 +662,6 @@ __device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, Chai
     }
 }
 
-// scans the tile in v (already loaded), looks back, stores; the barriers inside are met by every thread
-template <class T, class Op, bool NT, int R, int NW>
-__device__ __forceinline__ void chain_finish_tile(char* out, uint64_t first, uint32_t t, ChainVec<T> (&v)[R], const ScanChain<T>& c,
-                                                  T* s_wave_tot, T* s_prefix, ChainShared* sh) {
-    T total, wave_pre;
-    chain_scan_tile<T, Op, R, NW>(v, s_wave_tot, total, wave_pre);
-    if (threadIdx.x < 64) {
-        T pre;
-        bool pre_has;
-        chain_look_back<T, Op>(c, t, total, true, pre, pre_has);
-        if (threadIdx.x == 0) {
-            *s_prefix = pre;
-            sh->prefix_has = pre_has ? 1 : 0;
-        }
-    }
-    __syncthreads();
-    chain_store_tile<T, Op, NT, R>(out, first, v, *s_prefix, sh->prefix_has != 0, wave_pre, store_pieces(out));
-}
-
 // Many runs, each contiguous on both sides (64 vectors at least, aligned as their elements are):
 // one block per run, chunk after chunk of R * 256 vectors in the same wave-by-wave form,
 // the running value handed on in a register; the last chunk may be partly there.
@@ -711,58 +705,60 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
     }
 }
 
-template <class T, class Op, bool NT, int NW>
-__global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_kernel(const char* in, char* out, uint64_t n, ScanChain<T> c) {
+template <class T, class Op, bool NT, int NW, int R, bool MANY>
+__global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_kernel(ScanRowsParams p, ScanChain<T> c) {
     constexpr int V = ChainVec<T>::V;
-    constexpr int R = ScanChain<T>::TILE / (kScanBlock * V);   // rows of 64 vectors per wave
     constexpr int TILE = NW * R * 64 * V;
-    constexpr int PIECE = NW * 64 * kScanPer;                  // what the block-wide scan takes at a time
     __shared__ ChainShared sh;
     __shared__ T s_prefix;
     __shared__ T s_wave_tot[NW];
     if (threadIdx.x == 0) sh.tile = __hip_atomic_fetch_add(c.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - c.ticket_base;
     __syncthreads();
-    const uint32_t t = sh.tile;
+    // the first tile of every run, then the second of every run: runs come along side by side
+    uint32_t t = sh.tile;
+    const char* in = p.in;
+    char* out = p.out;
+    if constexpr (MANY) {
+        const uint32_t rows = (uint32_t)p.rows, row = t % rows;
+        t /= rows;
+        c.tile += (size_t)row * c.n_tiles * ScanChain<T>::W;
+        c.group += (size_t)row * c.n_groups * ScanChain<T>::W;
+        c.super += (size_t)row * c.n_supers * ScanChain<T>::W;
+        scan_run_start(p, row, in, out);
+    }
     const uint64_t first = (uint64_t)t * TILE;
-    if (first >= n) return;  // (the grid is exactly the tiles; a stray ticket does nothing)
-    if (n - first >= (uint64_t)TILE) {
-        ChainVec<T> v[R];
+    if (first >= p.n) return;  // (the grid is exactly the tiles; a stray ticket does nothing)
+    ChainVec<T> v[R];
+    // A run's last tile may be partly there. Loads and the scan stand in one branch each: where the branches met between them the
+    // compiler waited for all loads before the first addition (2^24 SFloat 28.4 -> 30.0 us). The look-back stands once: a second
+    // copy of it took registers that the tile needs.
+    const bool whole = p.n - first >= (uint64_t)TILE;
+    const uint32_t nelem = (uint32_t)(p.n - first);
+    T total, wave_pre;
+    if (whole) {
         chain_issue_loads<T, NT, R>(in, first, v);
-        chain_finish_tile<T, Op, NT, R, NW>(out, first, t, v, c, s_wave_tot, &s_prefix, &sh);
-        return;
+        total = chain_scan_wave<T, Op, R>(v);
+    } else {
+        chain_issue_loads<T, NT, R, true>(in, first, v, nelem);
+        total = chain_scan_wave<T, Op, R>(v);
     }
-    // the ragged last tile: its total first, then the scan from what the look-back gives
-    T total = T();
-    bool total_has = false;
-#pragma clang loop unroll(disable)
-    for (uint64_t f = first; f < n; f += PIECE) {
-        const uint64_t left = n - f;
-        const int cnt = left < (uint64_t)PIECE ? (int)left : PIECE;
-        T v[kScanPer];
-        scan_load<T>(in, (int64_t)sizeof(T), f, cnt, v);
-        scan_tile<T, Op, NW>(v, cnt, total, total_has);
-    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 0) s_wave_tot[w] = total;
+    __syncthreads();
+    chain_fold_waves<T, Op, NW>(s_wave_tot, w, total, wave_pre);
     if (threadIdx.x < 64) {
         T pre;
         bool pre_has;
-        chain_look_back<T, Op>(c, t, total, total_has, pre, pre_has);
+        chain_look_back<T, Op>(c, t, total, true, pre, pre_has);
         if (threadIdx.x == 0) {
             s_prefix = pre;
             sh.prefix_has = pre_has ? 1 : 0;
         }
     }
     __syncthreads();
-    T carry = s_prefix;
-    bool has_carry = sh.prefix_has != 0;
-#pragma clang loop unroll(disable)
-    for (uint64_t f = first; f < n; f += PIECE) {
-        const uint64_t left = n - f;
-        const int cnt = left < (uint64_t)PIECE ? (int)left : PIECE;
-        T v[kScanPer];
-        scan_load<T>(in, (int64_t)sizeof(T), f, cnt, v);
-        scan_tile<T, Op, NW>(v, cnt, carry, has_carry);
-        scan_store<T>(out, (int64_t)sizeof(T), f, cnt, v);
-    }
+    const bool pieces = p.through && store_pieces(out);
+    if (whole) chain_store_tile<T, Op, NT, R>(out, first, v, s_prefix, sh.prefix_has != 0, wave_pre, pieces);
+    else chain_store_tile<T, Op, NT, R, true>(out, first, v, s_prefix, sh.prefix_has != 0, wave_pre, pieces, nelem);
 }
 
 __global__ __launch_bounds__(256) void scan_chain_clear_kernel(uint64_t* words, uint64_t n) {
@@ -801,8 +797,8 @@ static bool chain_keep_enabled() {
     return on;
 }
 
-// words counts the head; tickets = blocks of the launch. False: no memory (the error is set).
-static bool chain_words_acquire(hipStream_t stream, uint64_t words, uint32_t tickets, ChainWords* w) {
+// words counts the head; tickets = blocks of the launch. False: no memory (the error is set), or, with kept_only, no region to keep them in.
+static bool chain_words_acquire(hipStream_t stream, uint64_t words, uint32_t tickets, ChainWords* w, bool kept_only = false) {
     w->flag = 1;
     w->ticket_base = 0;
     w->pooled = true;
@@ -866,6 +862,7 @@ static bool chain_words_acquire(hipStream_t stream, uint64_t words, uint32_t tic
         }
         g_chain_lock.unlock();
     }
+    if (kept_only) return false;
     w->ws = reinterpret_cast<uint64_t*>(cumo_cuda_runtime_malloc(words * sizeof(uint64_t)));
     if (!w->ws) return false;
     uint64_t clear_grid = (words + 255) / 256;
@@ -881,53 +878,69 @@ static void chain_words_release(const ChainWords& w) {
     else g_chain_lock.unlock();
 }
 
-// returns hipSuccess, or an error; -1 when the run does not suit this form
+// Whether the one pass is the better form for `rows` runs of `bytes` bytes than a block to each run: fewer runs than compute units,
+// and each longer than two small tiles and a KiB for every run that shares the device with it. A block to a run / one pass, us:
+// one run: SFloat 20000 6.4 / 4.7, 65013 14.6 / 4.9; several: SFloat [8,20000] 7.3 / 5.3, [100,40000] 12.2 / 10.7, [72,438001] 134 / 54;
+// DFloat [8,20000] 11.2 / 5.8, [32,10000] 7.7 / 6.5, [72,438001] 297 / 102, [200,40000] 33.0 / 30.6. On the other side SFloat [16,5001]
+// 4.3 / 5.4, [200,40000] 16.0 / 19.4, [256,30000] 15.8 / 15.8; DFloat [100,10000] 8.2 / 9.0, [250,20000] 20.5 / 22.6, [500,20000] 29 / 36.
+static bool scan_chain_pays(uint64_t rows, uint64_t bytes) { return rows < 256 && bytes > 2 * kChainSmallBytes + rows * 1024; }
+
+// The runs of p, contiguous and aligned as their elements are (p.through is set), in one pass; kept_only: with words that the stream
+// keeps or not at all.
+enum ChainLaunch { CHAIN_NOT_TAKEN, CHAIN_LAUNCHED, CHAIN_NO_MEMORY };
 template <class T, class Op>
-int scan_chain_launch(const char* p1, char* p2, ssize_t s1, ssize_t s2, uint64_t n, hipStream_t stream) {
+ChainLaunch scan_chain_launch(const ScanRowsParams& p, bool nt, bool kept_only, hipStream_t stream) {
     constexpr int W = ScanChain<T>::W;
-    // Blocks of eight waves and 128 KiB tiles wherever that leaves 64 tiles of four-byte elements or 128 to 3072 of eight-byte
-    // ones (half the tickets, which one word hands out at about 10 ns each, and half the look-backs per byte), else blocks of
-    // four waves and 64 KiB tiles. Wide / narrow, us on fresh operands: SFloat 2^22 11.2 / 11.6, 2^24 29.1 /
-    // 35.2, 2^26 103 / 109; DFloat 2^20 9.0 / 8.6, 2^21 11.8 / 12.2, 2^22 16.4 / 20.2, 2^24 56.5 / 63.2, 2^25 106 / 110, 2^26
-    // 207 / 202 (one wide block of doubles has a compute unit to itself, three narrow ones share it).
+    constexpr uint64_t E = 1024 / sizeof(T);  // elements of a row of 64 vectors
+    // Blocks of eight waves and 128 KiB tiles wherever that leaves 64 tiles of four-byte elements or 128 of eight-byte ones (half
+    // the tickets, which one word hands out at about 10 ns each, and half the look-backs per byte), else blocks of four waves and
+    // 64 KiB tiles, or 16 KiB ones where that makes 128 of them or fewer, so that a short run has more than a few blocks. One run,
+    // us on fresh operands, wide / narrow (small, where it is taken): SFloat 2^18 7.7 / 6.1 (4.9), 2^20 7.9 / 6.4 (256 small tiles 7.9), 2^22
+    // 10.4 / 10.9, 2^24 28.2 / 34.0, 2^26 96.5 / 102; DFloat 2^18 9.1 / 6.5 (6.2), 2^20 10.0 / 9.5, 2^21 11.2 / 11.0, 2^22 15.8 / 19.6,
+    // 2^24 54.2 / 60.7, 2^26 190 / 201.
     // CUMO_HIP_SCAN_CHAIN_WAVES=4 or 8, read once, fixes the choice.
     static const int forced_waves = [] {
         const char* e = std::getenv("CUMO_HIP_SCAN_CHAIN_WAVES");
         return e ? std::atoi(e) : 0;
     }();
-    const uint64_t wide_tile = 2ull * ScanChain<T>::TILE;
-    const uint64_t wide_tiles = (n + wide_tile - 1) / wide_tile;
-    const bool wide = forced_waves == 8 || (forced_waves != 4 && (sizeof(T) == 4 ? wide_tiles >= 64 : wide_tiles >= 128 && wide_tiles <= 3072));
-    const uint64_t tile = wide ? wide_tile : (uint64_t)ScanChain<T>::TILE;
-    const uint64_t n_tiles = (n + tile - 1) / tile;
-    if (n_tiles < 64 || n_tiles > kChainMaxTiles) return -1;
-    if (s1 != (ssize_t)sizeof(T) || s2 != (ssize_t)sizeof(T) || (((uintptr_t)p1 | (uintptr_t)p2) & 15) != 0) return -1;
+    constexpr uint64_t kSmall = kChainSmallBytes / sizeof(T), kNarrow = 4 * 16 * E, kWide = 8 * 16 * E;
+    const uint64_t wide_tiles = p.rows * ((p.n + kWide - 1) / kWide);
+    const bool wide = forced_waves == 8 || (forced_waves != 4 && wide_tiles >= (sizeof(T) == 4 ? 64u : 128u));
+    const bool small = !wide && forced_waves == 0 && p.rows * ((p.n + kSmall - 1) / kSmall) <= 128;
+    const uint64_t tile = wide ? kWide : small ? kSmall : kNarrow;
+    const uint64_t n_tiles = (p.n + tile - 1) / tile;
+    if (n_tiles < 2 || n_tiles > kChainMaxTiles || p.rows * n_tiles > 0x7fffffffull) return CHAIN_NOT_TAKEN;
     const uint64_t n_groups = (n_tiles + 63) / 64, n_supers = (n_groups + 63) / 64;
-    const uint64_t words = kChainHead + (n_tiles + n_groups + n_supers) * W;
+    const uint64_t words = kChainHead + p.rows * (n_tiles + n_groups + n_supers) * W;
     WaitCtl* wait = wait_ctl();
-    if (wait == nullptr) return -1;  // nowhere to report a wait that gives up: the form without waits
+    if (wait == nullptr) return CHAIN_NOT_TAKEN;  // nowhere to report a wait that gives up: the form without waits
     ChainWords cw;
-    if (!chain_words_acquire(stream, words, (uint32_t)n_tiles, &cw)) return (int)hipErrorOutOfMemory;
+    if (!chain_words_acquire(stream, words, (uint32_t)(p.rows * n_tiles), &cw, kept_only)) return kept_only ? CHAIN_NOT_TAKEN : CHAIN_NO_MEMORY;
     ScanChain<T> c;
     c.wait = wait;
     c.ticket = reinterpret_cast<uint32_t*>(cw.ws);
+    c.n_tiles = (uint32_t)n_tiles;
+    c.n_groups = (uint32_t)n_groups;
+    c.n_supers = (uint32_t)n_supers;
     c.tile = cw.ws + kChainHead;
-    c.group = c.tile + n_tiles * W;
-    c.super = c.group + n_groups * W;
+    c.group = c.tile + p.rows * n_tiles * W;
+    c.super = c.group + p.rows * n_groups * W;
     c.flag = cw.flag;
     c.ticket_base = cw.ticket_base;
-    const bool nt = stream_past_caches(2 * n * sizeof(T));
-    const uint64_t grid = n_tiles;
-    if (wide) {
-        if (nt) hipLaunchKernelGGL((scan_chain_kernel<T, Op, true, 8>), dim3((unsigned)grid), dim3(8 * 64), 0, stream, p1, p2, n, c);
-        else hipLaunchKernelGGL((scan_chain_kernel<T, Op, false, 8>), dim3((unsigned)grid), dim3(8 * 64), 0, stream, p1, p2, n, c);
-    } else {
-        if (nt) hipLaunchKernelGGL((scan_chain_kernel<T, Op, true, 4>), dim3((unsigned)grid), dim3(kScanBlock), 0, stream, p1, p2, n, c);
-        else hipLaunchKernelGGL((scan_chain_kernel<T, Op, false, 4>), dim3((unsigned)grid), dim3(kScanBlock), 0, stream, p1, p2, n, c);
-    }
-    const int st = (int)hipGetLastError();
+    const dim3 g((unsigned)(p.rows * n_tiles));
+#define CUMO_SCAN_CHAIN(NT_, NW_, R_)                                                                                                   \
+    do {                                                                                                                                \
+        if (p.rows > 1) hipLaunchKernelGGL((scan_chain_kernel<T, Op, NT_, NW_, R_, true>), g, dim3(NW_ * 64), 0, stream, p, c);        \
+        else hipLaunchKernelGGL((scan_chain_kernel<T, Op, NT_, NW_, R_, false>), g, dim3(NW_ * 64), 0, stream, p, c);                  \
+    } while (0)
+    if (small) CUMO_SCAN_CHAIN(false, 4, 4);
+    else if (wide && nt) CUMO_SCAN_CHAIN(true, 8, 16);
+    else if (wide) CUMO_SCAN_CHAIN(false, 8, 16);
+    else if (nt) CUMO_SCAN_CHAIN(true, 4, 16);
+    else CUMO_SCAN_CHAIN(false, 4, 16);
+#undef CUMO_SCAN_CHAIN
     chain_words_release(cw);
-    return st;
+    return CHAIN_LAUNCHED;
 }
 
 // ---- runs that lie across memory (the scan goes down the rows of a matrix) ------
@@ -1462,6 +1475,15 @@ void scan_cols_dispatch(int prod, int nan, ScanColsParams& p, hipStream_t stream
     }
 }
 
+// CUMO_HIP_SCAN_CHAIN=0 (read once): long runs take the three launches instead of the one pass
+static bool scan_chain_enabled() {
+    static const bool on = [] {
+        const char* e = std::getenv("CUMO_HIP_SCAN_CHAIN");
+        return !(e && e[0] == '0');
+    }();
+    return on;
+}
+
 template <class T, class Op>
 void scan_rows_launch(ScanRowsParams& p, hipStream_t stream) {
     if (p.rows == 0 || p.n == 0) return;
@@ -1478,6 +1500,10 @@ void scan_rows_launch(ScanRowsParams& p, hipStream_t stream) {
         StoreRows out_rows(p.out, p.n * sizeof(T));
         for (int d = 0; d < p.nouter; ++d) out_rows.dimension(p.oshape[d], p.ostep_out[d]);
         p.through = out_rows.through(nt);
+        // (the blocks that take a run each need no memory: neither does this call, under capture or on a stream without a slot)
+        if (scan_chain_enabled() && scan_chain_pays(p.rows, p.n * sizeof(T)) && !stream_under_capture() &&
+            scan_chain_launch<T, Op>(p, nt, true, stream) == CHAIN_LAUNCHED)
+            return;
         const dim3 g((unsigned)grid), b(kScanBlock);
 #define CUMO_SCAN_WHOLE(R_) do { if (nt) hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, true, R_>), g, b, 0, stream, p); \
                                  else hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, false, R_>), g, b, 0, stream, p); } while (0)
@@ -1492,37 +1518,30 @@ void scan_rows_launch(ScanRowsParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((scan_rows_kernel<T, Op>), dim3((unsigned)grid), dim3(kScanBlock), 0, stream, p);
 }
 
-// CUMO_HIP_SCAN_CHAIN=0 (read once): long runs take the three launches instead of the one pass
-static bool scan_chain_enabled() {
-    static const bool on = [] {
-        const char* e = std::getenv("CUMO_HIP_SCAN_CHAIN");
-        return !(e && e[0] == '0');
-    }();
-    return on;
-}
-
-// One run of n elements. Short runs take one block; from 64 tiles of 64 KiB on, contiguous and aligned, the one pass;
-// the three launches are what is left (runs beyond 2^30 elements, or the knob above).
+// One run of n elements: the one pass where it is contiguous; else one block where it is short, and three launches (also for runs
+// beyond 2^30 elements, and with the knob above).
 template <class T, class Op>
 int scan_run_launch(const char* p1, char* p2, ssize_t s1, ssize_t s2, uint64_t n) {
     if (n == 0) return 0;
     hipStream_t stream = current_stream();
     const uint64_t n_tiles = (n + kScanTile - 1) / kScanTile;
+    const bool contiguous = s1 == (ssize_t)sizeof(T) && s2 == (ssize_t)sizeof(T) && (((uintptr_t)p1 | (uintptr_t)p2) % sizeof(T)) == 0;
+    ScanRowsParams p;
+    std::memset(&p, 0, sizeof(p));
+    p.rows = 1;
+    p.n = n;
+    p.s_in = s1;
+    p.s_out = s2;
+    p.in = p1;
+    p.out = p2;
+    p.through = true;
     if (n_tiles <= 8) {
-        ScanRowsParams p;
-        std::memset(&p, 0, sizeof(p));
-        p.rows = 1;
-        p.n = n;
-        p.s_in = s1;
-        p.s_out = s2;
-        p.in = p1;
-        p.out = p2;
         scan_rows_launch<T, Op>(p, stream);
         return (int)hipGetLastError();
     }
-    if (scan_chain_enabled()) {
-        const int st = scan_chain_launch<T, Op>(p1, p2, s1, s2, n, stream);
-        if (st >= 0) return st;
+    if (contiguous && scan_chain_enabled()) {
+        const ChainLaunch how = scan_chain_launch<T, Op>(p, stream_past_caches(2 * n * sizeof(T)), false, stream);
+        if (how != CHAIN_NOT_TAKEN) return how == CHAIN_NO_MEMORY ? (int)hipErrorOutOfMemory : (int)hipGetLastError();
     }
     // One tile per block keeps the most loads in flight (a block that walks a stretch of
     // tiles waits at two barriers per tile: measured 15 % slower). The totals are scanned

@@ -283,8 +283,8 @@ def test_cum_along_contiguous_runs_of_whole_chunks(tname, dt):
 
 @pytest.mark.parametrize("tname,dt", ALL)
 def test_one_long_run_in_one_pass(tname, dt):
-    """Runs from 64 tiles of 64 KiB on are scanned in one pass (by blocks of eight waves with
-    tiles of 128 KiB once there are 64 of those, of eight-byte elements from 128 to 3072), tiles
+    """Long runs are scanned in one pass (by blocks of eight waves with tiles of 128 KiB once
+    there are 64 of those, 128 of eight-byte elements, else with tiles of 64 or 16 KiB), tiles
     handing their totals on through groups of 64 and supergroups of 64 groups: sizes that end
     exactly on a group, one element past it, the same for the larger tiles, and 4096 small
     (2048 large) tiles with a ragged tail; small integers (float sums
@@ -302,7 +302,7 @@ def test_one_long_run_in_one_pass(tname, dt):
         d = cls.cast(h)
         assert_bits_equal(d.cumsum().to_numpy(), oracle.cum("cumsum", h), (n, "cumsum"))
     if dt == np.float64:
-        # eight-byte elements: blocks of eight waves from 128 to 3072 of their tiles
+        # eight-byte elements: blocks of eight waves from 128 of their tiles on
         for n in (254 * tile, 254 * tile + 1, 257 * tile - 1, 6144 * tile, 6144 * tile + 1):
             h = rng.integers(-3, 4, size=n).astype(dt)
             assert_bits_equal(cls.cast(h).cumsum().to_numpy(), oracle.cum("cumsum", h), (n, "cumsum"))
@@ -328,6 +328,43 @@ def test_one_long_run_in_one_pass(tname, dt):
                 assert_bits_equal(d.cumsum().to_numpy(), first, (n, "same bits from launch to launch"))
             exact = np.cumsum(r.astype(np.float64)) if dt == np.float32 else np.asarray(np.cumsum(r.astype(np.longdouble))).astype(np.float64)
             _cum_close(first, exact, np.cumsum(np.abs(r).astype(np.float64)), n, dt, (n, "random floats"))
+
+
+@pytest.mark.parametrize("tname,dt", ALL)
+def test_runs_in_small_tiles_and_several_long_runs_in_one_pass(tname, dt):
+    """Runs of a few 16 KiB tiles: two tiles and what is just longer, one tile more, 128 tiles and one more; starts off a
+    16-byte boundary; and several long runs that share the device, whose tiles come level by level: rows that end inside a
+    vector, windows with gaps, one row more than a level of tiles. Small integers (float sums exact in any order) bit for bit,
+    products of 1, -1 and a few 2s, NaN carried and skipped."""
+    cls = cls_of(tname)
+    rng = np.random.default_rng(58)
+    tile = 16384 // np.dtype(dt).itemsize
+
+    def ints(shape):
+        h = rng.integers(-3, 4, size=shape).astype(dt)
+        return h
+
+    for n in (2 * tile, 2 * tile + 257, 3 * tile, 3 * tile + 1, 17 * tile - 1, 128 * tile, 128 * tile + 1):
+        h = ints(n + 3)
+        d = cls.cast(h)
+        for lead in (0, 1, 3):
+            assert_bits_equal(d[lead:lead + n].cumsum().to_numpy(), oracle.cum("cumsum", np.ascontiguousarray(h[lead:lead + n])), (n, lead))
+    for rows, n in ((2, 3 * tile + 5), (3, 65 * tile + 1), (7, 5 * tile), (31, 17 * tile + 3), (64, 33 * tile + 1)):
+        h = ints((rows, n + 5))
+        d = cls.cast(h)
+        for a, b in ((0, n + 5), (1, n + 1), (3, n - 2)):
+            hv = np.ascontiguousarray(h[:, a:b])
+            assert_bits_equal(d[:, a:b].cumsum(axis=1).to_numpy(), oracle.cum("cumsum", hv, axis=1), (rows, n, a, b))
+    f = rng.choice(np.array([1, -1], dtype=dt), size=(5, 9 * tile + 11))
+    f[rng.integers(0, 5, 20), rng.integers(0, 9 * tile, 20)] = 2
+    assert_bits_equal(cls.cast(f).cumprod(axis=1).to_numpy(), oracle.cum("cumprod", f, axis=1), "cumprod")
+    if dt != np.int32:
+        g = ints((5, 9 * tile + 11))
+        g[rng.integers(0, 5, 900), rng.integers(0, 9 * tile, 900)] = np.nan
+        g[2, :2 * tile] = np.nan
+        d = cls.cast(g)
+        assert_bits_equal(d.cumsum(axis=1, nan=True).to_numpy(), oracle.cum("cumsum", g, axis=1, nan=True), "nan: true")
+        assert_bits_equal(d.cumsum(axis=1).to_numpy(), oracle.cum("cumsum", g, axis=1), "NaN carried")
 
 
 @pytest.mark.parametrize("tname,dt", ALL)
