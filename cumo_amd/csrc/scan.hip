@@ -10,6 +10,7 @@
 // The forms, by layout:
 //   scan_rows_kernel        one block per run, tile after tile with the running value
 //                           carried along: many runs (an axis of a matrix), or short ones;
+//   scan_short_kernel       many short runs, as many to a wave as its registers hold (scan_short.hip);
 //   scan_rows_whole_kernel  the same for contiguous runs of whole 256-vector chunks, held
 //                           in registers wave by wave;
 //   scan_chain_kernel       one contiguous run, or a few long ones, in one pass: tiles hand their
@@ -25,6 +26,7 @@
 // totals through LDS. Everything is in a fixed order, so results do not change
 // from launch to launch.
 #include "common.h"
+#include "scan_ops.h"
 #include "wait_ctl.h"
 
 #include <cstdlib>
@@ -37,29 +39,6 @@ namespace {
 constexpr int kScanBlock = 256;
 constexpr int kScanPer = 8;                         // elements per lane
 constexpr int kScanTile = kScanBlock * kScanPer;    // 2048
-
-template <class T> __device__ __forceinline__ bool scan_is_nan(T x) { return x != x; }
-template <> __device__ __forceinline__ bool scan_is_nan<int32_t>(int32_t) { return false; }
-
-template <class T> struct scan_is_int { static constexpr bool value = false; };
-template <> struct scan_is_int<int32_t> { static constexpr bool value = true; };
-
-// OP: 0 sum, 1 prod. NANF: NaN is skipped.
-template <class T, int OP, bool NANF>
-struct ScanOp {
-    __device__ __forceinline__ static T apply(T a, T b) {
-        if (NANF) {
-            if (scan_is_nan(a)) return b;
-            if (scan_is_nan(b)) return a;
-        }
-        if constexpr (scan_is_int<T>::value) {
-            // Int32: wrapping arithmetic done in unsigned
-            return OP == 0 ? (T)((uint32_t)a + (uint32_t)b) : (T)((uint32_t)a * (uint32_t)b);
-        } else {
-            return OP == 0 ? a + b : a * b;
-        }
-    }
-};
 
 template <class T>
 __device__ __forceinline__ T scan_shfl_up(T v, unsigned d) {
@@ -186,33 +165,6 @@ __device__ __forceinline__ void scan_store(char* p, int64_t s, uint64_t first, i
 #pragma unroll
     for (int k = 0; k < kScanPer; ++k)
         if (base + k < cnt) *reinterpret_cast<T*>(p + (int64_t)(first + base + k) * s) = v[k];
-}
-
-struct ScanRowsParams {
-    int nouter;
-    uint64_t rows, n;
-    uint64_t oshape[CUMO_NA_MAX_DIMENSION];
-    int64_t ostep_in[CUMO_NA_MAX_DIMENSION], ostep_out[CUMO_NA_MAX_DIMENSION];
-    int64_t s_in, s_out;
-    const char* in;
-    char* out;
-    bool through;   // see StoreRows (scan_rows_whole_kernel)
-};
-
-// where run `row` starts on either side
-__device__ __forceinline__ void scan_run_start(const ScanRowsParams& p, uint64_t row, const char*& in, char*& out) {
-    int64_t oi = 0, oo = 0;
-#pragma unroll 1
-    for (int d = p.nouter - 1; d >= 0; --d) {
-        const uint64_t m = p.oshape[d];
-        const uint64_t q = row / m;
-        const int64_t k = (int64_t)(row - q * m);
-        row = q;
-        oi += k * p.ostep_in[d];
-        oo += k * p.ostep_out[d];
-    }
-    in = p.in + oi;
-    out = p.out + oo;
 }
 
 template <class T, class Op>
@@ -373,28 +325,6 @@ __device__ __forceinline__ void chain_join(T& a, bool& a_has, T b, bool b_has) {
     }
 }
 
-// v of another lane by data-parallel primitive (no trip through the LDS unit that shuffles take); lanes without a source keep their own
-template <int CTRL, class T>
-__device__ __forceinline__ T scan_dpp(T v) {
-    constexpr int W = (int)(sizeof(T) / 4);
-    union { T t; int w[W]; } a, b;
-    a.t = v;
-#pragma unroll
-    for (int i = 0; i < W; ++i) b.w[i] = __builtin_amdgcn_update_dpp(a.w[i], a.w[i], CTRL, 0xf, 0xf, false);
-    return b.t;
-}
-
-// v of one lane, the same lane for the whole wave
-template <class T>
-__device__ __forceinline__ T scan_read_lane(T v, uint32_t lane) {
-    constexpr int W = (int)(sizeof(T) / 4);
-    union { T t; int w[W]; } a;
-    a.t = v;
-#pragma unroll
-    for (int i = 0; i < W; ++i) a.w[i] = __builtin_amdgcn_readlane(a.w[i], (int)lane);
-    return a.t;
-}
-
 // Inclusive scan of K values of every lane across the wave, side by side: inside quarters of 16 lanes, then the
 // quarters' totals from lane 15 of the first and third, then the half's from lane 31.
 template <class T, class Op, int K>
@@ -525,13 +455,6 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
 // tiles; persistent blocks that stage the next tile into LDS with a wave of their own for tickets
 // and look-backs (2^24 DFloat 67 us with 64 KiB tiles, 89 with 32, 141 with 16: the tickets; with
 // tiles dealt out by block index, which could wait for a block that is not running, 63 with 32).
-template <class T>
-struct ChainVec {
-    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    static constexpr int V = 16 / (int)sizeof(T);
-    union { u4 q; T e[V]; };
-};
-
 struct ChainShared {
     uint32_t tile;
     int prefix_has;
@@ -541,9 +464,9 @@ struct ChainShared {
 // after everything that exists, so what they add to never reaches an element that is stored).
 // The one vector that is partly there goes element by element: nothing is read past the run.
 template <class T, bool NT, int R, bool RAGGED = false>
-__device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first, ChainVec<T> (&v)[R], uint32_t nelem = 0) {
-    typedef typename ChainVec<T>::u4 u4;
-    constexpr int V = ChainVec<T>::V;
+__device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first, ScanVec<T> (&v)[R], uint32_t nelem = 0) {
+    typedef typename ScanVec<T>::u4 u4;
+    constexpr int V = ScanVec<T>::V;
     const unsigned lane = threadIdx.x & 63u;
     const int w = threadIdx.x >> 6;
     const u4* src = reinterpret_cast<const u4*>(in + (first + (uint64_t)w * (R * 64 * V)) * sizeof(T)) + lane;
@@ -570,8 +493,8 @@ __device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first
 // The rows of one wave in v (already loaded) scanned by themselves; returns their total. Eight rows at a time, so that what
 // is in flight beside the tile stays in registers (a lane of doubles has 168 of them; none is spilled).
 template <class T, class Op, int R>
-__device__ __forceinline__ T chain_scan_wave(ChainVec<T> (&v)[R]) {
-    constexpr int V = ChainVec<T>::V;
+__device__ __forceinline__ T chain_scan_wave(ScanVec<T> (&v)[R]) {
+    constexpr int V = ScanVec<T>::V;
     constexpr int K = R < 8 ? R : 8;
     static_assert(R % K == 0, "rows in whole groups");
     const unsigned lane = threadIdx.x & 63u;
@@ -620,7 +543,7 @@ __device__ __forceinline__ void chain_fold_waves(const T* s_wave_tot, int w, T& 
 // value from the start of its wave's part, `total` is the tile's total and `wave_pre` the
 // total of the waves before this one (for wave 0: nothing). One barrier, met by every thread.
 template <class T, class Op, int R, int NW = kScanBlock / 64>
-__device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
+__device__ __forceinline__ void chain_scan_tile(ScanVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
     const int w = threadIdx.x >> 6;
     const T run = chain_scan_wave<T, Op, R>(v);
     if ((threadIdx.x & 63u) == 0) s_wave_tot[w] = run;
@@ -630,10 +553,10 @@ __device__ __forceinline__ void chain_scan_tile(ChainVec<T> (&v)[R], T* s_wave_t
 
 // adds what precedes the tile (if anything) and the earlier waves' total, and stores (pieces: see store_form.h)
 template <class T, class Op, bool NT, int R, bool RAGGED = false>
-__device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, ChainVec<T> (&v)[R], T head, bool head_has, T wave_pre, bool pieces,
+__device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, ScanVec<T> (&v)[R], T head, bool head_has, T wave_pre, bool pieces,
                                                  uint32_t nelem = 0) {
-    typedef typename ChainVec<T>::u4 u4;
-    constexpr int V = ChainVec<T>::V;
+    typedef typename ScanVec<T>::u4 u4;
+    constexpr int V = ScanVec<T>::V;
     const unsigned lane = threadIdx.x & 63u;
     const int w = threadIdx.x >> 6;
     if (w > 0) {
@@ -667,7 +590,7 @@ __device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, Chai
 // the running value handed on in a register; the last chunk may be partly there.
 template <class T, class Op, bool NT, int R>
 __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsParams p) {
-    constexpr int V = ChainVec<T>::V;
+    constexpr int V = ScanVec<T>::V;
     constexpr uint64_t CHUNK = (uint64_t)R * kScanBlock * V;
     __shared__ T s_wave_tot[kScanBlock / 64];
     for (uint64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
@@ -685,7 +608,7 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
         bool has_carry = false;
         const bool pieces = p.through && store_pieces(p.out + oo);
         for (uint64_t first = 0; first < p.n; first += CHUNK) {
-            ChainVec<T> v[R];
+            ScanVec<T> v[R];
             T total, wave_pre;
             if (p.n - first >= CHUNK) {
                 chain_issue_loads<T, NT, R>(p.in + oi, first, v);
@@ -707,7 +630,7 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
 
 template <class T, class Op, bool NT, int NW, int R, bool MANY>
 __global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_kernel(ScanRowsParams p, ScanChain<T> c) {
-    constexpr int V = ChainVec<T>::V;
+    constexpr int V = ScanVec<T>::V;
     constexpr int TILE = NW * R * 64 * V;
     __shared__ ChainShared sh;
     __shared__ T s_prefix;
@@ -728,7 +651,7 @@ __global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_ke
     }
     const uint64_t first = (uint64_t)t * TILE;
     if (first >= p.n) return;  // (the grid is exactly the tiles; a stray ticket does nothing)
-    ChainVec<T> v[R];
+    ScanVec<T> v[R];
     // A run's last tile may be partly there. Loads and the scan stand in one branch each: where the branches met between them the
     // compiler waited for all loads before the first addition (2^24 SFloat 28.4 -> 30.0 us). The look-back stands once: a second
     // copy of it took registers that the tile needs.
@@ -1660,6 +1583,10 @@ void cumo_hip_scan_rows_kernel_launch(int type, int prod, int nan, const cumo_hi
     p.s_out = d->s_out;
     p.in = d->in;
     p.out = d->out;
+    if (scan_short_launch(type, prod, nan, d)) {
+        cumo_cuda_runtime_check_kernel_launch();
+        return;
+    }
     hipStream_t stream = current_stream();
     switch (type) {
         case 0: scan_rows_dispatch<float>(prod, nan, p, stream); break;

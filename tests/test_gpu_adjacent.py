@@ -368,6 +368,46 @@ def test_runs_in_small_tiles_and_several_long_runs_in_one_pass(tname, dt):
 
 
 @pytest.mark.parametrize("tname,dt", ALL)
+def test_many_short_runs_share_a_wave(tname, dt):
+    """Runs of 1 element, of less than a vector, of odd lengths, of whole vectors, up to and just past 4 KiB, as many as end
+    inside a wave's share; one after another, with gaps between them, with gaps between their elements, from two outer
+    dimensions that are one step and from two that are not. Small integers bit for bit, products of 1, -1 and a few 2s, NaN
+    carried and skipped, infinities beside other runs."""
+    cls = cls_of(tname)
+    rng = np.random.default_rng(59)
+    es = np.dtype(dt).itemsize
+    for rows, n in ((9, 1), (5000, 1), (777, 2), (1001, 3), (64, 5), (700, 16), (1300, 37), (2100, 83), (500, 255), (300, 257), (90, 500), (40, 4096 // es - 1),
+                    (40, 4096 // es), (40, 4096 // es + 1), (2, 8), (3, 700)):
+        h = rng.integers(-3, 4, size=(rows, n)).astype(dt)
+        d = cls.cast(h)
+        assert_bits_equal(d.cumsum(axis=1).to_numpy(), oracle.cum("cumsum", h, axis=1), (rows, n))
+        if n > 4:
+            for sl in (np.s_[:, 1:n - 1], np.s_[:, ::2], np.s_[::3, 2:], np.s_[:, ::-1]):
+                hv = np.ascontiguousarray(h[sl])
+                got = (d.reverse(1) if sl[1].step == -1 else d[sl]).cumsum(axis=1).to_numpy()
+                assert_bits_equal(got, oracle.cum("cumsum", hv, axis=1), (rows, n, sl))
+    h = rng.integers(-3, 4, size=(40, 30, 29)).astype(dt)
+    for sl in (np.s_[:, :, :], np.s_[:, 1:29, :], np.s_[::2, :, 3:20]):
+        hv = np.ascontiguousarray(h[sl])
+        assert_bits_equal(cls.cast(h)[sl].cumsum(axis=2).to_numpy(), oracle.cum("cumsum", hv, axis=2), sl)
+    f = rng.choice(np.array([1, -1], dtype=dt), size=(600, 83))
+    f[rng.integers(0, 600, 900), rng.integers(0, 83, 900)] = 2
+    assert_bits_equal(cls.cast(f).cumprod(axis=1).to_numpy(), oracle.cum("cumprod", f, axis=1), "cumprod")
+    if dt != np.int32:
+        g = rng.integers(-3, 4, size=(600, 83)).astype(dt)
+        g[rng.integers(0, 600, 2000), rng.integers(0, 83, 2000)] = np.nan
+        g[5] = np.nan
+        g[7, 3] = np.inf
+        g[8, 82] = -np.inf
+        d = cls.cast(g)
+        assert_bits_equal(d.cumsum(axis=1, nan=True).to_numpy(), oracle.cum("cumsum", g, axis=1, nan=True), "nan: true")
+        assert_bits_equal(d.cumsum(axis=1).to_numpy(), oracle.cum("cumsum", g, axis=1), "NaN carried")
+        r = rng.standard_normal((900, 250)).astype(dt)
+        exact = np.cumsum(r.astype(np.longdouble), axis=1).astype(np.float64)
+        _cum_close(cls.cast(r).cumsum(axis=1).to_numpy(), exact, np.cumsum(np.abs(r).astype(np.float64), axis=1), 250, dt, "random floats")
+
+
+@pytest.mark.parametrize("tname,dt", ALL)
 def test_cum_along_columns_of_tall_wide_and_stacked_arrays(tname, dt):
     """Runs that lie across memory: few segments (the second pass folds their totals
     itself), many (the totals are scanned first, by the same routine), several planes.
