@@ -749,6 +749,16 @@ static inline ColumnSplit red_split_columns(uint64_t groups, uint64_t n, bool wh
     return c;
 }
 
+// Whether long rows that the planner would cut across blocks (fewer than 512 of them, of 16384 elements or more) go a row to
+// a block of kRsWide lanes instead: nothing to hand over between blocks, and 64 KiB of a row in flight on a compute unit. us of
+// sum / argmax on fresh operands, cut across blocks -> a row to a block:
+//  * more than 256 rows, where every block of a cut row would count in on tickets (and its last one fence): 394 x 54853
+//    SFloat 43.5 / 45.5 -> 17.2 / 20.8, 300 x 16384 18.2 / 18.2 -> 6.3 / 9.5, 474 x 23270 DFloat 39.4 / 41.2 -> 16.3 / 20.9;
+//  * 128 to 256 rows, against the hand-over words: 128 x 262144 25.6 / 27.9 -> 24.7 / 26.5, 200 x 100000 15.9 / 18.3 -> 14.7 / 16.1;
+//  * fewer leave compute units idle, which long rows cannot afford (96 x 300000 21.4 -> 27.6) and short ones can (80 x 16384
+//    5.7 -> 4.0, 64 x 40000 6.0 -> 4.9; 64 rows of 400 KB are even).
+static inline bool red_rows_wide(uint64_t rows, uint64_t row_bytes) { return rows >= 128 || (rows >= 48 && row_bytes <= (256u << 10)); }
+
 // The lean kernels of reduce_stream.h for the layouts they take. Returns 1 when the
 // reduction has been launched, 0 when the general kernels must take it, -1 when the
 // caller's fixed scratch is too small (nothing launched).
@@ -864,6 +874,14 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
         }
         if (force_bits >= 0 && force_bits <= 8 && plan.n_split <= 1) p.tpr_bits = (uint32_t)force_bits;
     }
+    if (plan.n_split > 1 && red_rows_wide(plan.out_total, plan.red_total * sizeof(In))) {
+        p.tpr_bits = 10;
+        const dim3 g((unsigned)plan.out_total), b2(kRsWide);
+        if (nt) hipLaunchKernelGGL((red_srow_kernel<Impl, V, true, kRsWide>), g, b2, 0, stream, p, impl);
+        else hipLaunchKernelGGL((red_srow_kernel<Impl, V, false, kRsWide>), g, b2, 0, stream, p, impl);
+        cumo_cuda_runtime_check_kernel_launch();
+        return 1;
+    }
     if (plan.n_split <= 1) {
         const uint64_t rpb = (uint64_t)kRedBlock >> p.tpr_bits;
         uint64_t grid = (plan.out_total + rpb - 1) / rpb;
@@ -875,7 +893,7 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
         return 1;
     }
 
-    // the axis cut over several blocks per output, one launch
+    // the axis cut over several blocks per output (127 of them at most), one launch
     // no more blocks than the axis has tiles (what a block loads in one step)
     const uint64_t tile = (uint64_t)kRedBlock * V * kRsUnroll;
     const uint64_t tiles = (plan.red_total + tile - 1) / tile;

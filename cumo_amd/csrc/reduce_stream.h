@@ -26,6 +26,7 @@
 namespace cumo_hip {
 
 constexpr int kRsUnroll = 4;            // 128-bit loads a lane keeps in flight
+constexpr int kRsWide = 1024;           // lanes of a block that has a long row to itself when there are a few hundred of them
 constexpr int kRsGroup = 32;            // blocks that count in on one first-level ticket when an output has more than kRsOneLevel
 constexpr int kRsOneLevel = 128;        // up to this many blocks per output count in on a single ticket
 constexpr uint32_t kRsTicketWords = 16384;  // ticket words per stream slot
@@ -151,10 +152,11 @@ __device__ __forceinline__ typename Impl::Acc rs_row_scan(const Impl& impl, cons
 
 // Lanes of one output combine; the group's first lane (thread 0 when a block shares the
 // output) ends up with everything, later lanes folded into earlier ones in a fixed order.
-template <class Impl>
+template <class Impl, int BLOCK = kRedBlock>
 __device__ __forceinline__ void rs_group_combine(const Impl& impl, typename Impl::Acc& acc, unsigned tpr_bits,
                                                  typename Impl::Acc* wave_slots) {
     typedef typename Impl::Acc Acc;
+    constexpr unsigned WAVES = BLOCK / 64;
     const unsigned TPR = 1u << tpr_bits;
     const unsigned span = TPR < 64 ? TPR : 64;
     for (unsigned d = span >> 1; d > 0; d >>= 1) {
@@ -164,21 +166,30 @@ __device__ __forceinline__ void rs_group_combine(const Impl& impl, typename Impl
     if (TPR > 64) {
         if ((threadIdx.x & 63) == 0) wave_slots[threadIdx.x >> 6] = acc;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            for (unsigned w = 1; w < kRedBlock / 64; ++w) impl.combine(wave_slots[w], acc);
+        if constexpr (WAVES > 4) {
+            // neighbours first, as within the wave
+            if (threadIdx.x < 64) {
+                acc = wave_slots[threadIdx.x & (WAVES - 1)];
+                for (unsigned d = WAVES >> 1; d > 0; d >>= 1) {
+                    const Acc other = shfl_down_any(acc, d);
+                    impl.combine(other, acc);
+                }
+            }
+        } else if (threadIdx.x == 0) {
+            for (unsigned w = 1; w < WAVES; ++w) impl.combine(wave_slots[w], acc);
         }
         __syncthreads();
     }
 }
 
 // scan + combine (+ the exact second fold where the impl asks for one)
-template <class Impl, int VEC, bool NT>
+template <class Impl, int VEC, bool NT, int BLOCK = kRedBlock>
 __device__ __forceinline__ typename Impl::Acc rs_row_reduce(const Impl& impl, const char* base, uint64_t first, uint64_t every, uint64_t end,
                                                             uint32_t tail, unsigned lane_r, unsigned tpr_bits, int64_t idx_base,
                                                             typename Impl::Acc* wave_slots, int* s_need) {
     typedef typename Impl::Acc Acc;
     Acc acc = rs_row_scan<Impl, VEC, NT>(impl, base, first, every, end, tail, lane_r, tpr_bits, idx_base);
-    rs_group_combine(impl, acc, tpr_bits, wave_slots);
+    rs_group_combine<Impl, BLOCK>(impl, acc, tpr_bits, wave_slots);
     if constexpr (has_exact<Impl>::value) {
         const unsigned TPR = 1u << tpr_bits;
         bool need;
@@ -195,23 +206,24 @@ __device__ __forceinline__ typename Impl::Acc rs_row_reduce(const Impl& impl, co
             typedef typename Impl::Exact Exact;
             const Exact ex = impl.exact();
             // the exact accumulator is wider: its own LDS slots
-            __shared__ typename Exact::Acc exact_slots[kRedBlock / 64];
+            __shared__ typename Exact::Acc exact_slots[BLOCK / 64];
             typename Exact::Acc e = rs_row_scan<Exact, VEC, false>(ex, base, first, every, end, tail, lane_r, tpr_bits, 0);
-            rs_group_combine(ex, e, tpr_bits, exact_slots);
+            rs_group_combine<Exact, BLOCK>(ex, e, tpr_bits, exact_slots);
             acc = impl.from_exact(e);
         }
     }
     return acc;
 }
 
-template <class Impl, int VEC, bool NT>
-__global__ __launch_bounds__(kRedBlock) void red_srow_kernel(RedSParams p, Impl impl) {
+// BLOCK: kRedBlock lanes, or kRsWide of them for a few hundred long rows (red_rows_wide)
+template <class Impl, int VEC, bool NT, int BLOCK = kRedBlock>
+__global__ __launch_bounds__(BLOCK) void red_srow_kernel(RedSParams p, Impl impl) {
     typedef typename Impl::In In;
     typedef typename Impl::Acc Acc;
-    __shared__ Acc wave_slots[kRedBlock / 64];
+    __shared__ Acc wave_slots[BLOCK / 64];
     __shared__ int s_need;
     const unsigned TPR = 1u << p.tpr_bits;
-    const unsigned RPB = (unsigned)kRedBlock >> p.tpr_bits;
+    const unsigned RPB = (unsigned)BLOCK >> p.tpr_bits;
     const unsigned lane_r = threadIdx.x & (TPR - 1);
     const unsigned row_in_block = threadIdx.x >> p.tpr_bits;
     const uint32_t n_rb = (p.n_out + RPB - 1) / RPB;
@@ -222,7 +234,7 @@ __global__ __launch_bounds__(kRedBlock) void red_srow_kernel(RedSParams p, Impl 
         rs_split_out(p, ok ? row : p.n_out - 1, o0, o1);
         const int64_t in_off = (int64_t)o0 * p.in_step[0] + (int64_t)o1 * p.in_step[1];
         const int64_t idx_base = p.index_mode == 2 ? in_off / (int64_t)sizeof(In) : 0;
-        const Acc acc = rs_row_reduce<Impl, VEC, NT>(impl, p.in + in_off, 0, 1, p.n, p.tail, lane_r, p.tpr_bits, idx_base, wave_slots, &s_need);
+        const Acc acc = rs_row_reduce<Impl, VEC, NT, BLOCK>(impl, p.in + in_off, 0, 1, p.n, p.tail, lane_r, p.tpr_bits, idx_base, wave_slots, &s_need);
         if (ok && lane_r == 0) {
             const int64_t a = (int64_t)o0 * p.out_step[0] + (int64_t)o1 * p.out_step[1];
             const int64_t b = (Impl::NOUT > 1) ? (int64_t)o0 * p.out2_step[0] + (int64_t)o1 * p.out2_step[1] : 0;

@@ -485,6 +485,14 @@ def test_runs_that_end_in_part_of_a_vector(tname, dt, shape, axis):
 
 
 @pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("shape,axis", [((48, 16387), 1), ((2, 128, 16384), 2), ((129, 16385), 1)])
+def test_long_rows_with_a_wide_block_each(tname, dt, shape, axis):
+    """Tens to hundreds of rows of 16384 elements or more: a block of 1024 lanes takes a row (four tiles or fewer of
+    it, the last one partly there). The same answers at the row's end as for any other run."""
+    test_runs_that_end_in_part_of_a_vector(tname, dt, shape, axis)
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
 def test_reductions_of_slices_that_start_off_a_16_byte_boundary(tname, dt):
     """Inner slices beginning at an odd column, with lengths that are whole 128-bit accesses: the
     kernels read them with wide loads on element boundaries; along the rows, down the columns, all."""
