@@ -16,8 +16,8 @@
 // in 10^4. Results differ from the chain through that and the order of the two row sums.
 //
 // The reference has no such entry point; the host layer (cumo_hip_na_softmax /
-// cumo_hip_na_layernorm) uses these for contiguous rows of up to 16384 elements and
-// composes the chain otherwise.
+// cumo_hip_na_layernorm) uses these for contiguous rows and composes the chain
+// otherwise.
 #include "common.h"
 #include "ew_ops.h"
 
@@ -45,23 +45,50 @@ __device__ __forceinline__ T fr_shfl_xor(T v, int m) {
 }
 
 // Combines one value per lane over the TPR lanes that share a row; every lane gets
-// the result. The order is fixed (butterfly within the wave, then the four waves in
+// the result. The order is fixed (butterfly within the wave, then the block's waves in
 // index order), so results do not vary from launch to launch.
-template <class T, int TPR, class F>
+template <class T, int TPR, int BLOCK = kFrBlock, class F>
 __device__ __forceinline__ T fr_allreduce(T v, F f) {
     constexpr int SPAN = TPR < 64 ? TPR : 64;
 #pragma unroll
     for (int m = SPAN >> 1; m > 0; m >>= 1) v = f(v, fr_shfl_xor(v, m));
     if constexpr (TPR > 64) {
-        __shared__ T slot[kFrBlock / 64];
+        __shared__ T slot[BLOCK / 64];
         __syncthreads();  // the slots may still be read from the previous use
         if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = v;
         __syncthreads();
         v = slot[0];
 #pragma unroll
-        for (int w = 1; w < kFrBlock / 64; ++w) v = f(v, slot[w]);
+        for (int w = 1; w < BLOCK / 64; ++w) v = f(v, slot[w]);
     }
     return v;
+}
+
+// The lanes' parts of a row's sum. DFloat carries what each addition rounds off (the two-sum of Knuth, The Art of Computer
+// Programming 2, 4.2.2) beside the sum: sixteen waves' parts one after the other would cost most of a last place. An infinite
+// sum has no such rest.
+template <class T, int LANES>
+__device__ __forceinline__ double fr_allsum(double v) {
+    if constexpr (sizeof(T) == 4) {
+        return fr_allreduce<double, LANES, LANES>(v, [](double a, double b) { return a + b; });
+    } else {
+        struct Sum { double s, r; };
+        auto add = [](Sum a, Sum b) {
+            const double s = a.s + b.s, bb = s - a.s;
+            return Sum{s, (a.r + b.r) + ((a.s - (s - bb)) + (b.s - bb))};
+        };
+        Sum t = {v, 0.0};
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1) t = add(t, Sum{fr_shfl_xor(t.s, m), fr_shfl_xor(t.r, m)});
+        __shared__ Sum slot[LANES / 64];
+        __syncthreads();  // the slots may still be read from the previous use
+        if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = t;
+        __syncthreads();
+        t = slot[0];
+#pragma unroll
+        for (int w = 1; w < LANES / 64; ++w) t = add(t, slot[w]);
+        return t.s - t.s == 0.0 ? t.s + t.r : t.s;
+    }
 }
 
 template <class T> __device__ __forceinline__ T fr_exp(T x);
@@ -85,7 +112,7 @@ template <class T> __device__ __forceinline__ T fr_fmax(T a, T b);
 template <> __device__ __forceinline__ float fr_fmax<float>(float a, float b) { return __builtin_fmaxf(a, b); }
 template <> __device__ __forceinline__ double fr_fmax<double>(double a, double b) { return __builtin_fmax(a, b); }
 
-// x / s for many x and one s, with the result of the IEEE division in T.
+// x / s for many x and one s, with the result of the IEEE division in T where s is a T.
 // float: x / s = float(double(x) * (1.0 / double(s))). The product is within 2^-52 of
 // the quotient, while the quotient of two 24-bit numbers is never closer than 2^-49
 // (relative) to the midpoint of two floats unless it is a float itself, so the one
@@ -94,7 +121,7 @@ template <> __device__ __forceinline__ double fr_fmax<double>(double a, double b
 template <class T> struct FrDivisor;
 template <> struct FrDivisor<float> {
     double r;
-    __device__ __forceinline__ explicit FrDivisor(float s) : r(1.0 / (double)s) {}
+    __device__ __forceinline__ explicit FrDivisor(double s) : r(1.0 / s) {}
     __device__ __forceinline__ float divide(float x) const { return (float)((double)x * r); }
 };
 template <> struct FrDivisor<double> {
@@ -190,7 +217,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
                 }
             }
             s = fr_allreduce<T, TPR>(s, [](T a, T b) { return a + b; });
-            const FrDivisor<T> by_s(s);
+            const FrDivisor<T> by_s((double)s);
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
                 if (cnt[k] > 0) {
@@ -235,23 +262,295 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
     }
 }
 
+// ---- rows that the registers of 256 lanes do not hold --------------------------------
+// One stretch of a row in the registers of a block: whole vectors, lane l holding vectors l, l + LANES, ..., and, one to a lane,
+// the elements behind the last whole one. A vector is there or not (one compare, whose outcome is not kept: with a count for
+// every vector and a mask for every element a block of 1024 lanes had 82 registers a lane instead of 64, and a compute unit
+// one such block instead of two).
+template <class T, int LANES, int NV>
+struct FrStretch {
+    static constexpr int V = 16 / (int)sizeof(T);
+    static constexpr uint32_t kElements = LANES * NV * V;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    union Vec { u4 q; T t[V]; __device__ Vec() {} };
+    Vec x[NV];
+    T last;
+    uint32_t vectors, rest;  // whole vectors of the stretch, elements behind them
+
+    __device__ __forceinline__ bool has(int k) const { return (uint32_t)k * LANES + threadIdx.x < vectors; }
+    __device__ __forceinline__ bool has_last() const { return threadIdx.x < rest; }
+
+    // `row`: the start of the row, which has one whole vector at least. A lane without a vector reads the stretch's first one, or
+    // the row's: no branch between the loads, and an address every lane of the block shares.
+    template <bool NT>
+    __device__ __forceinline__ void load(const char* row, uint64_t start, uint32_t held) {
+        const char* src = row + start * sizeof(T);
+        vectors = held / V;
+        rest = held % V;
+        const char* whole = vectors ? src : row;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const u4* ld = reinterpret_cast<const u4*>(whole + (has(k) ? ((uint32_t)k * LANES + threadIdx.x) * 16u : 0u));
+            x[k].q = NT ? __builtin_nontemporal_load(ld) : *ld;
+        }
+        last = *reinterpret_cast<const T*>(src + (has_last() ? (vectors * V + threadIdx.x) * (uint32_t)sizeof(T) : 0u));
+    }
+    __device__ __forceinline__ void fill(T none) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const bool there = has(k);
+#pragma unroll
+            for (int j = 0; j < V; ++j) x[k].t[j] = there ? x[k].t[j] : none;
+        }
+        last = has_last() ? last : none;
+    }
+    template <class F>
+    __device__ __forceinline__ void each(F f) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) f(x[k].t[j]);
+            if constexpr (NV > 8) __builtin_amdgcn_sched_barrier(0);
+        }
+        f(last);
+    }
+    // f of every element that is there, to memory
+    template <bool NT, class F>
+    __device__ __forceinline__ void store(char* row, uint64_t start, bool pieces, F f) {
+        char* dst = row + start * sizeof(T);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            if (has(k)) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) x[k].t[j] = f(x[k].t[j]);
+                store_vector<NT>(reinterpret_cast<u4*>(dst + ((uint32_t)k * LANES + threadIdx.x) * 16u), x[k].q, pieces);
+            }
+            if constexpr (NV > 8) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (has_last()) reinterpret_cast<T*>(dst)[vectors * V + threadIdx.x] = f(last);
+    }
+    // the largest element, NaN where there is one; wants absent elements to be -inf
+    __device__ __forceinline__ T maximum() {
+        T m = -INFINITY;
+        bool any_nan = false;
+        each([&](T& v) {
+            any_nan |= (v != v);
+            m = fr_fmax(m, v);
+        });
+        if (any_nan) m = (T)NAN;
+        return fr_allreduce<T, LANES, LANES>(m, [](T a, T b) { return fr_max_nan(a, b); });
+    }
+    // `part` gives what an element adds, which is 0 for one that is not there. A lane adds its elements as pairs of pairs in T,
+    // the lanes' sums meet in double.
+    template <class F>
+    __device__ __forceinline__ double sum(F part) {
+        T s = pairs<0, NV>(part);
+        s += part(last);
+        return fr_allsum<T, LANES>((double)s);
+    }
+    template <int FROM, int N, class F>
+    __device__ __forceinline__ T pairs(F& part) {
+        if constexpr (N == 1) {
+            T a[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) a[j] = part(x[FROM].t[j]);
+            if constexpr (NV > 8) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (V == 4) return (a[0] + a[1]) + (a[2] + a[3]);
+            else return a[0] + a[1];
+        } else {
+            const T low = pairs<FROM, N / 2>(part);
+            return low + pairs<FROM + N / 2, N / 2>(part);
+        }
+    }
+};
+
+template <class T, int MODE, int LANES, bool NT>
+__global__ __launch_bounds__(LANES, 4) void fused_wide_rows_kernel(FusedRowsParams p) {
+    if constexpr (MODE == 0 && sizeof(T) == 4) float_tables_prepare();
+    const bool pieces = p.through && store_pieces(p.out, p.out_row_step);
+    FrStretch<T, LANES, 16> a;
+    a.template load<NT>(p.in + (int64_t)blockIdx.x * p.in_row_step, 0, (uint32_t)p.n);
+    char* dst = p.out + (int64_t)blockIdx.x * p.out_row_step;
+    if constexpr (MODE == 0) {
+        a.fill(-INFINITY);
+        const T m = a.maximum();
+        const double s = a.sum([&](T& v) { return v = fr_exp<T>(v - m); });
+        const FrDivisor<T> by_s(s);
+        a.template store<NT>(dst, 0, pieces, [&](T v) { return by_s.divide(v); });
+    } else {
+        a.fill((T)0);
+        const T mean = (T)(a.sum([](T& v) { return v; }) / (double)p.n);
+        a.each([&](T& v) { v -= mean; });
+        a.fill((T)0);
+        const T var = (T)(a.sum([](T& v) { return v * v; }) / ((double)p.n - 1.0));
+        const T sd = fr_sqrt<T>(var + (T)p.eps);
+        a.template store<NT>(dst, 0, pieces, [&](T v) { return v / sd; });
+    }
+}
+
+// Longer rows, and few of them, are cut into pieces of 32 KiB, a block each, in two launches: the first leaves what the row
+// needs of every piece, the second folds a row's parts in every block again (sixteen bytes a piece, from the second-level cache)
+// and reads the piece once more, in the opposite order, since the pieces read last are still in the last-level cache.
+//   softmax    part {maximum of the piece, sum of exp(x - that maximum)}
+//   layernorm  part {sum of the piece, squared deviations from the piece's own mean}
+// Sums within a piece are the type's; parts are folded in double.
+template <class T> using FrPiece = FrStretch<T, kFrBlock, 8>;
+
+struct FusedSplitParams {
+    FusedRowsParams f;
+    uint32_t pieces;  // of a row
+    double* parts;    // two for each piece, row after row
+};
+
+template <class T>
+__device__ __forceinline__ uint32_t fr_piece_held(const FusedSplitParams& p, uint32_t piece) {
+    const uint64_t left = p.f.n - (uint64_t)piece * FrPiece<T>::kElements;
+    return left < FrPiece<T>::kElements ? (uint32_t)left : FrPiece<T>::kElements;
+}
+
+template <class T, int MODE>
+__global__ __launch_bounds__(kFrBlock) void fused_parts_kernel(FusedSplitParams p) {
+    if constexpr (MODE == 0 && sizeof(T) == 4) float_tables_prepare();
+    const uint32_t row = blockIdx.x / p.pieces, piece = blockIdx.x - row * p.pieces;
+    const uint32_t held = fr_piece_held<T>(p, piece);
+    FrPiece<T> a;
+    a.template load<false>(p.f.in + (int64_t)row * p.f.in_row_step, (uint64_t)piece * FrPiece<T>::kElements, held);
+    double* part = p.parts + 2 * (uint64_t)blockIdx.x;
+    if constexpr (MODE == 0) {
+        a.fill(-INFINITY);
+        const T m = a.maximum();
+        const double s = a.sum([&](T& v) { return fr_exp<T>(v - m); });
+        if (threadIdx.x == 0) {
+            part[0] = (double)m;
+            part[1] = m == (T)-INFINITY ? 0.0 : s;  // (nothing but -inf: adds 0 to a row that has more than that)
+        }
+    } else {
+        a.fill((T)0);
+        const T mean = (T)(a.sum([](T& v) { return v; }) / (double)held);
+        a.each([&](T& v) { v -= mean; });
+        a.fill((T)0);
+        const double q = a.sum([](T& v) { return v * v; });
+        const double r = a.sum([](T& v) { return v; });  // what rounding left of the sum: the deviations do not quite cancel
+        if (threadIdx.x == 0) {
+            part[0] = (double)mean * (double)held + r;
+            part[1] = q;
+        }
+    }
+}
+
+template <class T, int MODE, bool NT>
+__global__ __launch_bounds__(kFrBlock) void fused_apply_kernel(FusedSplitParams p) {
+    const uint32_t at = gridDim.x - 1 - blockIdx.x;
+    const uint32_t row = at / p.pieces, piece = at - row * p.pieces;
+    const uint64_t start = (uint64_t)piece * FrPiece<T>::kElements;
+    FrPiece<T> a;
+    a.template load<NT>(p.f.in + (int64_t)row * p.f.in_row_step, start, fr_piece_held<T>(p, piece));
+    if constexpr (MODE == 0 && sizeof(T) == 4) float_tables_prepare();
+    const double* part = p.parts + 2 * (uint64_t)row * p.pieces;
+    char* dst = p.f.out + (int64_t)row * p.f.out_row_step;
+    const bool pieces = p.f.through && store_pieces(p.f.out, p.f.out_row_step);
+    if constexpr (MODE == 0) {
+        double m = -INFINITY;
+        for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) m = fr_max_nan(m, part[2 * c]);
+        m = fr_allreduce<double, kFrBlock>(m, [](double u, double w) { return fr_max_nan(u, w); });
+        double s = 0.0;
+        for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) s += part[2 * c + 1] * exp(part[2 * c] - m);
+        s = fr_allsum<T, kFrBlock>(s);
+        const T mt = (T)m;  // (a maximum of T's)
+        const FrDivisor<T> by_s(s);
+        a.template store<NT>(dst, start, pieces, [&](T v) { return by_s.divide(fr_exp<T>(v - mt)); });
+    } else {
+        const double n = (double)p.f.n;
+        double s = 0.0;
+        for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) s += part[2 * c];
+        s = fr_allsum<T, kFrBlock>(s);
+        const double mean = s / n;
+        double q = 0.0;
+        for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) {
+            const double held = (double)fr_piece_held<T>(p, c);
+            const double away = part[2 * c] / held - mean;
+            q += part[2 * c + 1] + held * away * away;
+        }
+        q = fr_allsum<T, kFrBlock>(q);
+        const T var = (T)(q / (n - 1.0));
+        const T sd = fr_sqrt<T>(var + (T)p.f.eps);
+        const T mt = (T)mean;
+        a.template store<NT>(dst, start, pieces, [&](T v) { return (v - mt) / sd; });
+    }
+}
+
+// one read and one write of the array: beyond the 256 MB last-level cache, stream past it
+template <class T>
+bool fr_store_form(FusedRowsParams& p) {
+    const bool nt = stream_past_caches(2 * p.rows * p.n * sizeof(T));
+    StoreRows out_rows(p.out, p.n * sizeof(T));
+    out_rows.dimension(p.rows, p.out_row_step);
+    p.through = out_rows.through(nt);
+    return nt;
+}
+
 template <class T, int MODE, int TPR, int NV>
 void fr_launch_one(FusedRowsParams p, hipStream_t stream) {
     constexpr int RPB = kFrBlock / TPR;
     uint64_t grid = (p.rows + RPB - 1) / RPB;
     if (grid > 256u * 64u) grid = 256u * 64u;
-    // one read and one write of the array: beyond the 256 MB last-level cache, stream past it
-    const bool nt = stream_past_caches(2 * p.rows * p.n * sizeof(T));
-    StoreRows out_rows(p.out, p.n * sizeof(T));
-    out_rows.dimension(p.rows, p.out_row_step);
-    p.through = out_rows.through(nt);
-    if (nt) hipLaunchKernelGGL((fused_rows_kernel<T, MODE, TPR, NV, true>), dim3((unsigned)grid), dim3(kFrBlock), 0, stream, p);
+    if (fr_store_form<T>(p)) hipLaunchKernelGGL((fused_rows_kernel<T, MODE, TPR, NV, true>), dim3((unsigned)grid), dim3(kFrBlock), 0, stream, p);
     else hipLaunchKernelGGL((fused_rows_kernel<T, MODE, TPR, NV, false>), dim3((unsigned)grid), dim3(kFrBlock), 0, stream, p);
 }
 
-// picks lanes per row and vectors per lane for the row length (four vectors per lane
-// where the row allows, so that a lane has four loads in flight); false when the row
-// is too long
+// (a launch's lanes number less than 2^32; 2^22 blocks write 128 GiB and more)
+constexpr uint64_t kFrMostBlocks = 1u << 22;
+
+template <class T, int MODE, int LANES>
+void fr_launch_wide(FusedRowsParams p, hipStream_t stream) {
+    const dim3 grid((unsigned)p.rows), block(LANES);
+    if (fr_store_form<T>(p)) hipLaunchKernelGGL((fused_wide_rows_kernel<T, MODE, LANES, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((fused_wide_rows_kernel<T, MODE, LANES, false>), grid, block, 0, stream, p);
+}
+
+template <class T, int MODE>
+bool fr_launch_split(FusedRowsParams p, hipStream_t stream) {
+    const uint64_t pieces = (p.n + FrPiece<T>::kElements - 1) / FrPiece<T>::kElements;
+    if (pieces > kFrMostBlocks / p.rows) return false;
+    const bool nt = fr_store_form<T>(p);
+    char* parts = cumo_cuda_runtime_malloc(2 * sizeof(double) * p.rows * pieces);
+    if (!parts) return true;  // the pool has reported it
+    const FusedSplitParams q = {p, (uint32_t)pieces, reinterpret_cast<double*>(parts)};
+    const dim3 grid((unsigned)(p.rows * pieces)), block(kFrBlock);
+    hipLaunchKernelGGL((fused_parts_kernel<T, MODE>), grid, block, 0, stream, q);
+    cumo_cuda_runtime_check_kernel_launch();
+    if (nt) hipLaunchKernelGGL((fused_apply_kernel<T, MODE, true>), grid, block, 0, stream, q);
+    else hipLaunchKernelGGL((fused_apply_kernel<T, MODE, false>), grid, block, 0, stream, q);
+    cumo_cuda_runtime_free(parts);
+    return true;
+}
+
+// Rows of more than 64 KiB (DFloat 32) were taken to the chain, which has no trouble with a result that overlaps its operand in some other
+// way than element on element; what takes them here leaves those to it.
+template <class T>
+bool fr_apart(const FusedRowsParams& p) {
+    if (p.in == p.out && p.in_row_step == p.out_row_step) return true;
+    auto reach = [&](const char* at, int64_t step, uintptr_t* low, uintptr_t* high) {
+        const int64_t far = step * (int64_t)(p.rows - 1);
+        *low = (uintptr_t)at + (far < 0 ? far : 0);
+        *high = (uintptr_t)at + (far > 0 ? far : 0) + p.n * sizeof(T);
+    };
+    uintptr_t in_low, in_high, out_low, out_high;
+    reach(p.in, p.in_row_step, &in_low, &in_high);
+    reach(p.out, p.out_row_step, &out_low, &out_high);
+    return in_high <= out_low || out_high <= in_low;
+}
+
+// Picks lanes per row and vectors per lane for the row length (four vectors per lane
+// where the row allows, so that a lane has four loads in flight). Beyond 64 KiB (DFloat 32) lanes hold sixteen vectors, 64
+// registers: rows up to 128 KiB take 512 lanes, two blocks to a compute unit, so that one computes while the other's loads and
+// stores are under way; up to 256 KiB 1024 lanes, if there are rows enough; longer ones are cut. us, softmax / layernorm, the
+// chain that all of these took before, then 512 or 1024 lanes, then cut:
+//   SFloat [588,27696]  91.2 / 76.5, 32.8 / 26.6, 50.8 / 39.5     [8,20000]   19.6 / 22.0, 10.5 / 7.4, 11.4 / 10.3
+//   SFloat [400,65000]  211 / 190, 64.1 / 47.6, 66.6 / 55.8       [20,65000]  22.5 / 22.4, 19.2 / 12.7, 13.4 / 10.5
+//   DFloat [762,29665]  230 / 178, 92.9 / 90.5, 103 / 94.1        [33,29738]  24.6 / 26.4, 17.3 / 14.9, 14.3 / 11.6
+//   cut: SFloat [76,440000] 165 / 139, -, 80.0 / 67.0;  DFloat [108,128807] 146 / 123, -, 64.9 / 58.4
+// (1024 lanes with eight vectors each for [588,27696]: 45.5 / 32.1.) false when the shape is left to the chain.
 template <class T, int MODE>
 bool fr_launch(const FusedRowsParams& p, hipStream_t stream) {
     constexpr int V = 16 / (int)sizeof(T);
@@ -266,7 +565,10 @@ bool fr_launch(const FusedRowsParams& p, hipStream_t stream) {
     else if (nv <= 1024) fr_launch_one<T, MODE, 256, 4>(p, stream);
     else if (nv <= 2048) fr_launch_one<T, MODE, 256, 8>(p, stream);
     else if (nv <= 4096 && sizeof(T) == 4) fr_launch_one<T, MODE, 256, 16>(p, stream);
-    else return false;
+    else if (p.rows > kFrMostBlocks || !fr_apart<T>(p)) return false;
+    else if (nv <= 8192) fr_launch_wide<T, MODE, 512>(p, stream);
+    else if (nv <= 16384 && p.rows > 64) fr_launch_wide<T, MODE, 1024>(p, stream);
+    else return fr_launch_split<T, MODE>(p, stream);
     return true;
 }
 

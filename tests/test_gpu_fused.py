@@ -97,3 +97,65 @@ def test_layernorm_matches_the_chain(dt):
     # a row of one element has no variance: NaN from both
     one = cls.cast(np.array([[2.0], [3.0]], dtype=dt))
     assert np.isnan(m.Fused.layernorm(one).to_numpy()).all() and np.isnan(chain_layernorm(m, one, 1e-5).to_numpy()).all()
+
+
+# Rows beyond the registers of 256 lanes: a block of 1024 lanes up to 65536 SFloat / 32768 DFloat, pieces of 8192 / 4096 elements in
+# two launches beyond. Lengths at those edges, a last piece of one element, a last vector that is partly there.
+LONG_ROWS = [(3, 8193), (3, 16385), (5, 32768), (3, 32769), (2, 65533), (3, 65536), (300, 16390), (3, 65537), (7, 70001), (2, 3, 131073), (1, 1 << 20)]
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", LONG_ROWS)
+def test_long_rows_match_64_bit_arithmetic(dt, shape):
+    import cumo_amd as m
+    cls = m.SFloat if dt == np.float32 else m.DFloat
+    n = shape[-1]
+    h = (np.random.default_rng(n).standard_normal(shape) * 2 + 0.5).astype(dt)
+    x = cls.cast(h)
+    w = h.astype(np.longdouble)
+    e = np.exp(w - w.max(axis=-1, keepdims=True))
+    # per element: the difference's rounding (up to half an ulp of ~12), exp, the sum (pairwise, some 2^-23) and the division
+    tol = 16 * np.finfo(dt).eps
+    want = e / e.sum(axis=-1, keepdims=True)
+    assert (np.abs(m.Fused.softmax(x).to_numpy() - want) <= tol * want + np.finfo(dt).tiny).all()
+    c = w - w.mean(axis=-1, keepdims=True)
+    want = c / np.sqrt((c * c).sum(axis=-1, keepdims=True) / (n - 1) + dt(1e-5))
+    assert np.abs(m.Fused.layernorm(x, 1e-5).to_numpy() - want).max() <= tol
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [20001, 70001])
+def test_long_rows_special_values_views_and_overlap(dt, n):
+    import cumo_amd as m
+    cls = m.SFloat if dt == np.float32 else m.DFloat
+    h = (np.random.default_rng(n).standard_normal((6, n)) * 2).astype(dt)
+    h[0, n - 1] = np.nan
+    h[1, :] = -np.inf      # whole pieces of -inf, one of them with a number
+    h[1, 17] = 3.0
+    h[2, 11] = np.inf
+    h[3, :] = -np.inf
+    h[4, :] = 7.5
+    x = cls.cast(h)
+    for key in (slice(None), slice(1, None, 2), slice(None, None, -1)):
+        got = m.Fused.softmax(x[key]).to_numpy()
+        want = chain_softmax(m, x[key]).to_numpy()
+        close(got, want, n, dt, ("softmax", key))
+        got = m.Fused.layernorm(x[key], 1e-5).to_numpy()
+        assert (np.isnan(got) == np.isnan(chain_layernorm(m, x[key], 1e-5).to_numpy())).all()
+    want = m.Fused.softmax(x).to_numpy()
+    assert want[1, 17] == 1.0 and np.count_nonzero(want[1]) == 1 and np.isnan(want[[0, 2, 3]]).all()
+
+
+@pytest.mark.parametrize("n", [20001, 70001])
+def test_long_rows_into_their_operand_and_into_memory_that_overlaps_it(n):
+    import ctypes as C
+    import cumo_amd as m
+    from cumo_amd import _lib
+    h = (np.random.default_rng(n).standard_normal((5, n)) * 2).astype(np.float32)
+    want = m.Fused.softmax(m.SFloat.cast(h[:4])).to_numpy()
+    for down in (0, 1):
+        x = m.SFloat.cast(h)
+        operand, result = x[:4], x[down:4 + down]
+        d, z = operand._desc(), result._desc()
+        assert _lib.lib.cumo_hip_na_softmax(C.byref(d), C.byref(z)) == 0
+        close(x.to_numpy()[down:4 + down], want, n, np.float32, ("rows further down", down))
