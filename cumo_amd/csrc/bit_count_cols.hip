@@ -1,5 +1,6 @@
 // count_true / count_false down the rows of a Bit matrix (the counted dimension is the
-// slow one, the kept one runs along the words), for rows that start on word boundaries.
+// slow one, the kept one runs along the words), for rows that start on word boundaries and
+// short rows that follow one another (fold_rows).
 //
 // The reference has no kernel for this: its ndloop walks the outputs on the host and
 // launches tmpl_bit/bit_count_kernel.cu:4-78 once per output (narray/ndloop.c:1569-1613),
@@ -13,10 +14,13 @@
 // twenty-four a byte-sliced count needs, which alone would take as long as the rows take to
 // arrive. The stretches of a block (its groups of lanes) add their upright counters in a
 // binary tree through LDS, still as planes; only then a thread per column reads its count
-// off the planes. The blocks of a column group leave their counts in scratch, and the one
-// that counts in last (a ticket per column group) adds them up in order and writes the
-// results: no zero-fill launch before and no atomics on the results. count_false counts the
-// set bits too and takes them from the number of rows at the end.
+// off the planes. Where several blocks share columns they leave their counts in scratch, and a
+// second launch adds them up with every compute unit: no zero-fill launch before and no atomics
+// on the results. (The block that counted in last on a ticket added them up before: store,
+// acknowledgement, ticket, fence and reads one after the other in one block a column group. us,
+// that / this: [8192,4096] 10.8 / 9.4, [16384,32768] 18.0 / 16.4, [4096,65536] 13.6 / 10.7,
+// [32768,1024] 15.5 / 10.9, [28296,64] 15.3 / 9.9.) count_false counts the set bits too and takes
+// them from the number of rows at the end.
 #include "bit_common.h"
 
 #include <cstdlib>
@@ -25,7 +29,6 @@ using namespace cumo_hip;
 
 namespace {
 
-constexpr uint32_t kTicketWordsPerSlot = 16384;   // what red_ticket_words() hands out per stream slot (reduce_tickets.hip)
 constexpr int kVcRows = 16;            // rows a lane has in flight
 constexpr uint32_t kVcStretch = 240;   // rows between two additions to the long counter: 15 groups of 16, so planes 4..7 count to 15
 constexpr int kVcPlanes = 8;           // planes of the short counter: up to 255 rows
@@ -36,8 +39,7 @@ constexpr int kVcAuxNt = 2;                  // buffer load cache policy: non-te
 struct BitCountColsVc {
     const uint32_t* in;       // word of (row 0, column 0) of the first outer index
     char* out;
-    uint32_t* partial;        // [n_outer][parts][col_blocks][columns of a block], when parts > 1
-    uint32_t* tickets;        // [n_outer * col_blocks], zero between launches
+    uint32_t* partial;        // [n_outer][parts][col_blocks][columns of a block], where a second launch adds them up
     uint32_t cols, words, col_blocks, rows, rows_per_group, parts, n_outer;
     int64_t s_red_w, s_outer_w;   // steps in words
     int64_t o_outer, o_col;       // result steps in bytes
@@ -93,7 +95,6 @@ __global__ __launch_bounds__(BLOCK) void bit_count_cols_vc_kernel(BitCountColsVc
     static_assert((NG & (NG - 1)) == 0 && BC % BLOCK == 0, "the groups meet in a binary tree; whole columns per thread");
     __shared__ uint32_t planes[NG / 2][kVcBlockPlanes][LANES];   // the counters of the groups that hand theirs over
     __shared__ uint32_t total_planes[kVcBlockPlanes][LANES];
-    __shared__ int s_last;
     static_assert(LANES == 64, "a group is a wave: its rows are the same for every lane, so row addresses are scalar");
     const unsigned lane = threadIdx.x & 63u;
     const unsigned group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(BLOCK) void bit_count_cols_vc_kernel(BitCountColsVc
         for (int q = 0; q < kVcBlockPlanes; ++q) c |= ((total_planes[q][w] >> j) & 1u) << q;
         mine[k] = p.count_false ? rows_here - c : c;
     }
-    if (p.parts == 1) {
+    if (p.partial == nullptr) {
 #pragma unroll
         for (unsigned k = 0; k < CPT; ++k) {
             const uint32_t col = col0 + threadIdx.x + k * BLOCK;
@@ -208,55 +209,54 @@ __global__ __launch_bounds__(BLOCK) void bit_count_cols_vc_kernel(BitCountColsVc
         }
         return;
     }
-    // several blocks share these columns: the counts go to scratch, written through at agent scope,
-    // and the block that counts in last adds them up
-    uint32_t* scratch = p.partial + (((size_t)o * p.parts + part) * p.col_blocks + cb) * BC;
+    uint32_t* left = p.partial + (((size_t)o * p.parts + part) * p.col_blocks + cb) * BC;
 #pragma unroll
-    for (unsigned k = 0; k < CPT; ++k)
-        __hip_atomic_store(scratch + threadIdx.x + k * BLOCK, mine[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(0);   // this thread's stores are acknowledged
-    __syncthreads();                 // ... and every thread's
-    if (threadIdx.x == 0) {
-        uint32_t* t = p.tickets + (size_t)o * p.col_blocks + cb;
-        int last = 0;
-        if (__hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.parts - 1) {
-            __hip_atomic_store(t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last = 1;
-        }
-        s_last = last;
+    for (unsigned k = 0; k < CPT; ++k) left[threadIdx.x + k * BLOCK] = mine[k];
+}
+
+// The counts that blocks left, added up: `parts` of a column, and, where 2^fold_bits rows were taken as one, those of the columns
+// that it became; `rest` rows at the end were in none of them.
+struct FoldCounts {
+    const uint32_t* partial;   // [n_outer][parts][width]
+    const uint32_t* in;
+    char* out;
+    uint64_t rest_bit;         // of the first row left over
+    int64_t o_outer, o_col;
+    uint32_t cols, fold_bits, parts, width, rest, col_groups;
+    int count_false, overwrite;
+};
+
+constexpr uint32_t kFoldCols = 32;   // columns of a block
+
+// LANES lanes share a column
+template <uint32_t LANES>
+__global__ __launch_bounds__(kFoldCols * LANES) void bit_count_fold_kernel(FoldCounts p) {
+    __shared__ uint64_t sums[LANES][kFoldCols];
+    const uint32_t lane = threadIdx.x % kFoldCols, share = threadIdx.x / kFoldCols;
+    const uint32_t o = blockIdx.x / p.col_groups;
+    const uint32_t col = (blockIdx.x - o * p.col_groups) * kFoldCols + lane;
+    const uint32_t c = col < p.cols ? col : p.cols - 1;
+    const uint32_t* counts = p.partial + (uint64_t)o * p.parts * p.width + c;
+    uint64_t n = 0;
+    // eight trips to memory at a time: one after the other they are all that this kernel takes
+    const uint32_t terms = p.parts << p.fold_bits;
+#pragma unroll 8
+    for (uint32_t t = share; t < terms; t += LANES) {
+        const uint32_t q = t >> p.fold_bits, k = t - (q << p.fold_bits);
+        n += counts[(uint64_t)q * p.width + k * p.cols];
     }
+#pragma unroll 8
+    for (uint32_t k = share; k < p.rest; k += LANES) {
+        const uint64_t bit = p.rest_bit + (uint64_t)k * p.cols + c;
+        n += ((p.in[bit >> 5] >> (bit & 31u)) & 1u) ^ (uint32_t)(p.count_false != 0);
+    }
+    sums[share][lane] = n;
     __syncthreads();
-    if (!s_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    const uint32_t* all = p.partial + ((size_t)o * p.parts * p.col_blocks + cb) * BC;
-    const size_t part_step = (size_t)p.col_blocks * BC;
-    // sixteen blocks' counts of every column of this thread asked for at once: one after the other
-    // they cost a trip to memory each, and this block is the only one left running for its columns
-    unsigned long long total[CPT];
+    if (share != 0 || col >= p.cols) return;
 #pragma unroll
-    for (unsigned k = 0; k < CPT; ++k) total[k] = 0;
-    for (uint32_t q0 = 0; q0 < p.parts; q0 += 16) {
-        uint32_t v[CPT][16];
-#pragma unroll
-        for (unsigned k = 0; k < CPT; ++k)
-#pragma unroll
-            for (uint32_t u = 0; u < 16; ++u) {
-                const uint32_t q = q0 + u < p.parts ? q0 + u : p.parts - 1;
-                v[k][u] = all[(size_t)q * part_step + threadIdx.x + k * BLOCK];
-            }
-#pragma unroll
-        for (unsigned k = 0; k < CPT; ++k)
-#pragma unroll
-            for (uint32_t u = 0; u < 16; ++u) total[k] += q0 + u < p.parts ? v[k][u] : 0u;
-    }
-#pragma unroll
-    for (unsigned k = 0; k < CPT; ++k) {
-        const uint32_t col = col0 + threadIdx.x + k * BLOCK;
-        if (col >= p.cols) continue;
-        unsigned long long* dst = reinterpret_cast<unsigned long long*>(p.out + (int64_t)o * p.o_outer + (int64_t)col * p.o_col);
-        *dst = p.overwrite ? total[k] : *dst + total[k];
-    }
+    for (uint32_t k = 1; k < LANES; ++k) n += sums[k][lane];
+    uint64_t* dst = reinterpret_cast<uint64_t*>(p.out + (int64_t)o * p.o_outer + (int64_t)col * p.o_col);
+    *dst = p.overwrite ? n : *dst + n;
 }
 
 // geometry for blocks of BLOCK / LANES groups of LANES lanes; false when the launch does not fit
@@ -275,68 +275,96 @@ bool vc_geometry(BitCountColsVc& p, uint64_t want_blocks, uint64_t* blocks) {
     // offsets inside a stretch of rows are 32-bit operands of the loads
     if (((uint64_t)kVcStretch + kVcRows) * (uint64_t)p.s_red_w * 4 + (uint64_t)p.words * 4 >= 0x7fffffffull) return false;
     *blocks = across * p.parts;
-    return *blocks <= 0x7fffffffull && across <= kTicketWordsPerSlot;
+    return *blocks <= 0x3fffffull;   // (of 1024 lanes: a launch has less than 2^32)
 }
 
 }  // namespace
 
 namespace cumo_hip {
 
+// How many rows to take as one: rows that follow one another, off word boundaries or less than two words long, become the rows
+// of a matrix that is a whole number of words and two blocks wide at least, whose columns are counted in their place. Their counts
+// are 32 times the columns', so wide rows are left to the form that shifts their words into place (bit.hip), which keeps every
+// lane busy with them. us, that form / this: [24304,1066] 23.3 / 9.9, [3512,100] 21.9 / 9.5, [180232,137] 16.6 / 13.5,
+// [65536,33] 124.6 / 9.5, [11400,1903] 13.2 / 10.8, [1000,8001] 13.5 / 10.1, [136,9000] 7.3 / 7.8, [400,30001] 9.4 / 15.3. Rows on word
+// boundaries gain nothing from it: [32768,1024] 10.9 as they are, 14.2 so.
+static uint32_t fold_rows(const cumo_hip_bit_count_nd_t* d) {
+    const uint64_t cols = d->out_shape[d->out_ndim - 1], rows = d->red_shape[0];
+    if (d->out_ndim != 1 || cols > 8192 || (d->pos & 31) != 0 || d->in_red_step[0] != (ssize_t)cols) return 1;
+    if (cols >= 64 && cols % 32 == 0) return 1;
+    uint64_t fold = 1;
+    while ((cols * fold) % 32 != 0 || cols * fold < 4096) fold *= 2;
+    return rows < 4 * fold ? 1 : (uint32_t)fold;
+}
+
 // 1 when launched (the results are then stored or added as d->overwrite says, with no zero-fill
 // needed), 0 when the loop is not one this form takes
 int bit_count_cols_words_launch(const cumo_hip_bit_count_nd_t* d) {
     if (d->red_ndim != 1 || d->out_ndim < 1 || d->out_ndim > 2 || force_wide_indices()) return 0;
     const int L = d->out_ndim - 1;
-    if (d->in_out_step[L] != 1 || d->in_red_step[0] <= 0 || d->out_shape[L] < 64 || d->red_shape[0] < 2) return 0;
+    if (d->in_out_step[L] != 1 || d->in_red_step[0] <= 0 || d->out_shape[L] < 1 || d->red_shape[0] < 2) return 0;
     if (d->out_shape[L] >= 0x7fffffffull || d->red_shape[0] >= 0x7fffffffull) return 0;
     if (L == 1 && (d->in_out_step[0] < 0 || d->out_shape[0] >= 0x10000ull)) return 0;
-    // rows (and planes) that start on word boundaries
-    if ((d->pos & 31) != 0 || (d->in_red_step[0] & 31) != 0 || (L == 1 && (d->in_out_step[0] & 31) != 0)) return 0;
+    const uint32_t fold = fold_rows(d);
+    if (fold == 1) {
+        // rows (and planes) that start on word boundaries
+        if (d->out_shape[L] < 64 || (d->pos & 31) != 0 || (d->in_red_step[0] & 31) != 0 || (L == 1 && (d->in_out_step[0] & 31) != 0)) return 0;
+    }
     BitCountColsVc p;
     std::memset(&p, 0, sizeof(p));
     p.in = d->in + (d->pos >> 5);
     p.out = d->out;
-    p.cols = (uint32_t)d->out_shape[L];
+    p.cols = (uint32_t)d->out_shape[L] * fold;
     p.words = (p.cols + 31u) / 32u;
-    p.rows = (uint32_t)d->red_shape[0];
+    p.rows = (uint32_t)d->red_shape[0] / fold;
     p.n_outer = L == 1 ? (uint32_t)d->out_shape[0] : 1u;
-    p.s_red_w = d->in_red_step[0] >> 5;
+    p.s_red_w = (d->in_red_step[0] * (int64_t)fold) >> 5;
     p.s_outer_w = L == 1 ? (d->in_out_step[0] >> 5) : 0;
     p.o_outer = L == 1 ? d->out_step[0] : 0;
     p.o_col = d->out_step[L];
     p.overwrite = d->overwrite;
     p.count_false = d->count_false;
-    // A block is LANES lanes across and 1024 / LANES stretches of rows deep: the rows are cut
-    // inside the block, where the stretches meet in LDS, rather than across blocks, whose counts
-    // have to go through memory -- few blocks per column group, and many column groups to share
-    // the adding-up at the end. CUMO_HIP_BIT_COLS_LANES=32|64 and CUMO_HIP_BIT_COLS_BLOCKS (read
-    // once) fix the shape of a block and the number of blocks aimed at.
-    static const int forced_lanes = [] {
-        const char* e = std::getenv("CUMO_HIP_BIT_COLS_LANES");
-        return e ? std::atoi(e) : 0;
-    }();
+    // A block is 64 lanes across and 16 stretches of rows deep: the rows are cut inside the block first, where the stretches meet
+    // in LDS, and across blocks as far as there are compute units without one (CUMO_HIP_BIT_COLS_BLOCKS, read once, fixes the
+    // number of blocks aimed at).
     static const int forced_blocks = [] {
         const char* e = std::getenv("CUMO_HIP_BIT_COLS_BLOCKS");
         return e ? std::atoi(e) : 0;
     }();
     const uint64_t want_blocks = forced_blocks > 0 ? (uint64_t)forced_blocks : (uint64_t)kNumCU;
-    (void)forced_lanes;
-    const int lanes = 64;
     uint64_t blocks = 0;
     if (!vc_geometry<1024, 64>(p, want_blocks, &blocks)) return 0;
     hipStream_t stream = current_stream();
-    if (p.parts > 1) {
-        p.tickets = red_ticket_words(stream_slot(stream));
-        if (p.tickets == nullptr) return 0;
-        const size_t bytes = sizeof(uint32_t) * (size_t)blocks * lanes * 32;
-        p.partial = reinterpret_cast<uint32_t*>(cumo_cuda_runtime_malloc(bytes));
+    if (p.parts > 1 || fold > 1) {
+        p.partial = reinterpret_cast<uint32_t*>(cumo_cuda_runtime_malloc(sizeof(uint32_t) * (size_t)blocks * 64 * 32));
         if (p.partial == nullptr) return 0;
     }
-    const dim3 g((unsigned)blocks), b(1024);
-    hipLaunchKernelGGL((bit_count_cols_vc_kernel<1024, 64>), g, b, 0, stream, p);
-    // stream-ordered reuse: whoever gets the scratch next can only touch it from later work on this stream
-    if (p.partial) cumo_cuda_runtime_free(reinterpret_cast<char*>(p.partial));
+    hipLaunchKernelGGL((bit_count_cols_vc_kernel<1024, 64>), dim3((unsigned)blocks), dim3(1024), 0, stream, p);
     cumo_cuda_runtime_check_kernel_launch();
+    if (p.partial == nullptr) return 1;
+    FoldCounts f;
+    std::memset(&f, 0, sizeof(f));
+    f.partial = p.partial;
+    f.in = d->in;
+    f.out = d->out;
+    f.cols = (uint32_t)d->out_shape[L];
+    f.fold_bits = (uint32_t)__builtin_ctz(fold);
+    f.parts = p.parts;
+    f.width = p.col_blocks * 64 * 32;
+    f.rest = (uint32_t)d->red_shape[0] - p.rows * fold;
+    f.rest_bit = d->pos + (uint64_t)p.rows * fold * f.cols;
+    f.o_outer = p.o_outer;
+    f.o_col = p.o_col;
+    f.col_groups = (f.cols + kFoldCols - 1) / kFoldCols;
+    f.count_false = d->count_false;
+    f.overwrite = d->overwrite;
+    const dim3 g(f.col_groups * p.n_outer);
+    // as many lanes to a column as leave each about eight counts
+    if ((uint64_t)p.parts * fold > 64) hipLaunchKernelGGL((bit_count_fold_kernel<32>), g, dim3(kFoldCols * 32), 0, stream, f);
+    else hipLaunchKernelGGL((bit_count_fold_kernel<8>), g, dim3(kFoldCols * 8), 0, stream, f);
+    cumo_cuda_runtime_check_kernel_launch();
+    // stream-ordered reuse: whoever gets the scratch next can only touch it from later work on this stream
+    cumo_cuda_runtime_free(reinterpret_cast<char*>(p.partial));
     return 1;
 }
 

@@ -431,3 +431,27 @@ def test_all_any_along_word_aligned_rows():
     # shapes it leaves to the counts
     assert _lib.call(f, b._buf.ptr, 3, rows, cols, 4096, 1, out._buf.ptr, 0) == 0
     assert _lib.call(f, b._buf.ptr, 0, 100, cols, 4096, 1, out._buf.ptr, 0) == 0
+
+
+# (rows, columns): rows of less than a word, of whole words, a bit more and less; fewer rows than are taken as one, rows left over;
+# runs of 8129 and 8130 bits (the most that 64 lanes take, and one more)
+@pytest.mark.parametrize("shape", [(5, 3), (33, 31), (4096, 8), (2051, 33), (130, 64), (640, 32), (127, 1001), (128, 1001), (191, 1025), (4103, 137),
+                                   (200, 8191), (200, 8193), (3, 8129), (3, 8130), (40000, 20)])
+def test_counts_along_and_down_short_rows(shape):
+    import cumo_amd as m
+    rng = np.random.default_rng(shape[1])
+    rows, cols = shape
+    h = rng.random((rows + 2, cols + 5)) < 0.4
+    x = m.SFloat.cast(h.astype(np.float32)) > 0.5
+    whole = np.ascontiguousarray(h[:rows, :cols])
+    y = m.SFloat.cast(whole.astype(np.float32)) > 0.5
+    # one run without gaps, the same from a row further down (its first bit off a word), a window with gaps, rows backwards
+    for a, w in ((y, whole), (y[1:], whole[1:]), (x[1:rows + 1, 3:cols + 3], h[1:rows + 1, 3:cols + 3]), (y[::-1], whole[::-1])):
+        for axis in (0, 1):
+            for keep in (False, True):
+                assert (a.count_true(axis=axis, keepdims=keep).to_numpy() == w.sum(axis=axis, keepdims=keep)).all(), (axis, keep)
+            assert (a.count_false(axis=axis).to_numpy() == (~w).sum(axis=axis)).all(), axis
+    z = m.SFloat.cast(np.stack([whole, ~whole]).astype(np.float32)) > 0.5
+    assert (z.count_true(axis=2).to_numpy() == np.stack([whole, ~whole]).sum(axis=2)).all()
+    assert (z.count_true(axis=1).to_numpy() == np.stack([whole, ~whole]).sum(axis=1)).all()
+    assert (z.transpose(1, 0, 2).count_false(axis=2).to_numpy() == np.stack([~whole, whole]).transpose(1, 0, 2).sum(axis=2)).all()
