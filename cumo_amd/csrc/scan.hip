@@ -1062,8 +1062,9 @@ void scan_cols_launch_vec(ScanColsParams& p, hipStream_t stream) {
 
 // ---- long runs across memory in one pass ---------------------------------------
 // The matrix is cut into tiles of NW * 16 rows by 64 vectors (1 KiB of a row): wave w of
-// a block holds 16 rows of the tile, lane l their vector l, all in registers. A tile adds
-// up its columns (in the lane, then across the waves through LDS), publishes the column
+// a block holds 16 rows of the tile, lane l their vector l, all in registers. Of narrower
+// matrices a wave holds two, four or eight bands of 16 rows side by side. A tile adds
+// up its columns (in the lane, from band to band by shuffles, then across the waves through LDS), publishes the column
 // totals, gathers what the tiles above it published, and scans its rows from there: the
 // data is read once and written once. The published words are {the launch's number, 32 bits of
 // the value}, in the region the stream keeps (see above). Tiles take their places by ticket, level by level
@@ -1085,7 +1086,7 @@ struct ScanColsChain {
     uint64_t* tile;    // [strip][level][column][W]
     uint64_t* group;   // [strip][group][column][W]
     uint64_t* super;   // [strip][supergroup][column][W]
-    uint32_t depth, n_groups, n_supers;  // per strip
+    uint32_t depth, n_groups, n_supers;  // per strip; nothing is published or waited for where depth is 1
     uint32_t strips;                     // per plane
     uint32_t all_strips;                 // planes * strips
     uint32_t flag;                       // the upper half of a word of this launch
@@ -1142,17 +1143,33 @@ __device__ __forceinline__ bool cols_chain_gather(const uint64_t* base, size_t s
     return has;
 }
 
-template <class T, class Op, bool NT, int NW>
+// v of the lane `step` rows' lanes before this one
+template <class T>
+__device__ __forceinline__ T cols_chain_up(T v, int step) {
+    constexpr int N = (int)(sizeof(T) / 4);
+    union { T t; int w[N]; } u;
+    u.t = v;
+#pragma unroll
+    for (int i = 0; i < N; ++i) u.w[i] = __shfl_up(u.w[i], step);
+    return u.t;
+}
+
+// LPR lanes to a row of the tile, so 64 / LPR bands of 16 rows to a wave. ONE: one tile holds every row, nothing is published or
+// waited for. DEEP: more than 512 tiles down a column.
+template <class T, class Op, bool NT, int NW, int LPR, bool ONE, bool DEEP>
 __global__ __launch_bounds__(NW * 64) void scan_cols_chain_kernel(ScanColsParams p, ScanColsChain<T> c) {
-    constexpr int V = 16 / (int)sizeof(T), R = kColsChainRows, SW = 64 * V, W = ScanColsChain<T>::W;
+    constexpr int V = 16 / (int)sizeof(T), R = kColsChainRows, SW = LPR * V, SUB = 64 / LPR, W = ScanColsChain<T>::W;
     __shared__ T part[NW][SW];
     __shared__ T s_groups[SW], s_supers[SW];
     __shared__ uint32_t s_ticket;
-    static_assert(NW * 64 >= 3 * SW, "three roles of SW threads each");
-    const unsigned w = threadIdx.x >> 6, l = threadIdx.x & 63u;
-    if (threadIdx.x == 0) s_ticket = __hip_atomic_fetch_add(c.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - c.ticket_base;
-    __syncthreads();
-    const uint32_t id = s_ticket;
+    static_assert(NW * 64 >= (ONE ? 1 : 3) * SW, "three roles of SW threads each");
+    const unsigned w = threadIdx.x >> 6, l = threadIdx.x % LPR, sub = (threadIdx.x & 63u) / LPR;
+    uint32_t id = blockIdx.x;
+    if constexpr (!ONE) {
+        if (threadIdx.x == 0) s_ticket = __hip_atomic_fetch_add(c.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - c.ticket_base;
+        __syncthreads();
+        id = s_ticket;
+    }
     const uint32_t k = id / c.all_strips, ps = id - k * c.all_strips;
     const uint32_t plane = ps / c.strips, strip = ps - plane * c.strips;
     int64_t oi = 0, oo = 0;
@@ -1168,56 +1185,97 @@ __global__ __launch_bounds__(NW * 64) void scan_cols_chain_kernel(ScanColsParams
             oo += i * p.ostep_out[d];
         }
     }
-    const int64_t row0 = (int64_t)k * (NW * R) + (int64_t)w * R;
+    const int64_t row0 = (int64_t)k * (NW * SUB * R) + (int64_t)(w * SUB + sub) * R;
     const int64_t colb = ((int64_t)strip * SW + (int64_t)l * V) * (int64_t)sizeof(T);
-    const char* src = p.in + oi + row0 * p.s_in + colb;
     char* dst = p.out + oo + row0 * p.s_out + colb;
-    // A tile at the lower edge has fewer rows and one at the right edge fewer columns: this wave's first
-    // `rows` rows exist, and of this lane's columns the first ncol. What such a tile reads as missing is zeros;
-    // the totals they enter are only ever used by rows or columns that do not exist either.
+    // A tile at the lower edge has fewer rows and one at the right edge fewer columns: this lane's first `rows` rows exist, and of
+    // its columns the first ncol. What such a tile reads as missing is zeros; the totals they enter are only ever used by
+    // rows or columns that do not exist either. A lane that has anything sends all of its loads, from inside the array: a row that
+    // does not exist is read again from the last one, a vector that is partly there as the one that ends with the row. They go by
+    // the second-level cache: the lines hold the start of the next row as well, which another block reads (SFloat [131072,257] 66.5 us
+    // with non-temporal loads here).
     const int64_t rows_left = (int64_t)p.n - row0;
     const int rows = rows_left >= R ? R : (rows_left > 0 ? (int)rows_left : 0);
     const int64_t cols_left = (int64_t)p.cols - (int64_t)((uint64_t)strip * SW + (uint64_t)l * V);
     const int ncol = cols_left >= V ? V : (cols_left > 0 ? (int)cols_left : 0);  // this lane's columns that exist
-    const bool all_there = rows == R && __builtin_amdgcn_ballot_w64(ncol != V) == 0;
+    const bool all_there = __builtin_amdgcn_ballot_w64(rows != R || ncol != V) == 0;
     T raw[R][V];
     if (all_there) {
+        const char* src = p.in + oi + row0 * p.s_in + colb;
 #pragma unroll
         for (int r = 0; r < R; ++r) scan_cols_load<T, V, NT>(src + (int64_t)r * p.s_in, raw[r]);
     } else {
+        const char* src = p.in + oi + (ncol == V ? colb : ((int64_t)p.cols - V) * (int64_t)sizeof(T));
+        if (rows > 0 && ncol > 0) {
+            const int64_t last = (int64_t)p.n - 1;
+#pragma unroll
+            for (int r = 0; r < R; ++r) scan_cols_load<T, V>(src + (row0 + r < last ? row0 + r : last) * p.s_in, raw[r]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
+            T v[V];
 #pragma unroll
-            for (int j = 0; j < V; ++j) raw[r][j] = T();
-            if (r < rows) {
-                if (ncol == V) {
-                    scan_cols_load<T, V, NT>(src + (int64_t)r * p.s_in, raw[r]);
-                } else {
-                    // the row's last vector, partly there: element by element, nothing read past the row
+            for (int j = 0; j < V; ++j) v[j] = raw[r][j];
 #pragma unroll
-                    for (int j = 0; j < V; ++j)
-                        if (j < ncol) raw[r][j] = reinterpret_cast<const T*>(src + (int64_t)r * p.s_in)[j];
-                }
+            for (int j = 0; j < V; ++j) {
+                // column j is element j + V - ncol of the vector
+                T e = T();
+#pragma unroll
+                for (int n = 1; n <= V; ++n)
+                    if (j < n) e = ncol == n ? v[j + V - n] : e;
+                raw[r][j] = r < rows ? e : T();
             }
         }
     }
+    // This lane's rows are scanned by themselves, here, and take what lies above them when it is known: a value is rounded at the size
+    // of the whole sum once, not at every row, and nothing is left to do one after the other behind the wait. Their total, and, of
+    // a wave that holds several bands, that of the bands before, follow.
+#pragma unroll
+    for (int r = 1; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < V; ++j) raw[r][j] = Op::apply(raw[r - 1][j], raw[r][j]);
+    T above_lane[V];
     {
         T tot[V];
 #pragma unroll
-        for (int j = 0; j < V; ++j) tot[j] = raw[0][j];
+        for (int j = 0; j < V; ++j) tot[j] = raw[R - 1][j];
+        if constexpr (SUB > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r)
+            for (int d = 1; d < SUB; d *= 2) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) tot[j] = Op::apply(tot[j], raw[r][j]);
+                for (int j = 0; j < V; ++j) {
+                    const T before = cols_chain_up(tot[j], d * LPR);
+                    if ((int)sub >= d) tot[j] = Op::apply(before, tot[j]);
+                }
+            }
 #pragma unroll
-        for (int j = 0; j < V; ++j) part[w][l * V + j] = tot[j];
+            for (int j = 0; j < V; ++j) above_lane[j] = cols_chain_up(tot[j], LPR);
+        }
+        if (sub == SUB - 1) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) part[w][l * V + j] = tot[j];
+        }
     }
     __syncthreads();
     // Threads 0 .. SW-1 see to the tile's own totals and to the tiles before it in its group,
     // the next SW threads to the groups before its group, the SW after those to the supergroups:
     // the three waits run side by side in different waves, each with seven loads in flight.
     const unsigned col = threadIdx.x % SW, role = threadIdx.x / SW;
+    if constexpr (ONE) {
+        if (role == 0) {
+            T above = part[0][col];
+#pragma unroll
+            for (int ww = 1; ww < NW; ++ww) {
+                const T mine = part[ww][col];
+                part[ww][col] = above;
+                above = Op::apply(above, mine);
+            }
+        }
+        __syncthreads();
+    } else {
     const uint32_t pos = k % kColsChainFan, g = k / kColsChainFan, gpos = g % kColsChainFan, sg = g / kColsChainFan;
+    // (supergroups are as many as there are: they are gathered seven at a time)
     const size_t cw = (size_t)SW * W;  // words from one tile's (group's) totals to the next one's
     T gt = T();
     if (role == 0) {
@@ -1243,7 +1301,15 @@ __global__ __launch_bounds__(NW * 64) void scan_cols_chain_kernel(ScanColsParams
         count = 0;
     }
     T xs = T();
-    const bool xh = cols_chain_gather<T, Op>(from, cw, count, c.flag, c.wait, xs);
+    const bool xh = cols_chain_gather<T, Op>(from, cw, DEEP && count > kColsChainFan - 1 ? kColsChainFan - 1 : count, c.flag, c.wait, xs);
+    if constexpr (DEEP) {
+        for (uint32_t at = kColsChainFan - 1; at < count; at += kColsChainFan - 1) {
+            T more = T();
+            const uint32_t left = count - at;
+            cols_chain_gather<T, Op>(from + at * cw, cw, left < kColsChainFan - 1 ? left : kColsChainFan - 1, c.flag, c.wait, more);
+            xs = Op::apply(xs, more);
+        }
+    }
     if (role == 0) {
         if (xh) gt = Op::apply(xs, gt);  // the group's total so far
         if (pos == kColsChainFan - 1) chain_publish<T>(c.group + (((size_t)ps * c.n_groups + g) * SW + col) * W, gt, c.flag);
@@ -1272,52 +1338,37 @@ __global__ __launch_bounds__(NW * 64) void scan_cols_chain_kernel(ScanColsParams
         for (int ww = 1; ww < NW; ++ww) part[ww][col] = Op::apply(pre, part[ww][col]);
     }
     __syncthreads();
-    // The topmost wave of the topmost tile has nothing above it; it goes the same way as the others
-    // from a first row the compiler cannot see through (it would otherwise find this wave's running
-    // values equal to the column totals' and keep all sixteen of them in registers from there to here,
-    // beside the tile: there is no room for both).
-    T acc[V];
-    const bool topmost = k == 0 && w == 0;
+    }
+    const bool first_wave = k == 0 && w == 0, topmost = first_wave && sub == 0;   // (nothing above it)
+    T above[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-        const T above = topmost ? raw[0][j] : part[w][l * V + j];
-        acc[j] = topmost ? above : Op::apply(above, raw[0][j]);
-        if constexpr (sizeof(T) == 8) {
-            union { T t; uint64_t u; } o;
-            o.t = acc[j];
-            asm volatile("" : "+v"(o.u));
-            acc[j] = o.t;
-        } else {
-            union { T t; uint32_t u; } o;
-            o.t = acc[j];
-            asm volatile("" : "+v"(o.u));
-            acc[j] = o.t;
+        above[j] = first_wave ? T() : part[w][l * V + j];
+        if constexpr (SUB > 1) {
+            if (sub > 0) above[j] = first_wave ? above_lane[j] : Op::apply(above[j], above_lane[j]);
         }
     }
     if (all_there) {
-        scan_cols_store<T, V, NT>(dst, acc);
 #pragma unroll
-        for (int r = 1; r < R; ++r) {
+        for (int r = 0; r < R; ++r) {
+            T out[V];
 #pragma unroll
-            for (int j = 0; j < V; ++j) acc[j] = Op::apply(acc[j], raw[r][j]);
-            scan_cols_store<T, V, NT>(dst + (int64_t)r * p.s_out, acc);
+            for (int j = 0; j < V; ++j) out[j] = topmost ? raw[r][j] : Op::apply(above[j], raw[r][j]);
+            scan_cols_store<T, V, NT>(dst + (int64_t)r * p.s_out, out);
         }
-    } else if (ncol > 0) {
-        auto put = [&](int r) {
-            if (ncol == V) {
-                scan_cols_store<T, V, NT>(dst + (int64_t)r * p.s_out, acc);
-            } else {
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            T out[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) out[j] = topmost ? raw[r][j] : Op::apply(above[j], raw[r][j]);
+            if (r < rows && ncol == V) {
+                scan_cols_store<T, V, NT>(dst + (int64_t)r * p.s_out, out);
+            } else if (r < rows) {
 #pragma unroll
                 for (int j = 0; j < V; ++j)
-                    if (j < ncol) reinterpret_cast<T*>(dst + (int64_t)r * p.s_out)[j] = acc[j];
+                    if (j < ncol) reinterpret_cast<T*>(dst + (int64_t)r * p.s_out)[j] = out[j];
             }
-        };
-        if (rows > 0) put(0);
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-#pragma unroll
-            for (int j = 0; j < V; ++j) acc[j] = Op::apply(acc[j], raw[r][j]);
-            if (r < rows) put(r);
         }
     }
 }
@@ -1331,45 +1382,65 @@ static bool scan_cols_chain_enabled() {
 }
 
 // true when the launch was made (or failed: the error is left for the caller's check)
-template <class T, class Op>
-bool scan_cols_chain_launch(ScanColsParams& p, hipStream_t stream) {
-    constexpr int V = 16 / (int)sizeof(T), W = ScanColsChain<T>::W, NW = 16;
-    constexpr uint64_t SW = 64 * V, TR = (uint64_t)NW * kColsChainRows;
-    if (!scan_cols_chain_enabled()) return false;
-    if (p.cols < SW) return false;  // (a strip of 64 vectors is the unit: narrower arrays would leave most lanes idle)
-    const uint64_t depth = (p.n + TR - 1) / TR, strips = (p.cols + SW - 1) / SW;
+template <class T, class Op, int NW, int LPR, bool MAY_NT, bool ONE, bool DEEP>
+bool scan_cols_chain_go(const ScanColsParams& p, hipStream_t stream) {
+    constexpr int V = 16 / (int)sizeof(T), W = ScanColsChain<T>::W;
+    constexpr uint64_t SW = LPR * V, TR = (uint64_t)NW * (64 / LPR) * kColsChainRows;
     constexpr uint64_t F = kColsChainFan;
-    if (depth < 2 || depth > F * F * F) return false;
+    const uint64_t depth = (p.n + TR - 1) / TR, strips = (p.cols + SW - 1) / SW;
+    if (depth > F * F * F * (DEEP ? 8 : 1)) return false;
     const uint64_t all_strips = strips * p.planes;
     const uint64_t n_tiles = all_strips * depth;
-    // (worth it from few tiles on: SFloat [512, 4096], 32 tiles, 9.5 us against 11.7 us for the launches of
-    // the two-pass form; [4096, 4096], 256 tiles, 27 us against 51 us)
-    if (n_tiles < 16 || n_tiles > 0x7fffffffull) return false;
+    if (n_tiles > 0x3fffffull) return false;
     const uint64_t n_groups = (depth + F - 1) / F, n_supers = (n_groups + F - 1) / F;
-    const uint64_t words = kChainHead + all_strips * (depth + n_groups + n_supers) * SW * W;
-    WaitCtl* wait = wait_ctl();
-    if (wait == nullptr) return false;  // nowhere to report a wait that gives up: the form without waits
-    ChainWords cw;
-    if (!chain_words_acquire(stream, words, (uint32_t)n_tiles, &cw)) return true;
     ScanColsChain<T> c;
-    c.wait = wait;
-    c.ticket = reinterpret_cast<uint32_t*>(cw.ws);
-    c.tile = cw.ws + kChainHead;
-    c.flag = cw.flag;
-    c.ticket_base = cw.ticket_base;
-    c.group = c.tile + all_strips * depth * SW * W;
-    c.super = c.group + all_strips * n_groups * SW * W;
+    std::memset(&c, 0, sizeof(c));
+    ChainWords cw;
+    if constexpr (!ONE) {
+        const uint64_t words = kChainHead + all_strips * (depth + n_groups + n_supers) * SW * W;
+        c.wait = wait_ctl();
+        if (c.wait == nullptr) return false;  // nowhere to report a wait that gives up: the form without waits
+        if (!chain_words_acquire(stream, words, (uint32_t)n_tiles, &cw)) return true;
+        c.ticket = reinterpret_cast<uint32_t*>(cw.ws);
+        c.tile = cw.ws + kChainHead;
+        c.flag = cw.flag;
+        c.ticket_base = cw.ticket_base;
+        c.group = c.tile + all_strips * depth * SW * W;
+        c.super = c.group + all_strips * n_groups * SW * W;
+    }
     c.depth = (uint32_t)depth;
     c.n_groups = (uint32_t)n_groups;
     c.n_supers = (uint32_t)n_supers;
     c.strips = (uint32_t)strips;
     c.all_strips = (uint32_t)all_strips;
-    const bool nt = stream_past_caches(2 * p.planes * p.n * p.cols * sizeof(T));
+    const bool nt = MAY_NT && stream_past_caches(2 * p.planes * p.n * p.cols * sizeof(T));
     const dim3 g((unsigned)n_tiles), b(NW * 64);
-    if (nt) hipLaunchKernelGGL((scan_cols_chain_kernel<T, Op, true, NW>), g, b, 0, stream, p, c);
-    else hipLaunchKernelGGL((scan_cols_chain_kernel<T, Op, false, NW>), g, b, 0, stream, p, c);
-    chain_words_release(cw);
+    if (nt) hipLaunchKernelGGL((scan_cols_chain_kernel<T, Op, MAY_NT, NW, LPR, ONE, DEEP>), g, b, 0, stream, p, c);
+    else hipLaunchKernelGGL((scan_cols_chain_kernel<T, Op, false, NW, LPR, ONE, DEEP>), g, b, 0, stream, p, c);
+    if constexpr (!ONE) chain_words_release(cw);
     return true;
+}
+
+// Any matrix whose rows hold a vector: what this leaves to the two passes (totals, perhaps their own scan, and the data
+// again) is rows of less than that, and more than 4096 tiles down. Up to 256 rows are one tile, in blocks of four waves up to 64
+// rows. us, two passes / this:
+//   rows that are few    SFloat [208,53952] 29.2 / 15.4, [64,500000] 68.6 / 46.8, [31,32000] 8.3 / 5.5; DFloat [76,440000] 149 / 100
+//   columns that are few SFloat [234385,93] 94.5 / 39.2, [20000,130] 25.0 / 14.2, [1000000,16] 416 / 39.9; DFloat [131072,33] 44 / 20
+//   matrices of few tiles SFloat [619,640] 14.2 / 9.0, [100,100] 6.9 / 5.6, [3036,248] 15.5 / 10.5
+template <class T, class Op>
+bool scan_cols_chain_launch(ScanColsParams& p, hipStream_t stream) {
+    constexpr int V = 16 / (int)sizeof(T);
+    if (!scan_cols_chain_enabled() || p.cols < (uint64_t)V || p.n < 2) return false;
+    const uint64_t vectors = (p.cols + V - 1) / V;
+    if (vectors > 32) {
+        if (p.n <= 4 * kColsChainRows) return scan_cols_chain_go<T, Op, 4, 64, true, true, false>(p, stream);
+        if (p.n <= 16 * kColsChainRows) return scan_cols_chain_go<T, Op, 16, 64, true, true, false>(p, stream);
+        if (p.n <= 512 * 16 * kColsChainRows) return scan_cols_chain_go<T, Op, 16, 64, true, false, false>(p, stream);
+        return scan_cols_chain_go<T, Op, 16, 64, true, false, true>(p, stream);
+    }
+    if (vectors > 16) return scan_cols_chain_go<T, Op, 16, 32, true, false, true>(p, stream);
+    if (vectors > 8) return scan_cols_chain_go<T, Op, 16, 16, false, false, true>(p, stream);
+    return scan_cols_chain_go<T, Op, 16, 8, false, false, true>(p, stream);
 }
 
 template <class T, class Op>

@@ -669,3 +669,36 @@ def test_mulsum_of_such_a_view_can_be_replayed():
             del dirt
     finally:
         _lib.lib.cumo_hip_set_stream(None)
+
+
+# (rows, columns): a strip of 64, 32, 16 and 8 lanes and one column to either side, rows that end in part of a vector; one tile of few
+# rows, exactly one tile, one row more; tiles enough for groups and supergroups, and for more than seven of those
+COLUMN_SCANS = [(2, 4), (16, 5), (64, 300), (65, 300), (208, 5395), (256, 1024), (257, 257), (300, 129), (513, 128), (600, 127), (1025, 65), (1030, 64),
+                (5000, 63), (2049, 33), (2100, 32), (2100, 31), (9, 17), (20000, 9), (40000, 260), (140000, 130), (300000, 66)]
+
+
+@pytest.mark.parametrize("shape", COLUMN_SCANS)
+def test_scans_down_narrow_and_shallow_matrices(shape):
+    import cumo_amd as m
+    rng = np.random.default_rng(shape[0])
+    h = rng.integers(-9, 10, size=shape).astype(np.int32)
+    assert (m.Int32.cast(h).cumsum(axis=0).to_numpy() == np.cumsum(h, axis=0, dtype=np.int32)).all()
+    # whole numbers that stay below 2^24: exact in float, in any order
+    assert (m.SFloat.cast(h.astype(np.float32)).cumsum(axis=0).to_numpy() == np.cumsum(h, axis=0)).all()
+    assert (m.DFloat.cast(h.astype(np.float64)).cumsum(axis=0).to_numpy() == np.cumsum(h, axis=0)).all()
+    # signs alone: products are exact
+    s = np.where(h < 0, -1.0, 1.0)
+    assert (m.SFloat.cast(s.astype(np.float32)).cumprod(axis=0).to_numpy() == np.cumprod(s, axis=0)).all()
+    if h.size <= 1 << 20:
+        # planes, a window whose rows have gaps, rows backwards
+        three = np.stack([h, -h, h[::-1]]).astype(np.float64)
+        assert (m.DFloat.cast(three).cumsum(axis=1).to_numpy() == np.cumsum(three, axis=1)).all()
+        wide = np.pad(h, ((0, 0), (1, 2))).astype(np.float32)
+        x = m.SFloat.cast(wide)[:, 1:-2]
+        assert (x.cumsum(axis=0).to_numpy() == np.cumsum(h, axis=0)).all()
+        assert (x[::-1].cumsum(axis=0).to_numpy() == np.cumsum(h[::-1], axis=0)).all()
+        n = h.astype(np.float64)
+        n[rng.random(shape) < 0.2] = np.nan
+        assert_bits_equal(m.DFloat.cast(n).cumsum(axis=0, nan=True).to_numpy(), oracle.cum("cumsum", n, axis=0, nan=True), (shape, "nan: true"))
+        assert_bits_equal(m.DFloat.cast(n).cumsum(axis=0).to_numpy(), oracle.cum("cumsum", n, axis=0), (shape, "NaN carried"))
+
