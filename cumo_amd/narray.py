@@ -273,6 +273,9 @@ class NArray(_native.View):
         return key + (slice(None),) * (self.ndim - len(key))
 
     def __getitem__(self, key):
+        view = _native.window(self, key)  # whole numbers and slices; None: every other key
+        if view is not None:
+            return view
         if isinstance(key, NArray) and type(key).__name__ == "Bit":
             return key.mask(self)  # a[mask]: the elements where the mask is set
         if type(key) is np.ndarray:

@@ -596,6 +596,79 @@ PyObject* na_take(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// views
+// ---------------------------------------------------------------------------------------------------------------
+
+// (x, key): x[key] for a key of whole numbers, slices and True (the whole dimension), one or a tuple of them. None: a key that
+// the Python form answers (index arrays, an ellipsis, numpy numbers, positions out of range, too many of them) and arrays of a
+// derived class. x[::3] 2.3 us of the caller's time -> 0.13, x.T[:, ::2] 2.3 -> 0.16.
+PyObject* na_window(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (!arity(n, 2)) return nullptr;
+    const View* x = as_view(a[0]);
+    if (!x || x->code < 0 || x->code > 7 || !x->shape || !x->strides || !x->buf) Py_RETURN_NONE;
+    PyTypeObject* type = Py_TYPE(a[0]);
+    if (reinterpret_cast<PyObject*>(type) != g_class[x->code]) Py_RETURN_NONE;
+    const Py_ssize_t nd = PyTuple_GET_SIZE(x->shape);
+    const bool many = PyTuple_CheckExact(a[1]);
+    const Py_ssize_t given = many ? PyTuple_GET_SIZE(a[1]) : 1;
+    if (given > nd || nd > CUMO_NA_MAX_DIMENSION || PyTuple_GET_SIZE(x->strides) != nd) Py_RETURN_NONE;
+    Py_ssize_t shape[CUMO_NA_MAX_DIMENSION], strides[CUMO_NA_MAX_DIMENSION], offset = x->offset;
+    Py_ssize_t left = 0;
+    for (Py_ssize_t d = 0; d < nd; d++) {
+        const Py_ssize_t len = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->shape, d));
+        const Py_ssize_t step = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->strides, d));
+        if ((len == -1 || step == -1) && PyErr_Occurred()) return nullptr;
+        PyObject* k = d >= given ? Py_True : many ? PyTuple_GET_ITEM(a[1], d) : a[1];
+        if (k == Py_True) {
+            shape[left] = len;
+            strides[left++] = step;
+        } else if (PyLong_CheckExact(k)) {
+            Py_ssize_t at = PyLong_AsSsize_t(k);
+            if (at == -1 && PyErr_Occurred()) {
+                PyErr_Clear();
+                Py_RETURN_NONE;
+            }
+            if (at < 0) at += len;
+            if (at < 0 || at >= len) Py_RETURN_NONE;
+            offset += at * step;
+        } else if (PySlice_Check(k)) {
+            Py_ssize_t from, to, by;
+            if (PySlice_Unpack(k, &from, &to, &by) < 0) return nullptr;
+            shape[left] = PySlice_AdjustIndices(len, &from, &to, by);
+            offset += from * step;
+            if (by == PY_SSIZE_T_MAX || by == -PY_SSIZE_T_MAX || __builtin_mul_overflow(step, by, &strides[left++])) Py_RETURN_NONE;
+        } else {
+            Py_RETURN_NONE;
+        }
+    }
+    PyObject* self = type->tp_alloc(type, 0);
+    PyObject* new_shape = PyTuple_New(left);
+    PyObject* new_strides = PyTuple_New(left);
+    bool ok = self && new_shape && new_strides;
+    for (Py_ssize_t d = 0; ok && d < left; d++) {
+        PyObject* len = PyLong_FromSsize_t(shape[d]);
+        PyObject* step = PyLong_FromSsize_t(strides[d]);
+        PyTuple_SET_ITEM(new_shape, d, len);
+        PyTuple_SET_ITEM(new_strides, d, step);
+        ok = len && step;
+    }
+    if (!ok) {
+        Py_XDECREF(self);
+        Py_XDECREF(new_shape);
+        Py_XDECREF(new_strides);
+        return nullptr;
+    }
+    View* v = reinterpret_cast<View*>(self);
+    v->code = x->code;
+    v->buf = x->buf;
+    Py_INCREF(v->buf);
+    v->shape = new_shape;
+    v->strides = new_strides;
+    v->offset = offset;
+    return self;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // set-up
 // ---------------------------------------------------------------------------------------------------------------
 
@@ -635,7 +708,7 @@ PyObject* set_recording(PyObject*, PyObject* rec) {
 
 #define CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(na_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {CALL(binary), CALL(compare), CALL(unary), CALL(math), CALL(reduce), CALL(mulsum), CALL(cum), CALL(bit_binary),
-                         CALL(bit_count), CALL(take), {"setup", setup, METH_VARARGS, nullptr}, {"set_recording", set_recording, METH_O, nullptr}, {}};
+                         CALL(bit_count), CALL(take), CALL(window), {"setup", setup, METH_VARARGS, nullptr}, {"set_recording", set_recording, METH_O, nullptr}, {}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "cumo_amd._native", "Buffers, views and calls of the array classes.", -1, methods};
 
