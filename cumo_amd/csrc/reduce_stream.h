@@ -37,6 +37,10 @@ constexpr uint32_t kRsTicketWords = 16384;  // ticket words per stream slot
 template <class I, class = void> struct folds_columns_together { static constexpr bool value = false; };
 template <class I> struct folds_columns_together<I, decltype((void)I::COLUMNS_TOGETHER)> { static constexpr bool value = I::COLUMNS_TOGETHER; };
 
+// An Impl whose combine() goes without branches and that has a form with them, combine_seldom(), for parts that mostly change nothing.
+template <class I, class = void> struct combines_in_two_forms { static constexpr bool value = false; };
+template <class I> struct combines_in_two_forms<I, decltype((void)&I::combine_seldom)> { static constexpr bool value = true; };
+
 // An Impl whose accumulate_columns_by_position<U, VEC>(x[U][VEC], first position, acc[VEC]) folds U consecutive
 // positions of VEC neighbouring outputs without a branch
 template <class I, class = void> struct folds_columns_by_position { static constexpr bool value = false; };
@@ -414,7 +418,10 @@ __global__ __launch_bounds__(kRedBlock) void red_fold_parts_kernel(RedSParams p,
     const uint32_t k0 = pg * per < p.n_split ? pg * per : p.n_split;
     const uint32_t k1 = k0 + per < p.n_split ? k0 + per : p.n_split;
     const Acc* base = reinterpret_cast<const Acc*>(p.partial) + (ok ? o : p.n_out - 1);
-    Acc total = rs_fold_output(impl, base, row, k0, k1, pg, PG, OV, slots, [&](const Acc& v, uint32_t, Acc& t) { impl.combine(v, t); });
+    Acc total = rs_fold_output(impl, base, row, k0, k1, pg, PG, OV, slots, [&](const Acc& v, uint32_t, Acc& t) {
+        if constexpr (combines_in_two_forms<Impl>::value) impl.combine_seldom(v, t);
+        else impl.combine(v, t);
+    });
     if constexpr (has_exact<Impl>::value) {
         // the parts are plain values in axis order: where the fast fold cannot tell which of two equal
         // values came first, the exact rule over the same values, by the same lanes

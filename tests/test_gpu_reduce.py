@@ -684,3 +684,29 @@ def test_products_and_compensated_sums_down_columns_over_every_split(tname, dt, 
         h[r[:, 0], cols], h[r[:, 1], cols] = big, -big
         small[r[:, 0], cols] = small[r[:, 1], cols] = 0
         assert_bits_equal(cls_of(tname).cast(h).kahan_sum(axis=0).to_numpy() + 0.0, small.sum(axis=0) + 0.0, "kahan_sum")
+
+
+# where lanes that share an axis meet with the position of an extreme: ties, NaN (which loses, or with nan: true wins) and nothing but NaN
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32])
+@pytest.mark.parametrize("shape", [(500, 37), (64, 500), (3000, 64), (70, 20001)])
+def test_positions_of_extremes_with_ties_and_nan(dt, shape):
+    import cumo_amd as m
+    cls = {np.float32: m.SFloat, np.float64: m.DFloat, np.int32: m.Int32}[dt]
+    rng = np.random.default_rng(shape[0])
+    h = rng.integers(-3, 4, size=shape).astype(dt)
+    if dt != np.int32:
+        h[rng.random(shape) < 0.3] = np.nan
+        h[:, 0] = np.nan
+        h[0, :] = np.nan
+        h[h == 3] = np.inf
+        h[(h == 0) & (rng.random(shape) < 0.5)] = -0.0
+    x = cls.cast(h)
+    for axis in (0, 1, None):
+        for name in ("argmax", "argmin"):
+            got = getattr(x, name)(axis=axis)
+            got = got.to_numpy() if hasattr(got, "to_numpy") else got
+            assert np.array_equal(got, oracle.reduce(name, h, axis=axis)), (axis, name)
+            if dt != np.int32:
+                got = getattr(x, name)(axis=axis, nan=True)
+                got = got.to_numpy() if hasattr(got, "to_numpy") else got
+                assert np.array_equal(got, oracle.reduce(name, h, axis=axis, nan=True)), (axis, name, "nan: true")
