@@ -18,8 +18,8 @@
 // second launch adds them up with every compute unit: no zero-fill launch before and no atomics
 // on the results. (The block that counted in last on a ticket added them up before: store,
 // acknowledgement, ticket, fence and reads one after the other in one block a column group. us,
-// that / this: [8192,4096] 10.8 / 9.4, [16384,32768] 18.0 / 16.4, [4096,65536] 13.6 / 10.7,
-// [32768,1024] 15.5 / 10.9, [28296,64] 15.3 / 9.9.) count_false counts the set bits too and takes
+// that / this: [8192,4096] 10.8 / 9.0, [16384,32768] 18.0 / 16.4, [4096,65536] 13.6 / 10.7,
+// [32768,1024] 15.5 / 9.0, [26984,720] 13.2 / 9.7.) count_false counts the set bits too and takes
 // them from the number of rows at the end.
 #include "bit_common.h"
 
@@ -226,15 +226,13 @@ struct FoldCounts {
     int count_false, overwrite;
 };
 
-constexpr uint32_t kFoldCols = 32;   // columns of a block
-
-// LANES lanes share a column
-template <uint32_t LANES>
-__global__ __launch_bounds__(kFoldCols * LANES) void bit_count_fold_kernel(FoldCounts p) {
-    __shared__ uint64_t sums[LANES][kFoldCols];
-    const uint32_t lane = threadIdx.x % kFoldCols, share = threadIdx.x / kFoldCols;
+// COLS columns of a block, LANES lanes that share one
+template <uint32_t COLS, uint32_t LANES>
+__global__ __launch_bounds__(COLS * LANES) void bit_count_fold_kernel(FoldCounts p) {
+    __shared__ uint64_t sums[LANES][COLS];
+    const uint32_t lane = threadIdx.x % COLS, share = threadIdx.x / COLS;
     const uint32_t o = blockIdx.x / p.col_groups;
-    const uint32_t col = (blockIdx.x - o * p.col_groups) * kFoldCols + lane;
+    const uint32_t col = (blockIdx.x - o * p.col_groups) * COLS + lane;
     const uint32_t c = col < p.cols ? col : p.cols - 1;
     const uint32_t* counts = p.partial + (uint64_t)o * p.parts * p.width + c;
     uint64_t n = 0;
@@ -251,10 +249,19 @@ __global__ __launch_bounds__(kFoldCols * LANES) void bit_count_fold_kernel(FoldC
         n += ((p.in[bit >> 5] >> (bit & 31u)) & 1u) ^ (uint32_t)(p.count_false != 0);
     }
     sums[share][lane] = n;
+    // (eight are sooner read one after the other than met in three rounds)
+#pragma unroll
+    for (uint32_t half = LANES / 2; half >= 8; half /= 2) {
+        __syncthreads();
+        if (share < half) {
+            n += sums[share + half][lane];
+            sums[share][lane] = n;
+        }
+    }
     __syncthreads();
     if (share != 0 || col >= p.cols) return;
 #pragma unroll
-    for (uint32_t k = 1; k < LANES; ++k) n += sums[k][lane];
+    for (uint32_t k = 1; k < 8; ++k) n += sums[k][lane];
     uint64_t* dst = reinterpret_cast<uint64_t*>(p.out + (int64_t)o * p.o_outer + (int64_t)col * p.o_col);
     *dst = p.overwrite ? n : *dst + n;
 }
@@ -266,7 +273,8 @@ bool vc_geometry(BitCountColsVc& p, uint64_t want_blocks, uint64_t* blocks) {
     p.col_blocks = (p.words + (uint32_t)LANES - 1) / (uint32_t)LANES;
     const uint64_t across = (uint64_t)p.col_blocks * p.n_outer;
     uint64_t parts = (want_blocks + across - 1) / across;
-    const uint64_t most = ((uint64_t)p.rows + 32 * NG - 1) / (32 * NG);   // stretches of 32 rows or more
+    // stretches of sixteen rows or more, what a lane has in flight (us, 32 / 16: [32768,1024] 10.9 / 9.0, [26984,720] 12.0 / 9.7)
+    const uint64_t most = ((uint64_t)p.rows + kVcRows * NG - 1) / (kVcRows * NG);
     if (parts > most) parts = most;
     if (parts < 1) parts = 1;
     p.rows_per_group = (uint32_t)(((uint64_t)p.rows + parts * NG - 1) / (parts * NG));
@@ -285,9 +293,9 @@ namespace cumo_hip {
 // How many rows to take as one: rows that follow one another, off word boundaries or less than two words long, become the rows
 // of a matrix that is a whole number of words and two blocks wide at least, whose columns are counted in their place. Their counts
 // are 32 times the columns', so wide rows are left to the form that shifts their words into place (bit.hip), which keeps every
-// lane busy with them. us, that form / this: [24304,1066] 23.3 / 9.9, [3512,100] 21.9 / 9.5, [180232,137] 16.6 / 13.5,
-// [65536,33] 124.6 / 9.5, [11400,1903] 13.2 / 10.8, [1000,8001] 13.5 / 10.1, [136,9000] 7.3 / 7.8, [400,30001] 9.4 / 15.3. Rows on word
-// boundaries gain nothing from it: [32768,1024] 10.9 as they are, 14.2 so.
+// lane busy with them. us, that form / this: [24304,1066] 23.3 / 8.5, [3512,100] 21.9 / 9.3, [180232,137] 16.6 / 10.2,
+// [65536,33] 124.6 / 10.0, [11400,1903] 13.2 / 10.8, [1000,8001] 13.5 / 10.0; with stretches of 32 rows [136,9000] 7.3 / 7.8 and
+// [400,30001] 9.4 / 15.3. Rows on word boundaries gain nothing from it: [32768,1024] 10.9 as they are, 14.2 so.
 static uint32_t fold_rows(const cumo_hip_bit_count_nd_t* d) {
     const uint64_t cols = d->out_shape[d->out_ndim - 1], rows = d->red_shape[0];
     if (d->out_ndim != 1 || cols > 8192 || (d->pos & 31) != 0 || d->in_red_step[0] != (ssize_t)cols) return 1;
@@ -355,13 +363,17 @@ int bit_count_cols_words_launch(const cumo_hip_bit_count_nd_t* d) {
     f.rest_bit = d->pos + (uint64_t)p.rows * fold * f.cols;
     f.o_outer = p.o_outer;
     f.o_col = p.o_col;
-    f.col_groups = (f.cols + kFoldCols - 1) / kFoldCols;
     f.count_false = d->count_false;
     f.overwrite = d->overwrite;
-    const dim3 g(f.col_groups * p.n_outer);
-    // as many lanes to a column as leave each about eight counts
-    if ((uint64_t)p.parts * fold > 64) hipLaunchKernelGGL((bit_count_fold_kernel<32>), g, dim3(kFoldCols * 32), 0, stream, f);
-    else hipLaunchKernelGGL((bit_count_fold_kernel<8>), g, dim3(kFoldCols * 8), 0, stream, f);
+    // as many lanes to a column as leave each some eight counts, and so fewer columns to a block
+    auto add_up = [&](auto kernel, uint32_t cols, uint32_t lanes) {
+        f.col_groups = (f.cols + cols - 1) / cols;
+        hipLaunchKernelGGL(kernel, dim3(f.col_groups * p.n_outer), dim3(cols * lanes), 0, stream, f);
+    };
+    const uint64_t terms = (uint64_t)p.parts * fold;
+    if (terms > 256) add_up(bit_count_fold_kernel<8, 128>, 8, 128);
+    else if (terms > 64) add_up(bit_count_fold_kernel<32, 32>, 32, 32);
+    else add_up(bit_count_fold_kernel<32, 8>, 32, 8);
     cumo_cuda_runtime_check_kernel_launch();
     // stream-ordered reuse: whoever gets the scratch next can only touch it from later work on this stream
     cumo_cuda_runtime_free(reinterpret_cast<char*>(p.partial));
