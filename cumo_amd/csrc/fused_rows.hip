@@ -139,6 +139,11 @@ struct FusedRowsParams {
     bool through;  // see StoreRows
 };
 
+// whether rows of the result are written through (StoreRows)
+__device__ __forceinline__ bool fr_pieces(const FusedRowsParams& p) {
+    return p.through && store_pieces(p.out, p.out_row_step);
+}
+
 // MODE 0 softmax, 1 layernorm. TPR lanes share a row, each holding NV vectors of V
 // elements (TPR * NV * V >= n). Rows, vectors and the elements of a row's last vector beyond the data are masked.
 // NT: non-temporal accesses, for arrays larger than the last-level cache.
@@ -181,7 +186,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
         auto put = [&](int k) {
             const uint64_t col = ((uint64_t)k * TPR + lane_r) * V;
             if (cnt[k] == V) {
-                store_vector<NT>(reinterpret_cast<u4*>(dst + col * sizeof(T)), x[k].q, p.through && store_pieces(p.out, p.out_row_step));
+                store_vector<NT>(reinterpret_cast<u4*>(dst + col * sizeof(T)), x[k].q, fr_pieces(p));
             } else {
 #pragma unroll
                 for (int j = 0; j < V; ++j)
@@ -367,7 +372,7 @@ struct FrStretch {
 template <class T, int MODE, int LANES, bool NT>
 __global__ __launch_bounds__(LANES, 4) void fused_wide_rows_kernel(FusedRowsParams p) {
     if constexpr (MODE == 0 && sizeof(T) == 4) float_tables_prepare();
-    const bool pieces = p.through && store_pieces(p.out, p.out_row_step);
+    const bool pieces = fr_pieces(p);
     FrStretch<T, LANES, 16> a;
     a.template load<NT>(p.in + (int64_t)blockIdx.x * p.in_row_step, 0, (uint32_t)p.n);
     char* dst = p.out + (int64_t)blockIdx.x * p.out_row_step;
@@ -396,15 +401,14 @@ __global__ __launch_bounds__(LANES, 4) void fused_wide_rows_kernel(FusedRowsPara
 // Sums within a piece are the type's; parts are folded in double.
 template <class T> using FrPiece = FrStretch<T, kFrBlock, 8>;
 
-struct FusedSplitParams {
-    FusedRowsParams f;
+struct FusedSplitParams : FusedRowsParams {
     uint32_t pieces;  // of a row
     double* parts;    // two for each piece, row after row
 };
 
 template <class T>
 __device__ __forceinline__ uint32_t fr_piece_held(const FusedSplitParams& p, uint32_t piece) {
-    const uint64_t left = p.f.n - (uint64_t)piece * FrPiece<T>::kElements;
+    const uint64_t left = p.n - (uint64_t)piece * FrPiece<T>::kElements;
     return left < FrPiece<T>::kElements ? (uint32_t)left : FrPiece<T>::kElements;
 }
 
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_parts_kernel(FusedSplitParams 
     const uint32_t row = blockIdx.x / p.pieces, piece = blockIdx.x - row * p.pieces;
     const uint32_t held = fr_piece_held<T>(p, piece);
     FrPiece<T> a;
-    a.template load<false>(p.f.in + (int64_t)row * p.f.in_row_step, (uint64_t)piece * FrPiece<T>::kElements, held);
+    a.template load<false>(p.in + (int64_t)row * p.in_row_step, (uint64_t)piece * FrPiece<T>::kElements, held);
     double* part = p.parts + 2 * (uint64_t)blockIdx.x;
     if constexpr (MODE == 0) {
         a.fill(-INFINITY);
@@ -444,11 +448,11 @@ __global__ __launch_bounds__(kFrBlock) void fused_apply_kernel(FusedSplitParams 
     const uint32_t row = at / p.pieces, piece = at - row * p.pieces;
     const uint64_t start = (uint64_t)piece * FrPiece<T>::kElements;
     FrPiece<T> a;
-    a.template load<NT>(p.f.in + (int64_t)row * p.f.in_row_step, start, fr_piece_held<T>(p, piece));
+    a.template load<NT>(p.in + (int64_t)row * p.in_row_step, start, fr_piece_held<T>(p, piece));
     if constexpr (MODE == 0 && sizeof(T) == 4) float_tables_prepare();
     const double* part = p.parts + 2 * (uint64_t)row * p.pieces;
-    char* dst = p.f.out + (int64_t)row * p.f.out_row_step;
-    const bool pieces = p.f.through && store_pieces(p.f.out, p.f.out_row_step);
+    char* dst = p.out + (int64_t)row * p.out_row_step;
+    const bool pieces = fr_pieces(p);
     if constexpr (MODE == 0) {
         double m = -INFINITY;
         for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) m = fr_max_nan(m, part[2 * c]);
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_apply_kernel(FusedSplitParams 
         const FrDivisor<T> by_s(s);
         a.template store<NT>(dst, start, pieces, [&](T v) { return by_s.divide(fr_exp<T>(v - mt)); });
     } else {
-        const double n = (double)p.f.n;
+        const double n = (double)p.n;
         double s = 0.0;
         for (uint32_t c = threadIdx.x; c < p.pieces; c += kFrBlock) s += part[2 * c];
         s = fr_allsum<T, kFrBlock>(s);
@@ -473,7 +477,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_apply_kernel(FusedSplitParams 
         }
         q = fr_allsum<T, kFrBlock>(q);
         const T var = (T)(q / (n - 1.0));
-        const T sd = fr_sqrt<T>(var + (T)p.f.eps);
+        const T sd = fr_sqrt<T>(var + (T)p.eps);
         const T mt = (T)mean;
         a.template store<NT>(dst, start, pieces, [&](T v) { return (v - mt) / sd; });
     }
