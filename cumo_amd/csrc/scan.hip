@@ -18,8 +18,8 @@
 //   three launches          one long run that is strided: per-tile totals, a scan of the
 //                           totals, then every tile scans itself from its offset (reads the
 //                           input twice);
-//   scan_cols_chain_kernel  long runs that lie across memory (down the rows of a matrix) in
-//                           one pass, tiles of 256 rows handing on their column totals;
+//   scan_cols_chain_kernel  runs that lie across memory (down the rows of a matrix) in one
+//                           pass, tiles of 256 rows or more handing on their column totals;
 //   scan_cols_kernel        other runs across memory, in segments and two passes.
 // Inside a tile each lane owns 8 consecutive elements: it scans them in registers,
 // the lane totals are scanned across the wave with shuffles and the four wave
@@ -996,6 +996,7 @@ __global__ __launch_bounds__(kScanBlock) void scan_cols_kernel(ScanColsParams p,
 }
 
 constexpr uint64_t kScanLookbackSegs = 32;
+constexpr uint64_t kScanColsThreads = 256ull * 8 * kScanBlock;  // lanes that the segments are to make
 
 // Two passes over the data with the segment totals between them. With few segments
 // the second pass folds the totals of the segments before its own by itself (two
@@ -1011,7 +1012,7 @@ void scan_cols_launch_vec(ScanColsParams& p, hipStream_t stream) {
     // segments: enough threads for eight blocks on every compute unit, at least 16 rows each;
     // no more than the second pass folds by itself when those already give every compute unit four
     // blocks (with one block each, SFloat [8192,8192] ran its first pass at half the bandwidth)
-    const uint64_t want_threads = 256ull * 8 * kScanBlock;
+    const uint64_t want_threads = kScanColsThreads;
     const uint64_t lanes_per_seg = col_groups * p.planes;
     uint64_t n_seg = (want_threads + lanes_per_seg - 1) / lanes_per_seg;
     const uint64_t max_seg = (p.n + 15) / 16;
@@ -1421,23 +1422,34 @@ bool scan_cols_chain_go(const ScanColsParams& p, hipStream_t stream) {
     return true;
 }
 
-// Any matrix whose rows hold a vector: what this leaves to the two passes (totals, perhaps their own scan, and the data
-// again) is rows of less than that, and more than 4096 tiles down. Up to 256 rows are one tile, in blocks of four waves up to 64
+// Matrices whose rows hold a vector: what this leaves to the segments is rows of less than that, more than 4096 tiles down, and
+// what the tests below say. Up to 256 rows are one tile, in blocks of four waves up to 64
 // rows. us, two passes / this:
 //   rows that are few    SFloat [208,53952] 29.2 / 15.4, [64,500000] 68.6 / 46.8, [31,32000] 8.3 / 5.5; DFloat [76,440000] 149 / 100
 //   columns that are few SFloat [234385,93] 94.5 / 39.2, [20000,130] 25.0 / 14.2, [1000000,16] 416 / 39.9; DFloat [131072,33] 44 / 20
-//   matrices of few tiles SFloat [619,640] 14.2 / 9.0, [100,100] 6.9 / 5.6, [3036,248] 15.5 / 10.5
+//   matrices of few tiles SFloat [619,640] 14.2 / 9.0, [3036,248] 15.5 / 10.5, DFloat [20,700] 6.1 / 4.3
 template <class T, class Op>
 bool scan_cols_chain_launch(ScanColsParams& p, hipStream_t stream) {
     constexpr int V = 16 / (int)sizeof(T);
     if (!scan_cols_chain_enabled() || p.cols < (uint64_t)V || p.n < 2) return false;
     const uint64_t vectors = (p.cols + V - 1) / V;
+    // Up to sixteen rows, or columns enough for a lane each: the segments are one, a launch that reads and writes once (us, that /
+    // this: [12,100000] 4.3 / 5.1, [3,20] 3.3 / 5.7); rows of 64 vectors keep to the tiles where there are two of them.
+    const bool one_segment = p.n <= (uint64_t)kColsChainRows || vectors * p.planes >= kScanColsThreads;
+    if (one_segment && (vectors < 64 || p.n <= 16 * kColsChainRows)) return false;
+    // Up to 512 rows are two launches in segments, which small arrays are done with sooner than tiles hand on their totals ([300,200]
+    // 7.5 / 9.3, [500,130] 8.2 / 10.1; [300,3000] 9.3 / 8.6): one tile or a MiB of them.
+    const bool one_tile = vectors > 32 && p.n <= 16 * kColsChainRows;
+    if (!one_tile && p.n <= kScanLookbackSegs * 16 && p.planes * p.n * p.cols * sizeof(T) < (1u << 20)) return false;
     if (vectors > 32) {
         if (p.n <= 4 * kColsChainRows) return scan_cols_chain_go<T, Op, 4, 64, true, true, false>(p, stream);
         if (p.n <= 16 * kColsChainRows) return scan_cols_chain_go<T, Op, 16, 64, true, true, false>(p, stream);
         if (p.n <= 512 * 16 * kColsChainRows) return scan_cols_chain_go<T, Op, 16, 64, true, false, false>(p, stream);
         return scan_cols_chain_go<T, Op, 16, 64, true, false, true>(p, stream);
     }
+    // (many planes of fewer rows than a quarter of a tile would be tiles, and words, of nothing)
+    const uint64_t bands = vectors > 16 ? 2 : vectors > 8 ? 4 : 8;
+    if (p.n < 4 * bands * kColsChainRows) return false;
     if (vectors > 16) return scan_cols_chain_go<T, Op, 16, 32, true, false, true>(p, stream);
     if (vectors > 8) return scan_cols_chain_go<T, Op, 16, 16, false, false, true>(p, stream);
     return scan_cols_chain_go<T, Op, 16, 8, false, false, true>(p, stream);
