@@ -41,6 +41,11 @@ template <class I> struct folds_columns_together<I, decltype((void)I::COLUMNS_TO
 template <class I, class = void> struct combines_in_two_forms { static constexpr bool value = false; };
 template <class I> struct combines_in_two_forms<I, decltype((void)&I::combine_seldom)> { static constexpr bool value = true; };
 
+// An Impl whose accumulate_step<U, VEC>(x[U][VEC], vectors, acc) folds a step's elements, of which the first `vectors` vectors are
+// there, among themselves before they join the accumulator: what a long row's sum rounds off does not depend on how few lanes share it.
+template <class I, class = void> struct folds_steps { static constexpr bool value = false; };
+template <class I> struct folds_steps<I, decltype((void)I::STEPS)> { static constexpr bool value = I::STEPS; };
+
 // An Impl whose accumulate_columns_by_position<U, VEC>(x[U][VEC], first position, acc[VEC]) folds U consecutive
 // positions of VEC neighbouring outputs without a branch
 template <class I, class = void> struct folds_columns_by_position { static constexpr bool value = false; };
@@ -107,7 +112,11 @@ __device__ __forceinline__ void rs_split_out(const RedSParams& p, uint32_t o, ui
 // kRsUnroll vectors per lane. end is a multiple of VEC. Every lane of the group runs the
 // same number of steps. The run may go on for `tail` more elements, fewer than a vector: the
 // group's first lane folds those one by one when the group has the run's first tile (first == 0).
-template <class Impl, int VEC, bool NT>
+// In a wide block sums go step by step as pairs of pairs: its lanes are fewer than those of the blocks that would share the row, so
+// that one element after the other a lane's chain was up to four times as long. Error in norm, rows of zero mean, cut across
+// blocks / a wide block, one after the other / as pairs: SFloat 128 x 262144 1.5e-7 / 3.0e-7 / 1.3e-7, 200 x 100000 1.5e-7 / 2.0e-7 / 1.2e-7,
+// DFloat 200 x 100000 2.8e-16 / 3.7e-16 / 2.3e-16; the times are the same.
+template <class Impl, int VEC, bool NT, int BLOCK = kRedBlock>
 __device__ __forceinline__ typename Impl::Acc rs_row_scan(const Impl& impl, const char* base, uint64_t first, uint64_t every, uint64_t end,
                                                           uint32_t tail, unsigned lane_r, unsigned tpr_bits, int64_t idx_base) {
     typedef typename Impl::In In;
@@ -131,6 +140,13 @@ __device__ __forceinline__ typename Impl::Acc rs_row_scan(const Impl& impl, cons
         // every load of the step is issued before anything is folded (the scheduler would
         // otherwise start folding the first vector and hold the later loads back behind it)
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (BLOCK > kRedBlock && folds_steps<Impl>::value) {
+            uint32_t vectors = 0;
+#pragma unroll
+            for (int u = 0; u < kRsUnroll; ++u) vectors += i0 + (uint64_t)u * stride < end ? 1u : 0u;
+            impl.template accumulate_step<kRsUnroll, VEC>(x, vectors, acc);
+            continue;
+        }
         if constexpr (has_group<Impl>::value) {
             if (i0 + (uint64_t)(kRsUnroll - 1) * stride < end) {
                 int64_t idx[kRsUnroll];
@@ -171,7 +187,7 @@ __device__ __forceinline__ void rs_group_combine(const Impl& impl, typename Impl
         if ((threadIdx.x & 63) == 0) wave_slots[threadIdx.x >> 6] = acc;
         __syncthreads();
         if constexpr (WAVES > 4) {
-            // neighbours first, as within the wave
+            // the far half onto the near one, as within the wave
             if (threadIdx.x < 64) {
                 acc = wave_slots[threadIdx.x & (WAVES - 1)];
                 for (unsigned d = WAVES >> 1; d > 0; d >>= 1) {
@@ -192,7 +208,7 @@ __device__ __forceinline__ typename Impl::Acc rs_row_reduce(const Impl& impl, co
                                                             uint32_t tail, unsigned lane_r, unsigned tpr_bits, int64_t idx_base,
                                                             typename Impl::Acc* wave_slots, int* s_need) {
     typedef typename Impl::Acc Acc;
-    Acc acc = rs_row_scan<Impl, VEC, NT>(impl, base, first, every, end, tail, lane_r, tpr_bits, idx_base);
+    Acc acc = rs_row_scan<Impl, VEC, NT, BLOCK>(impl, base, first, every, end, tail, lane_r, tpr_bits, idx_base);
     rs_group_combine<Impl, BLOCK>(impl, acc, tpr_bits, wave_slots);
     if constexpr (has_exact<Impl>::value) {
         const unsigned TPR = 1u << tpr_bits;

@@ -601,6 +601,39 @@ def test_column_sums_lose_no_more_than_short_chains_do(tname, dt, shape, lanes):
         assert off(d.var(axis=0), h.astype(np.float64).var(axis=0, ddof=1)) <= u / 3 ** 0.5 * (0.63 * m ** (1 / 3) / lanes + 6) ** 0.5
 
 
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("rows,n", [(200, 262144), (240, 400003), (96, 40001)])
+def test_row_sums_of_wide_blocks_lose_no_more_than_pairs_do(tname, dt, rows, n):
+    """The rounding error of sums along long rows that a block of 1024 lanes takes, values of both signs, in norm."""
+    rng = np.random.default_rng(95)
+    n //= 2 if tname == "dfloat" else 1
+    h = rng.normal(size=(rows, n)).astype(dt)
+    d = cls_of(tname).cast(h)
+    k = h[:, ::7].copy()   # some of them NaN, for the sums that skip those
+    hn = h.copy()
+    hn[:, ::7] = np.nan
+    dn = cls_of(tname).cast(hn)
+    exact = h.astype(np.longdouble).sum(axis=1)
+    kept = exact - k.astype(np.longdouble).sum(axis=1)
+    # An addition whose result has the size S rounds by u / 2 * S at most in root mean square (u: half a unit in the last place; uniform
+    # in it, at mantissas from 1 to 2), each on its own. A sum of m such values has the size sqrt(m), so n elements paired up to runs
+    # twice as long lose u / 2 * sqrt(n), a lane's chain of s steps u / 2 * sqrt(n s / 2); sixteen elements (eight) to a step, 1024
+    # lanes. A quarter to spare, for the scatter of a few hundred rows. (One element after the other, a lane's chain alone is 16 s long
+    # and loses u / 2 * sqrt(8 n s): more than twice this bound at 262144.)
+    u = np.finfo(dt).eps / 2
+    step = 1024 * (16 if tname == "sfloat" else 8)
+    s = -(-n // step)
+    bound = 0.5 * u * (np.log2(step) + s / 2) ** 0.5 * 1.25
+
+    def off(got, want):
+        return float(np.linalg.norm((got.to_numpy().astype(np.longdouble) - want).astype(np.float64)) / np.linalg.norm(want.astype(np.float64)))
+
+    assert off(d.sum(axis=1), exact) <= bound
+    assert off(dn.sum(axis=1, nan=True), kept) <= bound
+    assert off(d.mean(axis=1), exact / n) <= bound + u
+    assert off(dn.mean(axis=1, nan=True), kept / (n - k.shape[1])) <= bound + u
+
+
 COLUMN_SPLITS = [(7, 40), (9, 17), (1024, 18), (1025, 19), (2047, 516), (2049, 1029), (5000, 64), (40003, 257), (9, 262149)]
 ROW_VIEWS = [lambda a: a, lambda a: a[1::2], lambda a: a[::-1], lambda a: a[:, 1:]]
 
