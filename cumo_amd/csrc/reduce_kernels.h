@@ -750,14 +750,30 @@ static inline ColumnSplit red_split_columns(uint64_t groups, uint64_t n, bool wh
 }
 
 // Whether long rows that the planner would cut across blocks (fewer than 512 of them, of 16384 elements or more) go a row to
-// a block of kRsWide lanes instead: nothing to hand over between blocks, and 64 KiB of a row in flight on a compute unit. us of
-// sum / argmax on fresh operands, cut across blocks -> a row to a block:
-//  * more than 256 rows, where every block of a cut row would count in on tickets (and its last one fence): 394 x 54853
-//    SFloat 43.5 / 45.5 -> 17.2 / 20.8, 300 x 16384 18.2 / 18.2 -> 6.3 / 9.5, 474 x 23270 DFloat 39.4 / 41.2 -> 16.3 / 20.9;
-//  * 128 to 256 rows, against the hand-over words: 128 x 262144 25.6 / 27.9 -> 24.7 / 26.5, 200 x 100000 15.9 / 18.3 -> 14.7 / 16.1;
-//  * fewer leave compute units idle, which long rows cannot afford (96 x 300000 21.4 -> 27.6) and short ones can (80 x 16384
-//    5.7 -> 4.0, 64 x 40000 6.0 -> 4.9; 64 rows of 400 KB are even).
-static inline bool red_rows_wide(uint64_t rows, uint64_t row_bytes) { return rows >= 128 || (rows >= 48 && row_bytes <= (256u << 10)); }
+// a block of kRsWide lanes instead: nothing to hand over between blocks, and 64 KiB of a row in flight on a compute unit. Against that
+// stand the compute units left idle or with one block more than the others, which cost in proportion to the row. `handed`: whether the
+// cut rows' accumulators would go through the hand-over words (256 rows at most), else every block counts in on tickets. us of
+// sum / var, cut across blocks -> a row to a block:
+//  * short rows always: 48 x 33280 SFloat 4.9 / 6.8 -> 4.5 / 5.8, 128 x 65536 9.2 / 10.9 -> 8.6 / 10.0; beyond 192 KiB fewer than 100
+//    are even or worse (64 x 65536 6.4 / 8.1 -> 7.1 / 8.6);
+//  * handed: 128 rows are worse (131405 SFloat 14.4 / 16.9 -> 17.8 / 18.8, 524621 44.4 / 48.2 -> 59.7 / 60.8), 144 and 160 of whole
+//    vectors better (144 x 131072 16.2 / 18.9 -> 15.3 / 16.8, 160 x 524288 53.5 / 56.3 -> 49.8 / 51.0) and others not (160 x 524621
+//    55.7 / 59.1 -> 60.2 / 60.3), 200 and more better (524288 66.4 / 69.7 -> 64.0 / 65.7; 240 x 2^20 157 / 162 -> 146 / 147), or even
+//    where they are no whole vectors;
+//  * with tickets: var of 128 x 98637 DFloat 33.7 -> 24.9, x 262477 52.6 -> 57.8, 200 x 524288 140 -> 122; 300 x 262144 SFloat
+//    75.8 / 76.6 -> 58.7 / 60.9, x 393549 95.5 / 95.7 -> 96.8 / 98.3, x 786765 164 / 165 -> 193 / 194; 257 x 524288 114 / 110 -> 102 /
+//    105; 350 x 524621 135 / 137 -> 133 / 134; 420 x 786765 224 / 227 -> 220 / 222.
+static inline bool red_rows_wide(uint64_t rows, uint64_t row_bytes, bool handed) {
+    const uint64_t kib = (row_bytes + 1023) >> 10;
+    const bool vectors = row_bytes % 16 == 0;
+    if (rows < 48) return false;
+    if (kib <= (rows < 100 ? 192u : 256u)) return true;
+    if (rows < 128) return false;
+    if (handed) return rows >= 192 ? kib <= 4096 : vectors && (rows >= 160 ? kib <= 4096 : rows >= 144 && kib <= 512);
+    if (rows < 160) return kib <= 1536;
+    if (rows > 256 && rows < 400) return kib <= (rows >= 320 || vectors ? 2048u : 1536u);
+    return kib <= 4096;
+}
 
 // The lean kernels of reduce_stream.h for the layouts they take. Returns 1 when the
 // reduction has been launched, 0 when the general kernels must take it, -1 when the
@@ -874,7 +890,13 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
         }
         if (force_bits >= 0 && force_bits <= 8 && plan.n_split <= 1) p.tpr_bits = (uint32_t)force_bits;
     }
-    if (plan.n_split > 1 && red_rows_wide(plan.out_total, plan.red_total * sizeof(In))) {
+    // no more blocks to a row than it has tiles (what a block loads in one step)
+    const uint64_t tile = (uint64_t)kRedBlock * V * kRsUnroll;
+    const uint64_t tiles = (plan.red_total + tile - 1) / tile;
+    p.n_split = (uint32_t)((uint64_t)plan.n_split < tiles ? (uint64_t)plan.n_split : tiles);
+    const bool words_hold = plan.out_total <= kRsHandoverOutputs && plan.out_total * (uint64_t)p.n_split * (sizeof(Acc) / 4) <= kRsHandoverWords;
+    // (by shape and type alone, not by whether the words are to be had: the same on every stream and under capture)
+    if (plan.n_split > 1 && red_rows_wide(plan.out_total, plan.red_total * sizeof(In), words_hold)) {
         p.tpr_bits = 10;
         const dim3 g((unsigned)plan.out_total), b2(kRsWide);
         if (nt) hipLaunchKernelGGL((red_srow_kernel<Impl, V, true, kRsWide>), g, b2, 0, stream, p, impl);
@@ -893,11 +915,7 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
         return 1;
     }
 
-    // the axis cut over several blocks per output (127 of them at most), one launch
-    // no more blocks than the axis has tiles (what a block loads in one step)
-    const uint64_t tile = (uint64_t)kRedBlock * V * kRsUnroll;
-    const uint64_t tiles = (plan.red_total + tile - 1) / tile;
-    p.n_split = (uint32_t)((uint64_t)plan.n_split < tiles ? (uint64_t)plan.n_split : tiles);
+    // the axis cut over several blocks per output, one launch
     if (p.n_split <= 1) return 0;
     // few outputs: the form without tickets, when the accumulators fit the hand-over words. Not while
     // the stream is being captured: a replayed launch would carry the same launch number again and
@@ -911,9 +929,8 @@ static int red_stream_launch(const ReducePlan& plan, const cumo_na_reduction_arg
     // certainly keeps resident beside them (two blocks of this size per compute unit): the blocks
     // they wait for then always find room. With fewer compute units than this build was tuned for
     // (a partitioned device) fewer outputs qualify.
-    const uint64_t poll_outputs_max = (uint64_t)device_compute_units() < 256 ? (uint64_t)device_compute_units() : 256;
-    if (!fixed && red_poll_enabled() && capturing == hipStreamCaptureStatusNone && plan.out_total <= poll_outputs_max &&
-        plan.out_total * (uint64_t)p.n_split * (sizeof(Acc) / 4) <= kRsHandoverWords) {
+    const uint64_t poll_outputs_max = (uint64_t)device_compute_units() < kRsHandoverOutputs ? (uint64_t)device_compute_units() : kRsHandoverOutputs;
+    if (!fixed && red_poll_enabled() && capturing == hipStreamCaptureStatusNone && plan.out_total <= poll_outputs_max && words_hold) {
         uint32_t launch = 0;
         uint64_t* words = red_handover_words(stream_slot(stream), &launch);
         p.wait = words != nullptr ? wait_ctl() : nullptr;

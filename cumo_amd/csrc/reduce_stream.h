@@ -504,6 +504,7 @@ __device__ __attribute__((noinline)) typename Impl::Acc rs_exact_refold_wave(con
 // anything, so the waiting blocks (which the dispatcher starts first) cannot hold the others up;
 // a wait gives up after kRsPollLimit looks, counts that and raises the host's give-up word (wait_ctl.h).
 constexpr uint32_t kRsHandoverWords = 8192;
+constexpr uint32_t kRsHandoverOutputs = 256;
 constexpr uint32_t kRsPollLimit = 1u << 24;
 
 template <class Acc>

@@ -222,7 +222,8 @@ def test_column_sums_of_rows_that_are_not_whole_vectors(tname, dt, shape):
 @pytest.mark.parametrize("tname,dt", FLOATS)
 @pytest.mark.parametrize("shape,axis", [((1000003,), None), ((7, 100000), 1), ((100000, 7), 0), ((3, 40000, 5), 1),
                                         ((64, 64, 64), (0, 2)), ((2, 3), None), ((1,), None), ((70000, 3), 1),
-                                        ((5, 8192), 1), ((4096, 33), 0), ((33, 4096), 0), ((3, 2000003), 1), ((130, 40000), 1), ((260, 30000), 1)])
+                                        ((5, 8192), 1), ((4096, 33), 0), ((33, 4096), 0), ((3, 2000003), 1), ((130, 40000), 1), ((260, 30000), 1),
+                                        ((100, 70001), 1)])
 def test_random_float_sums(tname, dt, shape, axis):
     rng = np.random.default_rng(201)
     cls = cls_of(tname)
@@ -490,6 +491,26 @@ def test_long_rows_with_a_wide_block_each(tname, dt, shape, axis):
     """Tens to hundreds of rows of 16384 elements or more: a block of 1024 lanes takes a row (four tiles or fewer of
     it, the last one partly there). The same answers at the row's end as for any other run."""
     test_runs_that_end_in_part_of_a_vector(tname, dt, shape, axis)
+
+
+@pytest.mark.parametrize("tname,dt", FLOATS)
+@pytest.mark.parametrize("rows,kib", [(47, 64), (48, 64), (99, 192), (99, 193), (100, 256), (127, 257), (128, 256), (128, 257), (144, 257), (159, 257), (160, 257), (191, 257),
+                                      (192, 257), (256, 257), (257, 257)])
+def test_long_rows_that_blocks_share_or_have_to_themselves(tname, dt, rows, kib):
+    """Either side of the sizes at which a block of 1024 lanes takes a whole row, rows of whole vectors and one element more or less."""
+    rng = np.random.default_rng(97)
+    cls = cls_of(tname)
+    for extra in (0, 1 if kib % 2 else -1):
+        n = kib * 1024 // np.dtype(dt).itemsize + extra
+        h = rng.integers(-64, 65, size=(rows, n)).astype(dt)   # (every sum, and every sum of squares, is a whole number that the type holds)
+        h[:, -1] = 64 + np.arange(rows) % 2
+        d = cls.cast(h)
+        assert_bits_equal(d.sum(axis=1).to_numpy(), h.astype(np.float64).sum(axis=1).astype(dt))
+        assert_bits_equal(d.max(axis=1).to_numpy(), h.max(axis=1))
+        assert_bits_equal(d.min(axis=1).to_numpy(), h.min(axis=1))
+        assert (d.argmax(axis=1).to_numpy() == h.argmax(axis=1)).all()
+        want = h.astype(np.float64).var(axis=1, ddof=1)
+        assert_reduction_close(d.var(axis=1).to_numpy(), want.astype(dt), n, want, "var")
 
 
 @pytest.mark.parametrize("tname,dt", FLOATS)
