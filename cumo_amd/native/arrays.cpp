@@ -612,33 +612,41 @@ PyObject* na_window(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const bool many = PyTuple_CheckExact(a[1]);
     const Py_ssize_t given = many ? PyTuple_GET_SIZE(a[1]) : 1;
     if (given > nd || nd > CUMO_NA_MAX_DIMENSION || PyTuple_GET_SIZE(x->strides) != nd) Py_RETURN_NONE;
+    // All that is asked of x and all that may send the key elsewhere comes first: a slice's numbers may be objects whose __index__
+    // runs, once, and may set x anew.
     Py_ssize_t shape[CUMO_NA_MAX_DIMENSION], strides[CUMO_NA_MAX_DIMENSION], offset = x->offset;
-    Py_ssize_t left = 0;
+    PyObject* part[CUMO_NA_MAX_DIMENSION];
     for (Py_ssize_t d = 0; d < nd; d++) {
-        const Py_ssize_t len = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->shape, d));
-        const Py_ssize_t step = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->strides, d));
-        if ((len == -1 || step == -1) && PyErr_Occurred()) return nullptr;
-        PyObject* k = d >= given ? Py_True : many ? PyTuple_GET_ITEM(a[1], d) : a[1];
-        if (k == Py_True) {
-            shape[left] = len;
-            strides[left++] = step;
-        } else if (PyLong_CheckExact(k)) {
-            Py_ssize_t at = PyLong_AsSsize_t(k);
+        shape[d] = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->shape, d));
+        strides[d] = PyLong_AsSsize_t(PyTuple_GET_ITEM(x->strides, d));
+        if ((shape[d] == -1 || strides[d] == -1) && PyErr_Occurred()) return nullptr;
+        PyObject* k = part[d] = d >= given ? Py_True : many ? PyTuple_GET_ITEM(a[1], d) : a[1];
+        if (PyLong_CheckExact(k)) {
+            const Py_ssize_t at = PyLong_AsSsize_t(k);
             if (at == -1 && PyErr_Occurred()) {
                 PyErr_Clear();
                 Py_RETURN_NONE;
             }
-            if (at < 0) at += len;
-            if (at < 0 || at >= len) Py_RETURN_NONE;
-            offset += at * step;
-        } else if (PySlice_Check(k)) {
+            if (at < -shape[d] || at >= shape[d]) Py_RETURN_NONE;
+        } else if (k != Py_True && !PySlice_Check(k)) {
+            Py_RETURN_NONE;
+        }
+    }
+    Py_ssize_t left = 0;   // (never past d: what stands there has been read)
+    for (Py_ssize_t d = 0; d < nd; d++) {
+        const Py_ssize_t len = shape[d], step = strides[d];
+        if (part[d] == Py_True) {
+            shape[left] = len;
+            strides[left++] = step;
+        } else if (PyLong_CheckExact(part[d])) {
+            const Py_ssize_t at = PyLong_AsSsize_t(part[d]);
+            offset += (at < 0 ? at + len : at) * step;
+        } else {
             Py_ssize_t from, to, by;
-            if (PySlice_Unpack(k, &from, &to, &by) < 0) return nullptr;
+            if (PySlice_Unpack(part[d], &from, &to, &by) < 0) return nullptr;
             shape[left] = PySlice_AdjustIndices(len, &from, &to, by);
             offset += from * step;
             if (by == PY_SSIZE_T_MAX || by == -PY_SSIZE_T_MAX || __builtin_mul_overflow(step, by, &strides[left++])) Py_RETURN_NONE;
-        } else {
-            Py_RETURN_NONE;
         }
     }
     PyObject* self = type->tp_alloc(type, 0);
