@@ -15,6 +15,7 @@
 //                           in registers wave by wave;
 //   scan_chain_kernel       one contiguous run, or a few long ones, in one pass: tiles hand their
 //                           totals on through words in memory (read once, written once);
+//   scan_chain_alone_kernel those few, a block to each, where the stream keeps no such words: the same bits;
 //   three launches          one long run that is strided: per-tile totals, a scan of the
 //                           totals, then every tile scans itself from its offset (reads the
 //                           input twice);
@@ -464,11 +465,10 @@ struct ChainShared {
 // after everything that exists, so what they add to never reaches an element that is stored).
 // The one vector that is partly there goes element by element: nothing is read past the run.
 template <class T, bool NT, int R, bool RAGGED = false>
-__device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first, ScanVec<T> (&v)[R], uint32_t nelem = 0) {
+__device__ __forceinline__ void chain_issue_loads(const char* in, uint64_t first, ScanVec<T> (&v)[R], uint32_t nelem = 0, int w = threadIdx.x >> 6) {
     typedef typename ScanVec<T>::u4 u4;
     constexpr int V = ScanVec<T>::V;
     const unsigned lane = threadIdx.x & 63u;
-    const int w = threadIdx.x >> 6;
     const u4* src = reinterpret_cast<const u4*>(in + (first + (uint64_t)w * (R * 64 * V)) * sizeof(T)) + lane;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -554,11 +554,10 @@ __device__ __forceinline__ void chain_scan_tile(ScanVec<T> (&v)[R], T* s_wave_to
 // adds what precedes the tile (if anything) and the earlier waves' total, and stores (pieces: see store_form.h)
 template <class T, class Op, bool NT, int R, bool RAGGED = false>
 __device__ __forceinline__ void chain_store_tile(char* out, uint64_t first, ScanVec<T> (&v)[R], T head, bool head_has, T wave_pre, bool pieces,
-                                                 uint32_t nelem = 0) {
+                                                 uint32_t nelem = 0, int w = threadIdx.x >> 6) {
     typedef typename ScanVec<T>::u4 u4;
     constexpr int V = ScanVec<T>::V;
     const unsigned lane = threadIdx.x & 63u;
-    const int w = threadIdx.x >> 6;
     if (w > 0) {
         head = head_has ? Op::apply(head, wave_pre) : wave_pre;
         head_has = true;
@@ -682,6 +681,79 @@ __global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_ke
     const bool pieces = p.through && store_pieces(out);
     if (whole) chain_store_tile<T, Op, NT, R>(out, first, v, s_prefix, sh.prefix_has != 0, wave_pre, pieces);
     else chain_store_tile<T, Op, NT, R, true>(out, first, v, s_prefix, sh.prefix_has != 0, wave_pre, pieces, nelem);
+}
+
+// a barrier for what is in LDS: __syncthreads() also waits for the block's loads and stores
+__device__ __forceinline__ void chain_meet() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The same without words in memory, for streams that keep none (a stream under capture: a replay would repeat the launch's number): a
+// block has a run to itself, STEP tiles at a time, and keeps the totals of its tiles, groups and supergroups in LDS. Tiles, and the order
+// in which their totals are folded, are those of the one pass, and so is every bit of the result; a few compute units do all the work.
+// us, this in a graph / scan_rows_whole_kernel there, whose bits are others / the one pass: SFloat [8,20000] 6.4 / 7.4 / 6.1, one run of
+// 65000 11.1 / 14.9 / 5.7, [100,40000] 11.9 / 11.1 / 10.9, [72,438001] 70 / 135 / 53; DFloat 10.0 / 11.6 / 6.3, 22.6 / 30.1 / 6.2,
+// 20.8 / 27.6 / 19.3, 200 / 300 / 101. Bound by what a step takes from its loads to its stores, some 1.5 us; tiles asked for a step
+// ahead did not shorten it, four small tiles or two of 64 KiB to a step did (one run of 65000: 23.1 and 47.6 with one).
+template <class T, class Op, int NW, int R, int STEP>
+__global__ __launch_bounds__(STEP * NW * 64) void scan_chain_alone_kernel(ScanRowsParams p) {
+    constexpr uint32_t TILE = NW * R * 64 * ScanVec<T>::V;
+    static_assert(64 % STEP == 0, "the tiles of a step are of one group");
+    __shared__ T s_tile[64], s_group[64], s_super[64];
+    __shared__ T s_wave_tot[STEP][NW];
+    const unsigned lane = threadIdx.x & 63u;
+    const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / (NW * 64)));   // this wave's tile of a step
+    const int w = (int)(threadIdx.x >> 6) % NW;                                                     // and its place in the tile
+    const char* in;
+    char* out;
+    scan_run_start(p, blockIdx.x, in, out);
+    const bool pieces = p.through && store_pieces(out);
+    uint32_t t = q;
+    for (uint64_t step = 0; step < p.n; step += (uint64_t)STEP * TILE, t += STEP) {
+        const uint64_t first = step + q * TILE;
+        ScanVec<T> v[R];
+        // (a tile that lies behind the run's end holds nothing)
+        const bool whole = first + TILE <= p.n;
+        const uint32_t nelem = first < p.n ? (uint32_t)(p.n - first) : 0;
+        T total, wave_pre;
+        if (whole) {
+            chain_issue_loads<T, false, R>(in, first, v, 0, w);
+            total = chain_scan_wave<T, Op, R>(v);
+        } else {
+            chain_issue_loads<T, false, R, true>(in, first, v, nelem, w);
+            total = chain_scan_wave<T, Op, R>(v);
+        }
+        if (lane == 0) s_wave_tot[q][w] = total;
+        chain_meet();
+        chain_fold_waves<T, Op, NW>(s_wave_tot[q], w, total, wave_pre);
+        const uint32_t pos = t & 63u, g = t >> 6, gpos = g & 63u, sg = g >> 6;
+        if (w == 0 && lane == 0) s_tile[pos] = total;
+        chain_meet();
+        T x = lane < pos ? s_tile[lane] : T(), y = lane < gpos ? s_group[lane] : T(), z = lane < sg ? s_super[lane] : T();
+        bool xh, yh, zh;
+        chain_fold_lanes<T, Op>(x, xh, pos);
+        chain_fold_lanes<T, Op>(y, yh, gpos);
+        chain_fold_lanes<T, Op>(z, zh, sg);
+        // (read from the step after the next barrier on)
+        if (pos == 63u && w == 0 && lane == 0) {
+            T sum = x;
+            bool has = xh;
+            chain_join<T, Op>(sum, has, total, true);
+            s_group[gpos] = sum;
+            if (gpos == 63u) {
+                T st = y;
+                has = yh;
+                chain_join<T, Op>(st, has, sum, true);
+                s_super[sg] = st;
+            }
+        }
+        chain_join<T, Op>(z, zh, y, yh);
+        chain_join<T, Op>(z, zh, x, xh);
+        if (whole) chain_store_tile<T, Op, false, R>(out, first, v, z, zh, wave_pre, pieces, 0, w);
+        else chain_store_tile<T, Op, false, R, true>(out, first, v, z, zh, wave_pre, pieces, nelem, w);
+    }
 }
 
 __global__ __launch_bounds__(256) void scan_chain_clear_kernel(uint64_t* words, uint64_t n) {
@@ -809,7 +881,7 @@ static void chain_words_release(const ChainWords& w) {
 static bool scan_chain_pays(uint64_t rows, uint64_t bytes) { return rows < 256 && bytes > 2 * kChainSmallBytes + rows * 1024; }
 
 // The runs of p, contiguous and aligned as their elements are (p.through is set), in one pass; kept_only: with words that the stream
-// keeps or not at all.
+// keeps, or, where it keeps none, tile after tile by one block a run, to the same bits.
 enum ChainLaunch { CHAIN_NOT_TAKEN, CHAIN_LAUNCHED, CHAIN_NO_MEMORY };
 template <class T, class Op>
 ChainLaunch scan_chain_launch(const ScanRowsParams& p, bool nt, bool kept_only, hipStream_t stream) {
@@ -835,10 +907,18 @@ ChainLaunch scan_chain_launch(const ScanRowsParams& p, bool nt, bool kept_only, 
     if (n_tiles < 2 || n_tiles > kChainMaxTiles || p.rows * n_tiles > 0x7fffffffull) return CHAIN_NOT_TAKEN;
     const uint64_t n_groups = (n_tiles + 63) / 64, n_supers = (n_groups + 63) / 64;
     const uint64_t words = kChainHead + p.rows * (n_tiles + n_groups + n_supers) * W;
-    WaitCtl* wait = wait_ctl();
-    if (wait == nullptr) return CHAIN_NOT_TAKEN;  // nowhere to report a wait that gives up: the form without waits
+    // (the wait's own memory is not asked for inside a capture either: first use allocates it)
+    WaitCtl* wait = kept_only && stream_under_capture() ? nullptr : wait_ctl();
+    if (wait == nullptr && !kept_only) return CHAIN_NOT_TAKEN;  // nowhere to report a wait that gives up: the form without waits
     ChainWords cw;
-    if (!chain_words_acquire(stream, words, (uint32_t)(p.rows * n_tiles), &cw, kept_only)) return kept_only ? CHAIN_NOT_TAKEN : CHAIN_NO_MEMORY;
+    if (wait == nullptr || !chain_words_acquire(stream, words, (uint32_t)(p.rows * n_tiles), &cw, kept_only)) {
+        if (!kept_only) return CHAIN_NO_MEMORY;
+        const dim3 rows((unsigned)p.rows);
+        if (small) hipLaunchKernelGGL((scan_chain_alone_kernel<T, Op, 4, 4, 4>), rows, dim3(1024), 0, stream, p);
+        else if (wide) hipLaunchKernelGGL((scan_chain_alone_kernel<T, Op, 8, 16, 1>), rows, dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL((scan_chain_alone_kernel<T, Op, 4, 16, 2>), rows, dim3(512), 0, stream, p);
+        return CHAIN_LAUNCHED;
+    }
     ScanChain<T> c;
     c.wait = wait;
     c.ticket = reinterpret_cast<uint32_t*>(cw.ws);
@@ -1506,10 +1586,8 @@ void scan_rows_launch(ScanRowsParams& p, hipStream_t stream) {
         StoreRows out_rows(p.out, p.n * sizeof(T));
         for (int d = 0; d < p.nouter; ++d) out_rows.dimension(p.oshape[d], p.ostep_out[d]);
         p.through = out_rows.through(nt);
-        // (the blocks that take a run each need no memory: neither does this call, under capture or on a stream without a slot)
-        if (scan_chain_enabled() && scan_chain_pays(p.rows, p.n * sizeof(T)) && !stream_under_capture() &&
-            scan_chain_launch<T, Op>(p, nt, true, stream) == CHAIN_LAUNCHED)
-            return;
+        // (the blocks that take a run each need no memory from the pool: neither does this call, under capture or on a stream without a slot)
+        if (scan_chain_enabled() && scan_chain_pays(p.rows, p.n * sizeof(T)) && scan_chain_launch<T, Op>(p, nt, true, stream) == CHAIN_LAUNCHED) return;
         const dim3 g((unsigned)grid), b(kScanBlock);
 #define CUMO_SCAN_WHOLE(R_) do { if (nt) hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, true, R_>), g, b, 0, stream, p); \
                                  else hipLaunchKernelGGL((scan_rows_whole_kernel<T, Op, false, R_>), g, b, 0, stream, p); } while (0)

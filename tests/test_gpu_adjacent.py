@@ -671,6 +671,54 @@ def test_mulsum_of_such_a_view_can_be_replayed():
         _lib.lib.cumo_hip_set_stream(None)
 
 
+# (rows, elements, offset into wider rows): tiles of 16 KiB, of 64 KiB, of 128 KiB; more than 64 tiles to a run; more than 4096, with a whole
+# supergroup; one run that the callers of several reach
+@pytest.mark.parametrize("rows,n,offset", [(8, 20001, 0), (40, 30001, 3), (72, 43801, 1), (3, 2200001, 0), (2, 134300001, 0), (1, 65013, 0)])
+@pytest.mark.parametrize("tname", ["sfloat", "dfloat"])
+def test_scans_of_several_long_runs_are_the_same_when_captured(tname, rows, n, offset):
+    """A stream under capture keeps no words for the one pass to hand its totals on through; what takes its place gives the same bits,
+    and nothing from the pool is part of the graph."""
+    import ctypes as C
+    import cumo_amd
+    from cumo_amd import _lib
+    from test_gpu_index import hip_runtime
+    hip = hip_runtime()
+    cls = cls_of(tname)
+    n = n if tname == "sfloat" else n // 2 + 1
+    # values of both signs and many sizes, so that another order of the additions would show; every 1000th a NaN for the scan that skips those
+    h = np.random.default_rng(57).standard_normal(min(rows * (n + offset), 1 << 22)).astype(cls.cast([0.0]).to_numpy().dtype)
+    x = cls(rows, n + offset)
+    flat, part = x.reshape(rows * (n + offset)), cls.cast(h)
+    for at in range(0, flat.size, h.size):
+        flat[at:at + h.size].store(part[:min(h.size, flat.size - at)])
+    x = x[:, offset:]
+    z = cls(rows, n).fill(55)
+    stream = C.c_void_p(_lib.lib.cumo_hip_stream_create())
+    for skip in (0, 1):
+        if skip:
+            flat[::1000].store(float("nan"))
+        want = x.cumsum(axis=1, nan=bool(skip))
+        graph, ready = C.c_void_p(), C.c_void_p()
+        d, o = x._desc(), z._desc()
+        cumo_amd.synchronize()
+        _lib.lib.cumo_hip_set_stream(stream)
+        try:
+            assert hip.hipStreamBeginCapture(stream, 2) == 0
+            _lib.call(_lib.lib.cumo_hip_na_cum, b"cumsum", C.byref(d), 2, skip, C.byref(o))
+            assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(ready), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(3):
+                z.fill(0)
+                dirt = [cls(k).fill(float("nan")) for k in (1, 1000, 100000)]
+                assert hip.hipGraphLaunch(ready, stream) == 0
+                [a.fill(1e30) for a in dirt]
+                cumo_amd.synchronize()
+                same = z.eq(want) | (z.ne(z) & want.ne(want))
+                assert int(same.count_false()) == 0
+        finally:
+            _lib.lib.cumo_hip_set_stream(None)
+
+
 # (rows, columns): a strip of 64, 32, 16 and 8 lanes and one column to either side, rows that end in part of a vector; one tile of few
 # rows, exactly one tile, one row more; tiles enough for groups and supergroups, and for more than seven of those
 COLUMN_SCANS = [(2, 4), (16, 5), (64, 300), (65, 300), (208, 5395), (256, 1024), (257, 257), (300, 129), (513, 128), (600, 127), (1025, 65), (1030, 64),

@@ -9,7 +9,7 @@ run on the ordinary suites' small inputs in child processes:
                            (4097 tiles of four: the second supergroup);
   CUMO_HIP_SCAN_COLS_CHAIN=0  long runs across memory scanned in two passes over segments;
   CUMO_HIP_SCAN_KEEP_WORDS=0  the one-pass scans with their words from the pool, cleared by a kernel
-                           before each launch (what a stream under capture gets);
+                           before each launch, and few long runs with a block to each (what a stream under capture gets);
   CUMO_HIP_EW_LEAN_ROWS=0  (with CUMO_HIP_NT=1) the general row kernel in its non-temporal forms;
   CUMO_HIP_BIT_VEC_GRID=1  (with CUMO_HIP_NT=1) the Bit vector kernels with one block per compute unit, whose lanes
                            then loop over the result's vectors (what an array beyond 2^37 bits gets) and carry a
@@ -74,7 +74,8 @@ def test_long_runs_scanned_by_three_launches():
 
 def test_one_pass_scans_with_cleared_words_from_the_pool():
     run_child({"CUMO_HIP_SCAN_KEEP_WORDS": "0"},
-              ["tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass", "tests/test_gpu_adjacent.py::test_long_columns_in_one_pass"])
+              ["tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass", "tests/test_gpu_adjacent.py::test_long_columns_in_one_pass",
+               "tests/test_gpu_adjacent.py::test_runs_in_small_tiles_and_several_long_runs_in_one_pass"])
 
 
 def test_one_long_run_by_blocks_of_four_waves():
