@@ -269,9 +269,8 @@ __global__ __launch_bounds__(kFrBlock) void fused_rows_kernel(FusedRowsParams p)
 
 // ---- rows that the registers of 256 lanes do not hold --------------------------------
 // One stretch of a row in the registers of a block: whole vectors, lane l holding vectors l, l + LANES, ..., and, one to a lane,
-// the elements behind the last whole one. A vector is there or not (one compare, whose outcome is not kept: with a count for
-// every vector and a mask for every element a block of 1024 lanes had 82 registers a lane instead of 64, and a compute unit
-// one such block instead of two).
+// the elements behind the last whole one. A vector is there or not: one compare, whose outcome is not kept, since counts and
+// masks would be registers beside those that hold the row (64 of a lane's 128 with sixteen vectors).
 template <class T, int LANES, int NV>
 struct FrStretch {
     static constexpr int V = 16 / (int)sizeof(T);
@@ -318,6 +317,18 @@ struct FrStretch {
             if constexpr (NV > 8) __builtin_amdgcn_sched_barrier(0);
         }
         f(last);
+    }
+    // every element that is there less `by`; absent ones, which are 0, stay so. (A second fill() after taking `by` from every element
+    // kept both copies of a vector: 26 registers of a lane of doubles were spilled.)
+    __device__ __forceinline__ void lessen(T by) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const T mine = has(k) ? by : (T)0;
+#pragma unroll
+            for (int j = 0; j < V; ++j) x[k].t[j] -= mine;
+            if constexpr (NV > 8) __builtin_amdgcn_sched_barrier(0);
+        }
+        last -= has_last() ? by : (T)0;
     }
     // f of every element that is there, to memory
     template <bool NT, class F>
@@ -385,8 +396,7 @@ __global__ __launch_bounds__(LANES, 4) void fused_wide_rows_kernel(FusedRowsPara
     } else {
         a.fill((T)0);
         const T mean = (T)(a.sum([](T& v) { return v; }) / (double)p.n);
-        a.each([&](T& v) { v -= mean; });
-        a.fill((T)0);
+        a.lessen(mean);
         const T var = (T)(a.sum([](T& v) { return v * v; }) / ((double)p.n - 1.0));
         const T sd = fr_sqrt<T>(var + (T)p.eps);
         a.template store<NT>(dst, 0, pieces, [&](T v) { return v / sd; });
@@ -431,8 +441,7 @@ __global__ __launch_bounds__(kFrBlock) void fused_parts_kernel(FusedSplitParams 
     } else {
         a.fill((T)0);
         const T mean = (T)(a.sum([](T& v) { return v; }) / (double)held);
-        a.each([&](T& v) { v -= mean; });
-        a.fill((T)0);
+        a.lessen(mean);
         const double q = a.sum([](T& v) { return v * v; });
         const double r = a.sum([](T& v) { return v; });  // what rounding left of the sum: the deviations do not quite cancel
         if (threadIdx.x == 0) {
@@ -550,9 +559,11 @@ bool fr_apart(const FusedRowsParams& p) {
 // registers: rows up to 128 KiB take 512 lanes, two blocks to a compute unit, so that one computes while the other's loads and
 // stores are under way; up to 256 KiB 1024 lanes, if there are rows enough; longer ones are cut. us, softmax / layernorm, the
 // chain that all of these took before, then 512 or 1024 lanes, then cut:
-//   SFloat [588,27696]  91.2 / 76.5, 32.8 / 26.6, 50.8 / 39.5     [8,20000]   19.6 / 22.0, 10.5 / 7.4, 11.4 / 10.3
-//   SFloat [400,65000]  211 / 190, 64.1 / 47.6, 66.6 / 55.8       [20,65000]  22.5 / 22.4, 19.2 / 12.7, 13.4 / 10.5
-//   DFloat [762,29665]  230 / 178, 92.9 / 90.5, 103 / 94.1        [33,29738]  24.6 / 26.4, 17.3 / 14.9, 14.3 / 11.6
+//   SFloat [588,27696]  91.2 / 76.5, 32.1 / 26.3, 46.7 / 39.1     [8,20000]   19.6 / 22.0, 10.5 / 7.4, 11.4 / 10.3
+//   SFloat [400,65000]  211 / 190, 62.4 / 46.8, 63.6 / 55.0       [20,65000]  22.5 / 22.4, 19.2 / 12.7, 13.4 / 10.5
+//   DFloat [762,29665]  230 / 178, 91.6 / 82.1, 99.7 / 95.1       [33,29738]  24.6 / 26.4, 17.3 / 14.9, 14.6 / 12.5
+//   DFloat [588,27696]  69.2 / 57.0 and 69.0 / 66.4 cut, [2000,10000] 63.6 / 55.0 and 90.1 / 86.2, [200,32768] 25.8 / 21.8 and 33.3 / 33.3,
+//   [70,20000] 16.3 / 12.0 and 14.4 / 12.4
 //   cut: SFloat [76,440000] 165 / 139, -, 80.0 / 67.0;  DFloat [108,128807] 146 / 123, -, 64.9 / 58.4
 // (1024 lanes with eight vectors each for [588,27696]: 45.5 / 32.1.) false when the shape is left to the chain.
 template <class T, int MODE>

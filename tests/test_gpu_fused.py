@@ -99,9 +99,11 @@ def test_layernorm_matches_the_chain(dt):
     assert np.isnan(m.Fused.layernorm(one).to_numpy()).all() and np.isnan(chain_layernorm(m, one, 1e-5).to_numpy()).all()
 
 
-# Rows beyond the registers of 256 lanes: a block of 1024 lanes up to 65536 SFloat / 32768 DFloat, pieces of 8192 / 4096 elements in
-# two launches beyond. Lengths at those edges, a last piece of one element, a last vector that is partly there.
-LONG_ROWS = [(3, 8193), (3, 16385), (5, 32768), (3, 32769), (2, 65533), (3, 65536), (300, 16390), (3, 65537), (7, 70001), (2, 3, 131073), (1, 1 << 20)]
+# Rows beyond the registers of 256 lanes, which hold 16384 SFloat / 4096 DFloat: a block of 512 lanes up to
+# 32768 / 16384 elements, of 1024 lanes up to 65536 / 32768 where there are more than 64 rows, and pieces of 8192 / 4096 elements in
+# two launches beyond and for fewer rows. Lengths at those edges, a last piece of one element, a last vector that is partly there.
+LONG_ROWS = [(3, 4097), (3, 8193), (3, 16385), (5, 32768), (3, 32769), (2, 65533), (3, 65536), (300, 16390), (3, 65537), (7, 70001), (2, 3, 131073), (1, 1 << 20),
+             (64, 16385), (65, 16385), (65, 32768), (64, 32769), (65, 32769), (65, 65533), (65, 65536)]
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
@@ -124,11 +126,11 @@ def test_long_rows_match_64_bit_arithmetic(dt, shape):
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
-@pytest.mark.parametrize("n", [20001, 70001])
-def test_long_rows_special_values_views_and_overlap(dt, n):
+@pytest.mark.parametrize("rows,n", [(6, 20001), (6, 70001), (140, 20001), (140, 40001)])   # (140: a block of 1024 lanes each, DFloat / SFloat)
+def test_long_rows_special_values_views_and_overlap(dt, rows, n):
     import cumo_amd as m
     cls = m.SFloat if dt == np.float32 else m.DFloat
-    h = (np.random.default_rng(n).standard_normal((6, n)) * 2).astype(dt)
+    h = (np.random.default_rng(n).standard_normal((rows, n)) * 2).astype(dt)
     h[0, n - 1] = np.nan
     h[1, :] = -np.inf      # whole pieces of -inf, one of them with a number
     h[1, 17] = 3.0
@@ -146,16 +148,16 @@ def test_long_rows_special_values_views_and_overlap(dt, n):
     assert want[1, 17] == 1.0 and np.count_nonzero(want[1]) == 1 and np.isnan(want[[0, 2, 3]]).all()
 
 
-@pytest.mark.parametrize("n", [20001, 70001])
-def test_long_rows_into_their_operand_and_into_memory_that_overlaps_it(n):
+@pytest.mark.parametrize("rows,n", [(4, 20001), (4, 70001), (65, 40001)])
+def test_long_rows_into_their_operand_and_into_memory_that_overlaps_it(rows, n):
     import ctypes as C
     import cumo_amd as m
     from cumo_amd import _lib
-    h = (np.random.default_rng(n).standard_normal((5, n)) * 2).astype(np.float32)
-    want = m.Fused.softmax(m.SFloat.cast(h[:4])).to_numpy()
+    h = (np.random.default_rng(n).standard_normal((rows + 1, n)) * 2).astype(np.float32)
+    want = m.Fused.softmax(m.SFloat.cast(h[:rows])).to_numpy()
     for down in (0, 1):
         x = m.SFloat.cast(h)
-        operand, result = x[:4], x[down:4 + down]
+        operand, result = x[:rows], x[down:rows + down]
         d, z = operand._desc(), result._desc()
         assert _lib.lib.cumo_hip_na_softmax(C.byref(d), C.byref(z)) == 0
-        close(x.to_numpy()[down:4 + down], want, n, np.float32, ("rows further down", down))
+        close(x.to_numpy()[down:rows + down], want, n, np.float32, ("rows further down", down))
