@@ -268,13 +268,12 @@ __global__ __launch_bounds__(COLS * LANES) void bit_count_fold_kernel(FoldCounts
 
 // geometry for blocks of BLOCK / LANES groups of LANES lanes; false when the launch does not fit
 template <int BLOCK, int LANES>
-bool vc_geometry(BitCountColsVc& p, uint64_t want_blocks, uint64_t* blocks) {
+bool vc_geometry(BitCountColsVc& p, uint64_t want_blocks, uint32_t rows_least, uint64_t* blocks) {
     constexpr uint32_t NG = BLOCK / LANES;
     p.col_blocks = (p.words + (uint32_t)LANES - 1) / (uint32_t)LANES;
     const uint64_t across = (uint64_t)p.col_blocks * p.n_outer;
     uint64_t parts = (want_blocks + across - 1) / across;
-    // stretches of sixteen rows or more, what a lane has in flight (us, 32 / 16: [32768,1024] 10.9 / 9.0, [26984,720] 12.0 / 9.7)
-    const uint64_t most = ((uint64_t)p.rows + kVcRows * NG - 1) / (kVcRows * NG);
+    const uint64_t most = ((uint64_t)p.rows + rows_least * NG - 1) / (rows_least * NG);
     if (parts > most) parts = most;
     if (parts < 1) parts = 1;
     p.rows_per_group = (uint32_t)(((uint64_t)p.rows + parts * NG - 1) / (parts * NG));
@@ -313,7 +312,10 @@ int bit_count_cols_words_launch(const cumo_hip_bit_count_nd_t* d) {
     if (d->in_out_step[L] != 1 || d->in_red_step[0] <= 0 || d->out_shape[L] < 1 || d->red_shape[0] < 2) return 0;
     if (d->out_shape[L] >= 0x7fffffffull || d->red_shape[0] >= 0x7fffffffull) return 0;
     if (L == 1 && (d->in_out_step[0] < 0 || d->out_shape[0] >= 0x10000ull)) return 0;
-    const uint32_t fold = fold_rows(d);
+    // Scratch of a captured launch goes back to the pool before the graph is replayed, so a capture asks for none that it can do
+    // without: short rows are not folded then, and up to 512 rows are one block's.
+    const bool capturing = stream_under_capture();
+    const uint32_t fold = capturing ? 1 : fold_rows(d);
     if (fold == 1) {
         // rows (and planes) that start on word boundaries
         if (d->out_shape[L] < 64 || (d->pos & 31) != 0 || (d->in_red_step[0] & 31) != 0 || (L == 1 && (d->in_out_step[0] & 31) != 0)) return 0;
@@ -341,7 +343,8 @@ int bit_count_cols_words_launch(const cumo_hip_bit_count_nd_t* d) {
     }();
     const uint64_t want_blocks = forced_blocks > 0 ? (uint64_t)forced_blocks : (uint64_t)kNumCU;
     uint64_t blocks = 0;
-    if (!vc_geometry<1024, 64>(p, want_blocks, &blocks)) return 0;
+    // stretches of sixteen rows or more, what a lane has in flight (us, 32 / 16: [32768,1024] 10.9 / 9.0, [26984,720] 12.0 / 9.7)
+    if (!vc_geometry<1024, 64>(p, want_blocks, capturing ? 2 * kVcRows : kVcRows, &blocks)) return 0;
     hipStream_t stream = current_stream();
     if (p.parts > 1 || fold > 1) {
         p.partial = reinterpret_cast<uint32_t*>(cumo_cuda_runtime_malloc(sizeof(uint32_t) * (size_t)blocks * 64 * 32));

@@ -85,8 +85,8 @@ void launch_short(const ShortRows& p, hipStream_t stream) {
 
 namespace cumo_hip {
 
-// Runs of up to 8129 bits that lie along memory, anywhere. 1 when launched (counts stored or added as d->overwrite says), 0 when
-// the loop is another.
+// Runs of up to 8161 bits that lie along memory, anywhere (256 words, with the first bit the last of its word). 1 when launched (counts
+// stored or added as d->overwrite says), 0 when the loop is another.
 int bit_count_short_rows_launch(const cumo_hip_bit_count_nd_t* d) {
     if (d->red_ndim != 1 || d->in_red_step[0] != 1 || d->out_ndim < 1 || force_wide_indices()) return 0;
     const uint64_t n = d->red_shape[0];

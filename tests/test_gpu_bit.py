@@ -434,9 +434,9 @@ def test_all_any_along_word_aligned_rows():
 
 
 # (rows, columns): rows of less than a word, of whole words, a bit more and less; fewer rows than are taken as one, rows left over;
-# runs of 8129 and 8130 bits (the most that 64 lanes take, and one more)
+# runs of 8161 and 8162 bits (the most that 64 lanes take wherever a run's first bit lies, and one more)
 @pytest.mark.parametrize("shape", [(5, 3), (33, 31), (4096, 8), (2051, 33), (130, 64), (640, 32), (127, 1001), (128, 1001), (191, 1025), (4103, 137),
-                                   (200, 8191), (200, 8193), (3, 8129), (3, 8130), (40000, 20)])
+                                   (200, 8191), (200, 8193), (3, 8129), (3, 8161), (3, 8162), (40000, 20)])
 def test_counts_along_and_down_short_rows(shape):
     import cumo_amd as m
     rng = np.random.default_rng(shape[1])
@@ -451,7 +451,48 @@ def test_counts_along_and_down_short_rows(shape):
             for keep in (False, True):
                 assert (a.count_true(axis=axis, keepdims=keep).to_numpy() == w.sum(axis=axis, keepdims=keep)).all(), (axis, keep)
             assert (a.count_false(axis=axis).to_numpy() == (~w).sum(axis=axis)).all(), axis
+    # rows whose first bits are the last but one and the last of a word
+    for at in (30, 31):
+        wide = rng.random((rows, -(-(cols + at) // 32) * 32)) < 0.4
+        a, w = (m.SFloat.cast(wide.astype(np.float32)) > 0.5)[:, at:at + cols], wide[:, at:at + cols]
+        assert (a.count_true(axis=1).to_numpy() == w.sum(axis=1)).all() and (a.count_false(axis=0).to_numpy() == (~w).sum(axis=0)).all(), at
     z = m.SFloat.cast(np.stack([whole, ~whole]).astype(np.float32)) > 0.5
     assert (z.count_true(axis=2).to_numpy() == np.stack([whole, ~whole]).sum(axis=2)).all()
     assert (z.count_true(axis=1).to_numpy() == np.stack([whole, ~whole]).sum(axis=1)).all()
     assert (z.transpose(1, 0, 2).count_false(axis=2).to_numpy() == np.stack([~whole, whole]).transpose(1, 0, 2).sum(axis=2)).all()
+
+
+# (columns that are taken many rows as one outside a capture, rows of whole words that several blocks share, few of those)
+@pytest.mark.parametrize("shape", [(24304, 1066), (65536, 33), (2051, 137), (400, 1024), (512, 64)])
+def test_counts_down_columns_can_be_replayed(shape):
+    """Captured into a given result and replayed, with the pool's memory in use in between: nothing of it is part of the graph."""
+    import ctypes as C
+    import cumo_amd as m
+    from cumo_amd import _lib
+    from test_gpu_index import hip_runtime
+    hip = hip_runtime()
+    h = np.random.default_rng(58).random(shape) < 0.4
+    x = m.SFloat.cast(h.astype(np.float32)) > 0.5
+    z = x.count_true(axis=0)
+    want = h.sum(axis=0)
+    assert (z.to_numpy() == want).all()
+    stream = C.c_void_p(_lib.lib.cumo_hip_stream_create())
+    graph, ready = C.c_void_p(), C.c_void_p()
+    d, o = x._desc(), z._desc()
+    m.synchronize()
+    _lib.lib.cumo_hip_set_stream(stream)
+    try:
+        x.count_true(axis=0)   # (what a stream's first launch allocates)
+        assert hip.hipStreamBeginCapture(stream, 2) == 0
+        _lib.call(_lib.lib.cumo_hip_na_bit_count, C.byref(d), 1, 0, 0, C.byref(o))
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(ready), graph, None, None, C.c_size_t(0)) == 0
+        # (every size of block that the pool could have kept from the capture, a few of each)
+        held = [m.Int32((512 << k) // 4).fill(77) for k in range(0, 15) for _ in range(4)]
+        for _ in range(3):
+            assert hip.hipGraphLaunch(ready, stream) == 0
+            m.synchronize()
+            assert (z.to_numpy() == want).all()
+            assert all(int(a.ne(77).count_true()) == 0 for a in held)
+    finally:
+        _lib.lib.cumo_hip_set_stream(None)
