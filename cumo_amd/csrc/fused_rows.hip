@@ -561,7 +561,7 @@ bool fr_apart(const FusedRowsParams& p) {
 // chain that all of these took before, then 512 or 1024 lanes, then cut:
 //   SFloat [588,27696]  91.2 / 76.5, 32.1 / 26.3, 46.7 / 39.1     [8,20000]   19.6 / 22.0, 10.5 / 7.4, 11.4 / 10.3
 //   SFloat [400,65000]  211 / 190, 62.4 / 46.8, 63.6 / 55.0       [20,65000]  22.5 / 22.4, 19.2 / 12.7, 13.4 / 10.5
-//   DFloat [762,29665]  230 / 178, 91.6 / 82.1, 99.7 / 95.1       [33,29738]  24.6 / 26.4, 17.3 / 14.9, 14.6 / 12.5
+//   DFloat [762,29665]  230 / 178, 91.6 / 82.1, 99.7 / 95.1       [33,29738]  24.6 / 26.4, -, 14.6 / 12.5
 //   DFloat [588,27696]  69.2 / 57.0 and 69.0 / 66.4 cut, [2000,10000] 63.6 / 55.0 and 90.1 / 86.2, [200,32768] 25.8 / 21.8 and 33.3 / 33.3,
 //   [70,20000] 16.3 / 12.0 and 14.4 / 12.4
 //   cut: SFloat [76,440000] 165 / 139, -, 80.0 / 67.0;  DFloat [108,128807] 146 / 123, -, 64.9 / 58.4

@@ -122,9 +122,29 @@ static std::mutex g_wait_lock;
 static WaitCtl* g_wait_dev = nullptr;
 static std::atomic<uint32_t*> g_wait_flag{nullptr};
 
+// `from` to device memory, by a stream of its own: a copy that waits for the device would end a capture
+static bool upload_apart(void* to, const void* from, size_t bytes) {
+    hipStream_t stream = nullptr;
+    if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return false;
+    bool ok = hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, stream) == hipSuccess;
+    ok = hipStreamSynchronize(stream) == hipSuccess && ok;
+    return hipStreamDestroy(stream) == hipSuccess && ok;
+}
+
+// While one lives, what this thread asks of the runtime is no part of a capture, and does not end one.
+struct ApartFromCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool changed;
+    ApartFromCapture() : changed(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~ApartFromCapture() {
+        if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 WaitCtl* wait_ctl() {
     std::lock_guard<std::mutex> hold(g_wait_lock);
     if (g_wait_dev) return g_wait_dev;
+    ApartFromCapture apart;   // (the first launch that may wait can be a captured one)
     void* flag = nullptr;
     if (hipHostMalloc(&flag, 64, hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
@@ -143,7 +163,7 @@ WaitCtl* wait_ctl() {
     const char* e = std::getenv("CUMO_HIP_WAIT_LIMIT");
     init.limit_scale = (e && e[0] == '0') ? 0u : 1u;
     init.host_flag = (uint32_t*)flag;
-    if (hipMemcpy(dev, &init, sizeof(init), hipMemcpyHostToDevice) != hipSuccess) {
+    if (!upload_apart(dev, &init, sizeof(init))) {
         (void)hipGetLastError();
         (void)hipFree(dev);
         (void)hipHostFree(flag);

@@ -907,8 +907,7 @@ ChainLaunch scan_chain_launch(const ScanRowsParams& p, bool nt, bool kept_only, 
     if (n_tiles < 2 || n_tiles > kChainMaxTiles || p.rows * n_tiles > 0x7fffffffull) return CHAIN_NOT_TAKEN;
     const uint64_t n_groups = (n_tiles + 63) / 64, n_supers = (n_groups + 63) / 64;
     const uint64_t words = kChainHead + p.rows * (n_tiles + n_groups + n_supers) * W;
-    // (the wait's own memory is not asked for inside a capture either: first use allocates it)
-    WaitCtl* wait = kept_only && stream_under_capture() ? nullptr : wait_ctl();
+    WaitCtl* wait = wait_ctl();
     if (wait == nullptr && !kept_only) return CHAIN_NOT_TAKEN;  // nowhere to report a wait that gives up: the form without waits
     ChainWords cw;
     if (wait == nullptr || !chain_words_acquire(stream, words, (uint32_t)(p.rows * n_tiles), &cw, kept_only)) {

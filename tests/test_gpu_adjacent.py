@@ -4,6 +4,9 @@ contiguous arrays, views and repeated operands. Bars: Int32 and clip/maximum/
 minimum bit-exact; Float ** Int32 (products in the element type) bit-exact;
 SFloat pow <= 1 ulp (the device evaluates pow in double and rounds once, as the
 host macro does); DFloat pow <= 2 ulp against glibc."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
@@ -717,6 +720,42 @@ def test_scans_of_several_long_runs_are_the_same_when_captured(tname, rows, n, o
                 assert int(same.count_false()) == 0
         finally:
             _lib.lib.cumo_hip_set_stream(None)
+
+
+FIRST_LAUNCH_CAPTURED = """
+import ctypes as C
+import numpy as np
+import cumo_amd
+from cumo_amd import _lib
+with open("/proc/self/maps") as f:
+    hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+h = np.random.default_rng(59).integers(-3, 4, SHAPE).astype(np.float32)
+x, z = cumo_amd.SFloat.cast(h), cumo_amd.SFloat(*SHAPE).fill(55)
+stream, graph, ready = C.c_void_p(_lib.lib.cumo_hip_stream_create()), C.c_void_p(), C.c_void_p()
+d, o = x._desc(), z._desc()
+cumo_amd.synchronize()
+_lib.lib.cumo_hip_set_stream(stream)
+assert hip.hipStreamBeginCapture(stream, 2) == 0
+_lib.call(_lib.lib.cumo_hip_na_cum, b"cumsum", C.byref(d), 1, 0, C.byref(o))
+assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+assert hip.hipGraphInstantiate(C.byref(ready), graph, None, None, C.c_size_t(0)) == 0
+for _ in range(3):
+    assert hip.hipGraphLaunch(ready, stream) == 0
+    cumo_amd.synchronize()
+    assert (z.to_numpy() == np.cumsum(h, axis=0)).all()
+    z.fill(0)
+print("replayed")
+"""
+
+
+@pytest.mark.parametrize("shape", [(5000, 20), (100001,)])
+def test_the_first_scan_of_a_process_can_be_captured(shape):
+    """What the kernels with waits report to is set up by the first of them; that must not end a capture."""
+    import subprocess
+    env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    p = subprocess.run([sys.executable, "-c", FIRST_LAUNCH_CAPTURED.replace("SHAPE", repr(shape))], env=env, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert p.returncode == 0 and "replayed" in p.stdout, p.stdout[-2000:]
 
 
 # (rows, columns): a strip of 64, 32, 16 and 8 lanes and one column to either side, rows that end in part of a vector; one tile of few
