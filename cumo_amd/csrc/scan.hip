@@ -11,8 +11,8 @@
 //   scan_rows_kernel        one block per run, tile after tile with the running value
 //                           carried along: many runs (an axis of a matrix), or short ones;
 //   scan_short_kernel       many short runs, as many to a wave as its registers hold (scan_short.hip);
-//   scan_rows_whole_kernel  the same for contiguous runs of whole 256-vector chunks, held
-//                           in registers wave by wave;
+//   scan_rows_whole_kernel  the same for contiguous runs of 64 vectors or more, a chunk of them at a time held in
+//                           registers wave by wave, the last chunk maybe partly there;
 //   scan_chain_kernel       one contiguous run, or a few long ones, in one pass: tiles hand their
 //                           totals on through words in memory (read once, written once);
 //   scan_chain_alone_kernel those few, a block to each, where the stream keeps no such words: the same bits;
@@ -62,8 +62,9 @@ __device__ __forceinline__ T scan_shfl_up(T v, unsigned d) {
 // `carry` is the running value before the tile and has_carry says whether there is
 // one. Returns the running value after the tile in every lane (has_carry becomes true
 // when the tile is not empty).
-template <class T, class Op, int NWAVES = kScanBlock / 64>
+template <class T, class Op>
 __device__ __forceinline__ void scan_tile(T (&v)[kScanPer], int cnt, T& carry, bool& has_carry) {
+    constexpr int NWAVES = kScanBlock / 64;
     __shared__ T wave_tot[NWAVES];
     __shared__ int wave_has[NWAVES];
     const int t = threadIdx.x;
@@ -127,7 +128,7 @@ __device__ __forceinline__ void scan_tile(T (&v)[kScanPer], int cnt, T& carry, b
     has_carry = run_has;
 }
 
-template <class T, bool NT = false>
+template <class T>
 __device__ __forceinline__ void scan_load(const char* p, int64_t s, uint64_t first, int cnt, T (&v)[kScanPer]) {
     const int base = threadIdx.x * kScanPer;
     if (s == (int64_t)sizeof(T) && base + kScanPer <= cnt && ((reinterpret_cast<uintptr_t>(p) + (first + base) * sizeof(T)) & 15) == 0) {
@@ -136,7 +137,7 @@ __device__ __forceinline__ void scan_load(const char* p, int64_t s, uint64_t fir
         union { T t[kScanPer]; u4 q[NV]; } u;
         const u4* src = reinterpret_cast<const u4*>(p + (first + base) * sizeof(T));
 #pragma unroll
-        for (int i = 0; i < NV; ++i) u.q[i] = NT ? __builtin_nontemporal_load(src + i) : src[i];
+        for (int i = 0; i < NV; ++i) u.q[i] = src[i];
 #pragma unroll
         for (int k = 0; k < kScanPer; ++k) v[k] = u.t[k];
         return;
@@ -146,7 +147,7 @@ __device__ __forceinline__ void scan_load(const char* p, int64_t s, uint64_t fir
         if (base + k < cnt) v[k] = *reinterpret_cast<const T*>(p + (int64_t)(first + base + k) * s);
 }
 
-template <class T, bool NT = false>
+template <class T>
 __device__ __forceinline__ void scan_store(char* p, int64_t s, uint64_t first, int cnt, const T (&v)[kScanPer]) {
     const int base = threadIdx.x * kScanPer;
     if (s == (int64_t)sizeof(T) && base + kScanPer <= cnt && ((reinterpret_cast<uintptr_t>(p) + (first + base) * sizeof(T)) & 15) == 0) {
@@ -157,10 +158,7 @@ __device__ __forceinline__ void scan_store(char* p, int64_t s, uint64_t first, i
         for (int k = 0; k < kScanPer; ++k) u.t[k] = v[k];
         u4* dst = reinterpret_cast<u4*>(p + (first + base) * sizeof(T));
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            if (NT) __builtin_nontemporal_store(u.q[i], dst + i);
-            else dst[i] = u.q[i];
-        }
+        for (int i = 0; i < NV; ++i) dst[i] = u.q[i];
         return;
     }
 #pragma unroll
@@ -362,7 +360,7 @@ __device__ __forceinline__ void chain_fold_lanes(T& x, bool& has, uint32_t count
 // pauses (64 lanes of every running block polling would flood the memory system); then every
 // lane looks at its own words, all in flight together, until they are there.
 template <class T, class Op>
-__device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t t, T total, bool total_has, T& prefix, bool& prefix_has) {
+__device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t t, T total, T& prefix, bool& prefix_has) {
     constexpr int W = ScanChain<T>::W;
     const unsigned lane = threadIdx.x & 63u;
     t = (uint32_t)__builtin_amdgcn_readfirstlane(t);
@@ -396,7 +394,6 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
     bool xh = false, yh = false, zh = false;
     bool x_folded = false, y_folded = false;
     T gt = T();
-    bool gt_has = false;
     for (;;) {
         if (need_x) need_x = !chain_peek<T>(px, x, c.flag);
         if (need_y) need_y = !chain_peek<T>(py, y, c.flag);
@@ -405,9 +402,7 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
             chain_fold_lanes<T, Op>(x, xh, pos);
             x_folded = true;
             if (!group_out) {
-                gt = x;
-                gt_has = xh;
-                chain_join<T, Op>(gt, gt_has, total, total_has);
+                gt = Op::apply(x, total);
                 if (lane == 0) chain_publish<T>(c.group + (size_t)g * W, gt, c.flag);
                 group_out = true;
             }
@@ -416,10 +411,7 @@ __device__ __forceinline__ void chain_look_back(const ScanChain<T>& c, uint32_t 
             chain_fold_lanes<T, Op>(y, yh, gpos);
             y_folded = true;
             if (!super_out) {
-                T st = y;
-                bool st_has = yh;
-                chain_join<T, Op>(st, st_has, gt, gt_has);
-                if (lane == 0) chain_publish<T>(c.super + (size_t)sg * W, st, c.flag);
+                if (lane == 0) chain_publish<T>(c.super + (size_t)sg * W, Op::apply(y, gt), c.flag);
                 super_out = true;
             }
         }
@@ -542,13 +534,13 @@ __device__ __forceinline__ void chain_fold_waves(const T* s_wave_tot, int w, T& 
 // The tile in v (already loaded) scanned by itself: afterwards every element holds the running
 // value from the start of its wave's part, `total` is the tile's total and `wave_pre` the
 // total of the waves before this one (for wave 0: nothing). One barrier, met by every thread.
-template <class T, class Op, int R, int NW = kScanBlock / 64>
+template <class T, class Op, int R>
 __device__ __forceinline__ void chain_scan_tile(ScanVec<T> (&v)[R], T* s_wave_tot, T& total, T& wave_pre) {
     const int w = threadIdx.x >> 6;
     const T run = chain_scan_wave<T, Op, R>(v);
     if ((threadIdx.x & 63u) == 0) s_wave_tot[w] = run;
     __syncthreads();
-    chain_fold_waves<T, Op, NW>(s_wave_tot, w, total, wave_pre);
+    chain_fold_waves<T, Op, kScanBlock / 64>(s_wave_tot, w, total, wave_pre);
 }
 
 // adds what precedes the tile (if anything) and the earlier waves' total, and stores (pieces: see store_form.h)
@@ -593,32 +585,25 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
     constexpr uint64_t CHUNK = (uint64_t)R * kScanBlock * V;
     __shared__ T s_wave_tot[kScanBlock / 64];
     for (uint64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
-        int64_t oi = 0, oo = 0;
-        uint64_t q = row;
-        for (int d = p.nouter - 1; d >= 0; --d) {
-            const uint64_t m = p.oshape[d];
-            const uint64_t qq = q / m;
-            const int64_t k = (int64_t)(q - qq * m);
-            q = qq;
-            oi += k * p.ostep_in[d];
-            oo += k * p.ostep_out[d];
-        }
+        const char* in;
+        char* out;
+        scan_run_start(p, row, in, out);
         T carry = T();
         bool has_carry = false;
-        const bool pieces = p.through && store_pieces(p.out + oo);
+        const bool pieces = p.through && store_pieces(out);
         for (uint64_t first = 0; first < p.n; first += CHUNK) {
             ScanVec<T> v[R];
             T total, wave_pre;
             if (p.n - first >= CHUNK) {
-                chain_issue_loads<T, NT, R>(p.in + oi, first, v);
+                chain_issue_loads<T, NT, R>(in, first, v);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces);
+                chain_store_tile<T, Op, NT, R>(out, first, v, carry, has_carry, wave_pre, pieces);
             } else {
                 // the run's last chunk, partly there
                 const uint32_t nelem = (uint32_t)(p.n - first);
-                chain_issue_loads<T, NT, R, true>(p.in + oi, first, v, nelem);
+                chain_issue_loads<T, NT, R, true>(in, first, v, nelem);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R, true>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces, nelem);
+                chain_store_tile<T, Op, NT, R, true>(out, first, v, carry, has_carry, wave_pre, pieces, nelem);
             }
             carry = has_carry ? Op::apply(carry, total) : total;
             has_carry = true;
@@ -671,7 +656,7 @@ __global__ __launch_bounds__(NW * 64, sizeof(T) == 8 ? 3 : 4) void scan_chain_ke
     if (threadIdx.x < 64) {
         T pre;
         bool pre_has;
-        chain_look_back<T, Op>(c, t, total, true, pre, pre_has);
+        chain_look_back<T, Op>(c, t, total, pre, pre_has);
         if (threadIdx.x == 0) {
             s_prefix = pre;
             sh.prefix_has = pre_has ? 1 : 0;
@@ -738,16 +723,9 @@ __global__ __launch_bounds__(STEP * NW * 64) void scan_chain_alone_kernel(ScanRo
         chain_fold_lanes<T, Op>(z, zh, sg);
         // (read from the step after the next barrier on)
         if (pos == 63u && w == 0 && lane == 0) {
-            T sum = x;
-            bool has = xh;
-            chain_join<T, Op>(sum, has, total, true);
+            const T sum = Op::apply(x, total);
             s_group[gpos] = sum;
-            if (gpos == 63u) {
-                T st = y;
-                has = yh;
-                chain_join<T, Op>(st, has, sum, true);
-                s_super[sg] = st;
-            }
+            if (gpos == 63u) s_super[sg] = Op::apply(y, sum);
         }
         chain_join<T, Op>(z, zh, y, yh);
         chain_join<T, Op>(z, zh, x, xh);

@@ -39,7 +39,8 @@ REDUCE = ["tests/test_gpu_reduce.py::test_float_reductions_every_axis", "tests/t
           "tests/test_gpu_reduce.py::test_min_max_keep_the_zero_that_came_first"]
 ADJACENT = ["tests/test_gpu_adjacent.py::test_clip_parity_over_views", "tests/test_gpu_adjacent.py::test_float_pow_parity",
             "tests/test_gpu_adjacent.py::test_cumsum_cumprod_parity", "tests/test_gpu_adjacent.py::test_cum_along_contiguous_runs_of_whole_chunks",
-            "tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass",
+            "tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass", "tests/test_gpu_adjacent.py::test_many_short_runs_share_a_wave",
+            "tests/test_gpu_adjacent.py::test_scans_down_narrow_and_shallow_matrices",
             "tests/test_gpu_adjacent.py::test_cum_along_columns_of_tall_wide_and_stacked_arrays", "tests/test_gpu_adjacent.py::test_mulsum_parity"]
 OTHERS = ["tests/test_gpu_index.py::test_gather_and_scatter_between_view_and_buffer", "tests/test_gpu_index.py::test_getitem_with_index_arrays",
           "tests/test_gpu_index.py::test_setitem_with_index_arrays_and_slices", "tests/test_gpu_fused.py", "tests/test_gpu_configs.py"]
@@ -83,7 +84,7 @@ def test_one_long_run_by_blocks_of_four_waves():
 
 
 def test_one_long_run_by_blocks_of_eight_waves():
-    """Also the sizes of eight-byte elements that take blocks of four: 64 to 127 large tiles, and more than 3072."""
+    """Also the sizes of eight-byte elements that take blocks of four: 64 to 127 large tiles."""
     run_child({"CUMO_HIP_SCAN_CHAIN_WAVES": "8"}, ["tests/test_gpu_adjacent.py::test_one_long_run_in_one_pass"])
 
 
