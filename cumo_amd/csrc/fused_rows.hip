@@ -613,7 +613,7 @@ extern "C" int cumo_hip_fused_rows_kernel_launch(int type, int mode, const cumo_
     p.in = d->in;
     p.out = d->out;
     p.eps = d->eps;
-    p.through = false;  // (fr_launch_one says)
+    p.through = false;  // (fr_store_form says)
     hipStream_t stream = current_stream();
     bool ok;
     if (type == 0) ok = mode == 0 ? fr_launch<float, 0>(p, stream) : fr_launch<float, 1>(p, stream);

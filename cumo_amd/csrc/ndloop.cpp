@@ -1536,7 +1536,7 @@ int cumo_hip_na_cum(const char* op, const cumo_hip_narray_t* x, unsigned int red
     runs.out = dst->ptr + dst->offset;
     const bool use_nan = nan && is_float(x->type);
     if (runs.rows == 1 && n > (1u << 16)) {
-        // one long run: the three-launch form
+        // one long run: in one pass, or by three launches where its elements are not side by side
         typedef int (*RunFn)(char*, char*, ssize_t, ssize_t, uint64_t);
         static const RunFn fns[3][4] = {
             {cumo_sfloat_cumsum_kernel_launch, cumo_sfloat_cumsum_nan_kernel_launch, cumo_sfloat_cumprod_kernel_launch, cumo_sfloat_cumprod_nan_kernel_launch},

@@ -718,8 +718,14 @@ def test_scans_of_several_long_runs_are_the_same_when_captured(tname, rows, n, o
                 cumo_amd.synchronize()
                 same = z.eq(want) | (z.ne(z) & want.ne(want))
                 assert int(same.count_false()) == 0
+                del dirt
         finally:
             _lib.lib.cumo_hip_set_stream(None)
+            if ready:
+                hip.hipGraphExecDestroy(ready)
+            if graph:
+                hip.hipGraphDestroy(graph)
+    _lib.lib.cumo_hip_stream_destroy(stream)
 
 
 FIRST_LAUNCH_CAPTURED = """

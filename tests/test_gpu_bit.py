@@ -494,5 +494,11 @@ def test_counts_down_columns_can_be_replayed(shape):
             m.synchronize()
             assert (z.to_numpy() == want).all()
             assert all(int(a.ne(77).count_true()) == 0 for a in held)
+        del held
     finally:
         _lib.lib.cumo_hip_set_stream(None)
+        if ready:
+            hip.hipGraphExecDestroy(ready)
+        if graph:
+            hip.hipGraphDestroy(graph)
+        _lib.lib.cumo_hip_stream_destroy(stream)
