@@ -585,25 +585,24 @@ __global__ __launch_bounds__(kScanBlock) void scan_rows_whole_kernel(ScanRowsPar
     constexpr uint64_t CHUNK = (uint64_t)R * kScanBlock * V;
     __shared__ T s_wave_tot[kScanBlock / 64];
     for (uint64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
-        const char* in;
-        char* out;
-        scan_run_start(p, row, in, out);
+        int64_t oi, oo;
+        scan_run_offsets(p, row, oi, oo);
         T carry = T();
         bool has_carry = false;
-        const bool pieces = p.through && store_pieces(out);
+        const bool pieces = p.through && store_pieces(p.out + oo);
         for (uint64_t first = 0; first < p.n; first += CHUNK) {
             ScanVec<T> v[R];
             T total, wave_pre;
             if (p.n - first >= CHUNK) {
-                chain_issue_loads<T, NT, R>(in, first, v);
+                chain_issue_loads<T, NT, R>(p.in + oi, first, v);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R>(out, first, v, carry, has_carry, wave_pre, pieces);
+                chain_store_tile<T, Op, NT, R>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces);
             } else {
                 // the run's last chunk, partly there
                 const uint32_t nelem = (uint32_t)(p.n - first);
-                chain_issue_loads<T, NT, R, true>(in, first, v, nelem);
+                chain_issue_loads<T, NT, R, true>(p.in + oi, first, v, nelem);
                 chain_scan_tile<T, Op, R>(v, s_wave_tot, total, wave_pre);
-                chain_store_tile<T, Op, NT, R, true>(out, first, v, carry, has_carry, wave_pre, pieces, nelem);
+                chain_store_tile<T, Op, NT, R, true>(p.out + oo, first, v, carry, has_carry, wave_pre, pieces, nelem);
             }
             carry = has_carry ? Op::apply(carry, total) : total;
             has_carry = true;

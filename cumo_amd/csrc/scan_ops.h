@@ -50,9 +50,9 @@ struct ScanRowsParams {
     bool through;   // see StoreRows (scan_rows_whole_kernel)
 };
 
-// where run `row` starts on either side
-__device__ __forceinline__ void scan_run_start(const ScanRowsParams& p, uint64_t row, const char*& in, char*& out) {
-    int64_t oi = 0, oo = 0;
+// where run `row` starts on either side, in bytes from the first one
+__device__ __forceinline__ void scan_run_offsets(const ScanRowsParams& p, uint64_t row, int64_t& oi, int64_t& oo) {
+    oi = oo = 0;
 #pragma unroll 1
     for (int d = p.nouter - 1; d >= 0; --d) {
         const uint64_t m = p.oshape[d];
@@ -62,6 +62,10 @@ __device__ __forceinline__ void scan_run_start(const ScanRowsParams& p, uint64_t
         oi += k * p.ostep_in[d];
         oo += k * p.ostep_out[d];
     }
+}
+__device__ __forceinline__ void scan_run_start(const ScanRowsParams& p, uint64_t row, const char*& in, char*& out) {
+    int64_t oi, oo;
+    scan_run_offsets(p, row, oi, oo);
     in = p.in + oi;
     out = p.out + oo;
 }
