@@ -436,7 +436,7 @@ def test_all_any_along_word_aligned_rows():
 # (rows, columns): rows of less than a word, of whole words, a bit more and less; fewer rows than are taken as one, rows left over;
 # runs of 8161 and 8162 bits (the most that 64 lanes take wherever a run's first bit lies, and one more)
 @pytest.mark.parametrize("shape", [(5, 3), (33, 31), (4096, 8), (2051, 33), (130, 64), (640, 32), (127, 1001), (128, 1001), (191, 1025), (4103, 137),
-                                   (200, 8191), (200, 8193), (3, 8129), (3, 8161), (3, 8162), (40000, 20)])
+                                   (200, 8191), (200, 8193), (3, 8129), (3, 8130), (3, 8161), (3, 8162), (40000, 20)])
 def test_counts_along_and_down_short_rows(shape):
     import cumo_amd as m
     rng = np.random.default_rng(shape[1])
